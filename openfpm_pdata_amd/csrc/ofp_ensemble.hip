@@ -73,6 +73,49 @@ __global__ __launch_bounds__(256) void k_ens_map(uint32_t N, size_t cap, const u
   }
 }
 
+// The stored particles into the domain-row order of the build they are in, with
+// that build kept: its sorted order, cells and Verlet rows are in sorted indices
+// and stay; only the storage indices it names change (row k's particle becomes
+// stored particle k).  inv[old storage index] = new one, for k_ens_relabel_ghosts.
+// Called with positions that are those of the build (xb equals them).  Bound by
+// the gather of the particles from the caller's order (one cache line per value
+// where that order is random); it is paid once, against nine gathered and six
+// scattered values per particle in every later step.
+template <class T>
+__global__ __launch_bounds__(256) void k_ens_relabel(uint32_t N, size_t cap, const uint32_t* __restrict__ dom,
+                                                     uint32_t* __restrict__ s2n, uint32_t* __restrict__ n2s,
+                                                     const T* __restrict__ pos, const T* __restrict__ vel,
+                                                     const T* __restrict__ frc, const uint32_t* __restrict__ gid,
+                                                     T* __restrict__ pos2, T* __restrict__ vel2,
+                                                     T* __restrict__ frc2, uint32_t* __restrict__ gid2,
+                                                     T* __restrict__ xb, uint32_t* __restrict__ inv) {
+  const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k >= N) return;
+  const uint32_t f = dom[k];
+  const uint32_t i = s2n[f];
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    const T x = pos[d * cap + i];
+    pos2[d * cap + k] = x;
+    xb[d * cap + k] = x;
+    vel2[d * cap + k] = vel[d * cap + i];
+    if (frc) frc2[d * cap + k] = frc[d * cap + i];
+  }
+  gid2[k] = gid[i];
+  inv[i] = k;
+  s2n[f] = k;
+  n2s[k] = f;
+}
+
+// The ghosts' sources by their new storage indices (the ghosts keep theirs).
+__global__ __launch_bounds__(256) void k_ens_relabel_ghosts(uint32_t N, const uint32_t* __restrict__ counts,
+                                                            const uint32_t* __restrict__ inv,
+                                                            uint32_t* __restrict__ opid) {
+  const uint32_t g = blockIdx.x * blockDim.x + threadIdx.x;
+  if (N + g >= counts[0]) return;
+  opid[g] = inv[opid[g]];
+}
+
 // Ghost count / emit of the one-system path with the boxes of each particle's
 // system; ghosts land at N + (scan of the counts), at most gcap of them.
 template <class T>
@@ -371,6 +414,8 @@ struct ofp_ens {
   ofp_cl* cl = nullptr;
   ofp_vl* vl = nullptr;
   bool have_pos = false, built = false, sized = false, rebuild_pending = true;
+  bool ordered = false;   // the stored particles are in cell order (a build's rows)
+  bool at_build = false;  // the stored positions are those of the last build
   int force_prec = -1;  // precision of the forces in frc (-1: none)
   uint64_t n_ghost = 0, n_entries = 0, rebuilds = 0, steps = 0, recaptures = 0;
   // graphs: [step variant][precision] step (variants: see step_variant),
@@ -615,6 +660,7 @@ static int ens_rebuild_t(ofp_ens* e, int sizing, hipStream_t s, bool keep_frc) {
                                     e->gid2.as<uint32_t>(), e->xb.as<T>(), sid, dyn);
     OFP_LAUNCHED();
     ens_swap_storage(e, keep_frc);
+    e->ordered = true;
   } else {
     k_ens_map<T><<<gN, 256, 0, s>>>(N, cap, nullptr, nullptr, e->pos.as<T>(), nullptr, nullptr, nullptr, nullptr,
                                     nullptr, nullptr, nullptr, e->xb.as<T>(), sid, dyn);
@@ -663,6 +709,7 @@ static int ens_rebuild_t(ofp_ens* e, int sizing, hipStream_t s, bool keep_frc) {
       e->sized = true;
     }
     e->built = true;
+    e->at_build = true;
     return OFP_OK;
   }
   // Verlet list
@@ -686,6 +733,36 @@ static int ens_rebuild_t(ofp_ens* e, int sizing, hipStream_t s, bool keep_frc) {
     e->sized = true;
   }
   e->built = true;
+  e->at_build = true;
+  return OFP_OK;
+}
+
+// A run's particles in the caller's order: put them in the order of the build's
+// rows before the steps (k_ens_relabel), so the first steps read and write them
+// as coalesced as those after the next rebuild do.
+template <class T>
+static int ens_relabel_t(ofp_ens* e, bool keep_frc, hipStream_t s) {
+  const uint32_t N = uint32_t(e->N);
+  const size_t cap = e->cap;
+  ofp_cl_view v;
+  OFP_TRY(ofp_cl_get_view(e->cl, &v));
+  // the ensemble's own list: its storage indices are rewritten here
+  uint32_t* s2n = const_cast<uint32_t*>(v.sort_to_nonsort);
+  uint32_t* n2s = const_cast<uint32_t*>(v.nonsort_to_sort);
+  uint32_t* inv = e->gcnt.as<uint32_t>();  // N + 1 entries, free between rebuilds
+  k_ens_relabel<T><<<grid_for(N, 256), 256, 0, s>>>(N, cap, v.dom_sort_ids, s2n, n2s, e->pos.as<T>(), e->vel.as<T>(),
+                                                    keep_frc ? e->frc.as<T>() : nullptr, e->gid.as<uint32_t>(),
+                                                    e->pos2.as<T>(), e->vel2.as<T>(),
+                                                    keep_frc ? e->frc2.as<T>() : nullptr, e->gid2.as<uint32_t>(),
+                                                    e->xb.as<T>(), inv);
+  OFP_LAUNCHED();
+  if (e->gcap > 0) {
+    k_ens_relabel_ghosts<<<grid_for(e->gcap, 256), 256, 0, s>>>(N, e->counts.as<uint32_t>(), inv,
+                                                                e->opid.as<uint32_t>());
+    OFP_LAUNCHED();
+  }
+  ens_swap_storage(e, keep_frc);
+  e->ordered = true;
   return OFP_OK;
 }
 
@@ -819,7 +896,11 @@ static int ens_rebuild(ofp_ens* e, int sizing, hipStream_t s, bool keep_frc = tr
   return e->dtype == OFP_F32 ? ens_rebuild_t<float>(e, sizing, s, keep_frc)
                              : ens_rebuild_t<double>(e, sizing, s, keep_frc);
 }
+static int ens_relabel(ofp_ens* e, bool keep_frc, hipStream_t s) {
+  return e->dtype == OFP_F32 ? ens_relabel_t<float>(e, keep_frc, s) : ens_relabel_t<double>(e, keep_frc, s);
+}
 static int ens_drift(ofp_ens* e, double dt, hipStream_t s) {
+  e->at_build = false;
   return e->dtype == OFP_F32 ? ens_drift_t<float>(e, dt, s) : ens_drift_t<double>(e, dt, s);
 }
 static int ens_step(ofp_ens* e, int prec, double dt, int last, int set, hipStream_t s) {
@@ -1013,6 +1094,8 @@ int ofp_ens_set(ofp_ens* e, const void* pos, const void* vel, size_t stride, voi
   e->have_pos = true;
   e->built = false;
   e->sized = false;
+  e->ordered = false;
+  e->at_build = false;
   e->rebuild_pending = true;
   e->force_prec = -1;
   return OFP_OK;
@@ -1082,6 +1165,10 @@ int ofp_ens_run(ofp_ens* e, int precision, double dt, int n_steps, int use_graph
   OFP_CHECK(dt >= 0 && n_steps >= 0, OFP_E_ARG, "dt and n_steps must be >= 0");
   hipStream_t s = as_stream(stream);
   if (!e->built || !e->sized) OFP_TRY(ens_sizing(e, s));
+  // particles still in the caller's order: one reordering pays from the first
+  // step that kicks inside the pair kernel (every step but a run's last), see
+  // ens_relabel; a run of one step has none
+  if (!e->ordered && e->at_build && n_steps >= 2) OFP_TRY(ens_relabel(e, e->force_prec == precision, s));
   if (e->force_prec != precision) {
     OFP_TRY(ens_forces(e, precision, nullptr, s));
     e->force_prec = precision;
