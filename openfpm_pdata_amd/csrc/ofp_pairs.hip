@@ -1072,9 +1072,7 @@ __global__ __launch_bounds__(kTileBlock) void k_tile_f32c(ClDev c, QGeom qg1, Ph
   int4* buf = lds[threadIdx.x / kWave];
   const uint32_t n_items = *n_items_p;
   for (;;) {
-    uint32_t it = 0;
-    if (lane == 0) it = atomicAdd(counter, 1u);
-    it = __builtin_amdgcn_readfirstlane(it);
+    const uint32_t it = next_unit(counter);
     if (it >= n_items) break;
     const TargetItem ti = items[it];
     const uint32_t sy = ti.ncx >> 8;
@@ -1149,9 +1147,7 @@ __global__ __launch_bounds__(kTileBlock) void k_tile_f64(ClDev c, const T* __res
   Pos3<T>* buf = lds[threadIdx.x / kWave];
   const uint32_t n_items = *n_items_p;
   for (;;) {
-    uint32_t it = 0;
-    if (lane == 0) it = atomicAdd(counter, 1u);
-    it = __builtin_amdgcn_readfirstlane(it);
+    const uint32_t it = next_unit(counter);
     if (it >= n_items) break;
     const TargetItem ti = items[it];
     const Ph ph = kMany ? tab[ti.ncx >> 8] : ph1;
@@ -1558,7 +1554,7 @@ struct TileQueue {
 static int tile_queue(const PairCtx& x, TileQueue* q, hipStream_t s) {
   size_t cap = 0;
   OFP_TRY(ofp_cl_items_(x.cl, &q->items, &q->n_items, &q->counter, &cap, s));
-  return fill_u32(q->counter, 0, 1, s);
+  return fill_u32(q->counter, 0, kQueueWords, s);
 }
 
 // Verlet-row launches: kRowLanes lanes per domain row.

@@ -104,9 +104,7 @@ __global__ __launch_bounds__(kVlBlock) void k_vl_count(ClDev c, const T* __restr
   const int lane = threadIdx.x & (kWave - 1);
   const uint32_t n_items = *n_items_p;
   for (;;) {
-    uint32_t it = 0;
-    if (lane == 0) it = atomicAdd(counter, 1u);
-    it = __builtin_amdgcn_readfirstlane(it);
+    const uint32_t it = next_unit(counter);
     if (it >= n_items) break;
     const TargetItem ti = items[it];
     const ItemGeom<T> G = item_geom(c, ti, r2_one, sys, r2_sys);
@@ -189,9 +187,7 @@ __global__ __launch_bounds__(kVlBlock) void k_vl_fill(ClDev c, const SysGrid<T>*
   const uint32_t n_items = *n_items_p;
   if (*e_total > e_cap || mstate[1] != 0ull) return;
   for (;;) {
-    uint32_t it = 0;
-    if (lane == 0) it = atomicAdd(counter, 1u);
-    it = __builtin_amdgcn_readfirstlane(it);
+    const uint32_t it = next_unit(counter);
     if (it >= n_items) break;
     const TargetItem ti = items[it];
     const ItemGeom<T> G = item_geom(c, ti, T(0), sys, static_cast<const T*>(nullptr));
@@ -599,7 +595,7 @@ static int vl_build_t(ofp_vl* h, const ofp_cl* cl, const void* pos_v, size_t str
   auto count = [&]() -> int {
     OFP_TRY(fill_u64(reinterpret_cast<uint64_t*>(mstate), 0, 2, s));
     if (n == 0) return OFP_OK;
-    OFP_TRY(fill_u32(counter, 0, 1, s));
+    OFP_TRY(fill_u32(counter, 0, kQueueWords, s));
     k_vl_count<T><<<grid, kVlBlock, 0, s>>>(c, h->xyz.as<T>(), r2_one, sys, r2_sys, items, n_items, counter,
                                             h->cnt.as<uint32_t>(), mstate, h->moff.as<unsigned long long>(),
                                             h->masks.as<uint2>(), (unsigned long long)h->mask_cap);
@@ -626,7 +622,7 @@ static int vl_build_t(ofp_vl* h, const ofp_cl* cl, const void* pos_v, size_t str
   const size_t e_cap = *e_cap_io;
   OFP_TRY(h->nbr.ensure((e_cap + 4) * 4));  // + 3: the one-lane row kernels read whole groups of four entries
   if (n > 0) {
-    OFP_TRY(fill_u32(counter, 0, 1, s));
+    OFP_TRY(fill_u32(counter, 0, kQueueWords, s));
     k_vl_fill<T><<<grid, kVlBlock, 0, s>>>(c, sys, items, n_items, counter, h->off.as<unsigned long long>(),
                                            h->off.as<unsigned long long>() + n, (unsigned long long)e_cap, mstate,
                                            h->moff.as<unsigned long long>(), h->masks.as<uint2>(),
