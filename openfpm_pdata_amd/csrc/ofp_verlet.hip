@@ -4,24 +4,25 @@
 //
 // A target item is up to 64 domain particles (one per lane) whose cells lie on
 // one x-row of the grid; its candidates are the (2B+1)^2 x-runs of the stencil
-// (B = box_nn), each a contiguous range of sorted indices.
-//  * count: the candidate index is wave-uniform, so the candidates' coordinates
-//    come in through scalar loads (8 candidates at a time, from an interleaved
-//    xyz copy of the sorted positions) and every lane tests its own
-//    target against every candidate with the reference's rounding (distance2
-//    unfused, in the position dtype).  Each compare appends one bit to the
-//    lane's mask of the chunk (64 candidates): one 64-bit mask per (target,
-//    chunk), kept in a region of a mask buffer taken by one atomic per item.
-//  * fill: the candidates are in the lanes; a target's mask of a chunk is the
-//    exec mask of the chunk's store into its row, and the lanes below each hit
-//    give its place, so no distance is tested twice.  A group of up to 8 chunks
-//    is read at once (lane t: target t's masks); a target's hits of the whole
-//    group are written back to back at its row's cursor, so the row grows by
-//    whole cache lines while the wave is on it.
+// (B = box_nn), each a contiguous range of sorted indices, cut into blocks of 32
+// candidates.  The blocks of an item are numbered through its runs; a target's
+// hits in a block are one 32-bit word, a target's words are consecutive, the
+// targets one after another.
+//  * count: the squared distances of 64 targets and the 64 candidates of two
+//    blocks come from the matrix cores (FP32, K = 4: 2 x 2 tiles of 32 x 32), the
+//    sign bits of d^2 - r^2 are the targets' words.  Blocks in which some square
+//    is too near r^2 for FP32 products to decide are tested again with the
+//    reference's rounding (distance2 unfused, in the position dtype), so the
+//    words are those of the exact test.
+//  * fill: an item's words, in order, are its rows, in order, so the wave takes 64
+//    words at a time, one per lane, finds each lane's place by a prefix sum of
+//    the bit counts, and expands the bits into LDS, from where whole 1 KB stores
+//    go to the list.
 // Entries of a row come out in ascending sorted index, which is the reference
 // traversal order (cells in ascending linear id, ascending index inside a cell).
-// Persistent waves: each wave takes the next item from an atomic counter and
-// leaves when the queue is empty, so every wave reaches its exit.
+// Persistent waves: each wave takes the next unit (an item, or a part of one
+// where there are too few items for the chip) from its queue and leaves when that
+// is empty, so every wave reaches its exit.
 // A mask buffer too small for the items is flagged (mstate[1]); the fill then
 // writes nothing and the host grows the buffer and counts again.
 #include "ofp_internal.hpp"
@@ -30,10 +31,10 @@
 #include <type_traits>
 
 struct ofp_vl {
-  ofp::DevBuf cnt, off, nbr, scantmp, masks, moff, mstate, xyz;
+  ofp::DevBuf cnt, off, nbr, scantmp, masks, place, mstate, xyz;
   ofp::DevBuf rmask;  // thread-per-row build: the rows' hit masks, count pass to fill
   ofp::DevBuf aux;  // pair kernels' per-particle gather stream over the rows
-  size_t mask_cap = 0;  // 8-byte masks the buffer holds
+  size_t mask_cap = 0;  // pairs of mask words (8 bytes) the buffer holds (0: not sized yet)
   bool rows_path = false;  // the last build ran the thread-per-row kernels
   uint64_t n_rows = 0, n_entries = 0;
   bool built = false;
@@ -44,21 +45,9 @@ struct ofp_vl {
 namespace ofp {
 
 constexpr int kVlBlock = 256;
-constexpr int kFillGroup = 8;  // chunks of 64 candidates per fill group
-
-// Lane `lane` (uniform) of the returned VGPR takes the uniform value sval; the
-// other lanes keep vdst (v_writelane_b32, a VALU op; the lane select goes
-// through M0 since gfx9 VOP3 reads one SGPR besides M0).
-__device__ __forceinline__ uint32_t write_lane(uint32_t vdst, uint32_t sval, uint32_t lane) {
-  asm("s_mov_b32 m0, %2\n\tv_writelane_b32 %0, %1, m0" : "+v"(vdst) : "s"(sval), "s"(lane) : "m0");
-  return vdst;
-}
-
-__device__ __forceinline__ unsigned long long uniform_u64(unsigned long long v) {
-  const uint32_t lo = __builtin_amdgcn_readfirstlane(uint32_t(v));
-  const uint32_t hi = __builtin_amdgcn_readfirstlane(uint32_t(v >> 32));
-  return (static_cast<unsigned long long>(hi) << 32) | lo;
-}
+constexpr int kVlWaves = kVlBlock / kWave;
+constexpr uint32_t kBlk = 32;  // candidates per block (bits of a mask word)
+typedef float v16f __attribute__((ext_vector_type(16)));
 
 // The coordinates of 8 consecutive particles, x y z interleaved (read with
 // scalar loads; the element alignment is all a scalar load needs).
@@ -66,6 +55,25 @@ template <class T>
 struct alignas(sizeof(T)) Run8 {
   T v[24];
 };
+template <class T>
+struct Run1 {
+  T v[3];
+};
+// A load of read-only data at a wave-uniform address, as scalar loads (the
+// constant address space tells the compiler that no store of the kernel changes
+// it).
+template <class S>
+__device__ __forceinline__ S scalar_load(const void* p) {
+  using W = const uint32_t __attribute__((address_space(4)));
+  static_assert(sizeof(S) % 4 == 0, "whole dwords");
+  W* q = (W*)(reinterpret_cast<uintptr_t>(p));
+  uint32_t w[sizeof(S) / 4];
+#pragma unroll
+  for (size_t i = 0; i < sizeof(S) / 4; ++i) w[i] = q[i];
+  S s;
+  __builtin_memcpy(&s, w, sizeof(S));
+  return s;
+}
 
 // Sorted positions (three planes of stride `stride`) to one interleaved xyz
 // stream: the count pass reads the candidates of a run as one contiguous range,
@@ -80,205 +88,478 @@ __global__ void k_vl_pack(const T* __restrict__ pos, size_t stride, uint32_t n, 
   xyz[3 * size_t(i) + 2] = pos[2 * stride + i];
 }
 
-// One target's masks of a full fill group (64 contiguous bytes).
-struct alignas(8) MaskRun {
-  uint2 v[kFillGroup];
+// An item's runs in the lanes: lane r < (2B+1)^2 holds run r (traversal order),
+// its bounds and the number of its first block; blocks = the item's total.
+struct ItemRuns {
+  uint32_t ja, jb, first, blocks;
+};
+template <class T>
+__device__ __forceinline__ ItemRuns item_runs(const ClDev& c, const ItemGeom<T>& G, int lane) {
+  const int B = int(c.box_nn), W = 2 * B + 1;
+  const int xa = G.cx0 - B > 0 ? G.cx0 - B : 0;
+  const int xe = G.cx0 + G.ncx - 1 + B;
+  const int xb = xe < int(G.d0) - 1 ? xe : int(G.d0) - 1;
+  const int zz = G.cz + lane / W - B, yy = G.cy + lane % W - B;
+  ItemRuns R{0, 0, 0, 0};
+  if (lane < W * W && zz >= 0 && zz < int(G.d2) && yy >= 0 && yy < int(G.d1)) {
+    const uint32_t rowc = G.cbase + G.d0 * (uint32_t(yy) + G.d1 * uint32_t(zz));
+    R.ja = uint32_t(c.cs[rowc + uint32_t(xa)]);
+    R.jb = uint32_t(c.cs[rowc + uint32_t(xb) + 1]);
+  }
+  const uint32_t nb = (R.jb - R.ja + kBlk - 1) / kBlk;
+  const uint32_t inc = wave_incl_scan(nb);
+  R.first = inc - nb;
+  R.blocks = __builtin_amdgcn_readlane(inc, kWave - 1);
+  return R;
+}
+static_assert((2 * kMaxBoxNN + 1) * (2 * kMaxBoxNN + 1) <= kWave, "one lane per run");
+
+// Orders a wave's LDS accesses for the compiler (the LDS itself serves a wave's
+// accesses in order).
+__device__ __forceinline__ void lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// The first candidates and lengths of blocks [w0, w0 + N) of the item into the
+// wave's LDS table (entries past the item's blocks are not written).
+template <uint32_t N>
+__device__ __forceinline__ void block_table(const ItemRuns& R, uint32_t w0, uint2* tab) {
+  lds_order();
+  uint32_t q = R.first > w0 ? R.first : w0;
+  uint32_t j = R.ja + (q - R.first) * kBlk;
+  for (; j < R.jb && q < w0 + N; ++q, j += kBlk) tab[q - w0] = make_uint2(j, R.jb - j < kBlk ? R.jb - j : kBlk);
+  lds_order();
+}
+
+// Lane halves: {a_lo, b_lo} and {a_hi, b_hi}.
+__device__ __forceinline__ void swap_halves(uint32_t& a, uint32_t& b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+  a = r[0];
+  b = r[1];
+}
+__device__ __forceinline__ void swap_halves(float& a, float& b) {
+  uint32_t x = __float_as_uint(a), y = __float_as_uint(b);
+  swap_halves(x, y);
+  a = __uint_as_float(x);
+  b = __uint_as_float(y);
+}
+// min(m, |a|, |b|) in one instruction (no canonicalisation of the operands)
+__device__ __forceinline__ float min3_abs(float m, float a, float b) {
+  float r;
+  asm("v_min3_f32 %0, %1, |%2|, |%3|" : "=v"(r) : "v"(m), "v"(a), "v"(b));
+  return r;
+}
+template <class T>
+__device__ __forceinline__ T lane_value(T v, uint32_t lane);
+template <>
+__device__ __forceinline__ float lane_value<float>(float v, uint32_t lane) {
+  return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), lane));
+}
+template <>
+__device__ __forceinline__ double lane_value<double>(double v, uint32_t lane) {
+  const unsigned long long u = static_cast<unsigned long long>(__double_as_longlong(v));
+  const uint32_t lo = __builtin_amdgcn_readlane(uint32_t(u), lane), hi = __builtin_amdgcn_readlane(uint32_t(u >> 32), lane);
+  return __longlong_as_double(static_cast<long long>((static_cast<unsigned long long>(hi) << 32) | lo));
+}
+
+// Part `part` of P of `total` (monotonic in part, 0 and total at the ends).
+__device__ __forceinline__ uint32_t part_begin(uint32_t total, uint32_t part, uint32_t P) {
+  return P == 1 ? (part ? total : 0u) : uint32_t(uint64_t(total) * part / P);
+}
+
+// An item's words in the mask buffer: the first (in pairs of words) and the words
+// per target, a multiple of four (16-byte stores).
+struct ItemPlace {
+  unsigned long long first;
+  uint32_t words;
+  uint32_t pad;
 };
 
-// Count pass with the targets in the lanes.  Lane t builds, per chunk of 64
-// candidates, the 64-bit mask of the candidates within r of target t (bit k:
-// candidate k of the chunk).  The masks of a fill group (up to kFillGroup
-// chunks of one run) are stored target-major, ng per target, so the fill reads
-// a group with one contiguous load per lane.  mstate[0]: mask cursor,
-// mstate[1]: overflow flag; item_moff[it] = the item's first mask.
+// The places of all items and their total (mstate[0], cleared before), a thread
+// per item and one atomic per block of threads.
 template <class T>
-__global__ __launch_bounds__(kVlBlock) void k_vl_count(ClDev c, const T* __restrict__ xyz,
-                                                       T r2_one, const SysGrid<T>* __restrict__ sys,
-                                                       const T* __restrict__ r2_sys,
+__global__ __launch_bounds__(kVlBlock) void k_vl_place(ClDev c, const SysGrid<T>* __restrict__ sys,
                                                        const TargetItem* __restrict__ items,
                                                        const uint32_t* __restrict__ n_items_p,
-                                                       uint32_t* __restrict__ counter, uint32_t* __restrict__ cnt,
                                                        unsigned long long* __restrict__ mstate,
-                                                       unsigned long long* __restrict__ item_moff,
-                                                       uint2* __restrict__ masks, unsigned long long mask_cap) {
-  const int lane = threadIdx.x & (kWave - 1);
+                                                       ItemPlace* __restrict__ place) {
+  __shared__ unsigned long long ws[kVlWaves + 1];
+  const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
   const uint32_t n_items = *n_items_p;
-  for (;;) {
-    const uint32_t it = next_unit(counter);
-    if (it >= n_items) break;
-    const TargetItem ti = items[it];
-    const ItemGeom<T> G = item_geom(c, ti, r2_one, sys, r2_sys);
-    const T r2 = G.r2;
-    const bool valid = uint32_t(lane) < ti.n;
-    const uint32_t row = ti.row0 + (valid ? uint32_t(lane) : 0u);
-    const uint32_t p = c.dom[row];
-    const T xp = xyz[3 * size_t(p)], yp = xyz[3 * size_t(p) + 1], zp = xyz[3 * size_t(p) + 2];
-    // the item's mask region: ti.n masks per chunk of 64 candidates
-    uint32_t nch = 0;
-    for_each_run(c, G, [&](uint32_t ja, uint32_t jb) { nch += (jb - ja + kWave - 1) / kWave; });
-    const unsigned long long need = static_cast<unsigned long long>(nch) * ti.n;
-    unsigned long long moff = 0;
-    if (lane == 0) moff = atomicAdd(&mstate[0], need);
-    moff = uniform_u64(moff);
-    const bool keep = moff + need <= mask_cap;
-    if (lane == 0) {
-      item_moff[it] = moff;
-      if (!keep) atomicOr(&mstate[1], 1ull);
-    }
-    // Hit bits of candidates j0 .. j0 + cnt - 1 (1 <= cnt <= 32, uniform), bit k
-    // for candidate j0 + k.  The candidate index is wave-uniform: coordinates come
-    // in through scalar loads (read-only data), 8 candidates at a time, and enter
-    // the VALU as SGPR operands.  Lanes past the item's targets compute bits that
-    // are never stored.
-    auto hit_word = [&](uint32_t j0, uint32_t cnt) -> uint32_t {
-      uint32_t w = 0;  // candidate j0 + k at bit (k' - 1 - k) after k' shifts
-      uint32_t k = 0;
-      for (; k + 8 <= cnt; k += 8) {
-        const Run8<T> R = *reinterpret_cast<const Run8<T>*>(xyz + 3 * size_t(j0 + k));
-#pragma unroll
-        for (int i = 0; i < 8; ++i)
-          w = shift_in(w, dist2_unfused<T>(R.v[3 * i] - xp, R.v[3 * i + 1] - yp, R.v[3 * i + 2] - zp) < r2);
-      }
-      for (; k < cnt; ++k) {
-        const T* q = xyz + 3 * size_t(j0 + k);
-        w = shift_in(w, dist2_unfused<T>(q[0] - xp, q[1] - yp, q[2] - zp) < r2);
-      }
-      return __builtin_bitreverse32(w << (32u - cnt));
-    };
-    uint32_t n = 0;
-    unsigned long long goff = moff;  // the group's first mask
-    for_each_run(c, G, [&](uint32_t ja, uint32_t jb) {
-      for (uint32_t g0 = ja; g0 < jb; g0 += kFillGroup * kWave) {
-        const uint32_t rem = jb - g0 < uint32_t(kFillGroup * kWave) ? jb - g0 : uint32_t(kFillGroup * kWave);
-        const uint32_t ng = (rem + kWave - 1) / kWave;  // chunks in the group
-        for (uint32_t i = 0; i < ng; ++i) {
-          const uint32_t m = rem - i * kWave < uint32_t(kWave) ? rem - i * kWave : uint32_t(kWave);
-          const uint32_t lo = hit_word(g0 + i * kWave, m < 32u ? m : 32u);
-          const uint32_t hi = m > 32u ? hit_word(g0 + i * kWave + 32u, m - 32u) : 0u;
-          n += uint32_t(__builtin_popcount(lo)) + uint32_t(__builtin_popcount(hi));
-          if (keep && valid) masks[goff + static_cast<unsigned long long>(lane) * ng + i] = make_uint2(lo, hi);
+  for (uint32_t i0 = blockIdx.x * kVlBlock; i0 < n_items; i0 += gridDim.x * kVlBlock) {
+    const uint32_t it = i0 + threadIdx.x;
+    uint32_t words = 0, n = 0;
+    if (it < n_items) {
+      const TargetItem ti = items[it];
+      const ItemGeom<T> G = item_geom(c, ti, T(0), sys, static_cast<const T*>(nullptr));
+      const int B = int(c.box_nn);
+      const int xa = G.cx0 - B > 0 ? G.cx0 - B : 0;
+      const int xe = G.cx0 + G.ncx - 1 + B;
+      const int xb = xe < int(G.d0) - 1 ? xe : int(G.d0) - 1;
+      for (int dz = -B; dz <= B; ++dz)
+        for (int dy = -B; dy <= B; ++dy) {
+          const int zz = G.cz + dz, yy = G.cy + dy;
+          if (zz < 0 || zz >= int(G.d2) || yy < 0 || yy >= int(G.d1)) continue;
+          const uint32_t rowc = G.cbase + G.d0 * (uint32_t(yy) + G.d1 * uint32_t(zz));
+          words += (uint32_t(c.cs[rowc + uint32_t(xb) + 1]) - uint32_t(c.cs[rowc + uint32_t(xa)]) + kBlk - 1) / kBlk;
         }
-        goff += static_cast<unsigned long long>(ng) * ti.n;
+      words = (words + 3u) & ~3u;
+      n = ti.n;
+    }
+    const unsigned long long need = static_cast<unsigned long long>(words / 2u) * n;
+    const unsigned long long inc = wave_incl_scan(need);
+    if (lane == kWave - 1) ws[w] = inc;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      unsigned long long all = 0;
+      for (int k = 0; k < kVlWaves; ++k) {
+        const unsigned long long x = ws[k];
+        ws[k] = all;
+        all += x;
       }
-    });
-    if (valid) cnt[row] = n;
+      ws[kVlWaves] = all ? atomicAdd(&mstate[0], all) : 0ull;
+    }
+    __syncthreads();
+    if (it < n_items) place[it] = ItemPlace{ws[kVlWaves] + ws[w] + inc - need, words, 0u};
+    __syncthreads();
   }
 }
 
-// Fill pass from the masks, candidates in the lanes: for each target t of the
-// item (uniform loop) and chunk, the lanes set in t's mask hit it; they are
-// written to row t at base + (number of mask bits below the lane), one
-// contiguous store per (chunk, target); lane t keeps row t's write cursor.  Same
-// runs, same order as the count pass, so each row ends exactly where the count
-// said.  e_total / e_cap: the list's entry count (device) and the capacity of
-// nbr; a list that does not fit, or whose masks did not, is not written.
+// Count pass.  Lane t builds the words of target t, two blocks at a time.  A unit
+// is a part (of P) of an item's words; with P > 1 the parts' hits are added to cnt
+// (cleared before).  mstate[0]: pairs of words of all items, mstate[1]: overflow
+// flag (then no words are stored).
+//
+// With coordinates relative to one of the item's targets, a tile of the matrix
+// product of (x, y, z, |c|^2) and (-2x, -2y, -2z, 1), on top of |t|^2 - r^2, is
+// d^2 - r^2 for 32 candidates (rows) and 32 targets (columns): 128 matrix-core
+// cycles per 1024 pairs, and the vector ALU is left one instruction per 64 pairs
+// for the sign bit and half a one for the smallest |d^2 - r^2|, where the
+// distance test in the vector ALU took ten.  Rows are assigned to candidates so
+// that a lane's 16 results of a tile are 16 consecutive candidates, highest
+// first.
+// Undecided squares: with S = (R_c + R_t)^2 + r^2, R the farthest candidate and
+// target from the origin, relative coordinates, norms and products in FP32
+// (unit roundoff u) differ from the exact square by less than 24 u S, and the
+// reference's own roundings by less than 6 u d^2; |d^2 - r^2| < 32 u S = 2^-19 S
+// is tested exactly.  R comes from the cell geometry; blocks or an item with a
+// particle beyond it (outside its cell, or not a number) are tested exactly too.
+// 4.2e6 clustered particles (cells of r/2, 150 words a target): 6.4 -> 3.8 ms; 3e5:
+// 0.46 -> 0.27 ms; 4e5 in FP64 0.85 -> 0.36 ms.
+template <class T>
+__global__ __launch_bounds__(kVlBlock, 4) void k_vl_count(ClDev c, const T* __restrict__ xyz, T r2_one, float spx,
+                                                       float spy, float spz, const SysGrid<T>* __restrict__ sys,
+                                                       const T* __restrict__ r2_sys,
+                                                       const TargetItem* __restrict__ items,
+                                                       const uint32_t* __restrict__ n_items_p, uint32_t P,
+                                                       uint32_t* __restrict__ counter, uint32_t* __restrict__ cnt,
+                                                       unsigned long long* __restrict__ mstate,
+                                                       const ItemPlace* __restrict__ place,
+                                                       unsigned long long* __restrict__ masks,
+                                                       unsigned long long mask_cap) {
+  __shared__ uint2 tabs[kVlWaves][kWave];
+  const int lane = threadIdx.x & (kWave - 1);
+  uint2* const tab = tabs[threadIdx.x / kWave];
+  const uint32_t n_units = *n_items_p * P;
+  const bool keep = mstate[0] <= mask_cap;  // grid-uniform
+  if (!keep && blockIdx.x == 0 && threadIdx.x == 0) atomicOr(&mstate[1], 1ull);
+  // the candidate of this lane's matrix row: row 8 q + 4 h + m of a 32-block is
+  // candidate 16 h + 15 - (4 q + m), so a lane's results i = 4 q + m (rows
+  // 8 (i / 4) + 4 (lane / 32) + i % 4) are candidates 15 - i of its half
+  const uint32_t mrow = uint32_t(lane) & 31u;
+  const uint32_t mine = 16u * ((mrow >> 2) & 1u) + 15u - (4u * (mrow >> 3) + (mrow & 3u));
+  for (;;) {
+    const uint32_t un = next_unit(counter);
+    if (un >= n_units) break;
+    const uint32_t it = P == 1 ? un : un / P, part = P == 1 ? 0u : un % P;
+    const TargetItem ti = items[it];
+    const ItemGeom<T> G = item_geom(c, ti, r2_one, sys, r2_sys);
+    const T r2 = G.r2;
+    if (sys) {
+      const uint32_t sy = ti.ncx >> 8;
+      spx = float(sys[sy].sp[0]);
+      spy = float(sys[sy].sp[1]);
+      spz = float(sys[sy].sp[2]);
+    }
+    const bool valid = uint32_t(lane) < ti.n;
+    const uint32_t row = ti.row0 + (valid ? uint32_t(lane) : 0u);
+    const uint32_t p = c.dom[row];
+    const ItemPlace at = place[it];
+    const ItemRuns R = item_runs(c, G, lane);
+    const T xp = xyz[3 * size_t(p)], yp = xyz[3 * size_t(p) + 1], zp = xyz[3 * size_t(p) + 2];
+    // targets relative to the middle one, and the bounds of the FP32 squares
+    const uint32_t mid = ti.n / 2;
+    const T ox = lane_value(xp, mid), oy = lane_value(yp, mid), oz = lane_value(zp, mid);
+    const float tx = float(xp - ox), ty = float(yp - oy), tz = float(zp - oz);
+    const float tn = __builtin_fmaf(tx, tx, __builtin_fmaf(ty, ty, tz * tz));
+    const float B1 = float(c.box_nn + 1u), nx = float(G.ncx), bx = nx + float(c.box_nn);
+    const float rt2 = nx * nx * spx * spx + spy * spy + spz * spz;
+    const float rc2 = bx * bx * spx * spx + B1 * B1 * (spy * spy + spz * spz);
+    const float r2f = float(r2);
+    const float lim_t = rt2 * 1.01f, lim_c = rc2 * 1.01f;
+    const float eps = (2.05f * (rt2 + rc2) + r2f) * 0x1p-19f;  // (a + b)^2 <= 2 a^2 + 2 b^2
+    const bool fast = __all(tn <= lim_t);
+    float b00 = -2.f * tx, b01 = -2.f * ty;  // columns of the target halves: k = 0, 1
+    swap_halves(b00, b01);
+    float b10 = -2.f * tz, b11 = 1.f;  // k = 2, 3
+    swap_halves(b10, b11);
+    float k0 = tn - r2f, k1 = k0;
+    swap_halves(k0, k1);
+    v16f C0, C1;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      C0[i] = k0;
+      C1[i] = k1;
+    }
+    // Exact hit bits of candidates j0 .. j0 + m - 1 (1 <= m <= 32, uniform), bit k
+    // for candidate j0 + k; the coordinates come in through scalar loads.  Lanes
+    // past the item's targets compute bits that are never stored.
+    auto hit_word = [&](uint32_t j0, uint32_t m) -> uint32_t {
+      uint32_t w = 0;  // candidate j0 + k at bit (k' - 1 - k) after k' shifts
+      uint32_t k = 0;
+      for (; k + 8 <= m; k += 8) {
+        const Run8<T> Q = scalar_load<Run8<T>>(xyz + 3 * size_t(j0 + k));
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+          w = shift_in(w, dist2_unfused<T>(Q.v[3 * i] - xp, Q.v[3 * i + 1] - yp, Q.v[3 * i + 2] - zp) < r2);
+      }
+      for (; k < m; ++k) {
+        const Run1<T> q = scalar_load<Run1<T>>(xyz + 3 * size_t(j0 + k));
+        w = shift_in(w, dist2_unfused<T>(q.v[0] - xp, q.v[1] - yp, q.v[2] - zp) < r2);
+      }
+      return __builtin_bitreverse32(w << (32u - m));
+    };
+    // one tile: bits of 16 candidates appended to w, the smallest |square| in dm
+    auto tile = [&](float a0, float a1, float b0, float b1, const v16f& K, uint32_t& w, float& dm) {
+      v16f D = __builtin_amdgcn_mfma_f32_32x32x2f32(a0, b0, K, 0, 0, 0);
+      D = __builtin_amdgcn_mfma_f32_32x32x2f32(a1, b1, D, 0, 0, 0);
+#pragma unroll
+      for (int i = 0; i < 16; ++i) w = __builtin_amdgcn_alignbit(w, __float_as_uint(D[i]), 31);
+#pragma unroll
+      for (int i = 0; i < 16; i += 2) dm = min3_abs(dm, D[i], D[i + 1]);
+    };
+    const bool two_t = ti.n > 32u;
+    uint32_t n = 0;
+    // the unit's words [wa, wb), whole quads; blocks past the item's last are empty
+    const uint32_t wa = 4u * part_begin(at.words / 4u, part, P), wb = 4u * part_begin(at.words / 4u, part + 1, P);
+    uint2 tv = make_uint2(0u, 0u);  // block (w & ~63) + lane: first candidate, length
+    T cx, cy, cz;                   // this lane's candidate of the next two blocks
+    struct Two {
+      uint32_t ja, ma, jb, mb;
+    };
+    auto fetch = [&](uint32_t w) {
+      if ((w & 63u) == 0u || w == wa) {
+        block_table<kWave>(R, w & ~63u, tab);
+        tv = (w & ~63u) + uint32_t(lane) < R.blocks ? tab[lane] : make_uint2(0u, 0u);
+      }
+      Two b;
+      b.ja = __builtin_amdgcn_readlane(tv.x, w & 63u);
+      b.ma = __builtin_amdgcn_readlane(tv.y, w & 63u);
+      b.jb = __builtin_amdgcn_readlane(tv.x, (w & 63u) + 1u);
+      b.mb = __builtin_amdgcn_readlane(tv.y, (w & 63u) + 1u);
+      const uint32_t j = lane < 32 ? b.ja : b.jb, m = lane < 32 ? b.ma : b.mb;
+      const T* s = xyz + 3 * size_t(j + (mine < m ? mine : (m ? m - 1u : 0u)));
+      cx = s[0];
+      cy = s[1];
+      cz = s[2];
+      return b;
+    };
+    Two cur{0, 0, 0, 0};
+    if (wa < wb) cur = fetch(wa);
+    uint32_t* const out = reinterpret_cast<uint32_t*>(masks + at.first) + size_t(lane) * at.words;
+    uint32_t q0 = 0, q1 = 0;  // the quad's first two words
+    for (uint32_t w = wa; w < wb; w += 2) {
+      const Two b = cur;
+      const float x0 = float(cx - ox), y0 = float(cy - oy), z0 = float(cz - oz);
+      if (w + 2 < wb) cur = fetch(w + 2);
+      uint32_t lo = 0, hi = 0;
+      if (b.ma) {
+        const float cn = __builtin_fmaf(x0, x0, __builtin_fmaf(y0, y0, z0 * z0));
+        bool exact = !fast;
+        if (!exact) {
+          float dm = cn <= lim_c ? __builtin_inff() : 0.f;
+          float a00 = x0, a01 = y0, a10 = z0, a11 = cn;
+          swap_halves(a00, a01);  // a00: x, y of the first block; a01: of the second
+          swap_halves(a10, a11);
+          uint32_t w0 = 0, w1 = 0;
+          if (b.mb) {
+            tile(a01, a11, b00, b10, C0, w0, dm);
+            if (two_t) tile(a01, a11, b01, b11, C1, w1, dm);
+          }
+          tile(a00, a10, b00, b10, C0, w0, dm);
+          if (two_t) tile(a00, a10, b01, b11, C1, w1, dm);
+          // w_k: targets 32 k + lane % 32; of each block candidates 16 h + (0-15), h =
+          // lane / 32, the second block's in the high half.  To lane = target: w0 the
+          // h = 0 bits, w1 the h = 1 bits
+          swap_halves(w0, w1);
+          lo = __builtin_amdgcn_perm(w1, w0, 0x05040100u);
+          hi = __builtin_amdgcn_perm(w1, w0, 0x07060302u);
+          exact = __any(dm < eps);
+        }
+        if (exact) {  // a few per hundred
+          lo = hit_word(b.ja, b.ma);
+          hi = b.mb ? hit_word(b.jb, b.mb) : 0u;
+        } else {
+          lo &= 0xFFFFFFFFu >> (32u - b.ma);
+          hi &= b.mb ? 0xFFFFFFFFu >> (32u - b.mb) : 0u;
+        }
+      }
+      n += uint32_t(__builtin_popcount(lo)) + uint32_t(__builtin_popcount(hi));
+      if ((w & 2u) == 0u) {
+        q0 = lo;
+        q1 = hi;
+      } else if (keep && valid) {
+        *reinterpret_cast<uint4*>(out + (w - 2u)) = make_uint4(q0, q1, lo, hi);
+      }
+    }
+    if (valid) {
+      if (P == 1)
+        cnt[row] = n;
+      else if (n)
+        atomicAdd(&cnt[row], n);
+    }
+  }
+}
+
+// Fill pass from the words.  A unit is the words of TQ consecutive targets of an
+// item, the wave's stream; its entries are consecutive in the list.  Words with a
+// hit are queued in LDS with their blocks' first candidates (in the clustered
+// workload half of all words are empty), and 64 queued words are expanded at a time:
+// a prefix sum of the bit counts gives each lane its place in the staged row, and
+// each lane writes out its own word's bits.  Staged entries go to the list 16
+// bytes per lane.
+// Storing each word's hits straight to the list, a chunk of 64 candidates in the
+// lanes and a target's mask as exec mask, was bound by the 20 cycles a store
+// takes of the CU's address unit, for 8 entries on average.
+// e_total / e_cap: the list's entry count (device) and the capacity of nbr; a list
+// that does not fit, or whose masks did not, is not written.
+// 4.2e6 clustered particles (4.4e9 entries, 17.7 GB): 8.4 -> 6.5 ms (2.7 TB/s
+// written; instructions of the expansion, 40 % of whose lanes have bits left on
+// average, and their LDS conflicts); 3e5: 0.58 -> 0.35 ms; 4e5 in FP64 0.83 -> 0.55 ms.
+// LDS: 24 KB a block, six blocks per CU (32 KB and five: 6.8 ms).
+constexpr uint32_t kStage = 1024;  // entries staged per wave
+constexpr uint32_t kTab = 192;     // blocks tabulated per item (more: searched in its runs)
 template <class T>
 __global__ __launch_bounds__(kVlBlock) void k_vl_fill(ClDev c, const SysGrid<T>* __restrict__ sys,
                                                       const TargetItem* __restrict__ items,
-                                                      const uint32_t* __restrict__ n_items_p,
+                                                      const uint32_t* __restrict__ n_items_p, uint32_t TQ,
                                                       uint32_t* __restrict__ counter,
                                                       const unsigned long long* __restrict__ off,
                                                       const unsigned long long* __restrict__ e_total,
                                                       unsigned long long e_cap,
                                                       const unsigned long long* __restrict__ mstate,
-                                                      const unsigned long long* __restrict__ item_moff,
-                                                      const uint2* __restrict__ masks, uint32_t* __restrict__ nbr) {
+                                                      const ItemPlace* __restrict__ place,
+                                                      const unsigned long long* __restrict__ masks,
+                                                      uint32_t* __restrict__ nbr) {
+  static_assert(kStage >= 32 * kWave / 2, "half a wave of full words fits the empty row");
+  __shared__ uint4 stages[kVlWaves][kStage / 4];
+  __shared__ uint2 queues[kVlWaves][2 * kWave];
+  __shared__ uint32_t tabs[kVlWaves][kTab];
   const int lane = threadIdx.x & (kWave - 1);
-  const uint32_t n_items = *n_items_p;
+  uint32_t* const tab = tabs[threadIdx.x / kWave];
+  uint2* const queue = queues[threadIdx.x / kWave];
+  uint4* const st4 = stages[threadIdx.x / kWave];
+  uint32_t* const st = reinterpret_cast<uint32_t*>(st4);
+  const uint32_t Q = kWave / TQ;  // units per item
+  const uint32_t n_units = *n_items_p * Q;
   if (*e_total > e_cap || mstate[1] != 0ull) return;
   for (;;) {
-    const uint32_t it = next_unit(counter);
-    if (it >= n_items) break;
+    const uint32_t un = next_unit(counter);
+    if (un >= n_units) break;
+    const uint32_t it = un / Q;
     const TargetItem ti = items[it];
+    const uint32_t ta = (un % Q) * TQ, tb = ta + TQ < ti.n ? ta + TQ : ti.n;
+    if (ta >= ti.n) continue;
+    const ItemPlace at = place[it];
+    const uint32_t W = at.words;
+    if (W == 0) continue;
+    const unsigned long long e0 = off[ti.row0 + ta];
+    const uint32_t* __restrict__ words = reinterpret_cast<const uint32_t*>(masks + at.first) + size_t(ta) * W;
+    const uint32_t total = (tb - ta) * W;
     const ItemGeom<T> G = item_geom(c, ti, T(0), sys, static_cast<const T*>(nullptr));
-    const int nt = int(ti.n);
-    const bool valid = lane < nt;
-    const uint32_t row = ti.row0 + (valid ? uint32_t(lane) : 0u);
-    // lane t: row t's write cursor (low, high word)
-    const unsigned long long w0 = off[row];
-    uint32_t wlo = uint32_t(w0), whi = uint32_t(w0 >> 32);
-    unsigned long long goff = uniform_u64(item_moff[it]);  // the group's first mask
-    // groups of up to kFillGroup chunks of one run: each target's hits in the
-    // group are written back to back (its row grows by whole cache lines while
-    // the wave is on it), one cursor update per target and group
-    for_each_run(c, G, [&](uint32_t ja, uint32_t jb) {
-      for (uint32_t g0 = ja; g0 < jb; g0 += kFillGroup * kWave) {
-        const uint32_t rem = jb - g0 < uint32_t(kFillGroup * kWave) ? jb - g0 : uint32_t(kFillGroup * kWave);
-        const int ng = int((rem + kWave - 1) / kWave);  // chunks in the group (uniform)
-        // Lane t holds target t's masks of the group (ng of them, stored back to
-        // back); chunk i's mask of target t, read out of lane t, is the exec mask
-        // of its store: the lanes (the candidates) below each hit give the
-        // entry's place.  Two targets per step, t and t + 32, whose chains are
-        // independent (their instructions interleave).  full: the group has all
-        // kFillGroup chunks.  A row's write position is a uniform pointer plus a
-        // byte offset below 4 KiB (at most kFillGroup * 64 entries per target and
-        // group).
-        uint2 mk[kFillGroup];
-        if (ng == kFillGroup) {
-          const MaskRun M = valid ? *reinterpret_cast<const MaskRun*>(masks + goff + uint32_t(lane) * uint32_t(kFillGroup))
-                                  : MaskRun{};
+    const ItemRuns R = item_runs(c, G, lane);
+    lds_order();
+    const bool small = W <= kTab;
+    if (small) {  // tab[block] = its first candidate
+      for (uint32_t q = R.first, j = R.ja; j < R.jb; ++q, j += kBlk) tab[q] = j;
+    } else {  // tab[run] = its first block, tab[64 + run] = its first candidate
+      tab[lane] = R.first;
+      tab[kWave + lane] = R.ja;
+    }
+    lds_order();
+    auto block_first = [&](uint32_t w) -> uint32_t {
+      if (small) return tab[w];
+      uint32_t lo = 0;  // the last run that starts at or before w (empty runs start where the next one does)
 #pragma unroll
-          for (int i = 0; i < kFillGroup; ++i) mk[i] = M.v[i];
-        } else {
-#pragma unroll
-          for (int i = 0; i < kFillGroup; ++i)
-            mk[i] = valid && i < ng ? masks[goff + uint32_t(lane) * uint32_t(ng) + uint32_t(i)] : make_uint2(0u, 0u);
-        }
-        auto targets = [&](auto full, auto two, int t) {
-          constexpr bool kTwo = decltype(two)::value;
-          const int u = t + 32;
-          const uint32_t lo0 = __builtin_amdgcn_readlane(wlo, t), hi0 = __builtin_amdgcn_readlane(whi, t);
-          const unsigned long long base0 = (static_cast<unsigned long long>(hi0) << 32) | lo0;
-          unsigned long long base1 = 0;
-          if constexpr (kTwo) {
-            const uint32_t lo1 = __builtin_amdgcn_readlane(wlo, u), hi1 = __builtin_amdgcn_readlane(whi, u);
-            base1 = (static_cast<unsigned long long>(hi1) << 32) | lo1;
-          }
-          char* const row0 = reinterpret_cast<char*>(nbr + base0);
-          char* const row1 = reinterpret_cast<char*>(nbr + base1);
-          uint32_t run0 = 0, run1 = 0;  // entries written for the targets in the group
-#pragma unroll
-          for (int i = 0; i < kFillGroup; ++i) {
-            if constexpr (!decltype(full)::value) {
-              if (i >= ng) break;
-            }
-            const uint32_t j = g0 + uint32_t(i) * kWave + uint32_t(lane);
-            const uint32_t m0l = __builtin_amdgcn_readlane(mk[i].x, t), m0h = __builtin_amdgcn_readlane(mk[i].y, t);
-            const unsigned long long m0 = (static_cast<unsigned long long>(m0h) << 32) | m0l;
-            const uint32_t b0 = __builtin_amdgcn_mbcnt_hi(m0h, __builtin_amdgcn_mbcnt_lo(m0l, 0u));
-            if (__builtin_amdgcn_inverse_ballot_w64(m0)) *reinterpret_cast<uint32_t*>(row0 + (run0 + b0) * 4u) = j;
-            run0 += uint32_t(__popcll(m0));
-            if constexpr (kTwo) {
-              const uint32_t m1l = __builtin_amdgcn_readlane(mk[i].x, u), m1h = __builtin_amdgcn_readlane(mk[i].y, u);
-              const unsigned long long m1 = (static_cast<unsigned long long>(m1h) << 32) | m1l;
-              const uint32_t b1 = __builtin_amdgcn_mbcnt_hi(m1h, __builtin_amdgcn_mbcnt_lo(m1l, 0u));
-              if (__builtin_amdgcn_inverse_ballot_w64(m1)) *reinterpret_cast<uint32_t*>(row1 + (run1 + b1) * 4u) = j;
-              run1 += uint32_t(__popcll(m1));
-            }
-          }
-          if (run0) {
-            const unsigned long long nb = base0 + run0;
-            wlo = write_lane(wlo, uint32_t(nb), uint32_t(t));
-            whi = write_lane(whi, uint32_t(nb >> 32), uint32_t(t));
-          }
-          if (kTwo && run1) {
-            const unsigned long long nb = base1 + run1;
-            wlo = write_lane(wlo, uint32_t(nb), uint32_t(u));
-            whi = write_lane(whi, uint32_t(nb >> 32), uint32_t(u));
-          }
-        };
-        auto all_targets = [&](auto full) {
-          const int pairs = nt > 32 ? nt - 32 : 0;  // t with a partner t + 32
-          for (int t = 0; t < pairs; ++t) targets(full, std::true_type{}, t);
-          for (int t = pairs; t < (nt < 32 ? nt : 32); ++t) targets(full, std::false_type{}, t);
-        };
-        if (ng == kFillGroup)
-          all_targets(std::true_type{});
-        else
-          all_targets(std::false_type{});
-        goff += static_cast<unsigned long long>(ng) * uint32_t(nt);
+      for (uint32_t d = kWave / 2; d > 0; d >>= 1) lo += tab[lo + d] <= w ? d : 0u;
+      return tab[kWave + lo] + (w - tab[lo]) * kBlk;
+    };
+    uint32_t* out = nbr + e0;
+    uint32_t staged = 0, queued = 0;
+    auto flush = [&]() {
+      lds_order();
+      for (uint32_t k = uint32_t(lane); k < (staged >> 2); k += kWave) {
+        const uint4 v = st4[k];
+        __builtin_memcpy(out + 4 * k, &v, sizeof(v));
       }
-    });
+      const uint32_t k = (staged & ~3u) + uint32_t(lane);
+      if (k < staged) out[k] = st[k];
+      out += staged;
+      staged = 0;
+      lds_order();
+    };
+    // the first m <= 64 queued words
+    auto expand = [&](uint32_t m) {
+      lds_order();
+      uint2 v = make_uint2(0u, 0u);
+      if (uint32_t(lane) < m) v = queue[lane];
+      const uint32_t pc = uint32_t(__builtin_popcount(v.x));
+      const uint32_t inc = wave_incl_scan(pc);
+      const uint32_t all = __builtin_amdgcn_readlane(inc, kWave - 1);
+      auto write = [&](uint32_t bits, uint32_t place_) {
+        uint32_t* p = st + place_;
+        while (bits) {
+          *p++ = v.y + uint32_t(__builtin_ctz(bits));
+          bits &= bits - 1u;
+        }
+      };
+      if (staged + all > kStage) flush();
+      if (all <= kStage) {
+        write(v.x, staged + inc - pc);
+        staged += all;
+      } else {  // more hits than the row holds: half a wave at a time
+        const uint32_t first = __builtin_amdgcn_readlane(inc, kWave / 2 - 1);
+        write(lane < kWave / 2 ? v.x : 0u, inc - pc);
+        staged = first;
+        flush();
+        write(lane < kWave / 2 ? 0u : v.x, inc - pc - first);
+        staged = all - first;
+      }
+    };
+    uint32_t w = uint32_t(lane) % W;  // this lane's word of its target
+    const uint32_t step = kWave % W;
+    uint32_t next = uint32_t(lane) < total ? words[lane] : 0u;
+    for (uint32_t f = 0; f < total; f += kWave) {
+      const uint32_t bits = next;
+      const uint32_t fn = f + kWave + uint32_t(lane);
+      next = fn < total ? words[fn] : 0u;
+      const unsigned long long nz = __ballot(bits != 0u);
+      if (bits) {
+        const uint32_t k = queued + __builtin_amdgcn_mbcnt_hi(uint32_t(nz >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(nz), 0u));
+        queue[k] = make_uint2(bits, block_first(w));
+      }
+      queued += uint32_t(__popcll(nz));
+      w += step;
+      w = w >= W ? w - W : w;
+      if (queued >= uint32_t(kWave)) {
+        expand(kWave);
+        queued -= kWave;
+        if (uint32_t(lane) < queued) queue[lane] = queue[kWave + lane];
+      }
+    }
+    if (queued) expand(queued);
+    if (staged) flush();
   }
 }
 
@@ -492,14 +773,37 @@ static unsigned persistent_grid() {
   return g;
 }
 
+// How the item kernels split their work: count units of 1/parts of an item's
+// words, fill units of `targets` of its targets.  Whole items (one prologue, no
+// atomic adds to the counts) where n targets, at about 32 per item, give the waves
+// of the grid several units each; below that an item's serial walk would leave
+// most of the chip idle.
+struct VlSplit {
+  uint32_t parts, targets;
+};
+static VlSplit vl_split(size_t n) {
+  VlSplit s{1u, 64u};
+  while (s.parts < 8u && n * s.parts < size_t(1) << 18) s.parts *= 2u;
+  while (s.targets > 4u && n * (64u / s.targets) < size_t(1) << 20) s.targets /= 2u;
+  return s;
+}
+
 // One build.  sys/r2_sys: ensemble tables (null: one grid, radius r2_one).
 // sync: the counts are read back (entries, mask total), nbr and the mask
 // buffer grow to fit (the count pass is repeated if the masks did not fit), and
 // e_cap_io becomes max(e_cap_io, E x headroom); without sync nothing is read
 // back and the capacities stay (a list that would not fit is flagged).
 // rows_mode: 1 = the item kernels (targets in the lanes), 2 = thread per row,
-// 0 = thread per row when the stencil holds fewer than a wave of candidates per
-// target on average (n_part (2B+1)^3 < 64 n_cells), the item kernels otherwise.
+// 0 = by the mean candidates per target, n_part (2B+1)^3 / n_cells: thread per row
+// below kRowsBelow, the item kernels from there on (their 64 x 64 tiles need
+// candidates to fill).  Rebuilds of 2^20 uniform particles, items against rows, ms:
+// at 48 candidates 0.58 / 0.42, 110 1.17 / 0.63, 180 0.61 / 0.55, 222 0.90 / 0.91,
+// 359 0.72 / 0.86 (110 and 222 on cells of r/2, the others on cells of r).  Fewer than
+// kRowsFrom rows leave most of the chip without a wave, which the item kernels'
+// parts fill: 3,000 particles at 124 candidates 0.249 / 0.277, 10,000 at 132 0.219 /
+// 0.224, 30,000 at 144 0.286 / 0.258; below kRowsBelowFew candidates rows win there too.
+constexpr double kRowsBelow = 200.0, kRowsBelowFew = 64.0;
+constexpr size_t kRowsFrom = 16384;
 template <class T>
 static int vl_build_t(ofp_vl* h, const ofp_cl* cl, const void* pos_v, size_t stride, T r2_one, const void* sys_v,
                       const void* r2_sys_v, bool sync, size_t* e_cap_io, double headroom, unsigned grid,
@@ -514,11 +818,11 @@ static int vl_build_t(ofp_vl* h, const ofp_cl* cl, const void* pos_v, size_t str
   OFP_TRY(h->cnt.ensure((n + 1) * 4));
   OFP_TRY(h->off.ensure((n + 1) * 8));
   OFP_TRY(h->scantmp.ensure(scan_tmp_bytes(n)));
-  OFP_TRY(h->moff.ensure((n + 1) * 8));
   OFP_TRY(h->mstate.ensure(16));
   OFP_TRY(h->xyz.ensure((v.n_part + kRowAhead) * 3 * sizeof(T)));  // the row count reads whole groups
   const double stencil = std::pow(2.0 * double(c.box_nn) + 1.0, 3.0);
-  const bool rows = rows_mode == 2 || (rows_mode == 0 && double(v.n_part) * stencil < 64.0 * double(v.n_cells));
+  const double below = n < kRowsFrom ? kRowsBelowFew : kRowsBelow;
+  const bool rows = rows_mode == 2 || (rows_mode == 0 && double(v.n_part) * stencil < below * double(v.n_cells));
   if (rows) {
     auto* mstate = h->mstate.as<unsigned long long>();
     OFP_TRY(fill_u64(reinterpret_cast<uint64_t*>(mstate), 0, 2, s));  // no masks: nothing to overflow
@@ -579,8 +883,6 @@ static int vl_build_t(ofp_vl* h, const ofp_cl* cl, const void* pos_v, size_t str
     return OFP_OK;
   }
   h->rows_path = false;
-  if (h->mask_cap == 0) h->mask_cap = 16 * n + 4096;  // grown after the first count if short
-  OFP_TRY(h->masks.ensure(h->mask_cap * 8));
   const TargetItem* items;
   const uint32_t* n_items;
   uint32_t* counter;
@@ -592,13 +894,35 @@ static int vl_build_t(ofp_vl* h, const ofp_cl* cl, const void* pos_v, size_t str
     k_vl_pack<T><<<grid_for(v.n_part, 256), 256, 0, s>>>(pos, stride, uint32_t(v.n_part), h->xyz.as<T>());
     OFP_LAUNCHED();
   }
+  const VlSplit sp = vl_split(n);
+  OFP_TRY(h->place.ensure((n + 1) * sizeof(ItemPlace)));
+  OFP_TRY(fill_u64(reinterpret_cast<uint64_t*>(mstate), 0, 2, s));
+  if (n > 0) {
+    k_vl_place<T><<<n < size_t(1) << 18 ? grid_for(n, kVlBlock) : 1024u, kVlBlock, 0, s>>>(
+        c, sys, items, n_items, mstate, h->place.as<ItemPlace>());
+    OFP_LAUNCHED();
+  }
+  if (h->mask_cap == 0) {
+    // a handle's first build: the words its items need (sync), or an estimate that
+    // a sizing build corrects
+    h->mask_cap = size_t(stencil) * n + 4096;
+    if (sync && n > 0) {
+      unsigned long long need = 0;
+      OFP_HIP(hipMemcpyAsync(&need, mstate, 8, hipMemcpyDeviceToHost, s));
+      OFP_HIP(hipStreamSynchronize(s));
+      h->mask_cap = size_t(double(need) * (headroom > 1.0 ? headroom : 1.0)) + 4096;
+    }
+  }
+  OFP_TRY(h->masks.ensure(h->mask_cap * 8));
   auto count = [&]() -> int {
-    OFP_TRY(fill_u64(reinterpret_cast<uint64_t*>(mstate), 0, 2, s));
     if (n == 0) return OFP_OK;
+    OFP_TRY(fill_u64(reinterpret_cast<uint64_t*>(mstate) + 1, 0, 1, s));
     OFP_TRY(fill_u32(counter, 0, kQueueWords, s));
-    k_vl_count<T><<<grid, kVlBlock, 0, s>>>(c, h->xyz.as<T>(), r2_one, sys, r2_sys, items, n_items, counter,
-                                            h->cnt.as<uint32_t>(), mstate, h->moff.as<unsigned long long>(),
-                                            h->masks.as<uint2>(), (unsigned long long)h->mask_cap);
+    if (sp.parts > 1) OFP_TRY(fill_u32(h->cnt.as<uint32_t>(), 0, n, s));
+    k_vl_count<T><<<grid, kVlBlock, 0, s>>>(c, h->xyz.as<T>(), r2_one, float(v.spacing[0]), float(v.spacing[1]),
+                                            float(v.spacing[2]), sys, r2_sys, items, n_items, sp.parts, counter,
+                                            h->cnt.as<uint32_t>(), mstate, h->place.as<ItemPlace>(),
+                                            h->masks.as<unsigned long long>(), (unsigned long long)h->mask_cap);
     OFP_LAUNCHED();
     return OFP_OK;
   };
@@ -623,10 +947,10 @@ static int vl_build_t(ofp_vl* h, const ofp_cl* cl, const void* pos_v, size_t str
   OFP_TRY(h->nbr.ensure((e_cap + 4) * 4));  // + 3: the one-lane row kernels read whole groups of four entries
   if (n > 0) {
     OFP_TRY(fill_u32(counter, 0, kQueueWords, s));
-    k_vl_fill<T><<<grid, kVlBlock, 0, s>>>(c, sys, items, n_items, counter, h->off.as<unsigned long long>(),
-                                           h->off.as<unsigned long long>() + n, (unsigned long long)e_cap, mstate,
-                                           h->moff.as<unsigned long long>(), h->masks.as<uint2>(),
-                                           h->nbr.as<uint32_t>());
+    k_vl_fill<T><<<grid, kVlBlock, 0, s>>>(c, sys, items, n_items, sp.targets, counter,
+                                           h->off.as<unsigned long long>(), h->off.as<unsigned long long>() + n,
+                                           (unsigned long long)e_cap, mstate, h->place.as<ItemPlace>(),
+                                           h->masks.as<unsigned long long>(), h->nbr.as<uint32_t>());
     OFP_LAUNCHED();
   }
   h->n_rows = n;
@@ -764,7 +1088,7 @@ int ofp_vl_create(ofp_vl** h) {
 
 int ofp_vl_destroy(ofp_vl* h) {
   if (!h) return OFP_OK;
-  DevBuf* bufs[] = {&h->cnt, &h->off, &h->nbr, &h->scantmp, &h->masks, &h->moff, &h->mstate, &h->xyz, &h->aux, &h->rmask};
+  DevBuf* bufs[] = {&h->cnt, &h->off, &h->nbr, &h->scantmp, &h->masks, &h->place, &h->mstate, &h->xyz, &h->aux, &h->rmask};
   for (DevBuf* b : bufs) b->release();
   delete h;
   return OFP_OK;

@@ -21,6 +21,64 @@ PATTERNS = {
 }
 
 
+def dense(rng):
+    """Cells of thousands: rows of more mask words than an item tabulates, words
+    full of hits and words without any."""
+    p = np.concatenate([rng.random((3, 2700)) * 0.4 + np.array([[10.0 + k], [1.0], [1.0]]) for k in range(3)], axis=1)
+    return np.concatenate([p, rng.random((3, 100)) * np.array([[30.0], [3.0], [3.0]])], axis=1)
+
+
+@pytest.mark.parametrize("box_nn", [1, 2, 3])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("r", [0.999, 0.3])
+def test_rows_of_dense_cells(r, dtype, box_nn):
+    npd = np.float32 if dtype == torch.float32 else np.float64
+    pos = np.ascontiguousarray(dense(np.random.default_rng(2)).astype(npd))
+    n = pos.shape[1]
+    vd = vdm.VectorDistGPU(n, (0.0,) * 3, (30.0, 3.0, 3.0), (0, 0, 0), 0.5, dtype=dtype)
+    vd.pos[:, :n] = torch.from_numpy(pos).cuda()
+    opt = vdm.CL_NON_SYMMETRIC | vdm.CL_GPU_REORDER_POSITION
+    cl = vd.updateCellListGPU(vd.getCellListGPU(1.0 / box_nn, opt, NNIteratorBox=box_nn))
+    vl = vdm.VerletListGPU()
+    vl.build(cl, vd.pos, r)
+    off, nbr = (t.cpu().numpy() for t in vl.arrays())
+    s2n = cl.arrays()["s2n"].cpu().numpy()
+    dom = cl.arrays()["dom"].cpu().numpy()
+    rng = np.random.default_rng(3)
+    for k in np.concatenate([np.arange(40), rng.integers(0, n, 400), [n - 1]]):
+        i = s2n[dom[k]]
+        d = pos - pos[:, i:i + 1]
+        near = (d[0] * d[0] + d[1] * d[1]) + d[2] * d[2] < npd(r) * npd(r)
+        row = nbr[off[k]:off[k + 1]]
+        assert np.all(np.diff(row) > 0)
+        np.testing.assert_array_equal(np.sort(s2n[row]), np.flatnonzero(near))
+
+
+@pytest.mark.parametrize("rel", [0.0, 2.0 ** -23, 2.0 ** -20, 2.0 ** -17])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+def test_distances_at_the_radius(dtype, rel):
+    """Pairs whose distance is the radius to within rel (up to and past what the
+    FP32 products can decide): every decision is the exact test's."""
+    npd = np.float32 if dtype == torch.float32 else np.float64
+    rng = np.random.default_rng(6)
+    r = 0.5
+    c = rng.random((3, 300)) * 2.0 + 1.0
+    v = rng.standard_normal((3, 300))
+    v *= r * (1.0 + rel * rng.uniform(-1.0, 1.0, 300)) / np.linalg.norm(v, axis=0)
+    pos = np.ascontiguousarray(np.concatenate([c, c + v], axis=1).astype(npd))
+    n = pos.shape[1]
+    vd = vdm.VectorDistGPU(n, (0.0,) * 3, (4.0,) * 3, (0, 0, 0), r, dtype=dtype)
+    vd.pos[:, :n] = torch.from_numpy(pos).cuda()
+    cl, vl = vd.getVerletGPU(r, sub=1)
+    off, nbr = (t.cpu().numpy() for t in vl.arrays())
+    s2n = cl.arrays()["s2n"].cpu().numpy()
+    dom = cl.arrays()["dom"].cpu().numpy()
+    for k in range(n):
+        d = pos - pos[:, s2n[dom[k]]][:, None]
+        near = (d[0] * d[0] + d[1] * d[1]) + d[2] * d[2] < npd(r) * npd(r)
+        np.testing.assert_array_equal(np.sort(s2n[nbr[off[k]:off[k + 1]]]), np.flatnonzero(near))
+
+
 @pytest.mark.parametrize("box_nn", [1, 2])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
 @pytest.mark.parametrize("pattern", sorted(PATTERNS))
