@@ -32,6 +32,7 @@
 #include <cstring>
 
 struct ofp_cl {
+  ofp::HandleLife life;
   int dtype = OFP_F32;
   uint32_t opt = 0;
   ofp::CellGeom<float> gf;
@@ -1130,7 +1131,7 @@ int ofp_cl_destroy(ofp_cl* h) {
   DevBuf* bufs[] = {&h->packed, &h->scan64, &h->keys,    &h->keys2, &h->s2n,        &h->vals2, &h->n2s,
                     &h->dom,    &h->quant,  &h->scantmp, &h->hist,  &h->sid_sorted, &h->items, &h->nitems,
                     &h->payload, &h->ctl, &h->colpart, &h->nz_flag, &h->nz_key, &h->nz_start, &h->nz_nn,
-                    &h->nz_inv};
+                    &h->nz_inv, &h->aux};
   for (DevBuf* b : bufs) b->release();
   delete h;
   return OFP_OK;

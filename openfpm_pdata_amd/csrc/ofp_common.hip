@@ -6,6 +6,8 @@
 
 #include <atomic>
 #include <cstring>
+#include <list>
+#include <mutex>
 
 namespace ofp {
 
@@ -15,6 +17,156 @@ uint64_t realloc_epoch() { return g_realloc_epoch.load(std::memory_order_acquire
 void bump_realloc_epoch() { g_realloc_epoch.fetch_add(1, std::memory_order_acq_rel); }
 
 static thread_local std::string g_last_error;
+
+// ---------------------------------------------------------- device blocks
+namespace {
+struct Kept {
+  void* p;
+  size_t cap;
+  int dev;
+  uint64_t stamp;  // number of the release
+};
+constexpr int kMaxPoolDevices = 64;
+struct Pool {
+  std::mutex m;
+  std::list<Kept> kept;  // oldest first
+  size_t held[kMaxPoolDevices] = {};
+  size_t limit[kMaxPoolDevices] = {};  // 0: not asked yet
+  uint64_t releases = 0;
+  uint64_t synced[kMaxPoolDevices] = {};  // releases the device is known to have finished before
+  size_t handles = 0;
+};
+Pool& pool() {
+  static Pool* p = new Pool();  // lives until the process ends
+  return *p;
+}
+// Sizes in steps of an eighth of their power of two, so counts that vary a
+// little from call to call meet the same blocks.
+size_t block_size(size_t b) {
+  size_t step = 256;
+  while (step * 16 < b) step *= 2;
+  return (b + step - 1) / step * step;
+}
+// Takes the kept blocks that `which` names out of the pool (under its lock).
+template <class F>
+std::list<Kept> take_out(Pool& P, F&& which) {
+  std::list<Kept> out;
+  for (auto it = P.kept.begin(); it != P.kept.end();) {
+    const auto next = std::next(it);
+    if (which(*it)) {
+      P.held[it->dev] -= it->cap;
+      out.splice(out.end(), P.kept, it);
+    }
+    it = next;
+  }
+  return out;
+}
+void give_back(const std::list<Kept>& blocks) {
+  for (const Kept& k : blocks) (void)hipFree(k.p);
+}
+}  // namespace
+
+int block_alloc(void** p, size_t bytes, size_t* cap, int* dev) {
+  *p = nullptr;
+  *cap = 0;
+  OFP_HIP(hipGetDevice(dev));
+  const size_t want = block_size(bytes);
+  Pool& P = pool();
+  const int d = *dev;
+  if (d >= 0 && d < kMaxPoolDevices) {
+    Kept best{nullptr, 0, 0, 0};
+    uint64_t before = 0;
+    {
+      std::lock_guard<std::mutex> lock(P.m);
+      auto found = P.kept.end();
+      for (auto it = P.kept.begin(); it != P.kept.end(); ++it)
+        if (it->dev == d && it->cap >= want && it->cap <= want + want / 4 &&
+            (found == P.kept.end() || it->cap < found->cap))
+          found = it;
+      if (found != P.kept.end()) {
+        best = *found;
+        P.held[d] -= best.cap;
+        P.kept.erase(found);
+        if (best.stamp > P.synced[d]) before = P.releases;
+      }
+    }
+    if (best.p) {
+      if (before) {
+        const hipError_t e = hipDeviceSynchronize();
+        std::lock_guard<std::mutex> lock(P.m);
+        if (e != hipSuccess) {  // a failed device, or a stream of this thread being captured: keep it for later
+          P.kept.push_back(best);
+          P.held[d] += best.cap;
+          return set_error(OFP_E_HIP, "hipDeviceSynchronize: %s", hipGetErrorString(e));
+        }
+        if (P.synced[d] < before) P.synced[d] = before;
+      }
+      *p = best.p;
+      *cap = best.cap;
+      return OFP_OK;
+    }
+  }
+  hipError_t e = hipMalloc(p, want);
+  if (e == hipErrorOutOfMemory) {
+    (void)hipGetLastError();
+    std::list<Kept> mine;
+    {
+      std::lock_guard<std::mutex> lock(P.m);
+      mine = take_out(P, [d](const Kept& k) { return k.dev == d; });
+    }
+    give_back(mine);
+    e = hipMalloc(p, want);
+  }
+  if (e != hipSuccess) {
+    *p = nullptr;
+    return set_error(OFP_E_HIP, "hipMalloc(%zu): %s", want, hipGetErrorString(e));
+  }
+  *cap = want;
+  return OFP_OK;
+}
+
+void block_free(void* p, size_t cap, int dev) {
+  Pool& P = pool();
+  std::list<Kept> out;
+  bool keep = false;
+  if (dev >= 0 && dev < kMaxPoolDevices) {
+    std::lock_guard<std::mutex> lock(P.m);
+    if (P.limit[dev] == 0) {
+      hipDeviceProp_t prop;
+      P.limit[dev] = hipGetDeviceProperties(&prop, dev) == hipSuccess ? prop.totalGlobalMem / 32 + 1 : 1;
+    }
+    const size_t limit = P.limit[dev];
+    if (P.handles > 0 && cap <= limit) {
+      keep = true;
+      P.kept.push_back(Kept{p, cap, dev, ++P.releases});
+      P.held[dev] += cap;
+      size_t over = P.held[dev] > limit ? P.held[dev] - limit : 0;
+      out = take_out(P, [dev, &over](const Kept& k) {
+        if (k.dev != dev || over == 0) return false;
+        over -= k.cap < over ? k.cap : over;
+        return true;
+      });
+    }
+  }
+  if (!keep) (void)hipFree(p);
+  give_back(out);
+}
+
+HandleLife::HandleLife() {
+  Pool& P = pool();
+  std::lock_guard<std::mutex> lock(P.m);
+  ++P.handles;
+}
+
+HandleLife::~HandleLife() {
+  Pool& P = pool();
+  std::list<Kept> out;
+  {
+    std::lock_guard<std::mutex> lock(P.m);
+    if (--P.handles == 0) out = take_out(P, [](const Kept&) { return true; });
+  }
+  give_back(out);
+}
 
 int set_error(int code, const char* fmt, ...) {
   char buf[1024];

@@ -386,6 +386,7 @@ __global__ __launch_bounds__(256) void k_ens_get(uint32_t N, size_t cap, const u
 using namespace ofp;
 
 struct ofp_ens {
+  ofp::HandleLife life;
   int dtype = OFP_F32;
   uint32_t S = 0;
   uint64_t N = 0;
@@ -1034,7 +1035,7 @@ int ofp_ens_destroy(ofp_ens* e) {
                     &e->ljq[0],  &e->ljq[1], &e->pos,    &e->vel,     &e->frc,    &e->xb,       &e->pos2,
                     &e->vel2,    &e->frc2,   &e->gid,    &e->gid2,    &e->sid,    &e->spos,     &e->fsorted,
                     &e->esorted, &e->energy_tmp, &e->gcnt, &e->gstart, &e->gtmp,  &e->opid,     &e->osid,
-                    &e->counts,  &e->flags,  &e->e_dev,  &e->nn};
+                    &e->counts,  &e->flags,  &e->e_dev,  &e->nn,      &e->spos2,   &e->quant2};
   for (DevBuf* b : bufs) b->release();
   delete e;
   return OFP_OK;

@@ -11,6 +11,7 @@
 #include <vector>
 
 struct ofp_ghost {
+  ofp::HandleLife life;
   int dtype = OFP_F32;
   ofp::GhostBoxes<float> bf;
   ofp::GhostBoxes<double> bd;

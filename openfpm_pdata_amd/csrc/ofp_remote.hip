@@ -76,6 +76,7 @@ struct RemoteBoxes {
 }  // namespace ofp
 
 struct ofp_map {
+  ofp::HandleLife life;
   int dtype = OFP_F32;
   uint32_t rank = 0;
   ofp::GeoGrid g{};
@@ -90,6 +91,7 @@ struct ofp_map {
 };
 
 struct ofp_ghost_remote {
+  ofp::HandleLife life;
   int dtype = OFP_F32;
   int n_boxes = 0;
   ofp::GeoGrid g{};

@@ -31,6 +31,7 @@
 #include <type_traits>
 
 struct ofp_vl {
+  ofp::HandleLife life;
   ofp::DevBuf cnt, off, nbr, scantmp, masks, place, mstate, xyz;
   ofp::DevBuf rmask;  // thread-per-row build: the rows' hit masks, count pass to fill
   ofp::DevBuf aux;  // pair kernels' per-particle gather stream over the rows
