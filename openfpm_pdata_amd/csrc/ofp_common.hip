@@ -1,7 +1,9 @@
 // ofp_common.hip -- error state, plane arguments, fills and exclusive scans.
 //
 // The scans are three-phase (block reduce -> scan of block sums in one block ->
-// block scan + offset): no inter-block waiting, so no kernel can spin.
+// block scan + offset), two-phase where the blocks are few enough that each sums
+// the earlier blocks' totals itself, and one block where one will do: no
+// inter-block waiting, so no kernel can spin.
 #include "ofp_internal.hpp"
 
 #include <atomic>
@@ -228,6 +230,12 @@ int fill_u64(uint64_t* p, uint64_t v, size_t n, hipStream_t s) { return fill_imp
 constexpr int kScanBlock = 256;
 constexpr int kScanItems = 16;
 constexpr size_t kScanTile = size_t(kScanBlock) * kScanItems;  // 4096 per block
+// One launch up to kScanOne elements, two up to kScanTwo tiles, three beyond.  A
+// launch costs about 2 us of kernel and as much again before the next one starts:
+// 8,192 elements 11.4 us in three launches, 7 in one.
+constexpr int kScanOneBlock = 1024;
+constexpr size_t kScanOne = size_t(kScanOneBlock) * kScanItems;
+constexpr size_t kScanTwo = 512;
 
 size_t scan_tmp_bytes(size_t n) {
   size_t nb = (n + kScanTile - 1) / kScanTile;
@@ -236,11 +244,11 @@ size_t scan_tmp_bytes(size_t n) {
 
 // Block-wide exclusive scan of one value per thread; returns the block total in
 // *total (all threads).
-template <class V>
+template <class V, int kBlock = kScanBlock>
 __device__ __forceinline__ V block_excl_scan(V v, V* lds, V* total) {
   const int lane = threadIdx.x & (kWave - 1);
   const int w = threadIdx.x / kWave;
-  constexpr int nw = kScanBlock / kWave;
+  constexpr int nw = kBlock / kWave;
   V inc = wave_incl_scan(v);
   if (lane == kWave - 1) lds[w] = inc;
   __syncthreads();
@@ -297,14 +305,11 @@ __global__ __launch_bounds__(kScanBlock) void k_scan_partials(V* partial, size_t
   if (threadIdx.x == 0) partial[nb] = tot;
 }
 
-// Each thread owns kScanItems consecutive elements, read and written as whole
-// 16-byte vectors in full tiles (the arrays are at least 4-byte aligned, which
-// gfx950's multi-dword loads and stores need).
-template <class In, class V>
-__global__ __launch_bounds__(kScanBlock) void k_scan_apply(const In* in, V* out, size_t n,
-                                                           const V* partial, size_t nb) {
-  __shared__ V lds[kScanBlock / kWave + 1];
-  const size_t base = size_t(blockIdx.x) * kScanTile + size_t(threadIdx.x) * kScanItems;
+// One tile: each thread owns kScanItems consecutive elements, read and written as
+// whole 16-byte vectors in full tiles (the arrays are at least 4-byte aligned,
+// which gfx950's multi-dword loads and stores need).  Returns the tile's total.
+template <class In, class V, int kBlock>
+__device__ __forceinline__ V scan_tile(const In* in, V* out, size_t n, size_t base, V before, V* lds) {
   const bool full = base + kScanItems <= n;
   In x[kScanItems];
   if (full) {
@@ -317,8 +322,8 @@ __global__ __launch_bounds__(kScanBlock) void k_scan_apply(const In* in, V* out,
 #pragma unroll
   for (int k = 0; k < kScanItems; ++k) acc += V(x[k]);
   V tot;
-  const V ex = block_excl_scan<V>(acc, lds, &tot);
-  V run = ex + partial[blockIdx.x];
+  const V ex = block_excl_scan<V, kBlock>(acc, lds, &tot);
+  V run = ex + before;
   V y[kScanItems];
 #pragma unroll
   for (int k = 0; k < kScanItems; ++k) {
@@ -332,7 +337,38 @@ __global__ __launch_bounds__(kScanBlock) void k_scan_apply(const In* in, V* out,
     for (int k = 0; k < kScanItems; ++k)
       if (base + k < n) out[base + k] = y[k];
   }
+  return tot;
+}
+
+template <class In, class V>
+__global__ __launch_bounds__(kScanBlock) void k_scan_apply(const In* in, V* out, size_t n,
+                                                           const V* partial, size_t nb) {
+  __shared__ V lds[kScanBlock / kWave + 1];
+  const size_t base = size_t(blockIdx.x) * kScanTile + size_t(threadIdx.x) * kScanItems;
+  (void)scan_tile<In, V, kScanBlock>(in, out, n, base, partial[blockIdx.x], lds);
   if (blockIdx.x == 0 && threadIdx.x == 0) out[n] = partial[nb];
+}
+
+// partial: the tiles' sums (not scanned), nb <= kScanTwo of them.
+template <class In, class V>
+__global__ __launch_bounds__(kScanBlock) void k_scan_apply_two(const In* in, V* out, size_t n, const V* partial) {
+  static_assert(kScanTwo == 2 * kScanBlock, "two sums per thread");
+  __shared__ V lds[kScanBlock / kWave + 1];
+  const uint32_t b = blockIdx.x, t = threadIdx.x;
+  V v = t < b ? partial[t] : V(0);
+  if (t + kScanBlock < b) v += partial[t + kScanBlock];
+  V before;
+  (void)block_excl_scan<V>(v, lds, &before);
+  const size_t base = size_t(b) * kScanTile + size_t(t) * kScanItems;
+  const V tot = scan_tile<In, V, kScanBlock>(in, out, n, base, before, lds);
+  if (b == gridDim.x - 1 && t == 0) out[n] = before + tot;
+}
+
+template <class In, class V>
+__global__ __launch_bounds__(kScanOneBlock) void k_scan_one(const In* in, V* out, size_t n) {
+  __shared__ V lds[kScanOneBlock / kWave + 1];
+  const V tot = scan_tile<In, V, kScanOneBlock>(in, out, n, size_t(threadIdx.x) * kScanItems, V(0), lds);
+  if (threadIdx.x == 0) out[n] = tot;
 }
 
 template <class In, class V>
@@ -342,8 +378,18 @@ static int scan_impl(const In* in, V* out, size_t n, void* tmp, hipStream_t s) {
   if (n == 0) {
     return fill_impl<V>(out, V(0), 1, s);
   }
+  if (n <= kScanOne) {
+    k_scan_one<In, V><<<1, kScanOneBlock, 0, s>>>(in, out, n);
+    OFP_LAUNCHED();
+    return OFP_OK;
+  }
   k_scan_reduce<In, V><<<unsigned(nb), kScanBlock, 0, s>>>(in, n, partial);
   OFP_LAUNCHED();
+  if (nb <= kScanTwo) {
+    k_scan_apply_two<In, V><<<unsigned(nb), kScanBlock, 0, s>>>(in, out, n, partial);
+    OFP_LAUNCHED();
+    return OFP_OK;
+  }
   k_scan_partials<V><<<1, kScanBlock, 0, s>>>(partial, nb);
   OFP_LAUNCHED();
   k_scan_apply<In, V><<<unsigned(nb), kScanBlock, 0, s>>>(in, out, n, partial, nb);

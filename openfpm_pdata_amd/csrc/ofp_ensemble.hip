@@ -129,11 +129,12 @@ __global__ __launch_bounds__(256) void k_ens_ghost_count(const GhostBoxes<T>* __
   auto count = [&](const GhostBoxes<T>& B) {
     uint32_t old = 0xFFFFFFFFu, n = 0;
     if (!no_box(B, x, y, z)) {
+#pragma unroll 4
       for (int b = 0; b < B.nb; ++b) {
-        if (inside_np(B, b, x, y, z) && B.sv[b] != old) {
-          old = B.sv[b];
-          ++n;
-        }
+        const uint32_t sv = B.sv[b];
+        const bool in = inside_np(B, b, x, y, z) & (sv != old);
+        old = in ? sv : old;
+        n += in ? 1u : 0u;
       }
     }
     return n;
@@ -159,8 +160,8 @@ __global__ __launch_bounds__(256) void k_ens_ghost_emit(const GhostBoxes<T>* __r
     const uint32_t base = gstart[p];
     uint32_t old = 0xFFFFFFFFu, n = 0;
     for (int b = 0; b < B.nb; ++b) {
-      if (inside_np(B, b, x, y, z) && B.sv[b] != old) {
-        const uint32_t sh = B.sv[b];
+      const uint32_t sh = B.sv[b];
+      if (inside_np(B, b, x, y, z) & (sh != old)) {
         const uint32_t g = base + n;
         if (g < gcap) {
           pos[N + g] = x - B.shift[sh][0];

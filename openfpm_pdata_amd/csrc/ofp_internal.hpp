@@ -221,11 +221,13 @@ struct GhostBoxes {
   T in_lo[3], in_hi[3];
 };
 
-// Box::isInsideNP: half-open on every side.
+// Box::isInsideNP: half-open on every side.  All six compares, no branches
+// between them: a box's bounds are scalar loads, and the loops over the boxes can
+// have several boxes' loads in flight.
 template <class T>
 __device__ __forceinline__ bool inside_np(const GhostBoxes<T>& B, int b, T x, T y, T z) {
-  return x >= B.lo[b][0] && x < B.hi[b][0] && y >= B.lo[b][1] && y < B.hi[b][1] &&
-         z >= B.lo[b][2] && z < B.hi[b][2];
+  return (x >= B.lo[b][0]) & (x < B.hi[b][0]) & (y >= B.lo[b][1]) & (y < B.hi[b][1]) & (z >= B.lo[b][2]) &
+         (z < B.hi[b][2]);
 }
 
 // True when (x, y, z) lies in the region no box reaches (no ghost).

@@ -27,17 +27,19 @@
 // writes nothing and the host grows the buffer and counts again.
 #include "ofp_internal.hpp"
 
+#include <algorithm>
 #include <cmath>
 #include <type_traits>
 
 struct ofp_vl {
   ofp::HandleLife life;
-  ofp::DevBuf cnt, off, nbr, scantmp, masks, place, mstate, xyz;
+  ofp::DevBuf cnt, off, nbr, scantmp, masks, place, xyz;
   ofp::DevBuf rmask;  // thread-per-row build: the rows' hit masks, count pass to fill
   ofp::DevBuf aux;  // pair kernels' per-particle gather stream over the rows
   size_t mask_cap = 0;  // pairs of mask words (8 bytes) the buffer holds (0: not sized yet)
   bool rows_path = false;  // the last build ran the thread-per-row kernels
   uint64_t n_rows = 0, n_entries = 0;
+  uint64_t n_state = 0;  // rows of the last build: mstate lies behind its offsets
   bool built = false;
   bool symmetric = false;  // built by ofp_vl_build_sym (each interaction once)
   const ofp_cl* cl = nullptr;
@@ -80,9 +82,13 @@ __device__ __forceinline__ S scalar_load(const void* p) {
 // stream: the count pass reads the candidates of a run as one contiguous range,
 // whatever the planes' stride (planes a large power of two apart would share
 // cache sets).
+// Also clears the build's counts (cnt) and control words (ctl).
 template <class T>
-__global__ void k_vl_pack(const T* __restrict__ pos, size_t stride, uint32_t n, T* __restrict__ xyz) {
+__global__ void k_vl_pack(const T* __restrict__ pos, size_t stride, uint32_t n, T* __restrict__ xyz,
+                          uint32_t* __restrict__ cnt, uint32_t n_cnt, uint32_t* __restrict__ ctl, uint32_t n_ctl) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n_cnt) cnt[i] = 0u;
+  if (i < n_ctl) ctl[i] = 0u;
   if (i >= n) return;
   xyz[3 * size_t(i)] = pos[i];
   xyz[3 * size_t(i) + 1] = pos[stride + i];
@@ -817,20 +823,23 @@ static int vl_build_t(ofp_vl* h, const ofp_cl* cl, const void* pos_v, size_t str
   const T* r2_sys = static_cast<const T*>(r2_sys_v);
   const size_t n = c.n_dom;
   OFP_TRY(h->cnt.ensure((n + 1) * 4));
-  OFP_TRY(h->off.ensure((n + 1) * 8));
+  // behind the n + 1 offsets: mstate[2] (read back with the last offset) and the
+  // queue heads of the count and fill passes
+  constexpr uint32_t kCtl = 4u + 2u * kQueueWords;
+  OFP_TRY(h->off.ensure((n + 1) * 8 + kCtl * 4));
+  h->n_state = n;
+  auto* mstate = h->off.as<unsigned long long>() + n + 1;
+  auto* heads = reinterpret_cast<uint32_t*>(mstate + 2);
   OFP_TRY(h->scantmp.ensure(scan_tmp_bytes(n)));
-  OFP_TRY(h->mstate.ensure(16));
   OFP_TRY(h->xyz.ensure((v.n_part + kRowAhead) * 3 * sizeof(T)));  // the row count reads whole groups
   const double stencil = std::pow(2.0 * double(c.box_nn) + 1.0, 3.0);
   const double below = n < kRowsFrom ? kRowsBelowFew : kRowsBelow;
   const bool rows = rows_mode == 2 || (rows_mode == 0 && double(v.n_part) * stencil < below * double(v.n_cells));
   if (rows) {
-    auto* mstate = h->mstate.as<unsigned long long>();
-    OFP_TRY(fill_u64(reinterpret_cast<uint64_t*>(mstate), 0, 2, s));  // no masks: nothing to overflow
-    if (v.n_part > 0) {
-      k_vl_pack<T><<<grid_for(v.n_part, 256), 256, 0, s>>>(pos, stride, uint32_t(v.n_part), h->xyz.as<T>());
-      OFP_LAUNCHED();
-    }
+    // no masks: mstate stays 0, nothing to overflow
+    k_vl_pack<T><<<grid_for(std::max<size_t>(v.n_part, 4), 256), 256, 0, s>>>(
+        pos, stride, uint32_t(v.n_part), h->xyz.as<T>(), nullptr, 0u, reinterpret_cast<uint32_t*>(mstate), 4u);
+    OFP_LAUNCHED();
     CellGeom<T> g1;
     for (int k = 0; k < 3; ++k) {
       g1.lo[k] = T(v.lo[k]);
@@ -886,18 +895,17 @@ static int vl_build_t(ofp_vl* h, const ofp_cl* cl, const void* pos_v, size_t str
   h->rows_path = false;
   const TargetItem* items;
   const uint32_t* n_items;
-  uint32_t* counter;
+  uint32_t* counter;  // the cell tiles' queue heads; a list's passes have their own
   size_t cap;
   OFP_TRY(ofp_cl_items_(cl, &items, &n_items, &counter, &cap, s));
   if (grid == 0) grid = persistent_grid();
-  auto* mstate = h->mstate.as<unsigned long long>();
-  if (v.n_part > 0) {
-    k_vl_pack<T><<<grid_for(v.n_part, 256), 256, 0, s>>>(pos, stride, uint32_t(v.n_part), h->xyz.as<T>());
-    OFP_LAUNCHED();
-  }
   const VlSplit sp = vl_split(n);
+  const bool add = sp.parts > 1;  // the parts add their hits to the counts
+  k_vl_pack<T><<<grid_for(std::max<size_t>(v.n_part, kCtl), 256), 256, 0, s>>>(
+      pos, stride, uint32_t(v.n_part), h->xyz.as<T>(), h->cnt.as<uint32_t>(), add ? uint32_t(n) : 0u,
+      reinterpret_cast<uint32_t*>(mstate), kCtl);
+  OFP_LAUNCHED();
   OFP_TRY(h->place.ensure((n + 1) * sizeof(ItemPlace)));
-  OFP_TRY(fill_u64(reinterpret_cast<uint64_t*>(mstate), 0, 2, s));
   if (n > 0) {
     k_vl_place<T><<<n < size_t(1) << 18 ? grid_for(n, kVlBlock) : 1024u, kVlBlock, 0, s>>>(
         c, sys, items, n_items, mstate, h->place.as<ItemPlace>());
@@ -915,30 +923,32 @@ static int vl_build_t(ofp_vl* h, const ofp_cl* cl, const void* pos_v, size_t str
     }
   }
   OFP_TRY(h->masks.ensure(h->mask_cap * 8));
-  auto count = [&]() -> int {
+  auto count = [&](bool again) -> int {
     if (n == 0) return OFP_OK;
-    OFP_TRY(fill_u64(reinterpret_cast<uint64_t*>(mstate) + 1, 0, 1, s));
-    OFP_TRY(fill_u32(counter, 0, kQueueWords, s));
-    if (sp.parts > 1) OFP_TRY(fill_u32(h->cnt.as<uint32_t>(), 0, n, s));
+    if (again) {
+      OFP_TRY(fill_u64(reinterpret_cast<uint64_t*>(mstate) + 1, 0, 1, s));
+      OFP_TRY(fill_u32(heads, 0, kQueueWords, s));
+      if (add) OFP_TRY(fill_u32(h->cnt.as<uint32_t>(), 0, n, s));
+    }
     k_vl_count<T><<<grid, kVlBlock, 0, s>>>(c, h->xyz.as<T>(), r2_one, float(v.spacing[0]), float(v.spacing[1]),
-                                            float(v.spacing[2]), sys, r2_sys, items, n_items, sp.parts, counter,
+                                            float(v.spacing[2]), sys, r2_sys, items, n_items, sp.parts, heads,
                                             h->cnt.as<uint32_t>(), mstate, h->place.as<ItemPlace>(),
                                             h->masks.as<unsigned long long>(), (unsigned long long)h->mask_cap);
     OFP_LAUNCHED();
     return OFP_OK;
   };
-  OFP_TRY(count());
+  OFP_TRY(count(false));
   OFP_TRY(scan_excl_u32_to_u64(h->cnt.as<uint32_t>(), h->off.as<uint64_t>(), n, h->scantmp.p, s));
   uint64_t E = 0;
   if (sync) {
-    unsigned long long ms[2] = {0, 0};
-    OFP_HIP(hipMemcpyAsync(&E, h->off.as<uint64_t>() + n, 8, hipMemcpyDeviceToHost, s));
-    OFP_HIP(hipMemcpyAsync(ms, mstate, 16, hipMemcpyDeviceToHost, s));
+    unsigned long long back[3] = {0, 0, 0};  // the last offset, mstate
+    OFP_HIP(hipMemcpyAsync(back, h->off.as<uint64_t>() + n, sizeof(back), hipMemcpyDeviceToHost, s));
     OFP_HIP(hipStreamSynchronize(s));
-    if (ms[1] != 0) {  // masks did not fit: grow to the exact total (+ headroom) and count again
-      h->mask_cap = size_t(double(ms[0]) * (headroom > 1.0 ? headroom : 1.0)) + 4096;
+    E = back[0];
+    if (back[2] != 0) {  // masks did not fit: grow to the exact total (+ headroom) and count again
+      h->mask_cap = size_t(double(back[1]) * (headroom > 1.0 ? headroom : 1.0)) + 4096;
       OFP_TRY(h->masks.ensure(h->mask_cap * 8));
-      OFP_TRY(count());
+      OFP_TRY(count(true));
     }
     const size_t want = size_t(double(E) * (headroom > 1.0 ? headroom : 1.0)) + 1024;
     if (want > *e_cap_io) *e_cap_io = want;
@@ -947,8 +957,7 @@ static int vl_build_t(ofp_vl* h, const ofp_cl* cl, const void* pos_v, size_t str
   const size_t e_cap = *e_cap_io;
   OFP_TRY(h->nbr.ensure((e_cap + 4) * 4));  // + 3: the one-lane row kernels read whole groups of four entries
   if (n > 0) {
-    OFP_TRY(fill_u32(counter, 0, kQueueWords, s));
-    k_vl_fill<T><<<grid, kVlBlock, 0, s>>>(c, sys, items, n_items, sp.targets, counter,
+    k_vl_fill<T><<<grid, kVlBlock, 0, s>>>(c, sys, items, n_items, sp.targets, heads + kQueueWords,
                                            h->off.as<unsigned long long>(), h->off.as<unsigned long long>() + n,
                                            (unsigned long long)e_cap, mstate, h->place.as<ItemPlace>(),
                                            h->masks.as<unsigned long long>(), h->nbr.as<uint32_t>());
@@ -1044,7 +1053,7 @@ int ofp::vl_offsets(const ofp_vl* h, const unsigned long long** off) {
 
 int ofp::vl_mask_state(const ofp_vl* h, const unsigned long long** mstate) {
   OFP_CHECK(h && h->built, OFP_E_STATE, "Verlet list not built");
-  *mstate = h->mstate.as<unsigned long long>();
+  *mstate = h->off.as<unsigned long long>() + h->n_state + 1;
   return OFP_OK;
 }
 
@@ -1089,7 +1098,8 @@ int ofp_vl_create(ofp_vl** h) {
 
 int ofp_vl_destroy(ofp_vl* h) {
   if (!h) return OFP_OK;
-  DevBuf* bufs[] = {&h->cnt, &h->off, &h->nbr, &h->scantmp, &h->masks, &h->place, &h->mstate, &h->xyz, &h->aux, &h->rmask};
+  DevBuf* bufs[] = {&h->cnt, &h->off, &h->nbr, &h->scantmp, &h->masks, &h->place,
+                    &h->xyz, &h->aux, &h->rmask};
   for (DevBuf* b : bufs) b->release();
   delete h;
   return OFP_OK;

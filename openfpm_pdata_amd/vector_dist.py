@@ -49,6 +49,8 @@ CL_QUANT = L.OFP_CL_QUANT
 PERIODIC = 1
 NON_PERIODIC = 0
 
+MAX_PLANES = 24  # planes per copy call (kMaxPlanes of the library)
+
 # getCellListGPU's default ghostEnlargeFactor is a float (vector_dist.hpp:1223)
 GHOST_ENLARGE_CL = float(np.float32(1.013))
 # getVerlet magnifies the ghost by the double literal 1.013 (vector_dist.hpp:1537)
@@ -444,13 +446,20 @@ class VectorDistGPU:
     def restoreOrder(self, cl: CellListGPU, props=()):
         """Scatter positions (if reordered) and props back to the original order."""
         assert self.sorted_by is cl, "vector is not in this cell list's order"
+        src, dst = [], []
         if cl.opt & CL_GPU_REORDER_POSITION:
-            cl.restore(planes_of(self.pos), planes_of(self.pos_sorted))
-            self.pos, self.pos_sorted = self.pos_sorted, self.pos
+            src += planes_of(self.pos)
+            dst += planes_of(self.pos_sorted)
         for nm in props:
             if nm not in self.prp_sorted or self.prp_sorted[nm].shape[1] != self.cap:
                 self.prp_sorted[nm] = torch.empty_like(self.prp[nm])
-            cl.restore(planes_of(self.prp[nm]), planes_of(self.prp_sorted[nm]))
+            src += planes_of(self.prp[nm])
+            dst += planes_of(self.prp_sorted[nm])
+        for k in range(0, len(src), MAX_PLANES):  # one launch for all planes, as a call takes up to MAX_PLANES
+            cl.restore(src[k:k + MAX_PLANES], dst[k:k + MAX_PLANES])
+        if cl.opt & CL_GPU_REORDER_POSITION:
+            self.pos, self.pos_sorted = self.pos_sorted, self.pos
+        for nm in props:
             self.prp[nm], self.prp_sorted[nm] = self.prp_sorted[nm], self.prp[nm]
         self.sorted_by = None
 
