@@ -5,10 +5,12 @@
 // come out in ascending original index (domain ids < ghost ids: domain first).
 // That is the canonical order, reached without atomics on cell counters.
 //   1. k_rx_hist     pass 0: cell id per particle (the key), and per tile of
-//                    4096 particles the histogram of the pass's digit (<= 8 bits),
-//                    counted per wave with ballots, one LDS add per digit run.
-//   2. column scan   of the [tile][digit] histogram table gives every (tile,
-//                    digit) its first output slot.
+//                    4096 particles (1024 in small builds) the histogram of the
+//                    pass's digit (<= 8 bits), counted per wave with ballots, one
+//                    LDS add per digit run.
+//   2. column sums   of the [tile][digit] histogram table give every (tile,
+//                    digit) its first output slot: summed in the scatter up to
+//                    kRxChunked tiles, in kernels of their own beyond.
 //   3. k_rx_scatter  per tile: stable rank of each key inside the tile (ballot
 //                    peer masks, per-wave running counts in LDS), staged in LDS in
 //                    digit order, then written out as contiguous runs.
@@ -27,6 +29,7 @@
 // past the count.
 #include "ofp_internal.hpp"
 
+#include <algorithm>
 #include <cmath>
 #include <cstddef>
 #include <cstring>
@@ -54,7 +57,6 @@ struct ofp_cl {
   bool items_valid = false;
   size_t items_cap = 0;
   ofp::DevBuf packed, scan64, keys, keys2, s2n, vals2, n2s, dom, quant, scantmp, hist, sid_sorted, payload;
-  ofp::DevBuf ctl;  // [0] descents counted by pass 0 (the payload decision)
   ofp::DevBuf colpart;  // chunk sums of the histogram table
   ofp::DevBuf items, nitems;  // nitems: the consumers' queue heads (kQueueWords), then the item count
   ofp::DevBuf aux;            // pair kernels' per-particle record stream (cell tiles)
@@ -69,9 +71,28 @@ namespace ofp {
 
 constexpr int kRxBlock = 256;
 constexpr int kRxWaves = kRxBlock / kWave;
-constexpr int kRxIters = 16;                        // 64-key rounds per wave
-constexpr uint32_t kRxTile = kRxBlock * kRxIters;  // keys per tile
+// 64-key rounds per wave, and so the keys per tile (256 x rounds): 4096 for long
+// runs per digit, 1024 below kRxSmall particles, where tiles of 4096 leave most
+// CUs without a block and a wave works through 16 rounds one after another (and
+// through four times the code, fetched cold): 17,000 keys, a scatter 26 -> 13 us.
+constexpr int kRxLong = 16, kRxShort = 4;
+constexpr size_t kRxSmall = size_t(1) << 20;
 constexpr int kRxMaxBits = 8;
+// Up to kRxDirect tiles a scatter block sums the tiles' histograms itself; up to
+// kRxChunked it sums those of its own chunk of tiles and the chunks' sums, which
+// the histogram blocks add up with atomics (at most 32 adds per word): two launches
+// per pass.  The rows a block sums are loaded kColBatch at a time, one batch after
+// another: at 65 tiles 2 batches with chunks, 5 without.  Beyond kRxChunked, the column kernels do it (four launches): a block would read
+// over 100 rows of 1 KB for its 4096 keys.
+constexpr uint32_t kRxDirect = 32;
+constexpr uint32_t kRxChunked = 2048;
+// Below this many particles nothing is read back between the order check and the
+// passes: the passes' kernels return at once if the check found the input in cell
+// order.  Whole builds with and without the read-back (us): input in order 47 and
+// 53 at 17,000 particles, 70 and 64 at 2^20, 133 and 134 at 8e6; one exchanged pair
+// 81 and 62, 186 and 163, 438 and 417.  From here on the empty grids cost more than
+// the read-back.
+constexpr size_t kRxNoSync = size_t(1) << 23;
 constexpr int kRxBins = 1 << kRxMaxBits;
 
 __device__ __forceinline__ uint32_t lanes_below(unsigned long long m) {
@@ -94,25 +115,39 @@ __device__ __forceinline__ uint32_t count_of(uint32_t n_host, const uint32_t* n_
 }
 
 
+// Grid-uniform: the order check (*check = its descents; null = no check was
+// made) found the input in cell order, so the build is done.
+__device__ __forceinline__ bool in_order(const unsigned long long* check) { return check && *check == 0ull; }
+
 // Tile histogram of one digit.  Pass 0 (kin == null) evaluates the key, stores
-// it to kout and adds the tile's descents (k[e] > k[e+1] inside each 64-key
-// round) to *disorder, which then tells how far the input is from cell order.
-template <class Key>
+// it to kout, clears the cells' counts (clear[0 .. n_clear), null: not needed),
+// adds the digits' counts to the tile's chunk (part != null; cleared before), and,
+// where no order check ran before (disorder != null), adds the tile's
+// descents (k[e] > k[e+1] inside each 64-key round) to *disorder, which then
+// tells how far the input is from cell order.
+template <class Key, int kIters>
 __global__ __launch_bounds__(kRxBlock) void k_rx_hist(Key key, const uint32_t* __restrict__ kin,
                                                       uint32_t* __restrict__ kout, uint32_t n_host,
                                                       const uint32_t* __restrict__ n_dev, int shift, int bits,
                                                       uint32_t n_tiles, uint32_t* __restrict__ hist,
-                                                      unsigned long long* __restrict__ disorder) {
+                                                      unsigned long long* __restrict__ disorder,
+                                                      const unsigned long long* __restrict__ check,
+                                                      unsigned long long* __restrict__ clear, uint64_t n_clear,
+                                                      uint32_t* __restrict__ part, uint32_t ch) {
+  if (in_order(check)) return;
+  constexpr uint32_t kRxTile = uint32_t(kRxBlock * kIters);
   __shared__ uint32_t h[kRxBins];
   __shared__ uint32_t wdesc[kRxWaves];
   const uint32_t n = count_of(n_host, n_dev);
   const uint32_t t = blockIdx.x;
+  if (clear)
+    for (uint64_t i = uint64_t(t) * kRxBlock + threadIdx.x; i < n_clear; i += uint64_t(gridDim.x) * kRxBlock) clear[i] = 0ull;
   for (int d = threadIdx.x; d < kRxBins; d += kRxBlock) h[d] = 0;
   __syncthreads();
   const int lane = threadIdx.x & (kWave - 1);
   const int w = threadIdx.x / kWave;
   const uint32_t mask = (1u << bits) - 1u;
-  const uint64_t base = uint64_t(t) * kRxTile + uint64_t(w) * (kRxIters * kWave);
+  const uint64_t base = uint64_t(t) * kRxTile + uint64_t(w) * (kIters * kWave);
   uint32_t desc = 0;
   // batches of rounds: the batch's loads first, then its stores, then the
   // counting; all 16 rounds at once for stored keys, 4 when the keys are
@@ -120,7 +155,7 @@ __global__ __launch_bounds__(kRxBlock) void k_rx_hist(Key key, const uint32_t* _
   auto rounds = [&](auto batch) {
     constexpr int kB = decltype(batch)::value;
 #pragma unroll 1
-    for (int b = 0; b < kRxIters; b += kB) {
+    for (int b = 0; b < kIters; b += kB) {
       uint32_t kr[kB];
 #pragma unroll
       for (int i = 0; i < kB; ++i) {
@@ -142,7 +177,7 @@ __global__ __launch_bounds__(kRxBlock) void k_rx_hist(Key key, const uint32_t* _
         const unsigned long long act = __ballot(v);
         if (act == 0ull) continue;  // wave-uniform: a round past n
         const uint32_t k = kr[i];
-        if (!kin) {
+        if (!kin && disorder) {
           const uint32_t next = __shfl_down(k, 1, kWave);
           const bool nv = lane + 1 < kWave && ((act >> (lane + 1)) & 1ull);
           desc += (v && nv && k > next) ? 1u : 0u;
@@ -154,16 +189,20 @@ __global__ __launch_bounds__(kRxBlock) void k_rx_hist(Key key, const uint32_t* _
     }
   };
   if (kin)
-    rounds(std::integral_constant<int, kRxIters>{});
+    rounds(std::integral_constant<int, kIters>{});
   else
     rounds(std::integral_constant<int, 4>{});
-  if (!kin) {
+  if (!kin && disorder) {
     desc = wave_sum(desc);
     if (lane == 0) wdesc[w] = desc;
   }
   __syncthreads();
-  for (int d = threadIdx.x; d < (1 << bits); d += kRxBlock) hist[size_t(t) * kRxBins + d] = h[d];
-  if (!kin && threadIdx.x == 0) {
+  for (int d = threadIdx.x; d < (1 << bits); d += kRxBlock) {
+    const uint32_t v = h[d];
+    hist[size_t(t) * kRxBins + d] = v;
+    if (part && v) atomicAdd(&part[size_t(t / ch) * kRxBins + d], v);
+  }
+  if (!kin && disorder && threadIdx.x == 0) {
     uint32_t s = 0;
     for (int ww = 0; ww < kRxWaves; ++ww) s += wdesc[ww];
     if (s) atomicAdd(disorder, static_cast<unsigned long long>(s));
@@ -182,83 +221,110 @@ __device__ __forceinline__ bool carry_positions(const unsigned long long* disord
 // coalesced rows): offs[t][d] = sum of all counts of digits < d + sum of the
 // counts of digit d in tiles < t.  The tiles form at most kColChunks chunks;
 // every loop below loads kColBatch rows before it uses them.
-constexpr uint32_t kColChunks = 256;
+constexpr uint32_t kColChunks = 64;
 constexpr uint32_t kColBatch = 16;
+constexpr int kColGroups = 4;  // of kRxBins threads
+
+// Sum of rows [a, b) of the table's column d.
+__device__ __forceinline__ uint32_t col_sum(const uint32_t* __restrict__ tab, uint32_t a, uint32_t b, int d) {
+  uint32_t s = 0;
+  for (uint32_t t = a; t < b; t += kColBatch) {
+    uint32_t v[kColBatch];
+#pragma unroll
+    for (uint32_t i = 0; i < kColBatch; ++i) v[i] = t + i < b ? tab[size_t(t + i) * kRxBins + d] : 0u;
+#pragma unroll
+    for (uint32_t i = 0; i < kColBatch; ++i) s += v[i];
+  }
+  return s;
+}
+
+// Exclusive scan of one value per digit over the first kRxBins threads of the
+// block (ws: a word per wave of them); every thread of the block calls it.
+__device__ __forceinline__ uint32_t digit_excl_scan(uint32_t v, uint32_t* ws) {
+  const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
+  const uint32_t inc = wave_incl_scan(v);
+  if (lane == kWave - 1 && w < kRxBins / kWave) ws[w] = inc;
+  __syncthreads();
+  uint32_t base = inc - v;
+  if (w < kRxBins / kWave)
+    for (int i = 0; i < w; ++i) base += ws[i];
+  __syncthreads();
+  return base;
+}
 
 // part[c][d] = counts of digit d in the tiles of chunk c
 __global__ __launch_bounds__(kRxBins) void k_rx_colsum(const uint32_t* __restrict__ tab, uint32_t n_tiles,
-                                                       uint32_t ch, int nb, uint32_t* __restrict__ part) {
+                                                       uint32_t ch, int nb, uint32_t* __restrict__ part,
+                                                       const unsigned long long* __restrict__ check) {
+  if (in_order(check)) return;
   const uint32_t c = blockIdx.x;
   const int d = threadIdx.x;
   const uint32_t t0 = c * ch;
   const uint32_t t1 = t0 + ch < n_tiles ? t0 + ch : n_tiles;
-  uint32_t s = 0;
-  if (d < nb) {
-    for (uint32_t t = t0; t < t1; t += kColBatch) {
-      uint32_t v[kColBatch];
-#pragma unroll
-      for (uint32_t i = 0; i < kColBatch; ++i) v[i] = t + i < t1 ? tab[size_t(t + i) * kRxBins + d] : 0u;
-#pragma unroll
-      for (uint32_t i = 0; i < kColBatch; ++i) s += v[i];
-    }
-  }
-  part[size_t(c) * kRxBins + d] = s;
+  part[size_t(c) * kRxBins + d] = d < nb ? col_sum(tab, t0, t1, d) : 0u;
 }
 
-// One block: part[c][d] becomes the count of digit d in the chunks before c, and
-// row kColChunks the digit bases (counts of all smaller digits).
-__global__ __launch_bounds__(kRxBins) void k_rx_colscan(uint32_t* __restrict__ part, uint32_t n_chunks) {
+// tab[t][d] of chunk c becomes offs[t][d].  Every block sums the chunks' counts
+// itself, a quarter of them per group of kRxBins threads (one batch of loads), so
+// no launch of one block stands between the sums and their use.
+__global__ __launch_bounds__(kColGroups* kRxBins) void k_rx_colapply(uint32_t* __restrict__ tab, uint32_t n_tiles,
+                                                                      uint32_t ch, int nb, uint32_t n_chunks,
+                                                                      const uint32_t* __restrict__ part,
+                                                                      const unsigned long long* __restrict__ check) {
+  if (in_order(check)) return;
+  __shared__ uint32_t below[kColGroups][kRxBins];  // chunks before c
+  __shared__ uint32_t total[kColGroups][kRxBins];
+  __shared__ uint32_t run_of[kColGroups][kRxBins];  // tiles of the chunk before the group's
   __shared__ uint32_t ws[kRxBins / kWave];
-  const int d = threadIdx.x;
-  uint32_t run = 0;
-  for (uint32_t c = 0; c < n_chunks; c += kColBatch) {
-    uint32_t v[kColBatch];
-#pragma unroll
-    for (uint32_t i = 0; i < kColBatch; ++i) v[i] = c + i < n_chunks ? part[size_t(c + i) * kRxBins + d] : 0u;
-#pragma unroll
-    for (uint32_t i = 0; i < kColBatch; ++i) {
-      if (c + i < n_chunks) part[size_t(c + i) * kRxBins + d] = run;
-      run += v[i];
-    }
-  }
-  // digit bases: exclusive scan of the digit totals over the block
-  const uint32_t inc = wave_incl_scan(run);
-  const int lane = d & (kWave - 1), w = d / kWave;
-  if (lane == kWave - 1) ws[w] = inc;
-  __syncthreads();
-  uint32_t base = inc - run;
-  for (int i = 0; i < w; ++i) base += ws[i];
-  part[size_t(kColChunks) * kRxBins + d] = base;
-}
-
-// tab[t][d] becomes offs[t][d]
-__global__ __launch_bounds__(kRxBins) void k_rx_colapply(uint32_t* __restrict__ tab, uint32_t n_tiles,
-                                                         uint32_t ch, int nb, const uint32_t* __restrict__ part) {
   const uint32_t c = blockIdx.x;
-  const int d = threadIdx.x;
-  if (d >= nb) return;
+  const int d = int(threadIdx.x) % kRxBins, g = int(threadIdx.x) / kRxBins;
+  const uint32_t per = (n_chunks + kColGroups - 1) / kColGroups;
+  const uint32_t a = uint32_t(g) * per, b = a + per < n_chunks ? a + per : n_chunks;
+  const uint32_t lo = c < a ? a : (c < b ? c : b);  // [a, lo) lie before c
+  const uint32_t s0 = a < b ? col_sum(part, a, lo, d) : 0u;
+  below[g][d] = s0;
+  total[g][d] = a < b ? s0 + col_sum(part, lo, b, d) : 0u;
+  // the chunk's tiles, a quarter per group
   const uint32_t t0 = c * ch;
   const uint32_t t1 = t0 + ch < n_tiles ? t0 + ch : n_tiles;
-  uint32_t run = part[size_t(c) * kRxBins + d] + part[size_t(kColChunks) * kRxBins + d];
-  for (uint32_t t = t0; t < t1; t += kColBatch) {
+  const uint32_t pt = (t1 - t0 + kColGroups - 1) / kColGroups;
+  const uint32_t ta = t0 + uint32_t(g) * pt < t1 ? t0 + uint32_t(g) * pt : t1;
+  const uint32_t tb = ta + pt < t1 ? ta + pt : t1;
+  run_of[g][d] = d < nb ? col_sum(tab, ta, tb, d) : 0u;
+  __syncthreads();
+  uint32_t all = 0, run = 0;
+#pragma unroll
+  for (int q = 0; q < kColGroups; ++q) {
+    all += total[q][d];
+    run += below[q][d];
+    if (q < g) run += run_of[q][d];
+  }
+  const uint32_t base = digit_excl_scan(all, ws);  // of group 0's threads
+  if (g == 0) below[0][d] = base;
+  __syncthreads();
+  if (d >= nb) return;
+  run += below[0][d];
+  for (uint32_t t = ta; t < tb; t += kColBatch) {
     uint32_t v[kColBatch];
 #pragma unroll
-    for (uint32_t i = 0; i < kColBatch; ++i) v[i] = t + i < t1 ? tab[size_t(t + i) * kRxBins + d] : 0u;
+    for (uint32_t i = 0; i < kColBatch; ++i) v[i] = t + i < tb ? tab[size_t(t + i) * kRxBins + d] : 0u;
 #pragma unroll
     for (uint32_t i = 0; i < kColBatch; ++i) {
-      if (t + i < t1) tab[size_t(t + i) * kRxBins + d] = run;
+      if (t + i < tb) tab[size_t(t + i) * kRxBins + d] = run;
       run += v[i];
     }
   }
 }
 
-// Stable scatter of one tile by one digit; offs = [tile][digit] offset table.
+// Stable scatter of one tile by one digit; offs = [tile][digit] offset table, or
+// (direct) the tiles' histograms, from which the block sums its row, with the sums
+// of the chunks of ch tiles where part is given.
 // vin == null stands for the identity (pass 0).  Payload: three planes of T
 // (positions) that travel with the keys, pin (stride si) in the input order,
 // pout (stride so) in the output order; null = none.  Keys, values and each
 // payload plane are read in input order (coalesced), placed in LDS at their
 // staged slot, and written out in staged order: runs of one digit each.
-template <class T>
+template <class T, int kIters>
 __global__ __launch_bounds__(kRxBlock) void k_rx_scatter(const uint32_t* __restrict__ kin,
                                                          const uint32_t* __restrict__ vin, uint32_t n_host,
                                                          const uint32_t* __restrict__ n_dev, int shift,
@@ -267,7 +333,12 @@ __global__ __launch_bounds__(kRxBlock) void k_rx_scatter(const uint32_t* __restr
                                                          uint32_t* __restrict__ kout,
                                                          uint32_t* __restrict__ vout, const T* __restrict__ pin,
                                                          size_t si, T* __restrict__ pout, size_t so,
-                                                         const unsigned long long* __restrict__ disorder) {
+                                                         const unsigned long long* __restrict__ disorder,
+                                                         const unsigned long long* __restrict__ check,
+                                                         int direct, const uint32_t* __restrict__ part,
+                                                         uint32_t ch, uint32_t n_chunks) {
+  if (in_order(check)) return;
+  constexpr uint32_t kRxTile = uint32_t(kRxBlock * kIters);
   __shared__ uint32_t wh[kRxWaves][kRxBins];  // running count per wave, then wave prefix
   __shared__ uint32_t tstart[kRxBins];        // first staged slot of each digit
   __shared__ uint32_t goff[kRxBins];          // first output slot of each digit
@@ -284,16 +355,33 @@ __global__ __launch_bounds__(kRxBlock) void k_rx_scatter(const uint32_t* __restr
   for (int d = threadIdx.x; d < kRxBins; d += kRxBlock) {
 #pragma unroll
     for (int w = 0; w < kRxWaves; ++w) wh[w][d] = 0;
-    goff[d] = d < nb ? offs[size_t(t) * kRxBins + d] : 0u;
+    if (!direct) goff[d] = d < nb ? offs[size_t(t) * kRxBins + d] : 0u;
+  }
+  if (direct) {
+    const int d = threadIdx.x;
+    static_assert(kRxBlock == kRxBins, "a thread per digit");
+    const uint32_t c = t / ch;
+    uint32_t before = 0, all = 0;
+    if (d < nb) {
+      if (part) {
+        before = col_sum(part, 0, c, d);
+        all = before + col_sum(part, c, n_chunks, d);
+        before += col_sum(offs, c * ch, t, d);
+      } else {
+        before = col_sum(offs, 0, t, d);
+        all = before + col_sum(offs, t, n_tiles, d);
+      }
+    }
+    goff[d] = digit_excl_scan(all, wsum) + before;
   }
   __syncthreads();
   const int lane = threadIdx.x & (kWave - 1);
   const int w = threadIdx.x / kWave;
-  const uint64_t base = tile0 + uint64_t(w) * (kRxIters * kWave);
-  uint32_t key[kRxIters], lr[kRxIters], val[kRxIters];
+  const uint64_t base = tile0 + uint64_t(w) * (kIters * kWave);
+  uint32_t key[kIters], lr[kIters], val[kIters];
   // all loads of the wave's rounds first
 #pragma unroll
-  for (int it = 0; it < kRxIters; ++it) {
+  for (int it = 0; it < kIters; ++it) {
     const uint64_t e = base + uint64_t(it) * kWave + uint64_t(lane);
     key[it] = 0u;
     val[it] = uint32_t(e);
@@ -303,7 +391,7 @@ __global__ __launch_bounds__(kRxBlock) void k_rx_scatter(const uint32_t* __restr
     }
   }
 #pragma unroll
-  for (int it = 0; it < kRxIters; ++it) {
+  for (int it = 0; it < kIters; ++it) {
     const uint64_t e = base + uint64_t(it) * kWave + uint64_t(lane);
     const bool v = e < n;
     const unsigned long long act = __ballot(v);
@@ -348,7 +436,7 @@ __global__ __launch_bounds__(kRxBlock) void k_rx_scatter(const uint32_t* __restr
   __syncthreads();
   // lr[it] becomes the staged slot of element it
 #pragma unroll
-  for (int it = 0; it < kRxIters; ++it) {
+  for (int it = 0; it < kIters; ++it) {
     const uint64_t e = base + uint64_t(it) * kWave + uint64_t(lane);
     if (e < n) {
       const uint32_t d = (key[it] >> shift) & mask;
@@ -376,7 +464,7 @@ __global__ __launch_bounds__(kRxBlock) void k_rx_scatter(const uint32_t* __restr
   for (int q = 0; q < 3; ++q) {
     __syncthreads();  // sv / the previous plane has been read
 #pragma unroll
-    for (int it = 0; it < kRxIters; ++it) {
+    for (int it = 0; it < kIters; ++it) {
       const uint64_t e = base + uint64_t(it) * kWave + uint64_t(lane);
       if (e < n) sp[lr[it]] = pin[size_t(q) * si + e];
     }
@@ -394,18 +482,18 @@ __global__ __launch_bounds__(kRxBlock) void k_rx_scatter(const uint32_t* __restr
 // wave into run segments, whose lengths and domain counts are bit counts.  A
 // segment that is a whole run is stored; the pieces of a run that crosses a
 // wave boundary are added atomically.  One coalesced read of keys and
-// sort_to_nonsort; empty cells keep 0.  A wave takes kRunRounds rounds of 64
+// sort_to_nonsort; empty cells keep 0.  A wave takes kRounds rounds of 64
 // slots with all loads issued first (the work per slot is a few bit operations,
 // so the loads' latency is what there is to hide).
-constexpr int kRunRounds = 16;
 
-// The runs of one wave's kRunRounds rounds of 64 consecutive sorted slots from
+// The runs of one wave's kRounds rounds of 64 consecutive sorted slots from
 // w0: kk = keys, kp = the previous slot's key, dmf = domain particle.  The run
 // that reaches the end of a round is carried (wave-uniform) into the next
 // round: only a run that crosses the wave's first or last slot is added
 // atomically, every other run is stored once.
-__device__ __forceinline__ void runs_of_wave(const uint32_t (&kk)[kRunRounds], const uint32_t (&kp)[kRunRounds],
-                                             const bool (&dmf)[kRunRounds], uint64_t w0, uint32_t n,
+template <int kRounds>
+__device__ __forceinline__ void runs_of_wave(const uint32_t (&kk)[kRounds], const uint32_t (&kp)[kRounds],
+                                             const bool (&dmf)[kRounds], uint64_t w0, uint32_t n,
                                              uint64_t n_cells, unsigned long long* __restrict__ packed) {
   const int lane = threadIdx.x & (kWave - 1);
   uint32_t ck = 0;              // carried run: key,
@@ -427,7 +515,7 @@ __device__ __forceinline__ void runs_of_wave(const uint32_t (&kk)[kRunRounds], c
     copen = false;
   };
 #pragma unroll
-  for (int r = 0; r < kRunRounds; ++r) {
+  for (int r = 0; r < kRounds; ++r) {
     const uint64_t f = w0 + uint64_t(r) * kWave + uint64_t(lane);
     const bool v = f < n;
     const uint32_t k = kk[r];
@@ -483,20 +571,23 @@ __device__ __forceinline__ void runs_of_wave(const uint32_t (&kk)[kRunRounds], c
 // per round; ballots of "a run of equal keys starts here" and "domain particle"
 // split the wave into run segments, whose lengths and domain counts are bit
 // counts (runs_of_wave).  One coalesced read of keys and sort_to_nonsort; empty
-// cells keep 0.  All loads of the wave's kRunRounds rounds are issued first
+// cells keep 0.  All loads of the wave's kRounds rounds are issued first
 // (the work per slot is a few bit operations, so the loads' latency is what
 // there is to hide).
+template <int kRounds>
 __global__ __launch_bounds__(256) void k_cl_runs(const uint32_t* __restrict__ keys,
                                                  const uint32_t* __restrict__ s2n, uint32_t n_host,
                                                  const uint32_t* __restrict__ n_dev, uint32_t gm,
-                                                 uint64_t n_cells, unsigned long long* __restrict__ packed) {
+                                                 uint64_t n_cells, unsigned long long* __restrict__ packed,
+                                                 const unsigned long long* __restrict__ check) {
+  if (in_order(check)) return;
   const int lane = threadIdx.x & (kWave - 1);
-  const uint64_t w0 = (uint64_t(blockIdx.x) * (blockDim.x / kWave) + threadIdx.x / kWave) * (kRunRounds * kWave);
+  const uint64_t w0 = (uint64_t(blockIdx.x) * (blockDim.x / kWave) + threadIdx.x / kWave) * (kRounds * kWave);
   const uint32_t n = count_of(n_host, n_dev);
-  uint32_t kk[kRunRounds], kp[kRunRounds];
-  bool dm[kRunRounds];
+  uint32_t kk[kRounds], kp[kRounds];
+  bool dm[kRounds];
 #pragma unroll
-  for (int r = 0; r < kRunRounds; ++r) {
+  for (int r = 0; r < kRounds; ++r) {
     const uint64_t f = w0 + uint64_t(r) * kWave + uint64_t(lane);
     kk[r] = 0u;
     kp[r] = ~0u;
@@ -507,7 +598,7 @@ __global__ __launch_bounds__(256) void k_cl_runs(const uint32_t* __restrict__ ke
       if (f > 0) kp[r] = keys[f - 1];
     }
   }
-  runs_of_wave(kk, kp, dm, w0, n, n_cells, packed);
+  runs_of_wave<kRounds>(kk, kp, dm, w0, n, n_cells, packed);
 }
 
 template <class T>
@@ -577,7 +668,9 @@ template <class T>
 __global__ __launch_bounds__(256) void k_cl_emit(EmitArgs<T> A, const uint32_t* __restrict__ keys,
                                                  const uint32_t* __restrict__ s2n, uint32_t n_host,
                                                  const uint32_t* __restrict__ n_dev,
-                                                 const unsigned long long* __restrict__ cs) {
+                                                 const unsigned long long* __restrict__ cs,
+                                                 const unsigned long long* __restrict__ check) {
+  if (in_order(check)) return;
   const uint32_t f = blockIdx.x * blockDim.x + threadIdx.x;
   const uint32_t n = count_of(n_host, n_dev);
   if (f >= n) return;
@@ -588,7 +681,7 @@ __global__ __launch_bounds__(256) void k_cl_emit(EmitArgs<T> A, const uint32_t* 
 }
 
 // The build of input already in cell order, speculatively, with the check of
-// that order.  Per tile of kRxTile particles: the cell keys and the descents
+// that order.  Per tile of 256 kIters particles: the cell keys and the descents
 // k[f-1] > k[f] (the key before a wave's first slot recomputed from its
 // position), added to *disorder.  A tile without descents writes what the
 // build gives for its particles when the whole input is in cell order: the
@@ -597,25 +690,25 @@ __global__ __launch_bounds__(256) void k_cl_emit(EmitArgs<T> A, const uint32_t* 
 // packed (cleared before).  If *disorder ends at zero these are the build's
 // results; otherwise the radix passes (from the positions: neither keys nor
 // histograms are kept here) and k_cl_emit overwrite every one of them.
-template <class T>
+template <class T, int kIters>
 __global__ __launch_bounds__(kRxBlock) void k_cl_first(CellGeom<T> g, EmitArgs<T> A, uint32_t n,
                                                        uint32_t* __restrict__ s2n,
                                                        unsigned long long* __restrict__ disorder,
                                                        unsigned long long* __restrict__ packed, uint64_t n_cells) {
-  static_assert(kRunRounds == kRxIters, "one wave's rounds are its run rounds");
+  constexpr uint32_t kRxTile = uint32_t(kRxBlock * kIters);
   __shared__ uint32_t wdesc[kRxWaves];
   const uint32_t t = blockIdx.x;
   const int lane = threadIdx.x & (kWave - 1);
   const int w = threadIdx.x / kWave;
-  const uint64_t base = uint64_t(t) * kRxTile + uint64_t(w) * (kRxIters * kWave);
+  const uint64_t base = uint64_t(t) * kRxTile + uint64_t(w) * (kIters * kWave);
   const T* pos = A.pos;
   const size_t st = A.stride;
-  uint32_t kk[kRxIters], kp[kRxIters];
+  uint32_t kk[kIters], kp[kIters];
   // keys, four rounds' loads at a time; the positions stay in registers for
   // the identity build below (read once from memory)
-  T x[kRxIters], y[kRxIters], z[kRxIters];
+  T x[kIters], y[kIters], z[kIters];
 #pragma unroll
-  for (int b = 0; b < kRxIters; b += 4) {
+  for (int b = 0; b < kIters; b += 4) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const uint64_t e = base + uint64_t(b + i) * kWave + uint64_t(lane);
@@ -642,7 +735,7 @@ __global__ __launch_bounds__(kRxBlock) void k_cl_first(CellGeom<T> g, EmitArgs<T
   }
   uint32_t desc = 0;
 #pragma unroll
-  for (int r = 0; r < kRxIters; ++r) {
+  for (int r = 0; r < kIters; ++r) {
     const uint64_t e = base + uint64_t(r) * kWave + uint64_t(lane);
     const uint32_t up = __shfl_up(kk[r], 1, kWave);
     const uint32_t prev_last = r == 0 ? before : uint32_t(__builtin_amdgcn_readlane(int(kk[r - 1]), kWave - 1));
@@ -657,9 +750,9 @@ __global__ __launch_bounds__(kRxBlock) void k_cl_first(CellGeom<T> g, EmitArgs<T
   if (threadIdx.x == 0 && tile_desc) atomicAdd(disorder, static_cast<unsigned long long>(tile_desc));
   if (tile_desc != 0) return;  // block-uniform
   // the identity build of this tile
-  bool dm[kRxIters];
+  bool dm[kIters];
 #pragma unroll
-  for (int r = 0; r < kRxIters; ++r) {
+  for (int r = 0; r < kIters; ++r) {
     const uint64_t e = base + uint64_t(r) * kWave + uint64_t(lane);
     dm[r] = e < A.gm;
     if (e >= n) continue;
@@ -680,7 +773,7 @@ __global__ __launch_bounds__(kRxBlock) void k_cl_first(CellGeom<T> g, EmitArgs<T
     }
     copy_planes(A.pa, f, f);
   }
-  runs_of_wave(kk, kp, dm, base, n, n_cells, packed);
+  runs_of_wave<kIters>(kk, kp, dm, base, n, n_cells, packed);
 }
 
 // out[j] = in[s2n[j]] (gather into sorted order)
@@ -699,6 +792,13 @@ __global__ __launch_bounds__(256) void k_cl_restore(uint32_t n, const uint32_t* 
   copy_planes(pa, j, s2n[j]);
 }
 
+// p[0 .. n) = 0 unless the order check found the input in cell order.
+__global__ __launch_bounds__(256) void k_clear_unless(unsigned long long* __restrict__ p, uint64_t n,
+                                                      const unsigned long long* __restrict__ check) {
+  if (in_order(check)) return;
+  for (uint64_t i = uint64_t(blockIdx.x) * 256 + threadIdx.x; i < n; i += uint64_t(gridDim.x) * 256) p[i] = 0ull;
+}
+
 // Digit widths of the radix passes for keys < n_cells: as few passes of at most
 // 8 bits as cover the key, widths as even as possible.
 static int radix_plan(uint64_t n_cells, int* widths) {
@@ -711,25 +811,32 @@ static int radix_plan(uint64_t n_cells, int* widths) {
 
 // n_cap: particles the buffers hold (the count itself is n_host or *n_dev).
 // g1 (one grid, count on the host): k_cl_first first checks the input's order
-// while writing the build of ordered input; the host reads its descent count
-// (one scalar) and, for input already in cell order, the build ends with the
-// scan of the cell counts it wrote; otherwise the radix build follows.
+// while writing the build of ordered input; for input already in cell order the
+// build ends with the scan of the cell counts it wrote, otherwise the radix build
+// follows (see kRxNoSync for how the two are told apart).
 // Ensembles (g1 null) keep every step on the device (their rebuilds are
 // captured in graphs).
-template <class T, class Key>
-static int cl_build(ofp_cl* h, const Key& key, const EmitArgs<T>& A0, size_t n_cap, uint32_t n_host,
-                    const uint32_t* n_dev, size_t gm, hipStream_t s, const CellGeom<T>* g1 = nullptr) {
+template <class T, int kIters, class Key>
+static int cl_build_t(ofp_cl* h, const Key& key, const EmitArgs<T>& A0, size_t n_cap, uint32_t n_host,
+                      const uint32_t* n_dev, size_t gm, hipStream_t s, const CellGeom<T>* g1) {
+  constexpr uint32_t kRxTile = uint32_t(kRxBlock * kIters);
   const uint64_t C = h->n_cells;
   const uint32_t n_tiles = uint32_t((n_cap + kRxTile - 1) / kRxTile);
   const size_t hist_n = size_t(kRxBins) * (n_tiles ? n_tiles : 1);
-  OFP_TRY(h->packed.ensure(C * 8));
+  int widths[4];
+  const int passes = radix_plan(C, widths);
+  // the descents counted and the chunks' sums lie behind the cells' counts, cleared
+  // with them
+  const int direct = n_tiles <= kRxChunked ? 1 : 0;
+  const bool chunked = direct && n_tiles > kRxDirect;
+  // the [tile][digit] table in at most kColChunks chunks of ch tiles
+  const uint32_t ch = std::max((n_tiles + kColChunks - 1) / kColChunks, kColBatch);
+  const uint32_t n_chunks = (n_tiles + ch - 1) / ch;
+  const uint64_t n_clear = C + 1 + (chunked ? uint64_t(passes) * n_chunks * (kRxBins / 2) : 0);
+  OFP_TRY(h->packed.ensure(n_clear * 8));
   OFP_TRY(h->scan64.ensure((C + 1) * 8));
   OFP_TRY(h->scantmp.ensure(scan_tmp_bytes(C)));
-  OFP_TRY(h->colpart.ensure(size_t(kColChunks + 1) * kRxBins * 4));
-  // the [tile][digit] table in chunks of ch tiles
-  const uint32_t ch = n_tiles ? (n_tiles + kColChunks - 1) / kColChunks : 1;
-  const uint32_t n_chunks = (n_tiles + ch - 1) / ch;
-  uint32_t* part = h->colpart.as<uint32_t>();
+  if (!direct) OFP_TRY(h->colpart.ensure(size_t(kColChunks) * kRxBins * 4));
   OFP_TRY(h->keys.ensure((n_cap + 1) * 4));
   OFP_TRY(h->keys2.ensure((n_cap + 1) * 4));
   OFP_TRY(h->s2n.ensure((n_cap + 1) * 4));
@@ -741,29 +848,24 @@ static int cl_build(ofp_cl* h, const Key& key, const EmitArgs<T>& A0, size_t n_c
   if (want_quant) OFP_TRY(h->quant.ensure((n_cap + 1) * 16));
   if (h->n_sys) OFP_TRY(h->sid_sorted.ensure((n_cap + 1) * 4));
 
-  int widths[4];
-  const int passes = radix_plan(C, widths);
   // With sorted positions requested they may travel with the keys as a payload
   // (the passes before the last alternate between two payload buffers, the last
-  // one writes the sorted positions); the kernels carry them only when pass 0
-  // finds the input far from cell order (carry_positions), else k_cl_emit
-  // gathers them.
+  // one writes the sorted positions); the kernels carry them only when the
+  // descents say the input is far from cell order (carry_positions), else
+  // k_cl_emit gathers them.
   const bool payload = A0.pos_sorted != nullptr;
   if (payload && passes > 1) OFP_TRY(h->payload.ensure(2 * 3 * n_cap * sizeof(T)));
   T* pbuf[2] = {h->payload.as<T>(), h->payload.as<T>() + 3 * n_cap};
-  OFP_TRY(h->ctl.ensure(sizeof(unsigned long long)));
-  auto* disorder = h->ctl.as<unsigned long long>();
   // ping-pong buffers chosen so that the last pass lands in keys / s2n
   uint32_t* kbuf[2] = {h->keys.as<uint32_t>(), h->keys2.as<uint32_t>()};
   uint32_t* vbuf[2] = {h->s2n.as<uint32_t>(), h->vals2.as<uint32_t>()};
   uint32_t* hist = h->hist.as<uint32_t>();
-  OFP_TRY(fill_u64(reinterpret_cast<uint64_t*>(disorder), 0, 1, s));
   auto* packed = h->packed.as<unsigned long long>();
+  auto* disorder = packed + C;
   auto* cs = h->scan64.as<unsigned long long>();
-  const bool want_quant_ = want_quant;
   auto emit_args = [&]() {
     EmitArgs<T> A = A0;
-    A.quant = want_quant_ ? h->quant.as<int4>() : nullptr;
+    A.quant = want_quant ? h->quant.as<int4>() : nullptr;
     A.gm = uint32_t(gm);
     A.n2s = h->n2s.as<uint32_t>();
     A.dom = h->dom.as<uint32_t>();
@@ -771,7 +873,9 @@ static int cl_build(ofp_cl* h, const Key& key, const EmitArgs<T>& A0, size_t n_c
     A.disorder = payload ? disorder : nullptr;
     return A;
   };
-  auto finish = [&]() {
+  auto scan_and_finish = [&]() -> int {
+    OFP_TRY(scan_excl_u64(reinterpret_cast<const uint64_t*>(packed), reinterpret_cast<uint64_t*>(cs), C,
+                          h->scantmp.p, s));
     h->n_part = n_dev ? n_cap : n_host;
     h->gm = gm;
     h->n_dev = n_dev;
@@ -780,79 +884,88 @@ static int cl_build(ofp_cl* h, const Key& key, const EmitArgs<T>& A0, size_t n_c
     h->items_valid = false;
     return OFP_OK;
   };
-  const bool first_fused = g1 != nullptr && n_dev == nullptr && n_tiles > 0;
-  if (first_fused) {
-    OFP_TRY(fill_u64(reinterpret_cast<uint64_t*>(packed), 0, C, s));
-    k_cl_first<T><<<n_tiles, kRxBlock, 0, s>>>(*g1, emit_args(), n_host, vbuf[0], disorder, packed, C);
-    OFP_LAUNCHED();
-    unsigned long long desc = 0;
-    OFP_HIP(hipMemcpyAsync(&desc, disorder, sizeof(desc), hipMemcpyDeviceToHost, s));
-    OFP_HIP(hipStreamSynchronize(s));
-    if (desc == 0) {  // input in cell order: every tile wrote its identity build
-      OFP_TRY(scan_excl_u64(reinterpret_cast<const uint64_t*>(packed), reinterpret_cast<uint64_t*>(cs), C,
-                            h->scantmp.p, s));
-      return finish();
-    }
-    // not in cell order: the radix build from the positions (its pass 0
-    // counts the descents again)
-    OFP_TRY(fill_u64(reinterpret_cast<uint64_t*>(disorder), 0, 1, s));
+  const bool first = g1 != nullptr && n_dev == nullptr;
+  if (first) {  // a build of a count on the host is none for a graph: the count and the buffers are this call's
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    OFP_HIP(hipStreamIsCapturing(s, &cap));
+    if (cap != hipStreamCaptureStatusNone) OFP_HIP(hipErrorStreamCaptureUnsupported);
   }
-  if (n_tiles > 0) {
-    uint32_t* kin = kbuf[passes % 2];  // pass-0 keys
-    const uint32_t* vin = nullptr;
-    const T* pin = payload ? A0.pos : nullptr;
-    size_t si = A0.stride;
-    int shift = 0;
-    for (int p = 0; p < passes; ++p) {
-      const int bits = widths[p];
-      uint32_t* kout = kbuf[(passes - 1 - p) % 2];
-      uint32_t* vout = vbuf[(passes - 1 - p) % 2];
-      T* pout = nullptr;
-      size_t so = 0;
-      if (payload) {
-        const bool last = p == passes - 1;
-        pout = last ? A0.pos_sorted : pbuf[p % 2];
-        so = last ? A0.sorted_stride : n_cap;
-      }
-      if (p == 0) {
-        k_rx_hist<Key><<<n_tiles, kRxBlock, 0, s>>>(key, nullptr, kin, n_host, n_dev, shift, bits, n_tiles, hist,
-                                                    disorder);
-        OFP_LAUNCHED();
-      } else {
-        k_rx_hist<Key><<<n_tiles, kRxBlock, 0, s>>>(key, kin, nullptr, n_host, n_dev, shift, bits, n_tiles, hist,
-                                                    nullptr);
-        OFP_LAUNCHED();
-      }
-      k_rx_colsum<<<n_chunks, kRxBins, 0, s>>>(hist, n_tiles, ch, 1 << bits, part);
-      OFP_LAUNCHED();
-      k_rx_colscan<<<1, kRxBins, 0, s>>>(part, n_chunks);
-      OFP_LAUNCHED();
-      k_rx_colapply<<<n_chunks, kRxBins, 0, s>>>(hist, n_tiles, ch, 1 << bits, part);
-      OFP_LAUNCHED();
-      k_rx_scatter<T><<<n_tiles, kRxBlock, 0, s>>>(kin, vin, n_host, n_dev, shift, bits, n_tiles, hist, kout, vout,
-                                                   pin, si, pout, so, disorder);
-      OFP_LAUNCHED();
-      kin = kout;
-      vin = vout;
-      pin = pout;
-      si = so;
-      shift += bits;
+  OFP_TRY(fill_u64(reinterpret_cast<uint64_t*>(packed), 0, n_clear, s));
+  if (n_tiles == 0) return scan_and_finish();
+  const unsigned long long* check = nullptr;  // the kernels below return if *check == 0
+  if (first) {
+    k_cl_first<T, kIters><<<n_tiles, kRxBlock, 0, s>>>(*g1, emit_args(), n_host, vbuf[0], disorder, packed, C);
+    OFP_LAUNCHED();
+    if (n_cap < kRxNoSync) {
+      check = disorder;
+    } else {
+      unsigned long long desc = 0;
+      OFP_HIP(hipMemcpyAsync(&desc, disorder, sizeof(desc), hipMemcpyDeviceToHost, s));
+      OFP_HIP(hipStreamSynchronize(s));
+      if (desc == 0) return scan_and_finish();  // every tile wrote its identity build
     }
   }
-  OFP_TRY(fill_u64(reinterpret_cast<uint64_t*>(packed), 0, C, s));
-  if (n_tiles > 0) {
-    k_cl_runs<<<grid_for(n_cap, 256 * kRunRounds), 256, 0, s>>>(h->keys.as<uint32_t>(), h->s2n.as<uint32_t>(),
-                                                                n_host, n_dev, uint32_t(gm), C, packed);
+  uint32_t* kin = kbuf[passes % 2];  // pass-0 keys
+  const uint32_t* vin = nullptr;
+  const T* pin = payload ? A0.pos : nullptr;
+  size_t si = A0.stride;
+  int shift = 0;
+  // pass 0 clears the counts that the order check's tiles wrote; many more cells
+  // than particles are left to a launch of their own
+  const bool clear_in_hist = first && C <= 16 * n_cap;
+  if (first && !clear_in_hist) {
+    k_clear_unless<<<2048, 256, 0, s>>>(packed, C, check);
     OFP_LAUNCHED();
   }
-  OFP_TRY(scan_excl_u64(reinterpret_cast<const uint64_t*>(packed), reinterpret_cast<uint64_t*>(cs), C,
-                        h->scantmp.p, s));
-  if (n_tiles > 0) {
-    k_cl_emit<T><<<grid_for(n_cap, 256), 256, 0, s>>>(emit_args(), h->keys.as<uint32_t>(), h->s2n.as<uint32_t>(),
-                                                       n_host, n_dev, cs);
+  for (int p = 0; p < passes; ++p) {
+    const int bits = widths[p];
+    uint32_t* kout = kbuf[(passes - 1 - p) % 2];
+    uint32_t* vout = vbuf[(passes - 1 - p) % 2];
+    T* pout = nullptr;
+    size_t so = 0;
+    if (payload) {
+      const bool last = p == passes - 1;
+      pout = last ? A0.pos_sorted : pbuf[p % 2];
+      so = last ? A0.sorted_stride : n_cap;
+    }
+    uint32_t* part = chunked ? reinterpret_cast<uint32_t*>(packed + C + 1) + size_t(p) * n_chunks * kRxBins
+                             : h->colpart.as<uint32_t>();
+    k_rx_hist<Key, kIters><<<n_tiles, kRxBlock, 0, s>>>(
+        key, p ? kin : nullptr, p ? nullptr : kin, n_host, n_dev, shift, bits, n_tiles, hist,
+        p || first ? nullptr : disorder, check, p == 0 && clear_in_hist ? packed : nullptr, C,
+        chunked ? part : nullptr, ch);
     OFP_LAUNCHED();
+    if (!direct) {
+      k_rx_colsum<<<n_chunks, kRxBins, 0, s>>>(hist, n_tiles, ch, 1 << bits, part, check);
+      OFP_LAUNCHED();
+      k_rx_colapply<<<n_chunks, kColGroups * kRxBins, 0, s>>>(hist, n_tiles, ch, 1 << bits, n_chunks, part, check);
+      OFP_LAUNCHED();
+    }
+    k_rx_scatter<T, kIters><<<n_tiles, kRxBlock, 0, s>>>(kin, vin, n_host, n_dev, shift, bits, n_tiles, hist, kout,
+                                                         vout, pin, si, pout, so, disorder, check, direct,
+                                                         chunked ? part : nullptr, ch, n_chunks);
+    OFP_LAUNCHED();
+    kin = kout;
+    vin = vout;
+    pin = pout;
+    si = so;
+    shift += bits;
   }
-  return finish();
+  k_cl_runs<kIters><<<grid_for(n_cap, 256 * kIters), 256, 0, s>>>(h->keys.as<uint32_t>(), h->s2n.as<uint32_t>(),
+                                                                  n_host, n_dev, uint32_t(gm), C, packed, check);
+  OFP_LAUNCHED();
+  OFP_TRY(scan_and_finish());
+  k_cl_emit<T><<<grid_for(n_cap, 256), 256, 0, s>>>(emit_args(), h->keys.as<uint32_t>(), h->s2n.as<uint32_t>(),
+                                                     n_host, n_dev, cs, check);
+  OFP_LAUNCHED();
+  return OFP_OK;
+}
+
+template <class T, class Key>
+static int cl_build(ofp_cl* h, const Key& key, const EmitArgs<T>& A0, size_t n_cap, uint32_t n_host,
+                    const uint32_t* n_dev, size_t gm, hipStream_t s, const CellGeom<T>* g1 = nullptr) {
+  if (n_cap < kRxSmall) return cl_build_t<T, kRxShort>(h, key, A0, n_cap, n_host, n_dev, gm, s, g1);
+  return cl_build_t<T, kRxLong>(h, key, A0, n_cap, n_host, n_dev, gm, s, g1);
 }
 
 template <class T>
@@ -1130,7 +1243,7 @@ int ofp_cl_destroy(ofp_cl* h) {
   if (!h) return OFP_OK;
   DevBuf* bufs[] = {&h->packed, &h->scan64, &h->keys,    &h->keys2, &h->s2n,        &h->vals2, &h->n2s,
                     &h->dom,    &h->quant,  &h->scantmp, &h->hist,  &h->sid_sorted, &h->items, &h->nitems,
-                    &h->payload, &h->ctl, &h->colpart, &h->nz_flag, &h->nz_key, &h->nz_start, &h->nz_nn,
+                    &h->payload, &h->colpart, &h->nz_flag, &h->nz_key, &h->nz_start, &h->nz_nn,
                     &h->nz_inv, &h->aux};
   for (DevBuf* b : bufs) b->release();
   delete h;
