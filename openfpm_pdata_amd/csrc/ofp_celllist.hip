@@ -24,6 +24,9 @@
 //                    word) and domain-id starts (high word).
 //   6. k_cl_emit     per sorted slot: nonsort_to_sort, domain sort ids, reordered
 //                    positions and planes, and the quantised cell-relative stream.
+//                    From 2^22 particles far from cell order, nonsort_to_sort and
+//                    the planes go by ranges of destinations (permute_far), as
+//                    restores and reorders then do.
 // The particle count may be read from device memory (ensembles whose ghost count
 // stays on the device): every kernel is launched for the capacity and returns
 // past the count.
@@ -33,6 +36,7 @@
 #include <cmath>
 #include <cstddef>
 #include <cstring>
+#include <mutex>
 
 struct ofp_cl {
   ofp::HandleLife life;
@@ -58,6 +62,16 @@ struct ofp_cl {
   size_t items_cap = 0;
   ofp::DevBuf packed, scan64, keys, keys2, s2n, vals2, n2s, dom, quant, scantmp, hist, sid_sorted, payload;
   ofp::DevBuf colpart;  // chunk sums of the histogram table
+  // the last construct's particles were many and far from cell order, and there is
+  // scratch for permute_far (payload, cursors).  It serves one call after another:
+  // restores and reorders may come from several threads and streams
+  bool far = false;
+  ofp::DevBuf cursors;
+  mutable std::mutex far_lock;
+  hipEvent_t far_done = nullptr;
+  // the order check's result on the host (pinned) and its event
+  unsigned long long* desc = nullptr;
+  hipEvent_t checked = nullptr;
   ofp::DevBuf items, nitems;  // nitems: the consumers' queue heads (kQueueWords), then the item count
   ofp::DevBuf aux;            // pair kernels' per-particle record stream (cell tiles)
   // sparse view (ofp_cl_build_sparse): non-empty cells only
@@ -86,12 +100,11 @@ constexpr int kRxMaxBits = 8;
 // over 100 rows of 1 KB for its 4096 keys.
 constexpr uint32_t kRxDirect = 32;
 constexpr uint32_t kRxChunked = 2048;
-// Below this many particles nothing is read back between the order check and the
-// passes: the passes' kernels return at once if the check found the input in cell
-// order.  Whole builds with and without the read-back (us): input in order 47 and
-// 53 at 17,000 particles, 70 and 64 at 2^20, 133 and 134 at 8e6; one exchanged pair
-// 81 and 62, 186 and 163, 438 and 417.  From here on the empty grids cost more than
-// the read-back.
+// Below this many particles the host does not wait for the order check before it
+// launches the passes: their kernels return at once if the check found the input in
+// cell order.  Whole builds with and without the wait (us): input in order 47 and 53
+// at 17,000 particles, 70 and 64 at 2^20, 133 and 134 at 8e6; one exchanged pair 81
+// and 62, 186 and 163, 438 and 417.  From here on the empty grids cost more.
 constexpr size_t kRxNoSync = size_t(1) << 23;
 constexpr int kRxBins = 1 << kRxMaxBits;
 
@@ -625,7 +638,7 @@ struct EmitArgs {
 template <class T>
 __device__ __forceinline__ void cl_emit(const EmitArgs<T>& A, uint32_t o, uint32_t f, uint32_t c,
                                         uint32_t dstart, uint32_t rank, bool pos_done) {
-  A.n2s[o] = f;
+  if (A.n2s) A.n2s[o] = f;  // else by permute_far
   if (o < A.gm) A.dom[dstart + rank] = f;
   uint32_t s = 0;
   if (A.sys) {
@@ -776,6 +789,210 @@ __global__ __launch_bounds__(kRxBlock) void k_cl_first(CellGeom<T> g, EmitArgs<T
   runs_of_wave<kIters>(kk, kp, dm, base, n, n_cells, packed);
 }
 
+// out[idx[j]] = in[j] for a permutation idx whose neighbours lie far apart, in two
+// steps.  A plain scatter over a plane much larger than the L2 (4 MB per XCD) writes
+// each value as a piece of a line of its own, 70e9 values/s.  Here the destinations
+// are cut into ranges of 32768, each as large as a block's LDS:
+//   k_far_stage  brings a tile of 32768 values into the order of their ranges in LDS
+//                and appends them, with their places in the range, to the ranges'
+//                parts of the scratch planes (2^25 values: runs of 32);
+//   k_far_place  brings a range's values into order in LDS and writes them out.
+// Each part is exactly as long as its range (idx is a permutation), so nothing is
+// counted in advance; the order inside a part does not matter.  Bound by memory:
+// each value is read and written twice, its place once.  A second step that
+// scattered in the L2 instead (128 ranges, all blocks of a range on one XCD) took
+// 200-230 us per 2^27 bytes, the L2's rate of partial stores.  Restore of 2^25
+// particles from random order, 5 planes of 24 bytes: 2.40 -> 1.03 ms.
+constexpr int kFarBlock = 1024;
+constexpr int kFarIters = 32;
+constexpr int kFarShift = 15;
+constexpr uint32_t kFarTile = uint32_t(kFarBlock * kFarIters);
+static_assert(kFarTile == 1u << kFarShift, "a range is a tile");
+constexpr uint32_t kFarRanges = 2 * kFarBlock;  // at most
+constexpr size_t kFarFrom = size_t(1) << 22;  // restore of 24 bytes: 128 us at 2^21 (143 direct), 156 (265) here
+constexpr size_t kFarTo = size_t(kFarRanges) << kFarShift;
+constexpr size_t kFarScratch = 10;  // least scratch, bytes per particle
+
+// Barrier over the block's LDS only: loads and stores of global memory stay in flight.
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// Two 16-bit values a register: 64 registers of a plane's values and a thread's
+// slots and runs have to fit into the 128 that 1024 threads leave.
+struct Halves {
+  uint32_t w[kFarIters / 2] = {};
+  __device__ __forceinline__ uint32_t get(int i) const { return i & 1 ? w[i / 2] >> 16 : w[i / 2] & 0xFFFFu; }
+  __device__ __forceinline__ void put(int i, uint32_t v) { w[i / 2] = i & 1 ? (w[i / 2] & 0xFFFFu) | v << 16 : (w[i / 2] & 0xFFFF0000u) | v; }
+  // opaque to the compiler, which would keep the 32 unpacked values across planes
+  __device__ __forceinline__ void hide() {
+#pragma unroll
+    for (int i = 0; i < kFarIters / 2; ++i) asm volatile("" : "+v"(w[i]));
+  }
+};
+
+// The planes of pa one after another through st: slot.get(i) is the place that value
+// i of the thread takes in st, to(i, l) the index that place l of st goes to.  Of a
+// last tile of len < kFarTile values the loads past the end read its last value,
+// which takes the place past the end that no value has.
+// 8-byte values pass in halves (32768 of them fill twice the LDS).
+template <class To>
+__device__ __forceinline__ void far_planes(const PlaneArgs& pa, uint32_t e0, uint32_t len, uint32_t (&st)[kFarTile],
+                                           Halves& slot, To&& to) {
+  uint32_t tid = threadIdx.x;
+  auto each = [&](auto&& f) {
+#pragma unroll
+    for (int i = 0; i < kFarIters; ++i) f(i, uint32_t(i) * kFarBlock + tid);
+  };
+  const uint32_t last = len - 1;
+  auto at = [&](uint32_t l) { return l < last ? l : last; };
+  for (int k = 0; k < pa.n; ++k) {
+    const uint64_t src = pa.src[k], dst = pa.dst[k];
+    slot.hide();
+    asm volatile("" : "+v"(tid));
+    uint32_t v[kFarIters];
+    if (pa.esz[k] == 4) {
+      const uint32_t* in = reinterpret_cast<const uint32_t*>(src) + e0;
+      each([&](int i, uint32_t l) { v[i] = src ? in[at(l)] : e0 + l; });
+      lds_barrier();  // st has been read
+      each([&](int i, uint32_t) { st[slot.get(i)] = v[i]; });
+      lds_barrier();
+      each([&](int i, uint32_t l) {
+        if (l < len) reinterpret_cast<uint32_t*>(dst)[to(i, l)] = st[l];
+      });
+    } else {
+      const uint2* in = reinterpret_cast<const uint2*>(src) + e0;
+      uint32_t hi[kFarIters];
+      each([&](int i, uint32_t l) {
+        const uint2 w = in[at(l)];
+        v[i] = w.x;
+        hi[i] = w.y;
+      });
+      lds_barrier();
+      each([&](int i, uint32_t) { st[slot.get(i)] = v[i]; });
+      lds_barrier();
+      each([&](int i, uint32_t l) { v[i] = st[l]; });
+      lds_barrier();
+      slot.hide();
+      each([&](int i, uint32_t) { st[slot.get(i)] = hi[i]; });
+      lds_barrier();
+      asm volatile("" : "+v"(tid));
+      each([&](int i, uint32_t l) {
+        if (l < len) reinterpret_cast<uint2*>(dst)[to(i, l)] = uint2{v[i], st[l]};
+      });
+    }
+  }
+}
+
+// pa: planes to stage (src 0: the values are the indexes j); dst: scratch planes.
+__global__ __launch_bounds__(kFarBlock) void k_far_stage(const uint32_t* __restrict__ idx, uint32_t n,
+                                                         uint32_t* __restrict__ cursor, PlaneArgs pa,
+                                                         uint16_t* __restrict__ place) {
+  __shared__ uint32_t st[kFarTile];
+  __shared__ uint32_t cnt[kFarRanges];   // counts, then the first slots of the runs
+  __shared__ uint32_t goff[kFarRanges];  // where slot 0 of the tile would go, by run
+  __shared__ uint32_t wsum[kFarBlock / kWave];
+  const uint32_t tid = threadIdx.x;
+  const uint32_t tile0 = blockIdx.x << kFarShift;
+  const uint32_t len = n - tile0 < kFarTile ? n - tile0 : kFarTile;
+  cnt[tid] = 0;
+  cnt[tid + kFarBlock] = 0;
+  uint32_t d[kFarIters];
+  Halves slot;
+#pragma unroll
+  for (int i = 0; i < kFarIters; ++i) {
+    const uint32_t l = uint32_t(i) * kFarBlock + tid;
+    d[i] = idx[tile0 + (l < len ? l : len - 1)];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < kFarIters; ++i)
+    slot.put(i, uint32_t(i) * kFarBlock + tid < len ? atomicAdd(&cnt[d[i] >> kFarShift], 1u) : 0u);
+  __syncthreads();
+  // first slots of the tile's runs, in the tile and in the ranges' parts: two ranges a thread
+  const uint32_t r0 = 2 * tid, r1 = r0 + 1;
+  const uint32_t c0 = cnt[r0], c1 = cnt[r1];
+  const uint32_t inc = wave_incl_scan(c0 + c1);
+  if ((tid & (kWave - 1)) == kWave - 1) wsum[tid / kWave] = inc;
+  const uint32_t g0 = (r0 << kFarShift) + (c0 ? atomicAdd(&cursor[r0], c0) : 0u);
+  const uint32_t g1 = (r1 << kFarShift) + (c1 ? atomicAdd(&cursor[r1], c1) : 0u);
+  __syncthreads();
+  uint32_t first = inc - c0 - c1;
+  for (uint32_t w = 0; w < tid / kWave; ++w) first += wsum[w];
+  cnt[r0] = first;
+  cnt[r1] = first + c0;
+  goff[r0] = g0 - first;
+  goff[r1] = g1 - first - c0;
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < kFarIters; ++i) {
+    const uint32_t l = uint32_t(i) * kFarBlock + tid;
+    const uint32_t t = l < len ? slot.get(i) + cnt[d[i] >> kFarShift] : l;
+    slot.put(i, t);
+    st[t] = d[i];
+  }
+  __syncthreads();
+  Halves run;
+#pragma unroll
+  for (int i = 0; i < kFarIters; ++i) {
+    const uint32_t l = uint32_t(i) * kFarBlock + tid;
+    const uint32_t v = st[l];
+    run.put(i, v >> kFarShift);
+    if (l < len) place[goff[v >> kFarShift] + l] = uint16_t(v & (kFarTile - 1));
+  }
+  auto to = [&](int i, uint32_t l) {
+    if (i == 0) run.hide();
+    return goff[run.get(i)] + l;
+  };
+  far_planes(pa, tile0, len, st, slot, to);
+}
+
+// pa: scratch planes (src) of values staged by range, brought into order to dst.
+__global__ __launch_bounds__(kFarBlock) void k_far_place(const uint16_t* __restrict__ place, uint32_t n,
+                                                         PlaneArgs pa) {
+  __shared__ uint32_t st[kFarTile];
+  const uint32_t e0 = blockIdx.x << kFarShift;
+  const uint32_t len = n - e0 < kFarTile ? n - e0 : kFarTile;
+  Halves d;
+#pragma unroll
+  for (int i = 0; i < kFarIters; ++i) {
+    const uint32_t l = uint32_t(i) * kFarBlock + threadIdx.x;
+    const uint32_t p = place[e0 + (l < len ? l : len - 1)];
+    d.put(i, l < len ? p : l);
+  }
+  auto to = [&](int, uint32_t l) { return e0 + l; };
+  far_planes(pa, e0, len, st, d, to);
+}
+
+// out[idx[j]] = in[j], j < n, for every plane (pa.src 0: in[j] = j), through
+// `scratch` (bytes >= kFarScratch (n + 8)); cursors: kFarRanges words.
+static int permute_far(const uint32_t* idx, uint32_t n, const PlaneArgs& pa, void* scratch, size_t bytes,
+                       uint32_t* cursors, hipStream_t s) {
+  const unsigned tiles = unsigned((uint64_t(n) + kFarTile - 1) >> kFarShift);
+  const size_t step = (size_t(n) + 7) & ~size_t(7);  // values per scratch plane
+  for (int k = 0; k < pa.n;) {
+    PlaneArgs in{}, out{};
+    size_t used = step * 2;
+    for (; k < pa.n && (in.n == 0 || used + step * pa.esz[k] <= bytes); ++k) {
+      const int m = in.n;
+      in.src[m] = pa.src[k];
+      in.dst[m] = out.src[m] = reinterpret_cast<uint64_t>(static_cast<char*>(scratch) + used);
+      out.dst[m] = pa.dst[k];
+      in.esz[m] = out.esz[m] = pa.esz[k];
+      in.n = out.n = m + 1;
+      used += step * pa.esz[k];
+    }
+    OFP_TRY(fill_u32(cursors, 0, kFarRanges, s));
+    k_far_stage<<<tiles, kFarBlock, 0, s>>>(idx, n, cursors, in, static_cast<uint16_t*>(scratch));
+    OFP_LAUNCHED();
+    k_far_place<<<tiles, kFarBlock, 0, s>>>(static_cast<const uint16_t*>(scratch), n, out);
+    OFP_LAUNCHED();
+  }
+  return OFP_OK;
+}
+
 // out[j] = in[s2n[j]] (gather into sorted order)
 __global__ __launch_bounds__(256) void k_cl_reorder(uint32_t n, const uint32_t* __restrict__ s2n,
                                                     PlaneArgs pa) {
@@ -790,6 +1007,33 @@ __global__ __launch_bounds__(256) void k_cl_restore(uint32_t n, const uint32_t* 
   uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
   if (j >= n) return;
   copy_planes(pa, j, s2n[j]);
+}
+
+// permute_far over the list's particles (h->far), with the list's scratch.
+static int go_far(ofp_cl* h, const uint32_t* idx, const PlaneArgs& pa, hipStream_t s) {
+  if (pa.n == 0) return OFP_OK;
+  std::lock_guard<std::mutex> lock(h->far_lock);
+  if (h->far_done)
+    OFP_HIP(hipStreamWaitEvent(s, h->far_done, 0));
+  else
+    OFP_HIP(hipEventCreateWithFlags(&h->far_done, hipEventDisableTiming));
+  OFP_TRY(permute_far(idx, uint32_t(h->n_part), pa, h->payload.p, h->payload.cap, h->cursors.as<uint32_t>(), s));
+  OFP_HIP(hipEventRecord(h->far_done, s));
+  return OFP_OK;
+}
+
+// A reorder or restore (out[idx[j]] = in[j]) by ranges, where the list's particles
+// are many and far from cell order; *done: it is.  A captured call takes the direct
+// kernel: the graph may be replayed beside other calls that use the scratch.
+static int permute_route(const ofp_cl* h, const uint32_t* idx, const PlaneArgs& pa, hipStream_t s, bool* done) {
+  *done = false;
+  if (!h->far) return OFP_OK;
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  OFP_HIP(hipStreamIsCapturing(s, &cap));
+  if (cap != hipStreamCaptureStatusNone) return OFP_OK;
+  OFP_TRY(go_far(const_cast<ofp_cl*>(h), idx, pa, s));  // its scratch only
+  *done = true;
+  return OFP_OK;
 }
 
 // p[0 .. n) = 0 unless the order check found the input in cell order.
@@ -823,6 +1067,12 @@ static int cl_build_t(ofp_cl* h, const Key& key, const EmitArgs<T>& A0, size_t n
   const uint64_t C = h->n_cells;
   const uint32_t n_tiles = uint32_t((n_cap + kRxTile - 1) / kRxTile);
   const size_t hist_n = size_t(kRxBins) * (n_tiles ? n_tiles : 1);
+  const bool first = g1 != nullptr && n_dev == nullptr;
+  if (first) {  // a build of a count on the host is none for a graph: the count and the buffers are this call's
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    OFP_HIP(hipStreamIsCapturing(s, &cap));
+    if (cap != hipStreamCaptureStatusNone) OFP_HIP(hipErrorStreamCaptureUnsupported);
+  }
   int widths[4];
   const int passes = radix_plan(C, widths);
   // the descents counted and the chunks' sums lie behind the cells' counts, cleared
@@ -884,25 +1134,26 @@ static int cl_build_t(ofp_cl* h, const Key& key, const EmitArgs<T>& A0, size_t n
     h->items_valid = false;
     return OFP_OK;
   };
-  const bool first = g1 != nullptr && n_dev == nullptr;
-  if (first) {  // a build of a count on the host is none for a graph: the count and the buffers are this call's
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    OFP_HIP(hipStreamIsCapturing(s, &cap));
-    if (cap != hipStreamCaptureStatusNone) OFP_HIP(hipErrorStreamCaptureUnsupported);
-  }
+  h->far = false;
   OFP_TRY(fill_u64(reinterpret_cast<uint64_t*>(packed), 0, n_clear, s));
   if (n_tiles == 0) return scan_and_finish();
   const unsigned long long* check = nullptr;  // the kernels below return if *check == 0
   if (first) {
     k_cl_first<T, kIters><<<n_tiles, kRxBlock, 0, s>>>(*g1, emit_args(), n_host, vbuf[0], disorder, packed, C);
     OFP_LAUNCHED();
+    if (n_cap >= kFarFrom) {
+      // the descents to the host, for the emission's route: read there while the passes run
+      if (!h->desc) OFP_HIP(hipHostMalloc(reinterpret_cast<void**>(&h->desc), sizeof(*h->desc)));
+      if (!h->checked) OFP_HIP(hipEventCreateWithFlags(&h->checked, hipEventDisableTiming));
+      OFP_HIP(hipMemcpyAsync(h->desc, disorder, sizeof(*h->desc), hipMemcpyDeviceToHost, s));
+      OFP_HIP(hipEventRecord(h->checked, s));
+    }
+    static_assert(kFarFrom <= kRxNoSync, "a build that waits has the descents");
     if (n_cap < kRxNoSync) {
       check = disorder;
     } else {
-      unsigned long long desc = 0;
-      OFP_HIP(hipMemcpyAsync(&desc, disorder, sizeof(desc), hipMemcpyDeviceToHost, s));
-      OFP_HIP(hipStreamSynchronize(s));
-      if (desc == 0) return scan_and_finish();  // every tile wrote its identity build
+      OFP_HIP(hipEventSynchronize(h->checked));
+      if (*h->desc == 0) return scan_and_finish();  // every tile wrote its identity build
     }
   }
   uint32_t* kin = kbuf[passes % 2];  // pass-0 keys
@@ -955,10 +1206,29 @@ static int cl_build_t(ofp_cl* h, const Key& key, const EmitArgs<T>& A0, size_t n
                                                                   n_host, n_dev, uint32_t(gm), C, packed, check);
   OFP_LAUNCHED();
   OFP_TRY(scan_and_finish());
-  k_cl_emit<T><<<grid_for(n_cap, 256), 256, 0, s>>>(emit_args(), h->keys.as<uint32_t>(), h->s2n.as<uint32_t>(),
-                                                     n_host, n_dev, cs, check);
+  EmitArgs<T> A = emit_args();
+  if (first && n_cap >= kFarFrom && n_cap <= kFarTo) {
+    OFP_HIP(hipEventSynchronize(h->checked));
+    if (*h->desc * kDisorderDen > n_cap) {
+      h->far = h->payload.ensure(kFarScratch * (n_cap + 8)) == OFP_OK &&
+               h->cursors.ensure(kFarRanges * 4) == OFP_OK;
+      if (!h->far) clear_error();  // no memory: without it
+    }
+  }
+  if (h->far) {
+    A.n2s = nullptr;
+    A.pa.n = 0;
+  }
+  k_cl_emit<T><<<grid_for(n_cap, 256), 256, 0, s>>>(A, h->keys.as<uint32_t>(), h->s2n.as<uint32_t>(), n_host, n_dev,
+                                                     cs, check);
   OFP_LAUNCHED();
-  return OFP_OK;
+  if (!h->far) return OFP_OK;
+  PlaneArgs index{};  // n2s[s2n[f]] = f
+  index.n = 1;
+  index.esz[0] = 4;
+  index.dst[0] = reinterpret_cast<uint64_t>(h->n2s.p);
+  OFP_TRY(go_far(h, h->s2n.as<uint32_t>(), index, s));
+  return go_far(h, h->n2s.as<uint32_t>(), A0.pa, s);
 }
 
 template <class T, class Key>
@@ -1243,9 +1513,12 @@ int ofp_cl_destroy(ofp_cl* h) {
   if (!h) return OFP_OK;
   DevBuf* bufs[] = {&h->packed, &h->scan64, &h->keys,    &h->keys2, &h->s2n,        &h->vals2, &h->n2s,
                     &h->dom,    &h->quant,  &h->scantmp, &h->hist,  &h->sid_sorted, &h->items, &h->nitems,
-                    &h->payload, &h->colpart, &h->nz_flag, &h->nz_key, &h->nz_start, &h->nz_nn,
+                    &h->payload, &h->colpart, &h->cursors, &h->nz_flag, &h->nz_key, &h->nz_start, &h->nz_nn,
                     &h->nz_inv, &h->aux};
   for (DevBuf* b : bufs) b->release();
+  if (h->far_done) (void)hipEventDestroy(h->far_done);
+  if (h->checked) (void)hipEventDestroy(h->checked);
+  if (h->desc) (void)hipHostFree(h->desc);
   delete h;
   return OFP_OK;
 }
@@ -1407,6 +1680,9 @@ int ofp_cl_restore(const ofp_cl* h, const ofp_plane* sorted_in, const ofp_plane*
   OFP_TRY(make_plane_args(sorted_in, orig_out, n_planes, &pa));  // every plane checked before any is written
   if (h->n_part == 0 || n_planes == 0) return OFP_OK;
   hipStream_t s = as_stream(stream);
+  bool done = false;
+  OFP_TRY(permute_route(h, h->s2n.as<uint32_t>(), pa, s, &done));
+  if (done) return OFP_OK;
   // planes scattered together while their destinations fit the Infinity Cache
   // (256 MB), where the scattered values of a line meet: 2^25 particles from random
   // order, 24 bytes each, 2.4 ms plane by plane, 3.2 ms with the three coordinates
@@ -1434,6 +1710,9 @@ int ofp_cl_reorder(const ofp_cl* h, const ofp_plane* orig_in, const ofp_plane* s
   OFP_TRY(make_plane_args(orig_in, sorted_out, n_planes, &pa));
   if (h->n_part == 0 || n_planes == 0) return OFP_OK;
   hipStream_t s = as_stream(stream);
+  bool done = false;
+  OFP_TRY(permute_route(h, h->n2s.as<uint32_t>(), pa, s, &done));
+  if (done) return OFP_OK;
   k_cl_reorder<<<grid_for(h->n_part, 256), 256, 0, s>>>(uint32_t(h->n_part), h->s2n.as<uint32_t>(), pa);
   OFP_LAUNCHED();
   return OFP_OK;
