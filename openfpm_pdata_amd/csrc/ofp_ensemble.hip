@@ -850,12 +850,12 @@ static int ens_forces_t(ofp_ens* e, int prec, int kick, double dt, void* energy,
                         static_cast<T*>(X.spos), prec == OFP_PREC_F32C ? X.quant : nullptr,
                         e->sysgrid.as<SysGrid<T>>()};
     return pair_lj_many(e->cl, e->vl, e->dtype, R.spos, cap, prec, e->ljtab[prec].p, e->ljq[prec].p,
-                        int(e->opt.lanes), e->ecap, 0, e->lj_cubic[prec], s, e->sysgrid.p, &K, R.quant);
+                        int(e->opt.lanes), e->ecap, 0, e->lj_cubic[prec], e->S == 1, s, e->sysgrid.p, &K, R.quant);
   }
   // a step (kick) needs the forces only; energy and neighbour counts are for
   // the explicit force pass
   OFP_TRY(pair_lj_many(e->cl, e->opt.pair_walk ? nullptr : e->vl, e->dtype, R.spos, cap, prec, e->ljtab[prec].p,
-                       e->ljq[prec].p, int(e->opt.lanes), e->ecap, kick ? 0 : 1, e->lj_cubic[prec], s,
+                       e->ljq[prec].p, int(e->opt.lanes), e->ecap, kick ? 0 : 1, e->lj_cubic[prec], e->S == 1, s,
                        e->sysgrid.p, nullptr, R.quant));
   const unsigned gN = grid_for(N, 256);
   T* en = static_cast<T*>(energy);
@@ -1158,7 +1158,7 @@ int ofp_ens_pair_pass(ofp_ens* e, int precision, int with_energy, void* stream) 
   const RecSet R = rec_set(e, e->rec_set, v);  // the positions of the last pass
   return pair_lj_many(e->cl, e->opt.pair_walk ? nullptr : e->vl, e->dtype, R.spos, e->cap, precision,
                       e->ljtab[precision].p, e->ljq[precision].p, int(e->opt.lanes), e->ecap, with_energy ? 1 : 0,
-                      e->lj_cubic[precision], as_stream(stream), e->sysgrid.p, nullptr, R.quant);
+                      e->lj_cubic[precision], e->S == 1, as_stream(stream), e->sysgrid.p, nullptr, R.quant);
 }
 
 int ofp_ens_run(ofp_ens* e, int precision, double dt, int n_steps, int use_graph, void* stream) {

@@ -313,16 +313,17 @@ __host__ __device__ __forceinline__ int32_t pack_cell(uint32_t cx, uint32_t cy, 
 // g = u + c 2^28 (mod 2^32) with u = rint((x - cell_low) / q), u clamped to
 // +-2^29 (a particle may drift past its cell between rebuilds).  qlo, qsp:
 // cell-list box low corner and spacing, qinv = 2^28 / spacing, cc = cell coords.
+__device__ __forceinline__ uint32_t quantise_one(double x, uint32_t cc, double qlo, double qsp, double qinv) {
+  const double org = qlo + double(int(cc) - 1) * qsp;
+  double u = rint((x - org) * qinv);
+  u = u < -536870912.0 ? -536870912.0 : (u > 536870912.0 ? 536870912.0 : u);
+  return uint32_t(int(u)) + (cc << kQuantBits);
+}
 __device__ __forceinline__ int4 quantise(const double xs[3], const uint32_t cc[3], const double qlo[3],
                                          const double qsp[3], const double qinv[3]) {
   uint32_t q[3];
 #pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    const double org = qlo[k] + double(int(cc[k]) - 1) * qsp[k];
-    double u = rint((xs[k] - org) * qinv[k]);
-    u = u < -536870912.0 ? -536870912.0 : (u > 536870912.0 ? 536870912.0 : u);
-    q[k] = uint32_t(int(u)) + (cc[k] << kQuantBits);
-  }
+  for (int k = 0; k < 3; ++k) q[k] = quantise_one(xs[k], cc[k], qlo[k], qsp[k], qinv[k]);
   return make_int4(int(q[0]), int(q[1]), int(q[2]), pack_cell(cc[0], cc[1], cc[2]));
 }
 
@@ -534,20 +535,24 @@ struct SysDyn {
 // when the squared displacement exceeds lim2).
 // The arithmetic on values: v, x updated in place; returns whether the
 // displacement exceeds the threshold.
+// One component; returns the square of its displacement since the build.
+template <class T>
+__device__ __forceinline__ T kick_kick_drift_one(T& v, T& x, T xb, const SysDyn<T>& D, T dt, T a) {
+#pragma clang fp contract(off)
+  const T h = (T(0.5) * dt) * D.inv_m;
+  const T v1 = v + h * a;  // end of this step
+  v = v1 + h * a;          // first half kick of the next
+  x = x + dt * v;
+  const T r = x - xb;
+  return r * r;
+}
 template <class T>
 __device__ __forceinline__ bool kick_kick_drift_v(T (&v)[3], T (&x)[3], const T (&xb)[3], const SysDyn<T>& D, T dt,
                                                   const T (&a)[3]) {
 #pragma clang fp contract(off)
-  const T h = (T(0.5) * dt) * D.inv_m;
   T dd = 0;
 #pragma unroll
-  for (int d = 0; d < 3; ++d) {
-    const T v1 = v[d] + h * a[d];  // end of this step
-    v[d] = v1 + h * a[d];          // first half kick of the next
-    x[d] = x[d] + dt * v[d];
-    const T r = x[d] - xb[d];
-    dd = dd + r * r;
-  }
+  for (int d = 0; d < 3; ++d) dd = dd + kick_kick_drift_one<T>(v[d], x[d], xb[d], D, dt, a[d]);
   return dd > D.lim2;
 }
 // xo: the new position.
@@ -575,19 +580,27 @@ __device__ inline void kick_kick_drift(uint32_t i, size_t cap, T* __restrict__ p
 // the particle of each row as soon as its force is summed (the force is not
 // stored).  s2n maps a row's sorted slot p to its storage index; per_sys = 0:
 // one system, constants dyn[0] / sys[0], else those of the row's system.  The
+// position of before is the sorted one that the pass has read anyway.  The
 // new position also goes to slot p of the next step's sorted positions (snext)
 // and, for FP32C, of its quantised records (qnext, against the cell of the
 // last build, w of the row's current record): the pair pass of the next step
 // reads those, while this one reads the current ones, which no lane changes.
+// Rows of kSplitLanes lanes and more: lane d takes component d (lanes past 2
+// repeat it for the loads), so that a wave's kick is 2 loads and 4 stores in
+// place of 6 and 10 of an eighth of the lanes each.
 struct NoKick {
   static constexpr bool kOn = false;
   struct Pre {};
   __device__ __forceinline__ uint32_t index(uint32_t) const { return 0u; }
-  __device__ __forceinline__ Pre prefetch(uint32_t) const { return Pre{}; }
+  template <int kLanes>
+  __device__ __forceinline__ Pre prefetch(uint32_t, unsigned) const {
+    return Pre{};
+  }
 };
 template <class T>
 struct StepKick {
   static constexpr bool kOn = true;
+  static constexpr int kSplitLanes = 4;
   using Tv = T;
   const uint32_t* s2n;
   T* pos;
@@ -601,28 +614,37 @@ struct StepKick {
   T* snext;
   int4* qnext;  // null: no quantised records (FP64 pass)
   const SysGrid<T>* sys;
-  // the particle's storage index and state, loaded ahead of the kick (the
-  // kernels issue these loads before their last gathers, so they wait once)
+  // the particle's storage index and state (component 0: the lane's own, of a
+  // split row), loaded ahead of the kick (the kernels issue these loads before
+  // their last gathers, so they wait once)
   struct Pre {
     uint32_t i;
-    T v[3], x[3], xb[3];
+    T v[3], xb[3];
   };
   __device__ __forceinline__ uint32_t index(uint32_t p) const { return s2n[p]; }
-  __device__ __forceinline__ Pre prefetch(uint32_t i) const {
+  template <int kLanes>
+  __device__ __forceinline__ Pre prefetch(uint32_t i, unsigned lane) const {
     Pre q;
     q.i = i;
+    if constexpr (kLanes >= kSplitLanes) {
+      const size_t at = (lane < 2u ? lane : 2u) * cap + i;
+      q.v[0] = vel[at];
+      q.xb[0] = xb[at];
+    } else {
 #pragma unroll
-    for (int d = 0; d < 3; ++d) {
-      q.v[d] = vel[d * cap + i];
-      q.x[d] = pos[d * cap + i];
-      q.xb[d] = xb[d * cap + i];
+      for (int d = 0; d < 3; ++d) {
+        q.v[d] = vel[d * cap + i];
+        q.xb[d] = xb[d * cap + i];
+      }
     }
     return q;
   }
-  __device__ __forceinline__ void apply(const Pre& q, uint32_t p, uint32_t sy, int w, const T (&a)[3]) const {
+  // One lane for all components.  xp: the current position.
+  __device__ __forceinline__ void apply(const Pre& q, uint32_t p, uint32_t sy, int w, const T (&a)[3],
+                                        const T (&xp)[3]) const {
     const uint32_t s = per_sys ? sy : 0u;
     T v[3] = {q.v[0], q.v[1], q.v[2]};
-    T x[3] = {q.x[0], q.x[1], q.x[2]};
+    T x[3] = {xp[0], xp[1], xp[2]};
     const bool far = kick_kick_drift_v<T>(v, x, q.xb, dyn[s], dt, a);
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
@@ -638,17 +660,46 @@ struct StepKick {
       qnext[p] = quantise(xs, cc, G.qlo, G.qsp, G.qinv);
     }
   }
+  // Lane d of a row for component d, called by every lane of the row; the
+  // arithmetic of apply.
+  template <int kLanes>
+  __device__ __forceinline__ void apply_split(const Pre& q, uint32_t p, uint32_t sy, int w, const T (&a)[3],
+                                              const T (&xp)[3], unsigned lane) const {
+    const uint32_t s = per_sys ? sy : 0u;
+    auto own = [&](auto a0, auto a1, auto a2) { return lane == 0 ? a0 : (lane == 1 ? a1 : a2); };
+    T v = q.v[0], x = own(xp[0], xp[1], xp[2]);
+    const T rr = kick_kick_drift_one<T>(v, x, q.xb[0], dyn[s], dt, own(a[0], a[1], a[2]));
+    T dd = T(0);
+#pragma unroll
+    for (int d = 0; d < 3; ++d) dd = dd + __shfl(rr, d, kLanes);
+    const bool far = dd > dyn[s].lim2;
+    if (lane < 3u) {
+      vel[lane * cap + q.i] = v;
+      pos[lane * cap + q.i] = x;
+      snext[lane * cap + p] = x;
+    }
+    if (far && lane == 0u) atomicOr(&flags[0], 1u);
+    if (qnext && lane < 4u) {
+      const SysGrid<T>& G = sys[s];
+      const uint32_t cc = own(uint32_t(w) & 2047u, (uint32_t(w) >> 11) & 2047u, (uint32_t(w) >> 22) & 1023u);
+      const uint32_t g = quantise_one(double(x), cc, own(G.qlo[0], G.qlo[1], G.qlo[2]),
+                                      own(G.qsp[0], G.qsp[1], G.qsp[2]), own(G.qinv[0], G.qinv[1], G.qinv[2]));
+      // (lane 3: the cell, as it was)
+      reinterpret_cast<uint32_t*>(qnext + p)[lane] = lane == 3u ? uint32_t(w) : g;
+    }
+  }
 };
 
 // vl == null: the cell-tile pass over the cell list's item queue (the cells of
 // the last build, whose stencil covers r_cut + skin), sysgrid = SysGrid<T>[n_sys]
-// of the position dtype.  kick (Verlet rows only, with_u = 0): a StepKick<T>
+// of the position dtype.  one_system: every row's constants are the tables' first
+// entry.  kick (Verlet rows only, with_u = 0): a StepKick<T>
 // of the position dtype, applied to every row in place of storing its force.
 // Over Verlet rows, pos_sorted (sorted positions, plane stride `stride`) and
 // quant (FP32C records; null: the cell list's own) are what the pass reads.
 int pair_lj_many(const ofp_cl* cl, const ofp_vl* vl, int dtype, const void* pos_sorted, size_t stride,
                  int precision, const void* tab, const void* qtab, int lanes, size_t e_cap, int with_u, int cubic,
-                 hipStream_t s, const void* sysgrid = nullptr, const void* kick = nullptr,
+                 bool one_system, hipStream_t s, const void* sysgrid = nullptr, const void* kick = nullptr,
                  const void* quant = nullptr);
 
 }  // namespace ofp

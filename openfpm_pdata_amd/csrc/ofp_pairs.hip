@@ -1250,9 +1250,11 @@ __device__ __forceinline__ void by_system(bool valid, uint32_t sy_lane, F&& f) {
 
 // The end of a row: its force stored (NoKick), or applied to the row's particle
 // by the step's kick (StepKick).
-template <class Ph, class K>
+// Called by every lane of the row.  x: the row's position.
+template <int kLanes, class Ph, class K, class T>
 __device__ __forceinline__ void finish_row(const Ph& ph, const typename Ph::St& st, uint32_t p, uint32_t sy, int w,
-                                           const K& kick, const typename K::Pre& pre) {
+                                           const K& kick, const typename K::Pre& pre, const T (&x)[3],
+                                           unsigned lane) {
   if constexpr (K::kOn) {
     typename K::Tv a[3];
     ph.force_as(st, a);
@@ -1261,15 +1263,19 @@ __device__ __forceinline__ void finish_row(const Ph& ph, const typename Ph::St& 
     // hold registers throughout
     uint32_t pk = p;
     int wk = w;
-    asm volatile("" : "+v"(pk), "+v"(wk));
-    kick.apply(pre, pk, sy, wk, a);
+    unsigned lk = lane;
+    asm volatile("" : "+v"(pk), "+v"(wk), "+v"(lk));
+    if constexpr (kLanes >= K::kSplitLanes)
+      kick.template apply_split<kLanes>(pre, pk, sy, wk, a, x, lk);
+    else if (lane == 0)
+      kick.apply(pre, pk, sy, wk, a, x);
   } else {
-    ph.finish(st, p);
+    if (lane == 0) ph.finish(st, p);
   }
 }
 
 // Verlet rows of an ensemble: the constants of row k are the table entry of its
-// system (sid_sorted of the row's particle); kLanes lanes per row.  K: NoKick
+// system (sid_sorted of the row's particle; null: one system); kLanes lanes per row.  K: NoKick
 // (forces stored) or StepKick<T> (the row's particle kicked and drifted).
 template <class T, class Ph, int kLanes, bool kCubic, class K>
 __global__ __launch_bounds__(256) void k_pairs_many_f32c(ClDev c, const Ph* __restrict__ tab,
@@ -1286,7 +1292,7 @@ __global__ __launch_bounds__(256) void k_pairs_many_f32c(ClDev c, const Ph* __re
   const int4 P = c.quant[p];
   const uint32_t ik = kick.index(p);
   const unsigned lane = threadIdx.x & (kLanes - 1);
-  by_system(valid, sid_sorted[p], [&](uint32_t sy) {
+  by_system(valid, sid_sorted ? sid_sorted[p] : 0u, [&](uint32_t sy) {
   const Ph ph = tab[sy];
   const QGeom qg = qtab[sy];
   // the stored position, for close pairs
@@ -1298,8 +1304,9 @@ __global__ __launch_bounds__(256) void k_pairs_many_f32c(ClDev c, const Ph* __re
   // hoisted above it, where their registers would be held throughout)
   auto prefetch = [&] {
     uint32_t i = ik;
-    asm volatile("" : "+v"(i));
-    pre = kick.prefetch(i);
+    unsigned l = lane;
+    asm volatile("" : "+v"(i), "+v"(l));
+    pre = kick.template prefetch<kLanes>(i, l);
   };
   if (kLanes == 1) {
     // e_lim: entries the list holds (a list that overflowed its capacity was not
@@ -1366,7 +1373,7 @@ __global__ __launch_bounds__(256) void k_pairs_many_f32c(ClDev c, const Ph* __re
     prefetch();
   }
   ph.reduce(st, kLanes);
-  if (lane == 0) finish_row(ph, st, p, sy, P.w, kick, pre);
+  finish_row<kLanes>(ph, st, p, sy, P.w, kick, pre, pp, lane);
   });
 }
 
@@ -1384,7 +1391,7 @@ __global__ __launch_bounds__(256) void k_pairs_many_f64(ClDev c, const Ph* __res
   const double xp = pos[p], yp = pos[stride + p], zp = pos[2 * stride + p];
   const uint32_t ik = kick.index(p);
   const unsigned lane = threadIdx.x & (kLanes - 1);
-  by_system(valid, sid_sorted[p], [&](uint32_t sy) {
+  by_system(valid, sid_sorted ? sid_sorted[p] : 0u, [&](uint32_t sy) {
   const Ph ph = tab[sy];
   typename Ph::St st;
   ph.start(st, p);
@@ -1433,9 +1440,10 @@ __global__ __launch_bounds__(256) void k_pairs_many_f64(ClDev c, const Ph* __res
   }
   uint32_t i = ik;  // opaque: the kick's loads stay after the loop
   asm volatile("" : "+v"(i));
-  const typename K::Pre pre = kick.prefetch(i);
+  const typename K::Pre pre = kick.template prefetch<kLanes>(i, lane);
   ph.reduce(st, kLanes);
-  if (lane == 0) finish_row(ph, st, p, sy, 0, kick, pre);
+  const T xr[3] = {T(xp), T(yp), T(zp)};  // stored in T
+  finish_row<kLanes>(ph, st, p, sy, 0, kick, pre, xr, lane);
   });
 }
 
@@ -1875,12 +1883,14 @@ static int launch_lj_tiles(const PairCtx& x, int precision, const void* pos_sort
 
 int ofp::pair_lj_many(const ofp_cl* cl, const ofp_vl* vl, int dtype, const void* pos_sorted, size_t stride,
                       int precision, const void* tab, const void* qtab, int lanes, size_t e_cap, int with_u,
-                      int cubic, hipStream_t s, const void* sysgrid, const void* kick, const void* quant) {
+                      int cubic, bool one_system, hipStream_t s, const void* sysgrid, const void* kick,
+                      const void* quant) {
   PairCtx x;
   OFP_TRY(pair_ctx(cl, vl, precision, 0.0, &x));
   if (quant) x.c.quant = static_cast<const int4*>(quant);
   const uint32_t* sid = nullptr;
   OFP_TRY(cl_sid_sorted(cl, &sid));
+  if (one_system) sid = nullptr;
   if (x.c.n_dom == 0) return OFP_OK;
   if (!vl) {
     OFP_CHECK(sysgrid, OFP_E_ARG, "ensemble cell-tile pass needs the systems' grids");
