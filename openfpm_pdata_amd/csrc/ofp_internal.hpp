@@ -406,6 +406,101 @@ __device__ __forceinline__ uint32_t next_unit(uint32_t* __restrict__ heads) {
   return __builtin_amdgcn_readfirstlane(k) * kQueues + q;
 }
 
+// ------------------------------------------- distances on the matrix cores
+typedef float v16f __attribute__((ext_vector_type(16)));
+// Lane halves: {a_lo, b_lo} and {a_hi, b_hi}.
+__device__ __forceinline__ void swap_halves(uint32_t& a, uint32_t& b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+  a = r[0];
+  b = r[1];
+}
+__device__ __forceinline__ void swap_halves(float& a, float& b) {
+  uint32_t x = __float_as_uint(a), y = __float_as_uint(b);
+  swap_halves(x, y);
+  a = __uint_as_float(x);
+  b = __uint_as_float(y);
+}
+template <class T>
+__device__ __forceinline__ T lane_value(T v, uint32_t lane);
+template <>
+__device__ __forceinline__ float lane_value<float>(float v, uint32_t lane) {
+  return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), lane));
+}
+template <>
+__device__ __forceinline__ double lane_value<double>(double v, uint32_t lane) {
+  const unsigned long long u = static_cast<unsigned long long>(__double_as_longlong(v));
+  const uint32_t lo = __builtin_amdgcn_readlane(uint32_t(u), lane);
+  const uint32_t hi = __builtin_amdgcn_readlane(uint32_t(u >> 32), lane);
+  return __longlong_as_double(static_cast<long long>((static_cast<unsigned long long>(hi) << 32) | lo));
+}
+
+
+// Row of this lane in a 32 x 32 product: row 8 q + 4 h + m of a 32-block is candidate
+// 16 h + 15 - (4 q + m), so a lane's results i = 4 q + m (rows 8 (i / 4) +
+// 4 (lane / 32) + i % 4) are candidates 15 - i of its half.
+__device__ __forceinline__ uint32_t matrix_candidate(uint32_t lane) {
+  const uint32_t r = lane & 31u;
+  return 16u * ((r >> 2) & 1u) + 15u - (4u * (r >> 3) + (r & 3u));
+}
+
+// Candidates that may lie within a cut-off of a wave's targets (target = lane), from
+// tiles of the matrix product of (x, y, z, |c|^2) and (-2x, -2y, -2z, 1) on top of
+// |t|^2 - r^2 (coordinates relative to a common origin): the sign of 32 x 32 squares
+// less r^2.  r2: the cut-off's square plus the bound of the FP32 error, 2^-19 S with
+// S = (R_c + R_t)^2 + r^2, R the farthest candidate's and target's distance from the
+// origin: every pair within the cut-off has its bit set, and a few beyond.
+struct MatrixTest {
+  v16f C0, C1;
+  float b00, b01, b10, b11, lim_c;
+  bool two;  // more than 32 targets
+  __device__ __forceinline__ void targets(float x, float y, float z, float r2, float lim, bool more_than_32) {
+    float k0 = __builtin_fmaf(x, x, __builtin_fmaf(y, y, z * z)) - r2, k1 = k0;
+    b00 = -2.f * x, b01 = -2.f * y;  // columns of the target halves: k = 0, 1
+    swap_halves(b00, b01);
+    b10 = -2.f * z, b11 = 1.f;  // k = 2, 3
+    swap_halves(b10, b11);
+    swap_halves(k0, k1);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      C0[i] = k0;
+      C1[i] = k1;
+    }
+    lim_c = lim;
+    two = more_than_32;
+  }
+  __device__ __forceinline__ void tile(float a0, float a1, float b0, float b1, const v16f& K, uint32_t& w) const {
+    v16f D = __builtin_amdgcn_mfma_f32_32x32x2f32(a0, b0, K, 0, 0, 0);
+    D = __builtin_amdgcn_mfma_f32_32x32x2f32(a1, b1, D, 0, 0, 0);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) w = __builtin_amdgcn_alignbit(w, __float_as_uint(D[i]), 31);
+  }
+  // (x, y, z): candidate matrix_candidate(lane) of the first block in the lower
+  // lanes, of the second (if any) in the upper.  Words of the two blocks for target
+  // = lane.  False (words void) if a candidate lies beyond the bound or is not a
+  // number.
+  __device__ __forceinline__ bool words(float x, float y, float z, bool second, uint32_t* lo, uint32_t* hi) const {
+    const float cn = __builtin_fmaf(x, x, __builtin_fmaf(y, y, z * z));
+    if (__ballot(!(cn <= lim_c)) != 0ull) return false;
+    float a00 = x, a01 = y, a10 = z, a11 = cn;
+    swap_halves(a00, a01);  // a00: x, y of the first block; a01: of the second
+    swap_halves(a10, a11);
+    uint32_t w0 = 0, w1 = 0;
+    if (second) {
+      tile(a01, a11, b00, b10, C0, w0);
+      if (two) tile(a01, a11, b01, b11, C1, w1);
+    }
+    tile(a00, a10, b00, b10, C0, w0);
+    if (two) tile(a00, a10, b01, b11, C1, w1);
+    // w_k: targets 32 k + lane % 32; of each block candidates 16 h + (0-15), h =
+    // lane / 32, the second block's in the high half.  To lane = target: w0 the
+    // h = 0 bits, w1 the h = 1 bits
+    swap_halves(w0, w1);
+    *lo = __builtin_amdgcn_perm(w1, w0, 0x05040100u);
+    *hi = __builtin_amdgcn_perm(w1, w0, 0x07060302u);
+    return true;
+  }
+};
+
 // ------------------------------------------------------ cell-list view
 // What the walkers need of a built cell list, passed to kernels by value.
 struct ClDev {
@@ -486,6 +581,21 @@ __device__ __forceinline__ void for_each_run(const ClDev& c, const ItemGeom<T>& 
     }
   }
 }
+
+// Run r of the item (traversal order) in lane r < (2B+1)^2: [x, y), empty outside the
+// grid and in the other lanes.
+template <class T>
+__device__ __forceinline__ uint2 lane_run(const ClDev& c, const ItemGeom<T>& G, int lane) {
+  const int B = int(c.box_nn), W = 2 * B + 1;
+  const int xa = G.cx0 - B > 0 ? G.cx0 - B : 0;
+  const int xe = G.cx0 + G.ncx - 1 + B;
+  const int xb = xe < int(G.d0) - 1 ? xe : int(G.d0) - 1;
+  const int zz = G.cz + lane / W - B, yy = G.cy + lane % W - B;
+  if (lane >= W * W || zz < 0 || zz >= int(G.d2) || yy < 0 || yy >= int(G.d1)) return make_uint2(0u, 0u);
+  const uint32_t rowc = G.cbase + G.d0 * (uint32_t(yy) + G.d1 * uint32_t(zz));
+  return make_uint2(uint32_t(c.cs[rowc + uint32_t(xa)]), uint32_t(c.cs[rowc + uint32_t(xb) + 1]));
+}
+static_assert((2 * kMaxBoxNN + 1) * (2 * kMaxBoxNN + 1) <= kWave, "one lane per run");
 
 // Ensemble cell lists: one sort over the grids of all systems (global cell ids).
 // sys_dev = SysGrid<T>[n_sys], rbase_dev = first global x-row of each system

@@ -1005,7 +1005,13 @@ __global__ __launch_bounds__(256) void k_rows_smooth(ClDev c, const unsigned lon
 // (the wrapped subtraction is exact) or its wrapped separation is still more
 // than B cells (one cell of slack for positions that have drifted since the
 // cells were built): no far candidate passes the check.
-constexpr int kTileChunk = 128;  // candidates staged per round (4 mask words)
+// Candidates staged per round: a lane's hits of a run of cells vary with its place
+// in y and z, those of several runs less, and a round takes as long as its busiest
+// lane.  Four blocks of four waves fit a CU's registers, 40 KB of LDS each.
+template <class R>
+constexpr int tile_chunk() {
+  return sizeof(R) <= 16 ? 384 : 256;
+}
 constexpr int kTileBlock = 256;  // four independent waves
 constexpr int kTileWaves = kTileBlock / kWave;
 static_assert(16 - (int(kItemMaxCells) - 1 + kMaxBoxNN) - 2 > kMaxBoxNN, "wrapped FP32C separations");
@@ -1024,35 +1030,72 @@ __device__ __forceinline__ uint32_t staged_hits(const R* buf, uint32_t k0, uint3
   return __builtin_bitreverse32(w << (32u - cnt));
 }
 
-// Calls fn(k) for the set bits k of the 128-bit mask (m[0] bits 0..31, ...),
-// lowest first, one bit per lane per round, until no lane has bits left.
+// Calls fn(k) for the set bits k of the lane's `words` 64-bit words (mk[q][lane]),
+// lowest first, one bit per lane per round, until no lane has bits left (an empty
+// word costs its lane a round).
 template <class F>
-__device__ __forceinline__ void for_each_hit(uint32_t m[4], F&& fn) {
-  unsigned long long lo = (static_cast<unsigned long long>(m[1]) << 32) | m[0];
-  unsigned long long hi = (static_cast<unsigned long long>(m[3]) << 32) | m[2];
-  while (__ballot((lo | hi) != 0ull) != 0ull) {
-    if ((lo | hi) != 0ull) {
-      uint32_t k;
-      if (lo != 0ull) {
-        k = uint32_t(__builtin_ctzll(lo));
-        lo &= lo - 1ull;
-      } else {
-        k = 64u + uint32_t(__builtin_ctzll(hi));
-        hi &= hi - 1ull;
-      }
+__device__ __forceinline__ void for_each_hit(const unsigned long long (*mk)[kWave], uint32_t words, int lane, F&& fn) {
+  unsigned long long w = mk[0][lane];
+  uint32_t q = 0;
+  for (;;) {
+    if (w == 0ull && q + 1 < words) w = mk[++q][lane];
+    if (__ballot(w != 0ull || q + 1 < words) == 0ull) return;
+    if (w != 0ull) {
+      const uint32_t k = q * 64u + uint32_t(__builtin_ctzll(w));
+      w &= w - 1ull;
       fn(k);
     }
   }
 }
 
-// Staging: records j0 .. j0 + m - 1 into the wave's buffer.  The wave's LDS
-// operations execute in issue order; the barriers keep the compiler from
-// moving the reads of one round across the writes of the next.
-template <class R>
-__device__ __forceinline__ void stage(R* buf, const R* __restrict__ src, uint32_t j0, uint32_t m, int lane) {
-  __builtin_amdgcn_wave_barrier();
-  for (uint32_t k = uint32_t(lane); k < m; k += kWave) buf[k] = src[j0 + k];
-  __builtin_amdgcn_wave_barrier();
+// The item's candidates through the wave's buffer, kChunk at a time across the
+// ends of the runs: put(slot, j) stages sorted index j, eval(m) takes the m staged.
+// Lane r holds run r.  The wave's LDS operations execute in issue order; the
+// barriers keep the compiler from moving the reads of one round across the writes
+// of the next.
+template <int kChunk, class T, class P, class E>
+__device__ __forceinline__ void for_each_chunk(const ClDev& c, const ItemGeom<T>& G, int lane, P&& put, E&& eval) {
+  const uint2 R = lane_run(c, G, lane);
+  const uint32_t runs = (2u * c.box_nn + 1u) * (2u * c.box_nn + 1u);
+  uint32_t r = 0, done = 0;  // the run in hand, and how much of it has been staged
+  for (;;) {
+    uint32_t m = 0;
+    __builtin_amdgcn_wave_barrier();
+    while (m < uint32_t(kChunk) && r < runs) {
+      const uint32_t ja = __builtin_amdgcn_readlane(R.x, r) + done, left = __builtin_amdgcn_readlane(R.y, r) - ja;
+      const uint32_t n = left < uint32_t(kChunk) - m ? left : uint32_t(kChunk) - m;
+      for (uint32_t k = uint32_t(lane); k < n; k += kWave) put(m + k, ja + k);
+      m += n;
+      done = n < left ? done + n : 0u;
+      r += n < left ? 0u : 1u;
+    }
+    __builtin_amdgcn_wave_barrier();
+    if (m == 0) return;
+    eval(m);
+  }
+}
+
+// Hit words of m staged candidates to mk: from the matrix cores, two blocks of 32 at
+// a time (rel: the coordinates of a staged candidate relative to the origin), or by
+// the exact test where they decline.
+template <class R, class Rel, class Test>
+__device__ __forceinline__ void chunk_hits(const MatrixTest& mt, bool fast, const R* buf, uint32_t m, int lane,
+                                           bool valid, unsigned long long (*mk)[kWave], Rel&& rel, Test&& test) {
+  const uint32_t mine = matrix_candidate(uint32_t(lane)) + (lane < 32 ? 0u : 32u);
+  for (uint32_t k0 = 0; k0 < m; k0 += 64u) {
+    const uint32_t n = m - k0 < 64u ? m - k0 : 64u;
+    float x, y, z;
+    rel(buf[k0 + (mine < n ? mine : n - 1u)], &x, &y, &z);
+    uint32_t lo = 0, hi = 0;
+    if (fast && mt.words(x, y, z, n > 32u, &lo, &hi)) {
+      lo &= n < 32u ? 0xFFFFFFFFu >> (32u - n) : 0xFFFFFFFFu;
+      hi &= n > 32u ? 0xFFFFFFFFu >> (64u - n) : 0u;
+    } else {
+      lo = staged_hits(buf, k0, n < 32u ? n : 32u, test);
+      hi = n > 32u ? staged_hits(buf, k0 + 32u, n - 32u, test) : 0u;
+    }
+    mk[k0 / 64u][lane] = valid ? static_cast<unsigned long long>(hi) << 32 | lo : 0ull;
+  }
 }
 
 // FP32C.  rec: per sorted particle the quantised record; with Ph::kAuxInQuant
@@ -1060,16 +1103,19 @@ __device__ __forceinline__ void stage(R* buf, const R* __restrict__ src, uint32_
 // the fourth word is not read.  kMany: ensembles, the physics and geometry of
 // an item come from the tables of its system (ncx >> 8).
 template <class T, class Ph, bool kCubic, bool kMany>
-__global__ __launch_bounds__(kTileBlock) void k_tile_f32c(ClDev c, QGeom qg1, Ph ph1, const Ph* __restrict__ tab,
+__global__ __launch_bounds__(kTileBlock, 4) void k_tile_f32c(ClDev c, QGeom qg1, Ph ph1, const Ph* __restrict__ tab,
                                                           const QGeom* __restrict__ qtab,
                                                           const SysGrid<T>* __restrict__ sys,
                                                           const int4* __restrict__ rec,
                                                           const TargetItem* __restrict__ items,
                                                           const uint32_t* __restrict__ n_items_p,
                                                           uint32_t* __restrict__ counter) {
-  __shared__ int4 lds[kTileWaves][kTileChunk];
+  constexpr int kChunk = tile_chunk<int4>();
+  __shared__ int4 lds[kTileWaves][kChunk];
+  __shared__ unsigned long long ldsm[kTileWaves][kChunk / 64][kWave];
   const int lane = threadIdx.x & (kWave - 1);
   int4* buf = lds[threadIdx.x / kWave];
+  unsigned long long(*mk)[kWave] = ldsm[threadIdx.x / kWave];
   const uint32_t n_items = *n_items_p;
   for (;;) {
     const uint32_t it = next_unit(counter);
@@ -1085,42 +1131,58 @@ __global__ __launch_bounds__(kTileBlock) void k_tile_f32c(ClDev c, QGeom qg1, Ph
     const float pre2 = ph.rc2 * kPreCut;
     typename Ph::St st;
     ph.start(st, p);
+    auto sep = [&](const int4& Q, int ox, int oy, int oz, float* x, float* y, float* z) {
+      *x = float(wrap_diff(Q.x, ox));
+      *y = kCubic ? float(wrap_diff(Q.y, oy)) : float(wrap_diff(Q.y, oy)) * qg.ry;
+      *z = kCubic ? float(wrap_diff(Q.z, oz)) : float(wrap_diff(Q.z, oz)) * qg.rz;
+    };
     auto test = [&](const int4& Q) {
-      const float fx = float(wrap_diff(Q.x, P.x));
-      const float fy = kCubic ? float(wrap_diff(Q.y, P.y)) : float(wrap_diff(Q.y, P.y)) * qg.ry;
-      const float fz = kCubic ? float(wrap_diff(Q.z, P.z)) : float(wrap_diff(Q.z, P.z)) * qg.rz;
+      float fx, fy, fz;
+      sep(Q, P.x, P.y, P.z, &fx, &fy, &fz);
       return __builtin_fmaf(fx, fx, __builtin_fmaf(fy, fy, fz * fz)) < pre2;
     };
-    for_each_run(c, G, [&](uint32_t ja, uint32_t jb) {
-      for (uint32_t j0 = ja; j0 < jb; j0 += kTileChunk) {
-        const uint32_t m = jb - j0 < uint32_t(kTileChunk) ? jb - j0 : uint32_t(kTileChunk);
-        stage(buf, rec, j0, m, lane);
-        uint32_t mk[4];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const uint32_t k0 = uint32_t(q) * 32u;
-          mk[q] = k0 < m ? staged_hits(buf, k0, m - k0 < 32u ? m - k0 : 32u, test) : 0u;
-          if (!valid) mk[q] = 0u;
-        }
-        for_each_hit(mk, [&](uint32_t k) {
-          const uint32_t j = j0 + k;
-          if (j == p) return;
-          const int4 Q = buf[k];
-          float a;
-          if constexpr (Ph::kAuxInQuant)
-            a = __int_as_float(Q.w);
-          else
-            a = ph.aux(j);
-          const int ix = wrap_diff(Q.x, P.x), iy = wrap_diff(Q.y, P.y), iz = wrap_diff(Q.z, P.z);
-          if constexpr (Ph::kSmooth)
-            smooth_pair<Ph, kCubic>(ph, st, qg, a, ix, iy, iz);
-          else
-            quant_pair<Ph, kCubic>(ph, st, qg, a, ix, iy, iz, p, j);
+    // the origin: the middle of the item's cells, at most ncx / 2 + 1 cells (drift
+    // included) from a target in x and B more from a candidate within its cut-off
+    const int ox = int(uint32_t(2 * G.cx0 + G.ncx) << (kQuantBits - 1));
+    const int oy = int(uint32_t(2 * G.cy + 1) << (kQuantBits - 1));
+    const int oz = int(uint32_t(2 * G.cz + 1) << (kQuantBits - 1));
+    constexpr float cell = float(kQuantOne);
+    const float ry2 = kCubic ? 1.f : qg.ry * qg.ry, rz2 = kCubic ? 1.f : qg.rz * qg.rz;
+    const float nx = 0.5f * float(G.ncx) + 1.f, bx = nx + float(c.box_nn), by = 1.5f + float(c.box_nn);
+    const float rt2 = cell * cell * (nx * nx + 2.25f * (ry2 + rz2));
+    const float rc2 = cell * cell * (bx * bx + by * by * (ry2 + rz2));
+    float tx, ty, tz;
+    sep(P, ox, oy, oz, &tx, &ty, &tz);
+    const bool fast = __ballot(!(__builtin_fmaf(tx, tx, __builtin_fmaf(ty, ty, tz * tz)) <= rt2 * 1.01f)) == 0ull;
+    MatrixTest mt;
+    mt.targets(tx, ty, tz, pre2 + (2.05f * (rt2 + rc2) + pre2) * 0x1p-19f, rc2 * 1.01f, ti.n > 32u);
+    bool seen = false;
+    for_each_chunk<kChunk>(
+        c, G, lane,
+        [&](uint32_t k, uint32_t j) {
+          int4 Q = rec[j];
+          if constexpr (!Ph::kAuxInQuant) Q.w = int(j);
+          buf[k] = Q;
+        },
+        [&](uint32_t m) {
+          chunk_hits(mt, fast, buf, m, lane, valid, mk,
+                     [&](const int4& Q, float* x, float* y, float* z) { sep(Q, ox, oy, oz, x, y, z); }, test);
+          for_each_hit(mk, (m + 63u) / 64u, lane, [&](uint32_t k) {
+            seen = true;
+            const int4 Q = buf[k];
+            const int ix = wrap_diff(Q.x, P.x), iy = wrap_diff(Q.y, P.y), iz = wrap_diff(Q.z, P.z);
+            if constexpr (Ph::kSmooth) {  // (the particle itself too)
+              float a = 0.f;
+              if constexpr (Ph::kAuxInQuant) a = __int_as_float(Q.w);
+              smooth_pair<Ph, kCubic>(ph, st, qg, a, ix, iy, iz);
+            } else {
+              const uint32_t j = uint32_t(Q.w);
+              if (j != p) quant_pair<Ph, kCubic>(ph, st, qg, ph.aux(j), ix, iy, iz, p, j);
+            }
+          });
         });
-      }
-    });
     if constexpr (Ph::kSmooth) {
-      if (valid) ph.finish(st, p, 1.0);
+      if (valid) ph.finish(st, p, seen ? 0.0 : 1.0);
     } else {
       if (valid) ph.finish(st, p);
     }
@@ -1136,15 +1198,20 @@ struct Pos3 {
 };
 
 template <class T, class Ph, bool kMany>
-__global__ __launch_bounds__(kTileBlock) void k_tile_f64(ClDev c, const T* __restrict__ pos, size_t stride,
-                                                         Ph ph1, const Ph* __restrict__ tab,
+__global__ __launch_bounds__(kTileBlock, 4) void k_tile_f64(ClDev c, const T* __restrict__ pos, size_t stride,
+                                                         float spx, float spy, float spz, Ph ph1, const Ph* __restrict__ tab,
                                                          const SysGrid<T>* __restrict__ sys,
                                                          const TargetItem* __restrict__ items,
                                                          const uint32_t* __restrict__ n_items_p,
                                                          uint32_t* __restrict__ counter) {
-  __shared__ Pos3<T> lds[kTileWaves][kTileChunk];
+  constexpr int kChunk = tile_chunk<Pos3<T>>();
+  __shared__ Pos3<T> lds[kTileWaves][kChunk];
+  __shared__ uint32_t ldsj[kTileWaves][kChunk];
+  __shared__ unsigned long long ldsm[kTileWaves][kChunk / 64][kWave];
   const int lane = threadIdx.x & (kWave - 1);
   Pos3<T>* buf = lds[threadIdx.x / kWave];
+  uint32_t* bufj = ldsj[threadIdx.x / kWave];
+  unsigned long long(*mk)[kWave] = ldsm[threadIdx.x / kWave];
   const uint32_t n_items = *n_items_p;
   for (;;) {
     const uint32_t it = next_unit(counter);
@@ -1160,35 +1227,56 @@ __global__ __launch_bounds__(kTileBlock) void k_tile_f64(ClDev c, const T* __res
     auto test = [&](const Pos3<T>& Q) {
       return dist2_unfused<double>(xp - double(Q.x), yp - double(Q.y), zp - double(Q.z)) < ph.rc2;
     };
-    for_each_run(c, G, [&](uint32_t ja, uint32_t jb) {
-      for (uint32_t j0 = ja; j0 < jb; j0 += kTileChunk) {
-        const uint32_t m = jb - j0 < uint32_t(kTileChunk) ? jb - j0 : uint32_t(kTileChunk);
-        __builtin_amdgcn_wave_barrier();
-        for (uint32_t k = uint32_t(lane); k < m; k += kWave) {
-          const uint32_t j = j0 + k;
+    if (kMany) {
+      const SysGrid<T>& S = sys[ti.ncx >> 8];
+      spx = float(S.sp[0]);
+      spy = float(S.sp[1]);
+      spz = float(S.sp[2]);
+    }
+    // relative to the middle target; the bounds as in the Verlet build's count pass
+    const uint32_t mid = ti.n / 2;
+    const double ox = lane_value(xp, mid), oy = lane_value(yp, mid), oz = lane_value(zp, mid);
+    const float tx = float(xp - ox), ty = float(yp - oy), tz = float(zp - oz);
+    const float B1 = float(c.box_nn + 1u), nx = float(G.ncx), bx = nx + float(c.box_nn);
+    const float rt2 = nx * nx * spx * spx + spy * spy + spz * spz;
+    const float rc2 = bx * bx * spx * spx + B1 * B1 * (spy * spy + spz * spz);
+    const float r2f = float(ph.rc2);
+    const bool fast = __ballot(!(__builtin_fmaf(tx, tx, __builtin_fmaf(ty, ty, tz * tz)) <= rt2 * 1.01f)) == 0ull;
+    MatrixTest mt;
+    mt.targets(tx, ty, tz, r2f + (2.05f * (rt2 + rc2) + r2f) * 0x1p-19f, rc2 * 1.01f, ti.n > 32u);
+    bool seen = false;
+    for_each_chunk<kChunk>(
+        c, G, lane,
+        [&](uint32_t k, uint32_t j) {
           buf[k] = Pos3<T>{pos[j], pos[stride + j], pos[2 * stride + j]};
-        }
-        __builtin_amdgcn_wave_barrier();
-        uint32_t mk[4];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const uint32_t k0 = uint32_t(q) * 32u;
-          mk[q] = k0 < m ? staged_hits(buf, k0, m - k0 < 32u ? m - k0 : 32u, test) : 0u;
-          if (!valid) mk[q] = 0u;
-        }
-        for_each_hit(mk, [&](uint32_t k) {
-          const uint32_t j = j0 + k;
-          if (j == p) return;
-          const Pos3<T> Q = buf[k];
-          const double rx = xp - double(Q.x), ry = yp - double(Q.y), rz = zp - double(Q.z);
-          double d2 = dist2_unfused<double>(rx, ry, rz);
-          if constexpr (Ph::kSmooth) d2 = __builtin_fmax(d2, 1e-280);  // coincident particles
-          ph.pair(st, ph.aux(j), rx, ry, rz, d2);
+          bufj[k] = j;
+        },
+        [&](uint32_t m) {
+          chunk_hits(
+              mt, fast, buf, m, lane, valid, mk,
+              [&](const Pos3<T>& Q, float* x, float* y, float* z) {
+                *x = float(double(Q.x) - ox);
+                *y = float(double(Q.y) - oy);
+                *z = float(double(Q.z) - oz);
+              },
+              test);
+          for_each_hit(mk, (m + 63u) / 64u, lane, [&](uint32_t k) {
+            const Pos3<T> Q = buf[k];
+            const uint32_t j = bufj[k];
+            const double rx = xp - double(Q.x), ry = yp - double(Q.y), rz = zp - double(Q.z);
+            double d2 = dist2_unfused<double>(rx, ry, rz);
+            if (!(d2 < ph.rc2)) return;
+            if constexpr (Ph::kSmooth) {
+              d2 = __builtin_fmax(d2, 1e-280);  // coincident particles, and the particle itself
+              seen = true;
+            } else {
+              if (j == p) return;
+            }
+            ph.pair(st, ph.aux(j), rx, ry, rz, d2);
+          });
         });
-      }
-    });
     if constexpr (Ph::kSmooth) {
-      if (valid) ph.finish(st, p, 1.0);
+      if (valid) ph.finish(st, p, seen ? 0.0 : 1.0);
     } else {
       if (valid) ph.finish(st, p);
     }
@@ -1585,8 +1673,9 @@ static int launch_f64(const PairCtx& x, const void* pos, size_t stride, const Ph
     } else {
       TileQueue q;
       OFP_TRY(tile_queue(x, &q, s));
-      k_tile_f64<T, Ph, false><<<tile_grid(), kTileBlock, 0, s>>>(x.c, P, stride, ph, nullptr, nullptr, q.items,
-                                                                   q.n_items, q.counter);
+      k_tile_f64<T, Ph, false><<<tile_grid(), kTileBlock, 0, s>>>(
+          x.c, P, stride, float(x.v.spacing[0]), float(x.v.spacing[1]), float(x.v.spacing[2]), ph, nullptr, nullptr,
+          q.items, q.n_items, q.counter);
     }
     OFP_LAUNCHED();
     return OFP_OK;
@@ -1873,7 +1962,8 @@ static int launch_lj_tiles(const PairCtx& x, int precision, const void* pos_sort
                                                                           q.items, q.n_items, q.counter);
   } else {
     using Ph = LJ64T<kU>;
-    k_tile_f64<T, Ph, true><<<tile_grid(), kTileBlock, 0, s>>>(x.c, static_cast<const T*>(pos_sorted), stride, Ph{},
+    k_tile_f64<T, Ph, true><<<tile_grid(), kTileBlock, 0, s>>>(x.c, static_cast<const T*>(pos_sorted), stride, 0.f,
+                                                               0.f, 0.f, Ph{},
                                                                static_cast<const Ph*>(tab), sys, q.items, q.n_items,
                                                                q.counter);
   }

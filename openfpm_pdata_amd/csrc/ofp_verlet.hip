@@ -50,7 +50,6 @@ namespace ofp {
 constexpr int kVlBlock = 256;
 constexpr int kVlWaves = kVlBlock / kWave;
 constexpr uint32_t kBlk = 32;  // candidates per block (bits of a mask word)
-typedef float v16f __attribute__((ext_vector_type(16)));
 
 // The coordinates of 8 consecutive particles, x y z interleaved (read with
 // scalar loads; the element alignment is all a scalar load needs).
@@ -102,24 +101,14 @@ struct ItemRuns {
 };
 template <class T>
 __device__ __forceinline__ ItemRuns item_runs(const ClDev& c, const ItemGeom<T>& G, int lane) {
-  const int B = int(c.box_nn), W = 2 * B + 1;
-  const int xa = G.cx0 - B > 0 ? G.cx0 - B : 0;
-  const int xe = G.cx0 + G.ncx - 1 + B;
-  const int xb = xe < int(G.d0) - 1 ? xe : int(G.d0) - 1;
-  const int zz = G.cz + lane / W - B, yy = G.cy + lane % W - B;
-  ItemRuns R{0, 0, 0, 0};
-  if (lane < W * W && zz >= 0 && zz < int(G.d2) && yy >= 0 && yy < int(G.d1)) {
-    const uint32_t rowc = G.cbase + G.d0 * (uint32_t(yy) + G.d1 * uint32_t(zz));
-    R.ja = uint32_t(c.cs[rowc + uint32_t(xa)]);
-    R.jb = uint32_t(c.cs[rowc + uint32_t(xb) + 1]);
-  }
+  const uint2 run = lane_run(c, G, lane);
+  ItemRuns R{run.x, run.y, 0, 0};
   const uint32_t nb = (R.jb - R.ja + kBlk - 1) / kBlk;
   const uint32_t inc = wave_incl_scan(nb);
   R.first = inc - nb;
   R.blocks = __builtin_amdgcn_readlane(inc, kWave - 1);
   return R;
 }
-static_assert((2 * kMaxBoxNN + 1) * (2 * kMaxBoxNN + 1) <= kWave, "one lane per run");
 
 // Orders a wave's LDS accesses for the compiler (the LDS itself serves a wave's
 // accesses in order).
@@ -139,37 +128,12 @@ __device__ __forceinline__ void block_table(const ItemRuns& R, uint32_t w0, uint
   lds_order();
 }
 
-// Lane halves: {a_lo, b_lo} and {a_hi, b_hi}.
-__device__ __forceinline__ void swap_halves(uint32_t& a, uint32_t& b) {
-  const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
-  a = r[0];
-  b = r[1];
-}
-__device__ __forceinline__ void swap_halves(float& a, float& b) {
-  uint32_t x = __float_as_uint(a), y = __float_as_uint(b);
-  swap_halves(x, y);
-  a = __uint_as_float(x);
-  b = __uint_as_float(y);
-}
 // min(m, |a|, |b|) in one instruction (no canonicalisation of the operands)
 __device__ __forceinline__ float min3_abs(float m, float a, float b) {
   float r;
   asm("v_min3_f32 %0, %1, |%2|, |%3|" : "=v"(r) : "v"(m), "v"(a), "v"(b));
   return r;
 }
-template <class T>
-__device__ __forceinline__ T lane_value(T v, uint32_t lane);
-template <>
-__device__ __forceinline__ float lane_value<float>(float v, uint32_t lane) {
-  return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), lane));
-}
-template <>
-__device__ __forceinline__ double lane_value<double>(double v, uint32_t lane) {
-  const unsigned long long u = static_cast<unsigned long long>(__double_as_longlong(v));
-  const uint32_t lo = __builtin_amdgcn_readlane(uint32_t(u), lane), hi = __builtin_amdgcn_readlane(uint32_t(u >> 32), lane);
-  return __longlong_as_double(static_cast<long long>((static_cast<unsigned long long>(hi) << 32) | lo));
-}
-
 // Part `part` of P of `total` (monotonic in part, 0 and total at the ends).
 __device__ __forceinline__ uint32_t part_begin(uint32_t total, uint32_t part, uint32_t P) {
   return P == 1 ? (part ? total : 0u) : uint32_t(uint64_t(total) * part / P);
@@ -271,11 +235,7 @@ __global__ __launch_bounds__(kVlBlock, 4) void k_vl_count(ClDev c, const T* __re
   const uint32_t n_units = *n_items_p * P;
   const bool keep = mstate[0] <= mask_cap;  // grid-uniform
   if (!keep && blockIdx.x == 0 && threadIdx.x == 0) atomicOr(&mstate[1], 1ull);
-  // the candidate of this lane's matrix row: row 8 q + 4 h + m of a 32-block is
-  // candidate 16 h + 15 - (4 q + m), so a lane's results i = 4 q + m (rows
-  // 8 (i / 4) + 4 (lane / 32) + i % 4) are candidates 15 - i of its half
-  const uint32_t mrow = uint32_t(lane) & 31u;
-  const uint32_t mine = 16u * ((mrow >> 2) & 1u) + 15u - (4u * (mrow >> 3) + (mrow & 3u));
+  const uint32_t mine = matrix_candidate(uint32_t(lane));
   for (;;) {
     const uint32_t un = next_unit(counter);
     if (un >= n_units) break;
