@@ -96,8 +96,9 @@ constexpr int kRxMaxBits = 8;
 // kRxChunked it sums those of its own chunk of tiles and the chunks' sums, which
 // the histogram blocks add up with atomics (at most 32 adds per word): two launches
 // per pass.  The rows a block sums are loaded kColBatch at a time, one batch after
-// another: at 65 tiles 2 batches with chunks, 5 without.  Beyond kRxChunked, the column kernels do it (four launches): a block would read
-// over 100 rows of 1 KB for its 4096 keys.
+// another: at 65 tiles 2 batches with chunks, 5 without.  Beyond kRxChunked, the
+// column kernels do it (four launches): a block would read over 100 rows of 1 KB
+// for its 4096 keys.
 constexpr uint32_t kRxDirect = 32;
 constexpr uint32_t kRxChunked = 2048;
 // Below this many particles the host does not wait for the order check before it
@@ -154,7 +155,8 @@ __global__ __launch_bounds__(kRxBlock) void k_rx_hist(Key key, const uint32_t* _
   const uint32_t n = count_of(n_host, n_dev);
   const uint32_t t = blockIdx.x;
   if (clear)
-    for (uint64_t i = uint64_t(t) * kRxBlock + threadIdx.x; i < n_clear; i += uint64_t(gridDim.x) * kRxBlock) clear[i] = 0ull;
+    for (uint64_t i = uint64_t(t) * kRxBlock + threadIdx.x; i < n_clear; i += uint64_t(gridDim.x) * kRxBlock)
+      clear[i] = 0ull;
   for (int d = threadIdx.x; d < kRxBins; d += kRxBlock) h[d] = 0;
   __syncthreads();
   const int lane = threadIdx.x & (kWave - 1);
@@ -825,7 +827,9 @@ __device__ __forceinline__ void lds_barrier() {
 struct Halves {
   uint32_t w[kFarIters / 2] = {};
   __device__ __forceinline__ uint32_t get(int i) const { return i & 1 ? w[i / 2] >> 16 : w[i / 2] & 0xFFFFu; }
-  __device__ __forceinline__ void put(int i, uint32_t v) { w[i / 2] = i & 1 ? (w[i / 2] & 0xFFFFu) | v << 16 : (w[i / 2] & 0xFFFF0000u) | v; }
+  __device__ __forceinline__ void put(int i, uint32_t v) {
+    w[i / 2] = i & 1 ? (w[i / 2] & 0xFFFFu) | v << 16 : (w[i / 2] & 0xFFFF0000u) | v;
+  }
   // opaque to the compiler, which would keep the 32 unpacked values across planes
   __device__ __forceinline__ void hide() {
 #pragma unroll
@@ -1577,10 +1581,9 @@ int ofp_cl_items_(const ofp_cl* hc, const TargetItem** items, const uint32_t** n
     const uint32_t off = h->dtype == OFP_F32 ? uint32_t(offsetof(SysGrid<float>, divc) / 4)
                                              : uint32_t(offsetof(SysGrid<double>, divc) / 4);
     const uint32_t* desc = h->n_sys ? static_cast<const uint32_t*>(h->sys) + off : nullptr;
-    k_cl_items<<<grid_for(h->n_rows, kItemRows), kItemRows * kWave, 0, s>>>(h->scan64.as<unsigned long long>(), h->divc[0],
-                                                                h->n_rows, h->n_sys, h->rbase, desc, words,
-                                                                h->items.as<TargetItem>(),
-                                                                h->nitems.as<uint32_t>() + kQueueWords);
+    k_cl_items<<<grid_for(h->n_rows, kItemRows), kItemRows * kWave, 0, s>>>(
+        h->scan64.as<unsigned long long>(), h->divc[0], h->n_rows, h->n_sys, h->rbase, desc, words,
+        h->items.as<TargetItem>(), h->nitems.as<uint32_t>() + kQueueWords);
     OFP_LAUNCHED();
     h->items_cap = need;
     h->items_valid = true;

@@ -560,28 +560,6 @@ __device__ __forceinline__ ItemGeom<T> item_geom(const ClDev& c, const TargetIte
   return g;
 }
 
-// The item's (2B+1)^2 x-runs in traversal order: fn(ja, jb) with wave-uniform
-// bounds of sorted indices.
-template <class T, class F>
-__device__ __forceinline__ void for_each_run(const ClDev& c, const ItemGeom<T>& G, F&& fn) {
-  const int B = int(c.box_nn);
-  const int xa = G.cx0 - B > 0 ? G.cx0 - B : 0;
-  const int xe = G.cx0 + G.ncx - 1 + B;
-  const int xb = xe < int(G.d0) - 1 ? xe : int(G.d0) - 1;
-  for (int dz = -B; dz <= B; ++dz) {
-    const int zz = G.cz + dz;
-    if (zz < 0 || zz >= int(G.d2)) continue;
-    for (int dy = -B; dy <= B; ++dy) {
-      const int yy = G.cy + dy;
-      if (yy < 0 || yy >= int(G.d1)) continue;
-      const uint32_t rowc = G.cbase + G.d0 * (uint32_t(yy) + G.d1 * uint32_t(zz));
-      const uint32_t ja = __builtin_amdgcn_readfirstlane(uint32_t(c.cs[rowc + uint32_t(xa)]));
-      const uint32_t jb = __builtin_amdgcn_readfirstlane(uint32_t(c.cs[rowc + uint32_t(xb) + 1]));
-      if (ja < jb) fn(ja, jb);
-    }
-  }
-}
-
 // Run r of the item (traversal order) in lane r < (2B+1)^2: [x, y), empty outside the
 // grid and in the other lanes.
 template <class T>

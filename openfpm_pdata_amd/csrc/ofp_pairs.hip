@@ -989,22 +989,32 @@ __global__ __launch_bounds__(256) void k_rows_smooth(ClDev c, const unsigned lon
 // target items from the cell list's item queue: up to 64 domain particles of
 // consecutive cells on one x-row of the grid, one per lane.  The item's
 // candidates are the (2B+1)^2 x-runs of its stencil, each a contiguous range
-// of sorted indices; they pass through the wave's LDS region kTileChunk at a
-// time (coalesced loads).  Check: every lane tests its own target against every
-// staged candidate (one broadcast LDS read per candidate), appending one bit
-// per candidate to its hit mask (the compare's lane mask as v_addc's carry).
+// of sorted indices; they pass through the wave's LDS region tile_chunk() at a
+// time (coalesced loads).  Check: the matrix cores give every target a bit per
+// staged candidate that may lie within the cut-off (MatrixTest; tested one by one
+// in the vector ALU where coordinates lie beyond its bounds).
 // Evaluate: each lane walks its own set bits in ascending order and evaluates
-// those pairs from the staged records.  A target's pairs are summed in one
+// those pairs from the staged records, deciding the cut-off where the physics does
+// not vanish there by itself.  A target's pairs are summed in one
 // lane in ascending sorted index, so the results do not depend on the order in
 // which the items are taken.  Candidates that lie in the union of the item's
 // stencils but outside a target's own stencil are more than B cells away in x
 // from it, so they are misses for it.
+// Bound by the evaluation's instructions (31 an entry of the density pass) and its
+// idle lanes (38 % busy with rounds of 128 candidates, whose runs' hits depend on a
+// target's place in its cell; larger rounds even that out).  Tests in the vector
+// ALU, eleven instructions per candidate and wave, took half of the passes.
+// 1,092,727 particles on a lattice (FP32C, density and force): 632 and 682 -> 372
+// and 391 us (128 candidates a round 445 and 453, 320: 380 and 402); 65,536 of a
+// gas, FP64 LJ: 112 -> 55 us.
 //
 // FP32C separations: the union spans at most kItemMaxCells - 1 + B cells in x
 // from any of the item's targets, so a candidate is either within 2^31 quanta
 // (the wrapped subtraction is exact) or its wrapped separation is still more
 // than B cells (one cell of slack for positions that have drifted since the
-// cells were built): no far candidate passes the check.
+// cells were built): no far candidate's pair is within the cut-off.  The masks'
+// coordinates are relative to the middle of the item's cells, from which no
+// candidate within a target's cut-off is 2^31 quanta away (static_assert below).
 // Candidates staged per round: a lane's hits of a run of cells vary with its place
 // in y and z, those of several runs less, and a round takes as long as its busiest
 // lane.  Four blocks of four waves fit a CU's registers, 40 KB of LDS each.
@@ -1014,6 +1024,7 @@ constexpr int tile_chunk() {
 }
 constexpr int kTileBlock = 256;  // four independent waves
 constexpr int kTileWaves = kTileBlock / kWave;
+static_assert(int(kItemMaxCells) / 2 + 1 + kMaxBoxNN <= 8, "wrapped FP32C coordinates of the masks");
 static_assert(16 - (int(kItemMaxCells) - 1 + kMaxBoxNN) - 2 > kMaxBoxNN, "wrapped FP32C separations");
 
 // Hit bits of staged candidates k0 .. k0 + cnt - 1 (cnt <= 32, uniform) for
@@ -1199,7 +1210,8 @@ struct Pos3 {
 
 template <class T, class Ph, bool kMany>
 __global__ __launch_bounds__(kTileBlock, 4) void k_tile_f64(ClDev c, const T* __restrict__ pos, size_t stride,
-                                                         float spx, float spy, float spz, Ph ph1, const Ph* __restrict__ tab,
+                                                         float spx, float spy, float spz, Ph ph1,
+                                                         const Ph* __restrict__ tab,
                                                          const SysGrid<T>* __restrict__ sys,
                                                          const TargetItem* __restrict__ items,
                                                          const uint32_t* __restrict__ n_items_p,

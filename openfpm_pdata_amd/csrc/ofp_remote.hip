@@ -52,7 +52,12 @@
 
 namespace ofp {
 
-constexpr int kRemoteTile = 1024;     // outputs per wave in the ordering passes
+// Outputs per wave in the ordering passes, in rounds of 64 one after another: at
+// least one round, and as few as keep the table of (slot, tile) counts within the
+// one-launch scan, at most kRemoteTile.  Tiles of 1024 leave most CUs without a
+// wave: a rank of 524,288 particles, map and ghosts, 67 -> 26 us.
+constexpr uint32_t kRemoteTile = 1024;
+constexpr uint32_t kRemoteTable = 16384;
 constexpr int kRemoteMaxSlots = 256;  // destination processors per rank
 constexpr uint32_t kGeoMaxDiv = 64;   // geometric cells per dimension
 
@@ -218,7 +223,7 @@ __global__ __launch_bounds__(256) void k_remote_emit(RemoteBoxes<T> B, const T* 
   });
 }
 
-// One wave per tile of kRemoteTile outputs, in rounds of 64 in output order.
+// One wave per tile of outputs, in rounds of 64 in output order.
 // kScatter = false: table[slot * n_tiles + tile] = outputs of the tile in slot.
 // kScatter = true: every output goes to toff[slot * n_tiles + tile] + (earlier
 // outputs of the tile in the same slot).
@@ -226,7 +231,7 @@ template <bool kScatter>
 __global__ __launch_bounds__(256) void k_remote_order(const uint32_t* __restrict__ oslot,
                                                       const uint32_t* __restrict__ oproc,
                                                       const unsigned long long* __restrict__ oid, uint32_t m,
-                                                      uint32_t n_slots, uint32_t n_tiles,
+                                                      uint32_t n_slots, uint32_t tile_size, uint32_t n_tiles,
                                                       uint32_t* __restrict__ table,
                                                       const uint32_t* __restrict__ toff,
                                                       uint32_t* __restrict__ sproc,
@@ -239,8 +244,8 @@ __global__ __launch_bounds__(256) void k_remote_order(const uint32_t* __restrict
   uint32_t* const r = run[w];
   for (uint32_t s = uint32_t(lane); s < n_slots; s += kWave) r[s] = kScatter ? toff[size_t(s) * n_tiles + tile] : 0u;
   __builtin_amdgcn_wave_barrier();
-  const uint32_t t0 = tile * uint32_t(kRemoteTile);
-  for (uint32_t i0 = t0; i0 < t0 + uint32_t(kRemoteTile) && i0 < m; i0 += kWave) {
+  const uint32_t t0 = tile * tile_size;
+  for (uint32_t i0 = t0; i0 < t0 + tile_size && i0 < m; i0 += kWave) {
     const uint32_t i = i0 + uint32_t(lane);
     const bool valid = i < m;
     const uint32_t key = valid ? oslot[i] : 0xFFFFFFFFu;
@@ -353,18 +358,20 @@ static int order_by_slot(DevBuf& table, DevBuf& toff, DevBuf& tmp, DevBuf& pcoun
                          uint32_t* sproc, unsigned long long* sid, std::vector<uint32_t>* starts, hipStream_t s) {
   starts->assign(n_slots + 1, 0u);
   if (m == 0) return OFP_OK;
-  const uint32_t n_tiles = (m + uint32_t(kRemoteTile) - 1) / uint32_t(kRemoteTile);
+  uint32_t tile = kWave;
+  while (tile < kRemoteTile && size_t(n_slots) * ((m + size_t(tile) - 1) / tile) > kRemoteTable) tile *= 2;
+  const uint32_t n_tiles = uint32_t((m + size_t(tile) - 1) / tile);
   const size_t tn = size_t(n_slots) * n_tiles;
   OFP_TRY(table.ensure((tn + 1) * sizeof(uint32_t)));
   OFP_TRY(toff.ensure((tn + 1) * sizeof(uint32_t)));
   OFP_TRY(tmp.ensure(scan_tmp_bytes(tn)));
   OFP_TRY(pcount.ensure((size_t(n_slots) + 1) * sizeof(uint32_t)));
   const unsigned grid = grid_for(n_tiles, 256 / kWave);
-  k_remote_order<false><<<grid, 256, 0, s>>>(oslot, nullptr, nullptr, m, n_slots, n_tiles, table.as<uint32_t>(),
+  k_remote_order<false><<<grid, 256, 0, s>>>(oslot, nullptr, nullptr, m, n_slots, tile, n_tiles, table.as<uint32_t>(),
                                              nullptr, nullptr, nullptr);
   OFP_LAUNCHED();
   OFP_TRY(scan_excl_u32(table.as<uint32_t>(), toff.as<uint32_t>(), tn, tmp.p, s));
-  k_remote_order<true><<<grid, 256, 0, s>>>(oslot, oproc, oid, m, n_slots, n_tiles, nullptr, toff.as<uint32_t>(),
+  k_remote_order<true><<<grid, 256, 0, s>>>(oslot, oproc, oid, m, n_slots, tile, n_tiles, nullptr, toff.as<uint32_t>(),
                                             sproc, sid);
   OFP_LAUNCHED();
   k_remote_slot_starts<<<grid_for(n_slots + 1, 256), 256, 0, s>>>(toff.as<uint32_t>(), n_slots, n_tiles,

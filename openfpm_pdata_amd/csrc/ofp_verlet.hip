@@ -513,7 +513,9 @@ __global__ __launch_bounds__(kVlBlock) void k_vl_fill(ClDev c, const SysGrid<T>*
       next = fn < total ? words[fn] : 0u;
       const unsigned long long nz = __ballot(bits != 0u);
       if (bits) {
-        const uint32_t k = queued + __builtin_amdgcn_mbcnt_hi(uint32_t(nz >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(nz), 0u));
+        const uint32_t lo = __builtin_amdgcn_mbcnt_lo(uint32_t(nz), 0u);
+        const uint32_t below = __builtin_amdgcn_mbcnt_hi(uint32_t(nz >> 32), lo);
+        const uint32_t k = queued + below;
         queue[k] = make_uint2(bits, block_first(w));
       }
       queued += uint32_t(__popcll(nz));
