@@ -633,8 +633,10 @@ struct EmitArgs {
   const SysGrid<T>* sys;
   const uint32_t* sid;
   uint32_t* sid_sorted;
-  // the passes carried the positions into pos_sorted when *disorder says so
+  // the passes carried the positions into pos_sorted when *disorder says so, or they
+  // have been placed there
   const unsigned long long* disorder;
+  bool placed;
 };
 
 template <class T>
@@ -689,7 +691,7 @@ __global__ __launch_bounds__(256) void k_cl_emit(EmitArgs<T> A, const uint32_t* 
   const uint32_t f = blockIdx.x * blockDim.x + threadIdx.x;
   const uint32_t n = count_of(n_host, n_dev);
   if (f >= n) return;
-  const bool pos_done = A.pos_sorted && carry_positions(A.disorder, n);
+  const bool pos_done = A.placed || (A.pos_sorted && carry_positions(A.disorder, n));
   const uint32_t c = keys[f];
   const unsigned long long s0 = cs[c];
   cl_emit(A, s2n[f], f, c, uint32_t(s0 >> 32), f - uint32_t(s0), pos_done);
@@ -804,16 +806,17 @@ __global__ __launch_bounds__(kRxBlock) void k_cl_first(CellGeom<T> g, EmitArgs<T
 // each value is read and written twice, its place once.  A second step that
 // scattered in the L2 instead (128 ranges, all blocks of a range on one XCD) took
 // 200-230 us per 2^27 bytes, the L2's rate of partial stores.  Restore of 2^25
-// particles from random order, 5 planes of 24 bytes: 2.40 -> 1.03 ms.
+// particles from random order, 5 planes of 24 bytes: 2.40 -> 0.94 ms.
 constexpr int kFarBlock = 1024;
 constexpr int kFarIters = 32;
 constexpr int kFarShift = 15;
 constexpr uint32_t kFarTile = uint32_t(kFarBlock * kFarIters);
 static_assert(kFarTile == 1u << kFarShift, "a range is a tile");
 constexpr uint32_t kFarRanges = 2 * kFarBlock;  // at most
-constexpr size_t kFarFrom = size_t(1) << 22;  // restore of 24 bytes: 128 us at 2^21 (143 direct), 156 (265) here
+constexpr size_t kFarFrom = size_t(1) << 22;  // restore of 24 bytes: 128 us at 2^21 (143 direct), 132 (265) here
 constexpr size_t kFarTo = size_t(kFarRanges) << kFarShift;
-constexpr size_t kFarScratch = 10;  // least scratch, bytes per particle
+constexpr size_t kFarScratch = 10;      // least scratch, bytes per particle
+constexpr size_t kFarScratchFull = 26;  // six 4-byte planes at a time
 
 // Barrier over the block's LDS only: loads and stores of global memory stay in flight.
 __device__ __forceinline__ void lds_barrier() {
@@ -1106,8 +1109,11 @@ static int cl_build_t(ofp_cl* h, const Key& key, const EmitArgs<T>& A0, size_t n
   // (the passes before the last alternate between two payload buffers, the last
   // one writes the sorted positions); the kernels carry them only when the
   // descents say the input is far from cell order (carry_positions), else
-  // k_cl_emit gathers them.
-  const bool payload = A0.pos_sorted != nullptr;
+  // k_cl_emit gathers them.  Few particles' positions stay in the caches and are
+  // gathered in any order (300,000 random ones: build 91 -> 82 us, 2^20: 205 -> 192);
+  // many are placed by permute_far (build of 2^25: 2.37 -> 1.92 ms).
+  const bool payload = A0.pos_sorted != nullptr && n_cap > kRxSmall &&
+                       !(first && n_cap >= kFarFrom && n_cap <= kFarTo);
   if (payload && passes > 1) OFP_TRY(h->payload.ensure(2 * 3 * n_cap * sizeof(T)));
   T* pbuf[2] = {h->payload.as<T>(), h->payload.as<T>() + 3 * n_cap};
   // ping-pong buffers chosen so that the last pass lands in keys / s2n
@@ -1214,25 +1220,51 @@ static int cl_build_t(ofp_cl* h, const Key& key, const EmitArgs<T>& A0, size_t n
   if (first && n_cap >= kFarFrom && n_cap <= kFarTo) {
     OFP_HIP(hipEventSynchronize(h->checked));
     if (*h->desc * kDisorderDen > n_cap) {
-      h->far = h->payload.ensure(kFarScratch * (n_cap + 8)) == OFP_OK &&
-               h->cursors.ensure(kFarRanges * 4) == OFP_OK;
-      if (!h->far) clear_error();  // no memory: without it
+      // scratch for five or six floats at a time, or for what there is memory
+      h->far = h->cursors.ensure(kFarRanges * 4) == OFP_OK &&
+               (h->payload.ensure(kFarScratchFull * (n_cap + 8)) == OFP_OK ||
+                h->payload.ensure(kFarScratch * (n_cap + 8)) == OFP_OK);
+      clear_error();  // without it, if there is none
     }
   }
   if (h->far) {
+    PlaneArgs index{};  // n2s[s2n[f]] = f
+    index.n = 1;
+    index.esz[0] = 4;
+    index.dst[0] = reinterpret_cast<uint64_t>(h->n2s.p);
+    OFP_TRY(go_far(h, h->s2n.as<uint32_t>(), index, s));
+    PlaneArgs planes = A0.pa;
+    if (A0.pos_sorted) {
+      PlaneArgs pos{};
+      for (int k = 0; k < 3; ++k) {
+        pos.src[k] = reinterpret_cast<uint64_t>(A0.pos + size_t(k) * A0.stride);
+        pos.dst[k] = reinterpret_cast<uint64_t>(A0.pos_sorted + size_t(k) * A0.sorted_stride);
+        pos.esz[k] = uint32_t(sizeof(T));
+      }
+      pos.n = 3;
+      for (int k = 0; k < planes.n && pos.n < kMaxPlanes; ++k, ++pos.n) {
+        pos.src[pos.n] = planes.src[k];
+        pos.dst[pos.n] = planes.dst[k];
+        pos.esz[pos.n] = planes.esz[k];
+      }
+      OFP_TRY(go_far(h, h->n2s.as<uint32_t>(), pos, s));
+      const int done = pos.n - 3;
+      planes.n -= done;
+      for (int k = 0; k < planes.n; ++k) {
+        planes.src[k] = planes.src[k + done];
+        planes.dst[k] = planes.dst[k + done];
+        planes.esz[k] = planes.esz[k + done];
+      }
+      A.placed = true;
+    }
+    OFP_TRY(go_far(h, h->n2s.as<uint32_t>(), planes, s));
     A.n2s = nullptr;
     A.pa.n = 0;
   }
   k_cl_emit<T><<<grid_for(n_cap, 256), 256, 0, s>>>(A, h->keys.as<uint32_t>(), h->s2n.as<uint32_t>(), n_host, n_dev,
                                                      cs, check);
   OFP_LAUNCHED();
-  if (!h->far) return OFP_OK;
-  PlaneArgs index{};  // n2s[s2n[f]] = f
-  index.n = 1;
-  index.esz[0] = 4;
-  index.dst[0] = reinterpret_cast<uint64_t>(h->n2s.p);
-  OFP_TRY(go_far(h, h->s2n.as<uint32_t>(), index, s));
-  return go_far(h, h->n2s.as<uint32_t>(), A0.pa, s);
+  return OFP_OK;
 }
 
 template <class T, class Key>

@@ -59,6 +59,22 @@ def test_far(n, order):
             assert torch.equal(a, b)
 
 
+def test_far_most_planes():
+    """24 planes, the most a call takes, with the positions (3 more)."""
+    n, side = (1 << 22) + 11, 64
+    pos = torch.rand((3, n), generator=torch.Generator(device="cuda").manual_seed(5), device="cuda") * side
+    cl = vdm.CellListGPU(torch.float32, (0.0,) * 3, (float(side),) * 3, (side,) * 3,
+                         vdm.CL_NON_SYMMETRIC | vdm.CL_GPU_REORDER, 1.0)
+    src = _planes(n, [4, 8, 4] * 8, 7)
+    dst = [torch.zeros_like(p) for p in src]
+    out = torch.empty_like(pos)
+    cl.construct(pos, n, n, out, _args(src), _args(dst))
+    s2n = cl.arrays()["s2n"].long()
+    assert torch.equal(out, pos[:, s2n])
+    for a, b in zip(src, dst):
+        assert torch.equal(b, a[s2n])
+
+
 def test_far_streams():
     """Restores of one list on two streams share its scratch one after another."""
     n, side = (1 << 22) + 3, 64
