@@ -1016,15 +1016,15 @@ __global__ __launch_bounds__(256) void k_cl_restore(uint32_t n, const uint32_t* 
   copy_planes(pa, j, s2n[j]);
 }
 
-// permute_far over the list's particles (h->far), with the list's scratch.
-static int go_far(ofp_cl* h, const uint32_t* idx, const PlaneArgs& pa, hipStream_t s) {
+// permute_far with the list's scratch (which is there).
+static int go_far(ofp_cl* h, const uint32_t* idx, uint32_t n, const PlaneArgs& pa, hipStream_t s) {
   if (pa.n == 0) return OFP_OK;
   std::lock_guard<std::mutex> lock(h->far_lock);
   if (h->far_done)
     OFP_HIP(hipStreamWaitEvent(s, h->far_done, 0));
   else
     OFP_HIP(hipEventCreateWithFlags(&h->far_done, hipEventDisableTiming));
-  OFP_TRY(permute_far(idx, uint32_t(h->n_part), pa, h->payload.p, h->payload.cap, h->cursors.as<uint32_t>(), s));
+  OFP_TRY(permute_far(idx, n, pa, h->payload.p, h->payload.cap, h->cursors.as<uint32_t>(), s));
   OFP_HIP(hipEventRecord(h->far_done, s));
   return OFP_OK;
 }
@@ -1038,7 +1038,7 @@ static int permute_route(const ofp_cl* h, const uint32_t* idx, const PlaneArgs& 
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   OFP_HIP(hipStreamIsCapturing(s, &cap));
   if (cap != hipStreamCaptureStatusNone) return OFP_OK;
-  OFP_TRY(go_far(const_cast<ofp_cl*>(h), idx, pa, s));  // its scratch only
+  OFP_TRY(go_far(const_cast<ofp_cl*>(h), idx, uint32_t(h->n_part), pa, s));  // its scratch only
   *done = true;
   return OFP_OK;
 }
@@ -1232,7 +1232,7 @@ static int cl_build_t(ofp_cl* h, const Key& key, const EmitArgs<T>& A0, size_t n
     index.n = 1;
     index.esz[0] = 4;
     index.dst[0] = reinterpret_cast<uint64_t>(h->n2s.p);
-    OFP_TRY(go_far(h, h->s2n.as<uint32_t>(), index, s));
+    OFP_TRY(go_far(h, h->s2n.as<uint32_t>(), n_host, index, s));
     PlaneArgs planes = A0.pa;
     if (A0.pos_sorted) {
       PlaneArgs pos{};
@@ -1247,7 +1247,7 @@ static int cl_build_t(ofp_cl* h, const Key& key, const EmitArgs<T>& A0, size_t n
         pos.dst[pos.n] = planes.dst[k];
         pos.esz[pos.n] = planes.esz[k];
       }
-      OFP_TRY(go_far(h, h->n2s.as<uint32_t>(), pos, s));
+      OFP_TRY(go_far(h, h->n2s.as<uint32_t>(), n_host, pos, s));
       const int done = pos.n - 3;
       planes.n -= done;
       for (int k = 0; k < planes.n; ++k) {
@@ -1257,7 +1257,7 @@ static int cl_build_t(ofp_cl* h, const Key& key, const EmitArgs<T>& A0, size_t n
       }
       A.placed = true;
     }
-    OFP_TRY(go_far(h, h->n2s.as<uint32_t>(), planes, s));
+    OFP_TRY(go_far(h, h->n2s.as<uint32_t>(), n_host, planes, s));
     A.n2s = nullptr;
     A.pa.n = 0;
   }
@@ -1488,6 +1488,33 @@ int ofp::cl_construct_many(ofp_cl* h, const void* pos, size_t stride, const uint
   if (h->dtype == OFP_F32)
     return ofp::cl_construct_many_t<float>(h, pos, stride, n_cap, n_dev, gm, pos_sorted, sorted_stride, s);
   return ofp::cl_construct_many_t<double>(h, pos, stride, n_cap, n_dev, gm, pos_sorted, sorted_stride, s);
+}
+
+int ofp::cl_far(const ofp_cl* h, size_t n, bool* far, hipStream_t s) {
+  *far = false;
+  if (!h->built || n < kFarFrom || n > kFarTo || h->payload.cap < kFarScratch * (n + 8)) return OFP_OK;
+  unsigned long long desc = 0;
+  OFP_HIP(hipMemcpyAsync(&desc, h->packed.as<unsigned long long>() + h->n_cells, sizeof(desc), hipMemcpyDeviceToHost,
+                         s));
+  OFP_HIP(hipStreamSynchronize(s));
+  *far = desc * kDisorderDen > n;
+  return OFP_OK;
+}
+
+int ofp::cl_permute(const ofp_cl* hc, const uint32_t* idx, size_t n, const PlaneArgs& pa, bool* done,
+                    hipStream_t s) {
+  *done = false;
+  ofp_cl* h = const_cast<ofp_cl*>(hc);  // its scratch only
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  OFP_HIP(hipStreamIsCapturing(s, &cap));
+  if (cap != hipStreamCaptureStatusNone || n > kFarTo || h->payload.cap < kFarScratch * (n + 8)) return OFP_OK;
+  {
+    std::lock_guard<std::mutex> lock(h->far_lock);
+    OFP_TRY(h->cursors.ensure(kFarRanges * 4));
+  }
+  OFP_TRY(go_far(h, idx, uint32_t(n), pa, s));
+  *done = true;
+  return OFP_OK;
 }
 
 int ofp::cl_sid_sorted(const ofp_cl* h, const uint32_t** sid_sorted) {
