@@ -168,13 +168,23 @@ __global__ __launch_bounds__(kVlBlock) void k_vl_place(ClDev c, const SysGrid<T>
       const int xa = G.cx0 - B > 0 ? G.cx0 - B : 0;
       const int xe = G.cx0 + G.ncx - 1 + B;
       const int xb = xe < int(G.d0) - 1 ? xe : int(G.d0) - 1;
-      for (int dz = -B; dz <= B; ++dz)
-        for (int dy = -B; dy <= B; ++dy) {
-          const int zz = G.cz + dz, yy = G.cy + dy;
-          if (zz < 0 || zz >= int(G.d2) || yy < 0 || yy >= int(G.d1)) continue;
-          const uint32_t rowc = G.cbase + G.d0 * (uint32_t(yy) + G.d1 * uint32_t(zz));
-          words += (uint32_t(c.cs[rowc + uint32_t(xb) + 1]) - uint32_t(c.cs[rowc + uint32_t(xa)]) + kBlk - 1) / kBlk;
+      for (int dz = -B; dz <= B; ++dz) {
+        const int zz = G.cz + dz;
+        if (zz < 0 || zz >= int(G.d2)) continue;
+        // a plane's rows at once, those outside the grid as an empty run of the
+        // item's own (small builds wait for nothing but these loads)
+        uint32_t ja[2 * kMaxBoxNN + 1], jb[2 * kMaxBoxNN + 1];
+#pragma unroll
+        for (int k = 0; k < 2 * kMaxBoxNN + 1; ++k) {
+          const int yy = G.cy - B + k;
+          const bool in = k <= 2 * B && yy >= 0 && yy < int(G.d1);
+          const uint32_t rowc = G.cbase + G.d0 * (uint32_t(in ? yy : G.cy) + G.d1 * uint32_t(zz));
+          ja[k] = uint32_t(c.cs[rowc + uint32_t(xa)]);
+          jb[k] = uint32_t(c.cs[rowc + (in ? uint32_t(xb) + 1u : uint32_t(xa))]);
         }
+#pragma unroll
+        for (int k = 0; k < 2 * kMaxBoxNN + 1; ++k) words += (jb[k] - ja[k] + kBlk - 1) / kBlk;
+      }
       words = (words + 3u) & ~3u;
       n = ti.n;
     }
