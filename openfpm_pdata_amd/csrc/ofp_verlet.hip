@@ -555,18 +555,24 @@ __global__ __launch_bounds__(kVlBlock) void k_vl_fill(ClDev c, const SysGrid<T>*
 //  * fill (kFill = true): the row's entries come from its mask words (the
 //    tests of candidates past kRowWords words are repeated), in ascending
 //    sorted index as the item kernels write them, gathered in LDS up to
-//    kRowSeg of them per wave and written out with coalesced stores; past
-//    kRowSeg they go straight to the list.
+//    kSeg of them per wave and written out with coalesced stores; past
+//    kSeg they go straight to the list.
 // Ensembles: the row's system from sid_sorted.
 constexpr int kRowAhead = 4;  // candidates in flight per thread
 constexpr uint32_t kRowWords = 16;  // mask words kept per row (32 candidates each)
-constexpr uint32_t kRowSeg = 1024;  // entries per wave staged in LDS
+// Entries per wave staged in LDS by the fill; the others go to the list one by one, a
+// line each.  The larger where the mean wave (the host knows the list's entries, or
+// its capacity) does not fit the smaller: 10 KB a wave are 16 waves per CU, with the
+// next run's bounds loaded ahead.  1e6 rows of 46 entries: fill 256 -> 167 us (3072:
+// 208, 5120: 253); the 857,000 rows of 64 boxes 247 -> 197 us.
+constexpr uint32_t kRowSegFew = 1024, kRowSegMany = 2560;
 constexpr int kRowWaves = 256 / kWave;
 
 // kB: the stencil half-width B (c.box_nn) as a constant, so the row's
 // (2B+1)^2 run bounds are all loaded before its first candidate is read.
 // masks: kRowWords x 64 words per wave of rows.
-template <class T, bool kFill, int kB>
+// kSeg: kRowSegFew or kRowSegMany.
+template <class T, bool kFill, int kB, uint32_t kSeg>
 __global__ __launch_bounds__(256) void k_vl_rows(ClDev c, CellGeom<T> g1, const T* __restrict__ xyz, T r2_one,
                                                  const SysGrid<T>* __restrict__ sys, const T* __restrict__ r2_sys,
                                                  const uint32_t* __restrict__ sid_sorted, uint32_t* __restrict__ cnt,
@@ -574,7 +580,7 @@ __global__ __launch_bounds__(256) void k_vl_rows(ClDev c, CellGeom<T> g1, const 
                                                  const unsigned long long* __restrict__ off,
                                                  const unsigned long long* __restrict__ e_total,
                                                  unsigned long long e_cap, uint32_t* __restrict__ nbr) {
-  __shared__ uint32_t lds[kRowWaves][kFill ? kRowSeg : kRowWords * kWave];
+  __shared__ uint32_t lds[kRowWaves][kFill ? kSeg : kRowWords * kWave];
   const int lane = threadIdx.x & (kWave - 1);
   const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
   const uint32_t k0 = k - uint32_t(lane);  // the wave's first row
@@ -630,10 +636,14 @@ __global__ __launch_bounds__(256) void k_vl_rows(ClDev c, CellGeom<T> g1, const 
 #pragma unroll
       for (int r = 0; r < kRuns; ++r) fn(run_a[r], run_b[r]);
     } else {
+      uint32_t a, b;
+      run_bounds(0, &a, &b);
       for (int r = 0; r < kRuns; ++r) {
-        uint32_t a, b;
-        run_bounds(r, &a, &b);
+        uint32_t na = 0, nb = 0;  // the next run's, loaded ahead
+        if (r + 1 < kRuns) run_bounds(r + 1, &na, &nb);
         fn(a, b);
+        a = na;
+        b = nb;
       }
     }
   };
@@ -695,7 +705,7 @@ __global__ __launch_bounds__(256) void k_vl_rows(ClDev c, CellGeom<T> g1, const 
     uint32_t i = 0;  // entries of the row written
     auto emit = [&](uint32_t j) {
       const unsigned long long at = lo + i;
-      if (at < kRowSeg)
+      if (at < kSeg)
         wl[at] = j;
       else
         nbr[base + at] = j;
@@ -734,7 +744,7 @@ __global__ __launch_bounds__(256) void k_vl_rows(ClDev c, CellGeom<T> g1, const 
     __builtin_amdgcn_wave_barrier();
     const uint32_t k1 = k0 + uint32_t(kWave) < c.n_dom ? k0 + uint32_t(kWave) : c.n_dom;
     const unsigned long long len = off[k1] - base;
-    const uint32_t ms = len < kRowSeg ? uint32_t(len) : kRowSeg;
+    const uint32_t ms = len < kSeg ? uint32_t(len) : kSeg;
     for (uint32_t e = uint32_t(lane); e < ms; e += kWave) nbr[base + e] = wl[e];
   }
 }
@@ -823,22 +833,24 @@ static int vl_build_t(ofp_vl* h, const ofp_cl* cl, const void* pos_v, size_t str
     const unsigned g = grid_for(n, 256);
     const size_t n_waves = (n + kWave - 1) / kWave;
     OFP_TRY(h->rmask.ensure(n_waves * kRowWords * kWave * 4 + 4));
-    auto launch = [&](auto fill, auto kb, size_t e_cap) {
-      k_vl_rows<T, decltype(fill)::value, decltype(kb)::value><<<g, 256, 0, s>>>(
+    auto launch = [&](auto fill, auto kb, auto seg, size_t e_cap) {
+      k_vl_rows<T, decltype(fill)::value, decltype(kb)::value, decltype(seg)::value><<<g, 256, 0, s>>>(
           c, g1, h->xyz.as<T>(), r2_one, sys, r2_sys, sid, h->cnt.as<uint32_t>(), h->rmask.as<uint32_t>(),
           h->off.as<unsigned long long>(), h->off.as<unsigned long long>() + n, (unsigned long long)e_cap,
           h->nbr.as<uint32_t>());
     };
-    auto pass = [&](auto fill, size_t e_cap) {
+    auto pass = [&](auto fill, auto seg, size_t e_cap) {
       if (c.box_nn == 1)
-        launch(fill, std::integral_constant<int, 1>{}, e_cap);
+        launch(fill, std::integral_constant<int, 1>{}, seg, e_cap);
       else if (c.box_nn == 2)
-        launch(fill, std::integral_constant<int, 2>{}, e_cap);
+        launch(fill, std::integral_constant<int, 2>{}, seg, e_cap);
       else
-        launch(fill, std::integral_constant<int, 3>{}, e_cap);
+        launch(fill, std::integral_constant<int, 3>{}, seg, e_cap);
     };
+    using Few = std::integral_constant<uint32_t, kRowSegFew>;
+    using Many = std::integral_constant<uint32_t, kRowSegMany>;
     if (n > 0) {
-      pass(std::false_type{}, 0);
+      pass(std::false_type{}, Few{}, 0);
       OFP_LAUNCHED();
     }
     OFP_TRY(scan_excl_u32_to_u64(h->cnt.as<uint32_t>(), h->off.as<uint64_t>(), n, h->scantmp.p, s));
@@ -853,7 +865,11 @@ static int vl_build_t(ofp_vl* h, const ofp_cl* cl, const void* pos_v, size_t str
     const size_t e_cap = *e_cap_io;
     OFP_TRY(h->nbr.ensure((e_cap + 4) * 4));  // + 3: the one-lane row kernels read whole groups of four entries
     if (n > 0) {
-      pass(std::true_type{}, e_cap);
+      const double entries = sync ? double(E) : double(e_cap) / std::max(1.0, headroom);
+      if (entries * kWave <= double(kRowSegFew) * double(n))
+        pass(std::true_type{}, Few{}, e_cap);
+      else
+        pass(std::true_type{}, Many{}, e_cap);
       OFP_LAUNCHED();
     }
     h->n_rows = n;
