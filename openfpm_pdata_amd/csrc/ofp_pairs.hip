@@ -1297,32 +1297,69 @@ __global__ __launch_bounds__(kTileBlock, 4) void k_tile_f64(ClDev c, const T* __
 
 // ------------------------------------------------------ ensemble kernels
 // One lane per Verlet row: the row's entries [e0, e1) are read in groups of
-// four from the row's first entry, one 16-byte load per group (4-byte aligned;
-// gfx950 takes dword-aligned multi-dword loads), so a wave's entry loads touch
-// a quarter of the cache lines that four 4-byte loads per lane would and a row
-// of L entries takes ceil(L / 4) groups.  The list buffer holds at least three
-// entries past the list's capacity, so the last group read stays inside it.
-// Slots of the last group past the row's end (the next row's entries, or
-// unwritten ones past the list's end) read as p, the row's own particle, which
-// the pair evaluation skips.  body(j, next) gets the group and a callable that
-// issues the next group's load; body calls it once its gathers are issued, so
-// that load is in flight during the evaluation.
-template <class F>
-__device__ __forceinline__ void row_groups(const uint32_t* __restrict__ vnbr, unsigned long long e0,
-                                           unsigned long long e1, uint32_t p, F&& body) {
-  auto load = [&](unsigned long long e) {
-    uint4 q;
-    __builtin_memcpy(&q, vnbr + e, sizeof(q));
-    return q;
-  };
-  uint4 Jn = load(e0 < e1 ? e0 : e1);
-  for (unsigned long long b = e0; b < e1; b += 4) {
-    const uint32_t raw[4] = {Jn.x, Jn.y, Jn.z, Jn.w};
-    uint32_t j[4];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) j[u] = b + u < e1 ? raw[u] : p;
-    body(j, [&] { Jn = load(b + 4 < e1 ? b + 4 : b); });
+// four from the row's first entry, so a row of L entries takes ceil(L / 4) groups.
+// A wave's rows are consecutive in the list: their entries, where kRowEntries hold
+// them, are staged in LDS (RowEntries), 16 bytes per lane of contiguous lines, and
+// the lanes read their groups there; else a lane loads a group from the list, 16
+// bytes (4-byte aligned; gfx950 takes dword-aligned multi-dword loads).  The list
+// buffer holds at least three entries past the list's capacity, so the last group
+// read stays inside it.  Slots of the last group past the row's end (the next row's
+// entries, or unwritten ones past the list's end) read as p, the row's own
+// particle, which the pair evaluation skips.  body(j, next) gets the group and a
+// callable that reads the next group; body calls it once its gathers are issued, so
+// that it is there after the evaluation.
+// The passes are bound by the texture path, which returns a wave's scattered 16-byte
+// groups in 64 clocks, against 48 for each of their four gathers.  Step pass of 2^23
+// particles, 19 entries a row: FP32C 538 -> 520 us; FP64 40 steps 29.8 -> 24.3 ms.
+// 6 KB a wave; 8 KB leave four blocks per CU (FP32C 590 us).
+constexpr uint32_t kRowEntries = 1532;
+struct RowEntries {
+  const uint32_t* lds;  // null: not staged
+  unsigned long long first;
+  // Called by the whole wave with its first row (kw).
+  __device__ __forceinline__ RowEntries(uint32_t* buf, const unsigned long long* __restrict__ voff,
+                                        const uint32_t* __restrict__ vnbr, unsigned long long e_lim, uint32_t kw,
+                                        uint32_t n_rows)
+      : lds(nullptr), first(0) {
+    if (kw >= n_rows) return;
+    first = voff[kw];
+    const unsigned long long end = voff[kw + kWave < n_rows ? kw + kWave : n_rows];
+    const unsigned long long lim = end < e_lim ? end : e_lim;
+    const unsigned long long n = first < lim ? lim - first : 0;
+    if (n > kRowEntries) return;
+    for (uint32_t i = (threadIdx.x & (kWave - 1)) * 4u; i < uint32_t(n); i += 4u * kWave) {
+      uint4 q;
+      __builtin_memcpy(&q, vnbr + first + i, sizeof(q));
+      *reinterpret_cast<uint4*>(buf + i) = q;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+    lds = buf;
   }
+};
+template <class F>
+__device__ __forceinline__ void row_groups(const RowEntries& staged, const uint32_t* __restrict__ vnbr,
+                                           unsigned long long e0, unsigned long long e1, uint32_t p, F&& body) {
+  auto walk = [&](auto&& load) {
+    uint4 Jn = load(e0 < e1 ? e0 : e1);
+    for (unsigned long long b = e0; b < e1; b += 4) {
+      const uint32_t raw[4] = {Jn.x, Jn.y, Jn.z, Jn.w};
+      uint32_t j[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) j[u] = b + u < e1 ? raw[u] : p;
+      body(j, [&] { Jn = load(b + 4 < e1 ? b + 4 : b); });
+    }
+  };
+  walk([&](unsigned long long e) {
+    uint4 q;
+    if (staged.lds) {
+      const uint32_t* s = staged.lds + uint32_t(e - staged.first);
+      q = make_uint4(s[0], s[1], s[2], s[3]);
+    } else {
+      __builtin_memcpy(&q, vnbr + e, sizeof(q));
+    }
+    return q;
+  });
 }
 
 // The systems of a wave's rows one at a time, so that a system's constants are
@@ -1392,6 +1429,9 @@ __global__ __launch_bounds__(256) void k_pairs_many_f32c(ClDev c, const Ph* __re
   const int4 P = c.quant[p];
   const uint32_t ik = kick.index(p);
   const unsigned lane = threadIdx.x & (kLanes - 1);
+  __shared__ __align__(16) uint32_t entries[kLanes == 1 ? 256 / kWave : 1][kLanes == 1 ? kRowEntries + 4 : 1];
+  RowEntries staged(entries[kLanes == 1 ? threadIdx.x / kWave : 0], voff, vnbr, e_lim,
+                    __builtin_amdgcn_readfirstlane(kLanes == 1 ? k : ~0u), c.n_dom);
   by_system(valid, sid_sorted ? sid_sorted[p] : 0u, [&](uint32_t sy) {
   const Ph ph = tab[sy];
   const QGeom qg = qtab[sy];
@@ -1414,7 +1454,7 @@ __global__ __launch_bounds__(256) void k_pairs_many_f32c(ClDev c, const Ph* __re
     const unsigned long long e0 = voff[k];
     const unsigned long long e1 = voff[k + 1] < e_lim ? voff[k + 1] : e_lim;
     Deferred df;
-    row_groups(vnbr, e0, e1, p, [&](const uint32_t (&j)[4], auto&& next) {
+    row_groups(staged, vnbr, e0, e1, p, [&](const uint32_t (&j)[4], auto&& next) {
       int4 Q[4];
       float a[4];
 #pragma unroll
@@ -1491,6 +1531,9 @@ __global__ __launch_bounds__(256) void k_pairs_many_f64(ClDev c, const Ph* __res
   const double xp = pos[p], yp = pos[stride + p], zp = pos[2 * stride + p];
   const uint32_t ik = kick.index(p);
   const unsigned lane = threadIdx.x & (kLanes - 1);
+  __shared__ __align__(16) uint32_t entries[kLanes == 1 ? 256 / kWave : 1][kLanes == 1 ? kRowEntries + 4 : 1];
+  RowEntries staged(entries[kLanes == 1 ? threadIdx.x / kWave : 0], voff, vnbr, e_lim,
+                    __builtin_amdgcn_readfirstlane(kLanes == 1 ? k : ~0u), c.n_dom);
   by_system(valid, sid_sorted ? sid_sorted[p] : 0u, [&](uint32_t sy) {
   const Ph ph = tab[sy];
   typename Ph::St st;
@@ -1504,7 +1547,7 @@ __global__ __launch_bounds__(256) void k_pairs_many_f64(ClDev c, const Ph* __res
   };
   if (kLanes == 1) {
     const unsigned long long e1 = voff[k + 1] < e_lim ? voff[k + 1] : e_lim;
-    row_groups(vnbr, voff[k], e1, p, [&](const uint32_t (&j)[4], auto&& next) {
+    row_groups(staged, vnbr, voff[k], e1, p, [&](const uint32_t (&j)[4], auto&& next) {
       T qx[4], qy[4], qz[4];
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
