@@ -72,7 +72,8 @@ struct ofp_cl {
   // the order check's result on the host (pinned) and its event
   unsigned long long* desc = nullptr;
   hipEvent_t checked = nullptr;
-  ofp::DevBuf items, nitems;  // nitems: the consumers' queue heads (kQueueWords), then the item count
+  ofp::DevBuf items;
+  uint64_t heads_at = 0;  // word of packed: the consumers' queue heads (kQueueWords), then the item count
   ofp::DevBuf aux;            // pair kernels' per-particle record stream (cell tiles)
   // sparse view (ofp_cl_build_sparse): non-empty cells only
   ofp::DevBuf nz_flag, nz_key, nz_start, nz_nn, nz_inv;
@@ -1082,15 +1083,17 @@ static int cl_build_t(ofp_cl* h, const Key& key, const EmitArgs<T>& A0, size_t n
   }
   int widths[4];
   const int passes = radix_plan(C, widths);
-  // the descents counted and the chunks' sums lie behind the cells' counts, cleared
-  // with them
+  // the descents counted, the chunks' sums, the items' queue heads and their count
+  // lie behind the cells' counts, cleared with them
   const int direct = n_tiles <= kRxChunked ? 1 : 0;
   const bool chunked = direct && n_tiles > kRxDirect;
   // the [tile][digit] table in at most kColChunks chunks of ch tiles
   const uint32_t ch = std::max((n_tiles + kColChunks - 1) / kColChunks, kColBatch);
   const uint32_t n_chunks = (n_tiles + ch - 1) / ch;
-  const uint64_t n_clear = C + 1 + (chunked ? uint64_t(passes) * n_chunks * (kRxBins / 2) : 0);
+  const uint64_t heads_at = C + 1 + (chunked ? uint64_t(passes) * n_chunks * (kRxBins / 2) : 0);
+  const uint64_t n_clear = heads_at + kQueueWords / 2 + 1;
   OFP_TRY(h->packed.ensure(n_clear * 8));
+  h->heads_at = heads_at;
   OFP_TRY(h->scan64.ensure((C + 1) * 8));
   OFP_TRY(h->scantmp.ensure(scan_tmp_bytes(C)));
   if (!direct) OFP_TRY(h->colpart.ensure(size_t(kColChunks) * kRxBins * 4));
@@ -1575,7 +1578,7 @@ int ofp_cl_create(ofp_cl** out, int dtype, const void* box_lo, const void* box_h
 int ofp_cl_destroy(ofp_cl* h) {
   if (!h) return OFP_OK;
   DevBuf* bufs[] = {&h->packed, &h->scan64, &h->keys,    &h->keys2, &h->s2n,        &h->vals2, &h->n2s,
-                    &h->dom,    &h->quant,  &h->scantmp, &h->hist,  &h->sid_sorted, &h->items, &h->nitems,
+                    &h->dom,    &h->quant,  &h->scantmp, &h->hist,  &h->sid_sorted, &h->items,
                     &h->payload, &h->colpart, &h->cursors, &h->nz_flag, &h->nz_key, &h->nz_start, &h->nz_nn,
                     &h->nz_inv, &h->aux};
   for (DevBuf* b : bufs) b->release();
@@ -1630,11 +1633,14 @@ int ofp_cl_items_(const ofp_cl* hc, const TargetItem** items, const uint32_t** n
                   uint32_t** counter, size_t* cap, hipStream_t s) {
   ofp_cl* h = const_cast<ofp_cl*>(hc);
   OFP_CHECK(h && h->built, OFP_E_STATE, "cell list not constructed");
+  uint32_t* heads = reinterpret_cast<uint32_t*>(h->packed.as<unsigned long long>() + h->heads_at);
   if (!h->items_valid) {
     size_t need = size_t(h->gm) + 1;
     OFP_TRY(h->items.ensure(need * sizeof(TargetItem)));
-    OFP_TRY(h->nitems.ensure((kQueueWords + 1) * sizeof(uint32_t)));
-    OFP_TRY(fill_u32(h->nitems.as<uint32_t>(), 0, kQueueWords + 1, s));
+    // cleared by the build, once: a captured call, which may be replayed, clears itself
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    OFP_HIP(hipStreamIsCapturing(s, &cap));
+    if (cap != hipStreamCaptureStatusNone) OFP_TRY(fill_u32(heads, 0, kQueueWords + 1, s));
     const uint32_t words = h->dtype == OFP_F32 ? uint32_t(sizeof(SysGrid<float>) / 4)
                                                : uint32_t(sizeof(SysGrid<double>) / 4);
     const uint32_t off = h->dtype == OFP_F32 ? uint32_t(offsetof(SysGrid<float>, divc) / 4)
@@ -1642,14 +1648,14 @@ int ofp_cl_items_(const ofp_cl* hc, const TargetItem** items, const uint32_t** n
     const uint32_t* desc = h->n_sys ? static_cast<const uint32_t*>(h->sys) + off : nullptr;
     k_cl_items<<<grid_for(h->n_rows, kItemRows), kItemRows * kWave, 0, s>>>(
         h->scan64.as<unsigned long long>(), h->divc[0], h->n_rows, h->n_sys, h->rbase, desc, words,
-        h->items.as<TargetItem>(), h->nitems.as<uint32_t>() + kQueueWords);
+        h->items.as<TargetItem>(), heads + kQueueWords);
     OFP_LAUNCHED();
     h->items_cap = need;
     h->items_valid = true;
   }
   *items = h->items.as<TargetItem>();
-  *n_items = h->nitems.as<uint32_t>() + kQueueWords;
-  *counter = h->nitems.as<uint32_t>();
+  *n_items = heads + kQueueWords;
+  *counter = heads;
   *cap = h->items_cap;
   return OFP_OK;
 }
