@@ -34,6 +34,7 @@
 extern "C" int ofp_vl_dev_(const ofp_vl* h, const ofp_cl* cl, int symmetric, const unsigned long long** off,
                            const uint32_t** nbr);
 extern "C" int ofp_vl_aux_(const ofp_vl* h, size_t bytes, void** p);
+extern "C" int ofp_vl_rec_(const ofp_vl* h, size_t bytes, void** p, hipStream_t s);
 
 namespace ofp {
 
@@ -876,11 +877,12 @@ __global__ __launch_bounds__(256) void k_pairs_f32c(ClDev c, QGeom qg, const uns
 // 8.2 ms.
 constexpr double kFar = 1e200;
 
-// FP32C: 12-byte (q_x, q_y, q_z) or 16-byte (q, pterm) records.
-template <class Ph, bool kCubic>
+// FP32C: 12-byte (q_x, q_y, q_z) or 16-byte (q, pterm) records; kWide: the
+// quantised stream itself, where there is no room for 12-byte records.
+template <class Ph, bool kCubic, bool kWide = false>
 struct QuantRows {
   using St = typename Ph::St;
-  using Rec = std::conditional_t<Ph::kAuxInQuant, int4, int3>;
+  using Rec = std::conditional_t<Ph::kAuxInQuant || kWide, int4, int3>;
   const Rec* rec;
   QGeom qg;
   Ph ph;
@@ -1771,7 +1773,8 @@ __global__ void k_quant_rec_aux(const int4* __restrict__ quant, const float* __r
   out[i] = make_int4(q.x, q.y, q.z, __float_as_int(aux[i]));
 }
 
-// rec: kSmooth physics over Verlet rows, int3 or (Ph::kAuxInQuant) int4 records;
+// rec: kSmooth physics over Verlet rows, int3 (null: the quantised stream) or
+// (Ph::kAuxInQuant) int4 records;
 // over cell tiles the int4 records (null: the quantised stream).
 template <class Ph>
 static int launch_f32c(const PairCtx& x, const Ph& ph, hipStream_t s, const void* rec = nullptr) {
@@ -1783,6 +1786,16 @@ static int launch_f32c(const PairCtx& x, const Ph& ph, hipStream_t s, const void
     if constexpr (Ph::kSmooth) {
       using R = typename QuantRows<Ph, true>::Rec;
       const R* r = static_cast<const R*>(rec);
+      if constexpr (!Ph::kAuxInQuant) {
+        if (!r) {
+          if (cubic)
+            k_rows_smooth<<<grid, 256, 0, s>>>(x.c, x.voff, x.vnbr, QuantRows<Ph, true, true>{x.c.quant, qg, ph});
+          else
+            k_rows_smooth<<<grid, 256, 0, s>>>(x.c, x.voff, x.vnbr, QuantRows<Ph, false, true>{x.c.quant, qg, ph});
+          OFP_LAUNCHED();
+          return OFP_OK;
+        }
+      }
       if (cubic)
         k_rows_smooth<<<grid, 256, 0, s>>>(x.c, x.voff, x.vnbr, QuantRows<Ph, true>{r, qg, ph});
       else
@@ -2213,9 +2226,12 @@ int ofp_sph_density(const ofp_cl* cl, const ofp_vl* vl, const void* pos, size_t 
   ph.rho = (double*)rho;
   void* rec = nullptr;
   if (x.voff && x.c.n_dom > 0) {
-    OFP_TRY(ofp_vl_aux_(vl, (x.v.n_part + 1) * sizeof(int4), &rec));
-    k_quant_rec<<<grid_for(x.v.n_part, 256), 256, 0, s>>>(x.c.quant, uint32_t(x.v.n_part), static_cast<int3*>(rec));
-    OFP_LAUNCHED();
+    OFP_TRY(ofp_vl_rec_(vl, (x.v.n_part + 1) * sizeof(int3), &rec, s));
+    if (rec) {
+      k_quant_rec<<<grid_for(x.v.n_part, 256), 256, 0, s>>>(x.c.quant, uint32_t(x.v.n_part),
+                                                            static_cast<int3*>(rec));
+      OFP_LAUNCHED();
+    }
   }
   return launch_f32c(x, ph, s, rec);
 }

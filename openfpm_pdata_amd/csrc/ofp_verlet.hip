@@ -36,6 +36,7 @@ struct ofp_vl {
   ofp::DevBuf cnt, off, nbr, scantmp, masks, place, xyz;
   ofp::DevBuf rmask;  // thread-per-row build: the rows' hit masks, count pass to fill
   ofp::DevBuf aux;  // pair kernels' per-particle gather stream over the rows
+  ofp::DevBuf rec;  // the density pass's 12-byte records
   size_t mask_cap = 0;  // pairs of mask words (8 bytes) the buffer holds (0: not sized yet)
   bool rows_path = false;  // the last build ran the thread-per-row kernels
   uint64_t n_rows = 0, n_entries = 0;
@@ -1078,6 +1079,27 @@ int ofp_vl_aux_(const ofp_vl* h, size_t bytes, void** p) {
   return OFP_OK;
 }
 
+// A buffer of the list for the density pass's records, apart from ofp_vl_aux_ so that
+// a density and a force pass may run side by side (density passes write the same
+// records).  Null where it would have to grow and cannot: in a captured call, or for
+// want of memory.
+int ofp_vl_rec_(const ofp_vl* h, size_t bytes, void** p, hipStream_t s) {
+  OFP_CHECK(h && p, OFP_E_ARG, "ofp_vl_rec_: null argument");
+  ofp_vl* m = const_cast<ofp_vl*>(h);
+  *p = nullptr;
+  if (m->rec.cap < bytes) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    OFP_HIP(hipStreamIsCapturing(s, &cap));
+    if (cap != hipStreamCaptureStatusNone) return OFP_OK;
+    if (m->rec.ensure(bytes) != OFP_OK) {
+      clear_error();
+      return OFP_OK;
+    }
+  }
+  *p = m->rec.p;
+  return OFP_OK;
+}
+
 int ofp_vl_create(ofp_vl** h) {
   OFP_CHECK(h, OFP_E_ARG, "ofp_vl_create: null handle pointer");
   *h = new ofp_vl();
@@ -1087,7 +1109,7 @@ int ofp_vl_create(ofp_vl** h) {
 int ofp_vl_destroy(ofp_vl* h) {
   if (!h) return OFP_OK;
   DevBuf* bufs[] = {&h->cnt, &h->off, &h->nbr, &h->scantmp, &h->masks, &h->place,
-                    &h->xyz, &h->aux, &h->rmask};
+                    &h->xyz, &h->aux, &h->rec, &h->rmask};
   for (DevBuf* b : bufs) b->release();
   delete h;
   return OFP_OK;
