@@ -813,7 +813,8 @@ constexpr int kFarIters = 32;
 constexpr int kFarShift = 15;
 constexpr uint32_t kFarTile = uint32_t(kFarBlock * kFarIters);
 static_assert(kFarTile == 1u << kFarShift, "a range is a tile");
-constexpr uint32_t kFarRanges = 2 * kFarBlock;  // at most
+constexpr int kFarPer = 3;  // ranges a thread counts: the most the LDS holds beside a tile
+constexpr uint32_t kFarRanges = kFarPer * kFarBlock;
 constexpr size_t kFarFrom = size_t(1) << 22;  // restore of 24 bytes: 128 us at 2^21 (143 direct), 132 (265) here
 constexpr size_t kFarTo = size_t(kFarRanges) << kFarShift;
 constexpr size_t kFarScratch = 10;      // least scratch, bytes per particle
@@ -905,8 +906,8 @@ __global__ __launch_bounds__(kFarBlock) void k_far_stage(const uint32_t* __restr
   const uint32_t tid = threadIdx.x;
   const uint32_t tile0 = blockIdx.x << kFarShift;
   const uint32_t len = n - tile0 < kFarTile ? n - tile0 : kFarTile;
-  cnt[tid] = 0;
-  cnt[tid + kFarBlock] = 0;
+#pragma unroll
+  for (int q = 0; q < kFarPer; ++q) cnt[tid + q * kFarBlock] = 0;
   uint32_t d[kFarIters];
   Halves slot;
 #pragma unroll
@@ -919,20 +920,27 @@ __global__ __launch_bounds__(kFarBlock) void k_far_stage(const uint32_t* __restr
   for (int i = 0; i < kFarIters; ++i)
     slot.put(i, uint32_t(i) * kFarBlock + tid < len ? atomicAdd(&cnt[d[i] >> kFarShift], 1u) : 0u);
   __syncthreads();
-  // first slots of the tile's runs, in the tile and in the ranges' parts: two ranges a thread
-  const uint32_t r0 = 2 * tid, r1 = r0 + 1;
-  const uint32_t c0 = cnt[r0], c1 = cnt[r1];
-  const uint32_t inc = wave_incl_scan(c0 + c1);
+  // first slots of the tile's runs, in the tile and in the ranges' parts: consecutive
+  // ranges a thread
+  uint32_t c[kFarPer], g[kFarPer], own = 0;
+#pragma unroll
+  for (int q = 0; q < kFarPer; ++q) {
+    const uint32_t r = kFarPer * tid + q;
+    c[q] = cnt[r];
+    own += c[q];
+    g[q] = (r << kFarShift) + (c[q] ? atomicAdd(&cursor[r], c[q]) : 0u);
+  }
+  const uint32_t inc = wave_incl_scan(own);
   if ((tid & (kWave - 1)) == kWave - 1) wsum[tid / kWave] = inc;
-  const uint32_t g0 = (r0 << kFarShift) + (c0 ? atomicAdd(&cursor[r0], c0) : 0u);
-  const uint32_t g1 = (r1 << kFarShift) + (c1 ? atomicAdd(&cursor[r1], c1) : 0u);
   __syncthreads();
-  uint32_t first = inc - c0 - c1;
+  uint32_t first = inc - own;
   for (uint32_t w = 0; w < tid / kWave; ++w) first += wsum[w];
-  cnt[r0] = first;
-  cnt[r1] = first + c0;
-  goff[r0] = g0 - first;
-  goff[r1] = g1 - first - c0;
+#pragma unroll
+  for (int q = 0; q < kFarPer; ++q) {
+    cnt[kFarPer * tid + q] = first;
+    goff[kFarPer * tid + q] = g[q] - first;
+    first += c[q];
+  }
   __syncthreads();
 #pragma unroll
   for (int i = 0; i < kFarIters; ++i) {

@@ -59,6 +59,28 @@ def test_far(n, order):
             assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("n", [3072 << 15, (3072 << 15) + 1])
+def test_far_most_particles(n):
+    """The most ranges (3072), and one particle more (the direct kernels again)."""
+    side = 200
+    pos = torch.rand((3, n), generator=torch.Generator(device="cuda").manual_seed(9), device="cuda") * side
+    cl = vdm.CellListGPU(torch.float32, (0.0,) * 3, (float(side),) * 3, (side,) * 3,
+                         vdm.CL_NON_SYMMETRIC | vdm.CL_GPU_REORDER, 1.0)
+    src = _planes(n, [4, 8], 11)
+    dst = [torch.zeros_like(p) for p in src]
+    out = torch.empty_like(pos)
+    cl.construct(pos, n, n, out, _args(src), _args(dst))
+    s2n = cl.arrays()["s2n"].long()
+    assert torch.equal(cl.arrays()["n2s"].long()[s2n], torch.arange(n, device="cuda"))
+    assert torch.equal(out, pos[:, s2n])
+    for a, b in zip(src, dst):
+        assert torch.equal(b, a[s2n])
+    back = [torch.zeros_like(p) for p in src]
+    cl.restore(_args(dst), _args(back))
+    for a, b in zip(src, back):
+        assert torch.equal(a, b)
+
+
 def test_far_most_planes():
     """24 planes, the most a call takes, with the positions (3 more)."""
     n, side = (1 << 22) + 11, 64
