@@ -1316,13 +1316,17 @@ __global__ __launch_bounds__(kTileBlock, 4) void k_tile_f64(ClDev c, const T* __
 // 6 KB a wave; 8 KB leave four blocks per CU (FP32C 590 us).
 constexpr uint32_t kRowEntries = 1532;
 struct RowEntries {
-  const uint32_t* lds;  // null: not staged
+  // (an LDS pointer by type: through a generic one the compiler makes one flat load
+  // of the two branches in row_groups)
+  typedef const uint32_t __attribute__((address_space(3))) Word;
+  Word* lds;
+  bool staged;  // wave-uniform
   unsigned long long first;
   // Called by the whole wave with its first row (kw).
   __device__ __forceinline__ RowEntries(uint32_t* buf, const unsigned long long* __restrict__ voff,
                                         const uint32_t* __restrict__ vnbr, unsigned long long e_lim, uint32_t kw,
                                         uint32_t n_rows)
-      : lds(nullptr), first(0) {
+      : lds((Word*)(buf)), staged(false), first(0) {
     if (kw >= n_rows) return;
     first = voff[kw];
     const unsigned long long end = voff[kw + kWave < n_rows ? kw + kWave : n_rows];
@@ -1336,14 +1340,16 @@ struct RowEntries {
     }
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
     __builtin_amdgcn_wave_barrier();
-    lds = buf;
+    staged = true;
   }
 };
 template <class F>
-__device__ __forceinline__ void row_groups(const RowEntries& staged, const uint32_t* __restrict__ vnbr,
+__device__ __forceinline__ void row_groups(const RowEntries& row, const uint32_t* __restrict__ vnbr,
                                            unsigned long long e0, unsigned long long e1, uint32_t p, F&& body) {
+  // (an empty row reads nothing: a list cut at its capacity ends before e0)
+  if (!(e0 < e1)) return;
   auto walk = [&](auto&& load) {
-    uint4 Jn = load(e0 < e1 ? e0 : e1);
+    uint4 Jn = load(e0);
     for (unsigned long long b = e0; b < e1; b += 4) {
       const uint32_t raw[4] = {Jn.x, Jn.y, Jn.z, Jn.w};
       uint32_t j[4];
@@ -1354,8 +1360,8 @@ __device__ __forceinline__ void row_groups(const RowEntries& staged, const uint3
   };
   walk([&](unsigned long long e) {
     uint4 q;
-    if (staged.lds) {
-      const uint32_t* s = staged.lds + uint32_t(e - staged.first);
+    if (row.staged) {
+      const RowEntries::Word* s = row.lds + uint32_t(e - row.first);
       q = make_uint4(s[0], s[1], s[2], s[3]);
     } else {
       __builtin_memcpy(&q, vnbr + e, sizeof(q));
