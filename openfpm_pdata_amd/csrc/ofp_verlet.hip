@@ -129,11 +129,11 @@ __device__ __forceinline__ void block_table(const ItemRuns& R, uint32_t w0, uint
   lds_order();
 }
 
-// min(m, |a|, |b|) in one instruction (no canonicalisation of the operands)
+// min(m, |a|, |b|): one instruction, which the compiler has to write itself.  Inline
+// asm would hide from it that a and b come out of the matrix cores, and the wait
+// states that such a read needs would be missing.
 __device__ __forceinline__ float min3_abs(float m, float a, float b) {
-  float r;
-  asm("v_min3_f32 %0, %1, |%2|, |%3|" : "=v"(r) : "v"(m), "v"(a), "v"(b));
-  return r;
+  return __builtin_fminf(__builtin_fminf(m, __builtin_fabsf(a)), __builtin_fabsf(b));
 }
 // Part `part` of P of `total` (monotonic in part, 0 and total at the ends).
 __device__ __forceinline__ uint32_t part_begin(uint32_t total, uint32_t part, uint32_t P) {
@@ -1097,6 +1097,14 @@ int ofp_vl_rec_(const ofp_vl* h, size_t bytes, void** p, hipStream_t s) {
     }
   }
   *p = m->rec.p;
+  return OFP_OK;
+}
+
+// Test hook (not in the public header): whether the last build ran the
+// thread-per-row kernels (else the item kernels).
+int ofp_vl_test_rows_(const ofp_vl* h, int* rows) {
+  OFP_CHECK(h && h->built && rows, OFP_E_STATE, "ofp_vl_test_rows_: list not built");
+  *rows = h->rows_path ? 1 : 0;
   return OFP_OK;
 }
 
