@@ -369,11 +369,13 @@ __device__ __forceinline__ V wave_sum(V x) {
 }
 
 // w * 2 + hit, per lane: the compare's lane mask enters v_addc as its carry-in,
-// so appending a hit bit costs one VALU op after the compare.
+// so appending a hit bit costs one VALU op after the compare.  (s_nop 1: the wait
+// states between a write of an SGPR by the vector ALU and a read of it there, which
+// the compiler does not add before inline asm.)
 __device__ __forceinline__ uint32_t shift_in(uint32_t w, bool hit) {
   const unsigned long long m = __ballot(hit);
   uint32_t r;
-  asm("v_addc_co_u32 %0, vcc, %1, %1, %2" : "=v"(r) : "v"(w), "s"(m) : "vcc");
+  asm("s_nop 1\n\tv_addc_co_u32 %0, vcc, %1, %1, %2" : "=v"(r) : "v"(w), "s"(m) : "vcc");
   return r;
 }
 

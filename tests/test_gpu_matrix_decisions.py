@@ -48,3 +48,25 @@ def test_distances_at_the_radius(dtype, rel, sub):
     vd.pos[:, :n] = torch.from_numpy(pos).cuda()
     cl, vl = vd.getVerletGPU(r, sub=sub)
     check_rows(pos, r, cl, vl, npd)
+
+
+@pytest.mark.parametrize("n", [333, 999, 3000])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+def test_particles_beyond_their_cells(dtype, n):
+    """Moved since the cells were built, further than the products' bound allows:
+    every pair is tested in the list's own rounding.  The stencil spans the grid."""
+    npd = np.float32 if dtype == torch.float32 else np.float64
+    rng = np.random.default_rng(n)
+    div, r = 4, 2.9
+    pos = torch.from_numpy(np.ascontiguousarray((rng.random((3, n)) * div).astype(npd))).cuda()
+    cl = vdm.CellListGPU(dtype, (0.0,) * 3, (float(div),) * 3, (div,) * 3,
+                         vdm.CL_NON_SYMMETRIC | vdm.CL_GPU_REORDER_POSITION, 0.9, box_nn=3)
+    out = torch.empty_like(pos)
+    cl.construct(pos, n, n, out)
+    s2n = cl.arrays()["s2n"].long()
+    out = (out * 9.0).contiguous()
+    pos = torch.empty_like(out)
+    pos[:, s2n[:n]] = out
+    vl = vdm.VerletListGPU()
+    vl.build(cl, out, r)
+    check_rows(pos.cpu().numpy(), r, cl, vl, npd)
