@@ -437,6 +437,13 @@ __device__ __forceinline__ double lane_value<double>(double v, uint32_t lane) {
 }
 
 
+// min(m, |a|, |b|): one instruction, which the compiler has to write itself.  Inline
+// asm would hide from it that a and b come out of the matrix cores, and the wait
+// states that such a read needs would be missing.
+__device__ __forceinline__ float min3_abs(float m, float a, float b) {
+  return __builtin_fminf(__builtin_fminf(m, __builtin_fabsf(a)), __builtin_fabsf(b));
+}
+
 // Row of this lane in a 32 x 32 product: row 8 q + 4 h + m of a 32-block is candidate
 // 16 h + 15 - (4 q + m), so a lane's results i = 4 q + m (rows 8 (i / 4) +
 // 4 (lane / 32) + i % 4) are candidates 15 - i of its half.
@@ -445,18 +452,39 @@ __device__ __forceinline__ uint32_t matrix_candidate(uint32_t lane) {
   return 16u * ((r >> 2) & 1u) + 15u - (4u * (r >> 3) + (r & 3u));
 }
 
+// The power of two that brings the largest of a grid's spacings to [1, 2): FP64
+// coordinates relative to an origin are multiplied by it before their conversion to
+// FP32, so that their squares stay in FP32's range whatever the unit of length
+// (squares of 1e-21 or 1e19 do not).  1 for spacings so small or large that FP64
+// squares leave FP64's range too (MatrixTest then declines).
+__device__ __forceinline__ double matrix_unit(double spx, double spy, double spz) {
+  const double m = __builtin_fmax(spx, __builtin_fmax(spy, spz));
+  const int e = int((static_cast<unsigned long long>(__double_as_longlong(m)) >> 52) & 0x7FFull) - 1023;
+  if (e < -500 || e > 500) return 1.0;
+  return __longlong_as_double(static_cast<long long>(1023 - e) << 52);
+}
+
 // Candidates that may lie within a cut-off of a wave's targets (target = lane), from
 // tiles of the matrix product of (x, y, z, |c|^2) and (-2x, -2y, -2z, 1) on top of
 // |t|^2 - r^2 (coordinates relative to a common origin): the sign of 32 x 32 squares
-// less r^2.  r2: the cut-off's square plus the bound of the FP32 error, 2^-19 S with
-// S = (R_c + R_t)^2 + r^2, R the farthest candidate's and target's distance from the
-// origin: every pair within the cut-off has its bit set, and a few beyond.
+// less r^2.  eps, the bound of the FP32 error: 2^-19 S with S = (R_c + R_t)^2 + r^2, R
+// the farthest candidate's and target's distance from the origin.
 struct MatrixTest {
   v16f C0, C1;
-  float b00, b01, b10, b11, lim_c;
+  float b00, b01, b10, b11, lim_c, eps;
   bool two;  // more than 32 targets
-  __device__ __forceinline__ void targets(float x, float y, float z, float r2, float lim, bool more_than_32) {
-    float k0 = __builtin_fmaf(x, x, __builtin_fmaf(y, y, z * z)) - r2, k1 = k0;
+  // (x, y, z): the lane's target; rt2, rc2: squares of the farthest target's and
+  // candidate's distance from the origin by the cell geometry; r2: the cut-off's
+  // square.  kWide: every pair within the cut-off gets its bit, and a few beyond
+  // (r2 + eps).  False if a target lies beyond its bound or is not a number, or if the
+  // squares are not FP32's: from 2^-100 to 2^100, eps is normal and no smaller than
+  // what the flush of denormals could cost, and no product overflows.
+  template <bool kWide>
+  __device__ __forceinline__ bool targets(float x, float y, float z, float rt2, float rc2, float r2,
+                                          bool more_than_32) {
+    eps = (2.05f * (rt2 + rc2) + r2) * 0x1p-19f;  // (a + b)^2 <= 2 a^2 + 2 b^2
+    const float tn = __builtin_fmaf(x, x, __builtin_fmaf(y, y, z * z));
+    float k0 = tn - (kWide ? r2 + eps : r2), k1 = k0;
     b00 = -2.f * x, b01 = -2.f * y;  // columns of the target halves: k = 0, 1
     swap_halves(b00, b01);
     b10 = -2.f * z, b11 = 1.f;  // k = 2, 3
@@ -467,38 +495,49 @@ struct MatrixTest {
       C0[i] = k0;
       C1[i] = k1;
     }
-    lim_c = lim;
+    lim_c = rc2 * 1.01f;
     two = more_than_32;
+    return eps >= 0x1p-100f && eps <= 0x1p100f && __ballot(!(tn <= rt2 * 1.01f)) == 0ull;
   }
-  __device__ __forceinline__ void tile(float a0, float a1, float b0, float b1, const v16f& K, uint32_t& w) const {
+  // kNear: the smallest |square less r^2| in dm too.
+  template <bool kNear>
+  __device__ __forceinline__ void tile(float a0, float a1, float b0, float b1, const v16f& K, uint32_t& w,
+                                       float& dm) const {
     v16f D = __builtin_amdgcn_mfma_f32_32x32x2f32(a0, b0, K, 0, 0, 0);
     D = __builtin_amdgcn_mfma_f32_32x32x2f32(a1, b1, D, 0, 0, 0);
 #pragma unroll
     for (int i = 0; i < 16; ++i) w = __builtin_amdgcn_alignbit(w, __float_as_uint(D[i]), 31);
+    if constexpr (kNear) {
+#pragma unroll
+      for (int i = 0; i < 16; i += 2) dm = min3_abs(dm, D[i], D[i + 1]);
+    }
   }
   // (x, y, z): candidate matrix_candidate(lane) of the first block in the lower
   // lanes, of the second (if any) in the upper.  Words of the two blocks for target
   // = lane.  False (words void) if a candidate lies beyond the bound or is not a
-  // number.
+  // number, or (kNear) some square is too near r^2 for FP32 products to decide.
+  template <bool kNear>
   __device__ __forceinline__ bool words(float x, float y, float z, bool second, uint32_t* lo, uint32_t* hi) const {
     const float cn = __builtin_fmaf(x, x, __builtin_fmaf(y, y, z * z));
     if (__ballot(!(cn <= lim_c)) != 0ull) return false;
+    float dm = __builtin_inff();
     float a00 = x, a01 = y, a10 = z, a11 = cn;
     swap_halves(a00, a01);  // a00: x, y of the first block; a01: of the second
     swap_halves(a10, a11);
     uint32_t w0 = 0, w1 = 0;
     if (second) {
-      tile(a01, a11, b00, b10, C0, w0);
-      if (two) tile(a01, a11, b01, b11, C1, w1);
+      tile<kNear>(a01, a11, b00, b10, C0, w0, dm);
+      if (two) tile<kNear>(a01, a11, b01, b11, C1, w1, dm);
     }
-    tile(a00, a10, b00, b10, C0, w0);
-    if (two) tile(a00, a10, b01, b11, C1, w1);
+    tile<kNear>(a00, a10, b00, b10, C0, w0, dm);
+    if (two) tile<kNear>(a00, a10, b01, b11, C1, w1, dm);
     // w_k: targets 32 k + lane % 32; of each block candidates 16 h + (0-15), h =
     // lane / 32, the second block's in the high half.  To lane = target: w0 the
     // h = 0 bits, w1 the h = 1 bits
     swap_halves(w0, w1);
     *lo = __builtin_amdgcn_perm(w1, w0, 0x05040100u);
     *hi = __builtin_amdgcn_perm(w1, w0, 0x07060302u);
+    if constexpr (kNear) return !__any(dm < eps);
     return true;
   }
 };

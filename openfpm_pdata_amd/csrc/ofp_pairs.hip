@@ -1100,7 +1100,7 @@ __device__ __forceinline__ void chunk_hits(const MatrixTest& mt, bool fast, cons
     float x, y, z;
     rel(buf[k0 + (mine < n ? mine : n - 1u)], &x, &y, &z);
     uint32_t lo = 0, hi = 0;
-    if (fast && mt.words(x, y, z, n > 32u, &lo, &hi)) {
+    if (fast && mt.words<false>(x, y, z, n > 32u, &lo, &hi)) {
       lo &= n < 32u ? 0xFFFFFFFFu >> (32u - n) : 0xFFFFFFFFu;
       hi &= n > 32u ? 0xFFFFFFFFu >> (64u - n) : 0u;
     } else {
@@ -1166,9 +1166,8 @@ __global__ __launch_bounds__(kTileBlock, 4) void k_tile_f32c(ClDev c, QGeom qg1,
     const float rc2 = cell * cell * (bx * bx + by * by * (ry2 + rz2));
     float tx, ty, tz;
     sep(P, ox, oy, oz, &tx, &ty, &tz);
-    const bool fast = __ballot(!(__builtin_fmaf(tx, tx, __builtin_fmaf(ty, ty, tz * tz)) <= rt2 * 1.01f)) == 0ull;
     MatrixTest mt;
-    mt.targets(tx, ty, tz, pre2 + (2.05f * (rt2 + rc2) + pre2) * 0x1p-19f, rc2 * 1.01f, ti.n > 32u);
+    const bool fast = mt.targets<true>(tx, ty, tz, rt2, rc2, pre2, ti.n > 32u);
     bool seen = false;
     for_each_chunk<kChunk>(
         c, G, lane,
@@ -1212,7 +1211,7 @@ struct Pos3 {
 
 template <class T, class Ph, bool kMany>
 __global__ __launch_bounds__(kTileBlock, 4) void k_tile_f64(ClDev c, const T* __restrict__ pos, size_t stride,
-                                                         float spx, float spy, float spz, Ph ph1,
+                                                         double spx, double spy, double spz, Ph ph1,
                                                          const Ph* __restrict__ tab,
                                                          const SysGrid<T>* __restrict__ sys,
                                                          const TargetItem* __restrict__ items,
@@ -1243,21 +1242,21 @@ __global__ __launch_bounds__(kTileBlock, 4) void k_tile_f64(ClDev c, const T* __
     };
     if (kMany) {
       const SysGrid<T>& S = sys[ti.ncx >> 8];
-      spx = float(S.sp[0]);
-      spy = float(S.sp[1]);
-      spz = float(S.sp[2]);
+      spx = double(S.sp[0]);
+      spy = double(S.sp[1]);
+      spz = double(S.sp[2]);
     }
     // relative to the middle target; the bounds as in the Verlet build's count pass
     const uint32_t mid = ti.n / 2;
     const double ox = lane_value(xp, mid), oy = lane_value(yp, mid), oz = lane_value(zp, mid);
-    const float tx = float(xp - ox), ty = float(yp - oy), tz = float(zp - oz);
+    const double unit = matrix_unit(spx, spy, spz);
+    const float ux = float(spx * unit), uy = float(spy * unit), uz = float(spz * unit);
     const float B1 = float(c.box_nn + 1u), nx = float(G.ncx), bx = nx + float(c.box_nn);
-    const float rt2 = nx * nx * spx * spx + spy * spy + spz * spz;
-    const float rc2 = bx * bx * spx * spx + B1 * B1 * (spy * spy + spz * spz);
-    const float r2f = float(ph.rc2);
-    const bool fast = __ballot(!(__builtin_fmaf(tx, tx, __builtin_fmaf(ty, ty, tz * tz)) <= rt2 * 1.01f)) == 0ull;
+    const float rt2 = nx * nx * ux * ux + uy * uy + uz * uz;
+    const float rc2 = bx * bx * ux * ux + B1 * B1 * (uy * uy + uz * uz);
     MatrixTest mt;
-    mt.targets(tx, ty, tz, r2f + (2.05f * (rt2 + rc2) + r2f) * 0x1p-19f, rc2 * 1.01f, ti.n > 32u);
+    const bool fast = mt.targets<true>(float((xp - ox) * unit), float((yp - oy) * unit), float((zp - oz) * unit), rt2,
+                                       rc2, float(ph.rc2 * unit * unit), ti.n > 32u);
     bool seen = false;
     for_each_chunk<kChunk>(
         c, G, lane,
@@ -1269,9 +1268,9 @@ __global__ __launch_bounds__(kTileBlock, 4) void k_tile_f64(ClDev c, const T* __
           chunk_hits(
               mt, fast, buf, m, lane, valid, mk,
               [&](const Pos3<T>& Q, float* x, float* y, float* z) {
-                *x = float(double(Q.x) - ox);
-                *y = float(double(Q.y) - oy);
-                *z = float(double(Q.z) - oz);
+                *x = float((double(Q.x) - ox) * unit);
+                *y = float((double(Q.y) - oy) * unit);
+                *z = float((double(Q.z) - oz) * unit);
               },
               test);
           for_each_hit(mk, (m + 63u) / 64u, lane, [&](uint32_t k) {
@@ -1737,8 +1736,8 @@ static int launch_f64(const PairCtx& x, const void* pos, size_t stride, const Ph
       TileQueue q;
       OFP_TRY(tile_queue(x, &q, s));
       k_tile_f64<T, Ph, false><<<tile_grid(), kTileBlock, 0, s>>>(
-          x.c, P, stride, float(x.v.spacing[0]), float(x.v.spacing[1]), float(x.v.spacing[2]), ph, nullptr, nullptr,
-          q.items, q.n_items, q.counter);
+          x.c, P, stride, x.v.spacing[0], x.v.spacing[1], x.v.spacing[2], ph, nullptr, nullptr, q.items, q.n_items,
+          q.counter);
     }
     OFP_LAUNCHED();
     return OFP_OK;
@@ -2036,8 +2035,8 @@ static int launch_lj_tiles(const PairCtx& x, int precision, const void* pos_sort
                                                                           q.items, q.n_items, q.counter);
   } else {
     using Ph = LJ64T<kU>;
-    k_tile_f64<T, Ph, true><<<tile_grid(), kTileBlock, 0, s>>>(x.c, static_cast<const T*>(pos_sorted), stride, 0.f,
-                                                               0.f, 0.f, Ph{},
+    k_tile_f64<T, Ph, true><<<tile_grid(), kTileBlock, 0, s>>>(x.c, static_cast<const T*>(pos_sorted), stride, 0.0,
+                                                               0.0, 0.0, Ph{},
                                                                static_cast<const Ph*>(tab), sys, q.items, q.n_items,
                                                                q.counter);
   }

@@ -129,12 +129,6 @@ __device__ __forceinline__ void block_table(const ItemRuns& R, uint32_t w0, uint
   lds_order();
 }
 
-// min(m, |a|, |b|): one instruction, which the compiler has to write itself.  Inline
-// asm would hide from it that a and b come out of the matrix cores, and the wait
-// states that such a read needs would be missing.
-__device__ __forceinline__ float min3_abs(float m, float a, float b) {
-  return __builtin_fminf(__builtin_fminf(m, __builtin_fabsf(a)), __builtin_fabsf(b));
-}
 // Part `part` of P of `total` (monotonic in part, 0 and total at the ends).
 __device__ __forceinline__ uint32_t part_begin(uint32_t total, uint32_t part, uint32_t P) {
   return P == 1 ? (part ? total : 0u) : uint32_t(uint64_t(total) * part / P);
@@ -226,12 +220,15 @@ __global__ __launch_bounds__(kVlBlock) void k_vl_place(ClDev c, const SysGrid<T>
 // (unit roundoff u) differ from the exact square by less than 24 u S, and the
 // reference's own roundings by less than 6 u d^2; |d^2 - r^2| < 32 u S = 2^-19 S
 // is tested exactly.  R comes from the cell geometry; blocks or an item with a
-// particle beyond it (outside its cell, or not a number) are tested exactly too.
+// particle beyond it (outside its cell, or not a number) are tested exactly too, and
+// so are items whose squares FP32 cannot hold: FP64 coordinates are scaled by
+// matrix_unit first, FP32 ones are not, for the reference's own squares of them leave
+// the range where those of the products do.
 // 4.2e6 clustered particles (cells of r/2, 150 words a target): 6.4 -> 3.8 ms; 3e5:
 // 0.46 -> 0.27 ms; 4e5 in FP64 0.85 -> 0.36 ms.
 template <class T>
-__global__ __launch_bounds__(kVlBlock, 4) void k_vl_count(ClDev c, const T* __restrict__ xyz, T r2_one, float spx,
-                                                       float spy, float spz, const SysGrid<T>* __restrict__ sys,
+__global__ __launch_bounds__(kVlBlock, 4) void k_vl_count(ClDev c, const T* __restrict__ xyz, T r2_one, T spx,
+                                                       T spy, T spz, const SysGrid<T>* __restrict__ sys,
                                                        const T* __restrict__ r2_sys,
                                                        const TargetItem* __restrict__ items,
                                                        const uint32_t* __restrict__ n_items_p, uint32_t P,
@@ -256,9 +253,9 @@ __global__ __launch_bounds__(kVlBlock, 4) void k_vl_count(ClDev c, const T* __re
     const T r2 = G.r2;
     if (sys) {
       const uint32_t sy = ti.ncx >> 8;
-      spx = float(sys[sy].sp[0]);
-      spy = float(sys[sy].sp[1]);
-      spz = float(sys[sy].sp[2]);
+      spx = sys[sy].sp[0];
+      spy = sys[sy].sp[1];
+      spz = sys[sy].sp[2];
     }
     const bool valid = uint32_t(lane) < ti.n;
     const uint32_t row = ti.row0 + (valid ? uint32_t(lane) : 0u);
@@ -269,27 +266,18 @@ __global__ __launch_bounds__(kVlBlock, 4) void k_vl_count(ClDev c, const T* __re
     // targets relative to the middle one, and the bounds of the FP32 squares
     const uint32_t mid = ti.n / 2;
     const T ox = lane_value(xp, mid), oy = lane_value(yp, mid), oz = lane_value(zp, mid);
-    const float tx = float(xp - ox), ty = float(yp - oy), tz = float(zp - oz);
-    const float tn = __builtin_fmaf(tx, tx, __builtin_fmaf(ty, ty, tz * tz));
+    const T unit = std::is_same_v<T, double> ? T(matrix_unit(spx, spy, spz)) : T(1);
+    auto rel = [&](T a, T o) {
+      if constexpr (std::is_same_v<T, double>) return float((a - o) * unit);
+      return float(a - o);
+    };
+    const float ux = float(spx * unit), uy = float(spy * unit), uz = float(spz * unit);
     const float B1 = float(c.box_nn + 1u), nx = float(G.ncx), bx = nx + float(c.box_nn);
-    const float rt2 = nx * nx * spx * spx + spy * spy + spz * spz;
-    const float rc2 = bx * bx * spx * spx + B1 * B1 * (spy * spy + spz * spz);
-    const float r2f = float(r2);
-    const float lim_t = rt2 * 1.01f, lim_c = rc2 * 1.01f;
-    const float eps = (2.05f * (rt2 + rc2) + r2f) * 0x1p-19f;  // (a + b)^2 <= 2 a^2 + 2 b^2
-    const bool fast = __all(tn <= lim_t);
-    float b00 = -2.f * tx, b01 = -2.f * ty;  // columns of the target halves: k = 0, 1
-    swap_halves(b00, b01);
-    float b10 = -2.f * tz, b11 = 1.f;  // k = 2, 3
-    swap_halves(b10, b11);
-    float k0 = tn - r2f, k1 = k0;
-    swap_halves(k0, k1);
-    v16f C0, C1;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      C0[i] = k0;
-      C1[i] = k1;
-    }
+    const float rt2 = nx * nx * ux * ux + uy * uy + uz * uz;
+    const float rc2 = bx * bx * ux * ux + B1 * B1 * (uy * uy + uz * uz);
+    MatrixTest mt;
+    const bool fast = mt.template targets<false>(rel(xp, ox), rel(yp, oy), rel(zp, oz), rt2, rc2,
+                                                 float(r2 * unit * unit), ti.n > 32u);
     // Exact hit bits of candidates j0 .. j0 + m - 1 (1 <= m <= 32, uniform), bit k
     // for candidate j0 + k; the coordinates come in through scalar loads.  Lanes
     // past the item's targets compute bits that are never stored.
@@ -308,16 +296,6 @@ __global__ __launch_bounds__(kVlBlock, 4) void k_vl_count(ClDev c, const T* __re
       }
       return __builtin_bitreverse32(w << (32u - m));
     };
-    // one tile: bits of 16 candidates appended to w, the smallest |square| in dm
-    auto tile = [&](float a0, float a1, float b0, float b1, const v16f& K, uint32_t& w, float& dm) {
-      v16f D = __builtin_amdgcn_mfma_f32_32x32x2f32(a0, b0, K, 0, 0, 0);
-      D = __builtin_amdgcn_mfma_f32_32x32x2f32(a1, b1, D, 0, 0, 0);
-#pragma unroll
-      for (int i = 0; i < 16; ++i) w = __builtin_amdgcn_alignbit(w, __float_as_uint(D[i]), 31);
-#pragma unroll
-      for (int i = 0; i < 16; i += 2) dm = min3_abs(dm, D[i], D[i + 1]);
-    };
-    const bool two_t = ti.n > 32u;
     uint32_t n = 0;
     // the unit's words [wa, wb), whole quads; blocks past the item's last are empty
     const uint32_t wa = 4u * part_begin(at.words / 4u, part, P), wb = 4u * part_begin(at.words / 4u, part + 1, P);
@@ -349,33 +327,11 @@ __global__ __launch_bounds__(kVlBlock, 4) void k_vl_count(ClDev c, const T* __re
     uint32_t q0 = 0, q1 = 0;  // the quad's first two words
     for (uint32_t w = wa; w < wb; w += 2) {
       const Two b = cur;
-      const float x0 = float(cx - ox), y0 = float(cy - oy), z0 = float(cz - oz);
+      const float x0 = rel(cx, ox), y0 = rel(cy, oy), z0 = rel(cz, oz);
       if (w + 2 < wb) cur = fetch(w + 2);
       uint32_t lo = 0, hi = 0;
       if (b.ma) {
-        const float cn = __builtin_fmaf(x0, x0, __builtin_fmaf(y0, y0, z0 * z0));
-        bool exact = !fast;
-        if (!exact) {
-          float dm = cn <= lim_c ? __builtin_inff() : 0.f;
-          float a00 = x0, a01 = y0, a10 = z0, a11 = cn;
-          swap_halves(a00, a01);  // a00: x, y of the first block; a01: of the second
-          swap_halves(a10, a11);
-          uint32_t w0 = 0, w1 = 0;
-          if (b.mb) {
-            tile(a01, a11, b00, b10, C0, w0, dm);
-            if (two_t) tile(a01, a11, b01, b11, C1, w1, dm);
-          }
-          tile(a00, a10, b00, b10, C0, w0, dm);
-          if (two_t) tile(a00, a10, b01, b11, C1, w1, dm);
-          // w_k: targets 32 k + lane % 32; of each block candidates 16 h + (0-15), h =
-          // lane / 32, the second block's in the high half.  To lane = target: w0 the
-          // h = 0 bits, w1 the h = 1 bits
-          swap_halves(w0, w1);
-          lo = __builtin_amdgcn_perm(w1, w0, 0x05040100u);
-          hi = __builtin_amdgcn_perm(w1, w0, 0x07060302u);
-          exact = __any(dm < eps);
-        }
-        if (exact) {  // a few per hundred
+        if (!fast || !mt.template words<true>(x0, y0, z0, b.mb != 0u, &lo, &hi)) {  // a few per hundred
           lo = hit_word(b.ja, b.ma);
           hi = b.mb ? hit_word(b.jb, b.mb) : 0u;
         } else {
@@ -919,8 +875,8 @@ static int vl_build_t(ofp_vl* h, const ofp_cl* cl, const void* pos_v, size_t str
       OFP_TRY(fill_u32(heads, 0, kQueueWords, s));
       if (add) OFP_TRY(fill_u32(h->cnt.as<uint32_t>(), 0, n, s));
     }
-    k_vl_count<T><<<grid, kVlBlock, 0, s>>>(c, h->xyz.as<T>(), r2_one, float(v.spacing[0]), float(v.spacing[1]),
-                                            float(v.spacing[2]), sys, r2_sys, items, n_items, sp.parts, heads,
+    k_vl_count<T><<<grid, kVlBlock, 0, s>>>(c, h->xyz.as<T>(), r2_one, T(v.spacing[0]), T(v.spacing[1]),
+                                            T(v.spacing[2]), sys, r2_sys, items, n_items, sp.parts, heads,
                                             h->cnt.as<uint32_t>(), mstate, h->place.as<ItemPlace>(),
                                             h->masks.as<unsigned long long>(), (unsigned long long)h->mask_cap);
     OFP_LAUNCHED();

@@ -70,3 +70,39 @@ def test_particles_beyond_their_cells(dtype, n):
     vl = vdm.VerletListGPU()
     vl.build(cl, out, r)
     check_rows(pos.cpu().numpy(), r, cl, vl, npd)
+
+
+def scaled(dtype, scale, n=4000):
+    """Particles in cells of 20 and more, and their lists' radius, in units of 1 / scale
+    (a power of two: the same bits in the mantissas)."""
+    rng = np.random.default_rng(11)
+    p = np.concatenate([rng.random((3, n // 2)) * 3.4, 1.0 + rng.random((3, n // 2))], axis=1)
+    npd = np.float32 if dtype == torch.float32 else np.float64
+    pos = np.ascontiguousarray(p.astype(npd) * npd(scale))
+    r = 0.6 * scale
+    vd = vdm.VectorDistGPU(n, (0.0,) * 3, (3.5 * scale,) * 3, (0, 0, 0), r, dtype=dtype)
+    vd.pos[:, :n] = torch.from_numpy(pos).cuda()
+    return pos, r, vd, npd
+
+
+@pytest.mark.parametrize("exponent", [0, -40, -50, -63, -70, -100, -480, -505, 40, 60, 64, 100, 480, 505])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+def test_units_of_length(dtype, exponent):
+    """Lengths whose squares FP32 (and at the ends FP64) cannot hold: the rows are the
+    direct search's in the positions' own arithmetic, the cell tiles' neighbour counts
+    that of FP64."""
+    if dtype == torch.float32 and abs(exponent) > 100:
+        pytest.skip("FP32 holds no such length")
+    pos, r, vd, npd = scaled(dtype, 2.0 ** exponent)
+    n = pos.shape[1]
+    cl, vl = vd.getVerletGPU(r, sub=1)
+    with np.errstate(over="ignore", under="ignore"):
+        check_rows(pos, r, cl, vl, npd)
+    nn = torch.zeros(vd.cap, dtype=torch.int32, device="cuda")
+    L.call("ofp_pair_lj", cl.h, None, vd.pos.data_ptr(), vd.cap, L.OFP_PREC_F64, L.LJParams(r, 0.1 * r, 1.0), None, None,
+           None, None, nn.data_ptr(), vdm._stream())
+    got = nn[cl.arrays()["n2s"].long()[:n]].cpu().numpy()
+    x = pos.astype(np.float64)
+    for i in range(n):
+        d = x - x[:, i:i + 1]
+        assert got[i] == np.count_nonzero((d[0] * d[0] + d[1] * d[1]) + d[2] * d[2] < r * r) - 1, i
