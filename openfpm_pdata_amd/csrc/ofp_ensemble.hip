@@ -19,6 +19,8 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <initializer_list>
+#include <utility>
 #include <vector>
 
 namespace ofp {
@@ -470,12 +472,12 @@ static int ens_destroy_graphs(ofp_ens* e) {
   return OFP_OK;
 }
 
-// The permuted copies become the stored particles (the forces too when they
-// were permuted).
-static void ens_swap_storage(ofp_ens* e, bool with_frc) {
+// The permuted copies become the stored particles.  The forces do not swap: the step
+// graphs, which are kept per spar, name their buffer, and a rebuild within a run
+// leaves them where they are; a permutation of them is copied back.
+static void ens_swap_storage(ofp_ens* e) {
   std::swap(e->pos, e->pos2);
   std::swap(e->vel, e->vel2);
-  if (with_frc) std::swap(e->frc, e->frc2);
   std::swap(e->gid, e->gid2);
   e->spar ^= 1;
 }
@@ -654,6 +656,32 @@ static int ens_alloc(ofp_ens* e, hipStream_t s) {
   return OFP_OK;
 }
 
+template <class U>
+static void add_plane(PlaneArgs* pa, const U* src, U* dst) {
+  pa->src[pa->n] = reinterpret_cast<uint64_t>(src);
+  pa->dst[pa->n] = reinterpret_cast<uint64_t>(dst);
+  pa->esz[pa->n] = uint32_t(sizeof(U));
+  ++pa->n;
+}
+
+__global__ __launch_bounds__(256) void k_ens_copy(uint32_t n, PlaneArgs pa) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) copy_planes(pa, i, i);
+}
+
+// Domain particles of 3-plane arrays: first = second of each pair.
+template <class T>
+static int ens_copy_back(const ofp_ens* e, std::initializer_list<std::pair<DevBuf*, const DevBuf*>> arrays,
+                         hipStream_t s) {
+  PlaneArgs pa{};
+  for (const auto& a : arrays)
+    for (size_t d = 0; d < 3; ++d)
+      add_plane(&pa, static_cast<const T*>(a.second->p) + d * e->cap, static_cast<T*>(a.first->p) + d * e->cap);
+  k_ens_copy<<<grid_for(e->N, 256), 256, 0, s>>>(uint32_t(e->N), pa);
+  OFP_LAUNCHED();
+  return OFP_OK;
+}
+
 // The rebuild: map (+ storage permutation), ghosts, cell list, Verlet list.
 // sizing: counts read back and capacities grown (synchronous, not capturable).
 // keep_frc = false: the stored forces are not read before they are written
@@ -677,7 +705,8 @@ static int ens_rebuild_t(ofp_ens* e, int sizing, hipStream_t s, bool keep_frc) {
                                     e->vel2.as<T>(), keep_frc ? e->frc2.as<T>() : nullptr,
                                     e->gid2.as<uint32_t>(), e->xb.as<T>(), sid, dyn);
     OFP_LAUNCHED();
-    ens_swap_storage(e, keep_frc);
+    ens_swap_storage(e);
+    if (keep_frc) OFP_TRY(ens_copy_back<T>(e, {{&e->frc, &e->frc2}}, s));
     e->ordered = true;
   } else {
     k_ens_map<T><<<gN, 256, 0, s>>>(N, cap, nullptr, nullptr, e->pos.as<T>(), nullptr, nullptr, nullptr, nullptr,
@@ -755,14 +784,6 @@ static int ens_rebuild_t(ofp_ens* e, int sizing, hipStream_t s, bool keep_frc) {
   return OFP_OK;
 }
 
-template <class U>
-static void add_plane(PlaneArgs* pa, const U* src, U* dst) {
-  pa->src[pa->n] = reinterpret_cast<uint64_t>(src);
-  pa->dst[pa->n] = reinterpret_cast<uint64_t>(dst);
-  pa->esz[pa->n] = uint32_t(sizeof(U));
-  ++pa->n;
-}
-
 // A run's particles in the caller's order: put them in the order of the build's
 // rows before the steps (k_ens_relabel), so the first steps read and write them
 // as coalesced as those after the next rebuild do.
@@ -810,7 +831,8 @@ static int ens_relabel_t(ofp_ens* e, bool keep_frc, hipStream_t s) {
                                                                 e->opid.as<uint32_t>());
     OFP_LAUNCHED();
   }
-  ens_swap_storage(e, keep_frc);
+  ens_swap_storage(e);
+  if (keep_frc) OFP_TRY(ens_copy_back<T>(e, {{&e->frc, &e->frc2}}, s));
   e->ordered = true;
   return OFP_OK;
 }
@@ -1277,7 +1299,7 @@ int ofp_ens_run(ofp_ens* e, int precision, double dt, int n_steps, int use_graph
           OFP_TRY(capture(e, &e->g_rebuild[q], &e->g_rebuild_epoch[q],
                           [&](hipStream_t cs) { return ens_rebuild(e, 0, cs, false); }));
         else
-          ens_swap_storage(e, false);
+          ens_swap_storage(e);
         OFP_HIP(hipGraphLaunch(e->g_rebuild[q], s));
       } else {
         OFP_TRY(ens_rebuild(e, 0, s, false));
