@@ -514,7 +514,12 @@ typedef struct ofp_ens_state {
   uint32_t rebuild_pending, overflow;
 } ofp_ens_state;
 
-/* Device arrays of an ensemble (storage order, `cap` = plane stride). */
+/* Device arrays of an ensemble (storage order, `cap` = plane stride).  The pointers
+ * hold until the next ofp_ens_set, ofp_ens_rebuild, ofp_ens_forces or ofp_ens_run: a
+ * rebuild, also one within a run, permutes the particles into other buffers, and one
+ * that grows a capacity allocates them anew.  The storage order changes with every
+ * rebuild and, without one, when a run of two or more steps starts with the particles
+ * still in the order of ofp_ens_set; gid follows. */
 typedef struct ofp_ens_arrays {
   void* pos;           /* 3 planes, domain then ghosts */
   void* vel;           /* 3 planes, domain */

@@ -78,7 +78,9 @@ __global__ __launch_bounds__(256) void k_ens_map(uint32_t N, size_t cap, const u
 // The stored particles into the domain-row order of the build they are in, with
 // that build kept: its sorted order, cells and Verlet rows are in sorted indices
 // and stay; only the storage indices it names change (row k's particle becomes
-// stored particle k).  inv[old storage index] = new one, for k_ens_relabel_ghosts.
+// stored particle k; written to the *2 arrays and copied back, for a run moves no
+// buffer unless it rebuilds).  inv[old storage index] = new one, for
+// k_ens_relabel_ghosts.
 // Called with positions that are those of the build (xb equals them).  It is paid
 // once, against nine gathered and six scattered values per particle in every later
 // step: 40 steps of 2^23 particles given in random order 108.7 -> 28.7 ms.  Bound by
@@ -669,14 +671,15 @@ __global__ __launch_bounds__(256) void k_ens_copy(uint32_t n, PlaneArgs pa) {
   if (i < n) copy_planes(pa, i, i);
 }
 
-// Domain particles of 3-plane arrays: first = second of each pair.
+// Domain particles of 3-plane arrays: first = second of each pair; and ids, if any.
 template <class T>
 static int ens_copy_back(const ofp_ens* e, std::initializer_list<std::pair<DevBuf*, const DevBuf*>> arrays,
-                         hipStream_t s) {
+                         DevBuf* ids, const DevBuf* ids2, hipStream_t s) {
   PlaneArgs pa{};
   for (const auto& a : arrays)
     for (size_t d = 0; d < 3; ++d)
       add_plane(&pa, static_cast<const T*>(a.second->p) + d * e->cap, static_cast<T*>(a.first->p) + d * e->cap);
+  if (ids) add_plane(&pa, static_cast<const uint32_t*>(ids2->p), static_cast<uint32_t*>(ids->p));
   k_ens_copy<<<grid_for(e->N, 256), 256, 0, s>>>(uint32_t(e->N), pa);
   OFP_LAUNCHED();
   return OFP_OK;
@@ -706,7 +709,7 @@ static int ens_rebuild_t(ofp_ens* e, int sizing, hipStream_t s, bool keep_frc) {
                                     e->gid2.as<uint32_t>(), e->xb.as<T>(), sid, dyn);
     OFP_LAUNCHED();
     ens_swap_storage(e);
-    if (keep_frc) OFP_TRY(ens_copy_back<T>(e, {{&e->frc, &e->frc2}}, s));
+    if (keep_frc) OFP_TRY(ens_copy_back<T>(e, {{&e->frc, &e->frc2}}, nullptr, nullptr, s));
     e->ordered = true;
   } else {
     k_ens_map<T><<<gN, 256, 0, s>>>(N, cap, nullptr, nullptr, e->pos.as<T>(), nullptr, nullptr, nullptr, nullptr,
@@ -831,8 +834,11 @@ static int ens_relabel_t(ofp_ens* e, bool keep_frc, hipStream_t s) {
                                                                 e->opid.as<uint32_t>());
     OFP_LAUNCHED();
   }
-  ens_swap_storage(e);
-  if (keep_frc) OFP_TRY(ens_copy_back<T>(e, {{&e->frc, &e->frc2}}, s));
+  // the stored particles keep their buffers (pointers taken after ofp_ens_set)
+  if (keep_frc)
+    OFP_TRY(ens_copy_back<T>(e, {{&e->pos, &e->pos2}, {&e->vel, &e->vel2}, {&e->frc, &e->frc2}}, &e->gid, &e->gid2, s));
+  else
+    OFP_TRY(ens_copy_back<T>(e, {{&e->pos, &e->pos2}, {&e->vel, &e->vel2}}, &e->gid, &e->gid2, s));
   e->ordered = true;
   return OFP_OK;
 }

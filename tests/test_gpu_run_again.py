@@ -6,6 +6,7 @@ import torch
 
 from openfpm_pdata_amd import _lib as L
 from openfpm_pdata_amd import ensemble as E
+from openfpm_pdata_amd import vector_dist as vdm
 
 pytestmark = pytest.mark.gpu
 
@@ -45,3 +46,29 @@ def test_set_forces_run_again(prec, steps, explicit):
                 out.append(e.get())
             for name, a, b in zip(("pos", "vel", "force"), *out):
                 assert torch.equal(a, b), (rnd, again, name)
+
+
+@pytest.mark.parametrize("with_forces", [False, True])
+@pytest.mark.parametrize("n", [2000, 1 << 22])
+def test_arrays_of_a_run_without_rebuild(n, with_forces):
+    """A run that needs no rebuild reorders the stored particles but moves no buffer."""
+    m = round(n ** (1.0 / 3.0)) + 1
+    systems = [E.System(n, 1.5 / m, 0.5 / m, 1.0, 1.0)]
+    ens = E.Ensemble(systems, torch.float32, E.Options(skin=0.3, sub=1, lanes=1))
+    x, v = gas(systems, m, 1)
+    ens.set(x, v)
+    if with_forces:
+        ens.force_pass(L.OFP_PREC_F64)
+    else:
+        ens.rebuild()
+    a = ens.arrays()
+    before = ens.status()["rebuilds"]
+    ens.run(L.OFP_PREC_F64, 1e-6 / m, 3)
+    assert ens.status()["rebuilds"] == before
+    b = ens.arrays()
+    assert (a.pos, a.vel, a.force, a.gid, a.cap) == (b.pos, b.vel, b.force, b.gid, b.cap)
+    gid = ens.gid().long()
+    assert torch.equal(torch.sort(gid).values, torch.arange(n, device="cuda"))
+    for ptr, want in zip((a.pos, a.vel, a.force), ens.get()):
+        got = vdm.device_view(ptr, 3 * int(a.cap), torch.float32).view(3, -1)[:, :n]
+        assert torch.equal(got, want[:, gid])
