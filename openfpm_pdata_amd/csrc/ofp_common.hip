@@ -68,11 +68,22 @@ void give_back(const std::list<Kept>& blocks) {
 }
 }  // namespace
 
+// Test hook: the next `count` allocations of lo to hi bytes fail, as on a full device
+// (the runtime is asked for more than any device has).
+namespace {
+std::atomic<size_t> g_fail_lo{0}, g_fail_hi{0};
+std::atomic<int> g_fail_count{0};
+bool test_fails(size_t bytes) {
+  if (g_fail_count.load(std::memory_order_relaxed) <= 0 || bytes < g_fail_lo || bytes > g_fail_hi) return false;
+  return g_fail_count.fetch_sub(1) > 0;
+}
+}  // namespace
+
 int block_alloc(void** p, size_t bytes, size_t* cap, int* dev) {
   *p = nullptr;
   *cap = 0;
   OFP_HIP(hipGetDevice(dev));
-  const size_t want = block_size(bytes);
+  const size_t want = test_fails(bytes) ? size_t(1) << 60 : block_size(bytes);
   Pool& P = pool();
   const int d = *dev;
   if (d >= 0 && d < kMaxPoolDevices) {
@@ -120,6 +131,9 @@ int block_alloc(void** p, size_t bytes, size_t* cap, int* dev) {
     e = hipMalloc(p, want);
   }
   if (e != hipSuccess) {
+    // the return code alone carries the error: a caller that goes on without the
+    // block would find the runtime's at its next launch
+    (void)hipGetLastError();
     *p = nullptr;
     return set_error(OFP_E_HIP, "hipMalloc(%zu): %s", want, hipGetErrorString(e));
   }
@@ -415,6 +429,14 @@ extern "C" {
 const char* ofp_last_error(void) { return ofp::g_last_error.c_str(); }
 
 int ofp_abi_version(void) { return OFP_ABI_VERSION; }
+
+// Test hook (not in the public header), see test_fails.
+int ofp_test_fail_alloc_(size_t lo, size_t hi, int count) {
+  ofp::g_fail_lo = lo;
+  ofp::g_fail_hi = hi;
+  ofp::g_fail_count = count;
+  return OFP_OK;
+}
 
 int ofp_device_info(int* device, int* n_cu, char* arch, size_t arch_len) {
   int dev = 0;

@@ -1,0 +1,83 @@
+"""Allocations that a call can do without, refused as on a full device: the call goes
+on without them and its results are those of an undisturbed call; one that it cannot
+do without is an error of that call alone."""
+from contextlib import contextmanager
+
+import numpy as np
+import pytest
+import torch
+
+from openfpm_pdata_amd import _lib as L
+from openfpm_pdata_amd import vector_dist as vdm
+
+pytestmark = pytest.mark.gpu
+
+
+@contextmanager
+def refused(lo, hi, count):
+    """The library's next `count` allocations of lo to hi bytes fail."""
+    L.call("ofp_test_fail_alloc_", lo, hi, count)
+    try:
+        yield
+    finally:
+        L.call("ofp_test_fail_alloc_", 0, 0, 0)
+
+
+def verlet(n=5000, r=0.09, seed=3):
+    x = np.random.default_rng(seed).random((3, n)).astype(np.float32)
+    vd = vdm.VectorDistGPU(n, (0.0,) * 3, (1.0,) * 3, (0, 0, 0), r, dtype=torch.float32)
+    vd.pos[:, :n] = torch.from_numpy(x).cuda()
+    cl, vl = vd.getVerletGPU(r, vdm.CL_NON_SYMMETRIC | vdm.CL_QUANT)
+    return vd, cl, vl
+
+
+def density(made, h=0.04):
+    vd, cl, vl = made
+    rho = torch.zeros(vd.cap, dtype=torch.float64, device="cuda")
+    L.call("ofp_sph_density", cl.h, vl.h, vd.pos.data_ptr(), vd.cap, L.OFP_PREC_F32C, L.SPHParams(h, 0.1, 1000.0, 10.0),
+           rho.data_ptr(), vdm._stream())
+    return rho
+
+
+def test_density_without_its_records():
+    want = density(verlet())
+    made = verlet()
+    n = int(made[1].view().n_part)
+    with refused(12 * n, 12 * (n + 2), 1):
+        got = density(made)
+    assert torch.equal(got, want)
+    assert torch.equal(density(made), want)  # with them
+
+
+@pytest.mark.parametrize("refusals", [1, 2])
+def test_far_build_with_little_or_no_scratch(refusals):
+    n = (1 << 22) + 12345
+    gen = torch.Generator(device="cuda").manual_seed(4)
+    pos = torch.rand((3, n), generator=gen, device="cuda")
+    idx = torch.arange(n, device="cuda", dtype=torch.int32)
+    out = []
+    for k in (0, refusals):
+        cl = vdm.CellListGPU(torch.float32, (0.0,) * 3, (1.0,) * 3, (78,) * 3, vdm.CL_NON_SYMMETRIC | vdm.CL_GPU_REORDER,
+                             1.0 / 78)
+        srt, idx_s = torch.empty_like(pos), torch.empty_like(idx)
+        with refused(30_000_000, 125_000_000, k):
+            cl.construct(pos, n, n, srt, [(idx.data_ptr(), 4)], [(idx_s.data_ptr(), 4)])
+        back = torch.empty_like(pos)
+        cl.restore(vdm.planes_of(srt), vdm.planes_of(back))
+        a = cl.arrays()
+        out.append([a["s2n"].clone(), a["n2s"].clone(), srt, idx_s])
+        assert torch.equal(back, pos)
+    for a, b in zip(*out):
+        assert torch.equal(a, b)
+
+
+def test_a_refused_call_leaves_no_error_behind():
+    made = verlet()
+    with refused(1, 1 << 40, 1):
+        with pytest.raises(L.OfpError):
+            vdm.VerletListGPU().build(made[1], made[0].pos, 0.09)
+    off, nbr = (t.clone() for t in made[2].arrays())
+    made[2].build(made[1], made[0].pos, 0.09)
+    for a, b in zip((off, nbr), made[2].arrays()):
+        assert torch.equal(a, b)
+    torch.cuda.synchronize()
