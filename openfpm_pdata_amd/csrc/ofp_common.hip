@@ -79,6 +79,17 @@ bool test_fails(size_t bytes) {
 }
 }  // namespace
 
+// Waits for everything submitted to the current device.  By hipFree, which waits
+// implicitly, on an allocation made for it (3 us on an idle device): a
+// hipDeviceSynchronize would end any capture under way, this thread's or another's,
+// that allows hipMalloc.
+static bool device_wait() {
+  void* p = nullptr;
+  if (hipMalloc(&p, 256) == hipSuccess && hipFree(p) == hipSuccess) return true;
+  (void)hipGetLastError();
+  return false;
+}
+
 int block_alloc(void** p, size_t bytes, size_t* cap, int* dev) {
   *p = nullptr;
   *cap = 0;
@@ -105,18 +116,21 @@ int block_alloc(void** p, size_t bytes, size_t* cap, int* dev) {
     }
     if (best.p) {
       if (before) {
-        const hipError_t e = hipDeviceSynchronize();
+        const bool waited = device_wait();
         std::lock_guard<std::mutex> lock(P.m);
-        if (e != hipSuccess) {  // a failed device, or a stream of this thread being captured: keep it for later
+        if (waited) {
+          if (P.synced[d] < before) P.synced[d] = before;
+        } else {  // kept for later
           P.kept.push_back(best);
           P.held[d] += best.cap;
-          return set_error(OFP_E_HIP, "hipDeviceSynchronize: %s", hipGetErrorString(e));
+          best.p = nullptr;
         }
-        if (P.synced[d] < before) P.synced[d] = before;
       }
-      *p = best.p;
-      *cap = best.cap;
-      return OFP_OK;
+      if (best.p) {
+        *p = best.p;
+        *cap = best.cap;
+        return OFP_OK;
+      }
     }
   }
   hipError_t e = hipMalloc(p, want);

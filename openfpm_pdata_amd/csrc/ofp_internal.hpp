@@ -57,9 +57,9 @@ void bump_realloc_epoch();
 // in hipMalloc and hipFree (LJ over a new list of 1e6 particles: 9.3 -> 1.26 ms a call,
 // up to 41 ms before where calls follow each other without a wait).
 //  * A block is handed out again only after the device has finished everything
-//    submitted before the block's release (one hipDeviceSynchronize covers all
-//    earlier releases; hipFree waits the same way), so its former users may have
-//    run on any stream and been called from any thread.
+//    submitted before the block's release (one wait covers all earlier releases;
+//    hipFree waits the same way), so its former users may have run on any stream and
+//    been called from any thread.
 //  * Kept blocks are bounded (1/32 of the device's memory; the oldest go first),
 //    given back when an allocation fails, and all given back when the library's
 //    last handle is destroyed.
