@@ -145,6 +145,12 @@ int ofp_abi_version(void);
 /* Allocates nothing; reports the device the library will use (hipGetDevice). */
 int ofp_device_info(int* device, int* n_cu, char* arch, size_t arch_len);
 
+/* Device blocks of destroyed handles stay with the library for its next handles: at
+ * most 1/128 of a device's memory, until the last handle is destroyed or an
+ * allocation of the library fails.  ofp_trim gives them back now, for allocators that
+ * run out beside it; *bytes (may be NULL): how much.  Waits for the device. */
+int ofp_trim(size_t* bytes);
+
 /* -------------------------------------------------------------- geometry
  * Host-only; write results into host arrays (values of type dtype). */
 

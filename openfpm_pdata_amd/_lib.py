@@ -122,6 +122,7 @@ _u32p = C.POINTER(C.c_uint32)
 SIGNATURES = {
     "ofp_last_error": (C.c_char_p, []),
     "ofp_abi_version": (_i, []),
+    "ofp_trim": (_i, [C.POINTER(_sz)]),
     "ofp_device_info": (_i, [C.POINTER(C.c_int), C.POINTER(C.c_int), C.c_char_p, _sz]),
     "ofp_shift_vectors": (_i, [_i, _vp, _vp, _vp]),
     "ofp_local_ghost_boxes": (_i, [_i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, C.POINTER(C.c_int)]),

@@ -42,9 +42,22 @@ Pool& pool() {
   static Pool* p = new Pool();  // lives until the process ends
   return *p;
 }
+// Most bytes kept on a device (under the lock): 1/128 of its memory.  Another
+// allocator of the program cannot reach kept blocks, so the bound is what the lists
+// that programs make anew need (2e6 particles with 46 entries: 0.8 GB), 2.25 GB of
+// 288; larger blocks go back at once.
+size_t keep_limit(Pool& P, int dev) {
+  if (P.limit[dev] == 0) {
+    hipDeviceProp_t prop;
+    P.limit[dev] = hipGetDeviceProperties(&prop, dev) == hipSuccess ? prop.totalGlobalMem / 128 + 1 : 1;
+  }
+  return P.limit[dev];
+}
 // Sizes in steps of an eighth of their power of two, so counts that vary a
-// little from call to call meet the same blocks.
-size_t block_size(size_t b) {
+// little from call to call meet the same blocks; blocks too large to be kept have
+// the size asked for.
+size_t block_size(size_t b, size_t limit) {
+  if (b > limit) return b;
   size_t step = 256;
   while (step * 16 < b) step *= 2;
   return (b + step - 1) / step * step;
@@ -94,7 +107,7 @@ int block_alloc(void** p, size_t bytes, size_t* cap, int* dev) {
   *p = nullptr;
   *cap = 0;
   OFP_HIP(hipGetDevice(dev));
-  const size_t want = test_fails(bytes) ? size_t(1) << 60 : block_size(bytes);
+  size_t want = bytes;
   Pool& P = pool();
   const int d = *dev;
   if (d >= 0 && d < kMaxPoolDevices) {
@@ -102,6 +115,8 @@ int block_alloc(void** p, size_t bytes, size_t* cap, int* dev) {
     uint64_t before = 0;
     {
       std::lock_guard<std::mutex> lock(P.m);
+      want = block_size(bytes, keep_limit(P, d));
+      if (test_fails(bytes)) bytes = want = size_t(1) << 60;
       auto found = P.kept.end();
       for (auto it = P.kept.begin(); it != P.kept.end(); ++it)
         if (it->dev == d && it->cap >= want && it->cap <= want + want / 4 &&
@@ -143,6 +158,7 @@ int block_alloc(void** p, size_t bytes, size_t* cap, int* dev) {
     }
     give_back(mine);
     e = hipMalloc(p, want);
+    if (e == hipErrorOutOfMemory && want > bytes) e = hipMalloc(p, want = bytes);
   }
   if (e != hipSuccess) {
     // the return code alone carries the error: a caller that goes on without the
@@ -161,11 +177,7 @@ void block_free(void* p, size_t cap, int dev) {
   bool keep = false;
   if (dev >= 0 && dev < kMaxPoolDevices) {
     std::lock_guard<std::mutex> lock(P.m);
-    if (P.limit[dev] == 0) {
-      hipDeviceProp_t prop;
-      P.limit[dev] = hipGetDeviceProperties(&prop, dev) == hipSuccess ? prop.totalGlobalMem / 32 + 1 : 1;
-    }
-    const size_t limit = P.limit[dev];
+    const size_t limit = keep_limit(P, dev);
     if (P.handles > 0 && cap <= limit) {
       keep = true;
       P.kept.push_back(Kept{p, cap, dev, ++P.releases});
@@ -443,6 +455,20 @@ extern "C" {
 const char* ofp_last_error(void) { return ofp::g_last_error.c_str(); }
 
 int ofp_abi_version(void) { return OFP_ABI_VERSION; }
+
+int ofp_trim(size_t* bytes) {
+  ofp::Pool& P = ofp::pool();
+  std::list<ofp::Kept> out;
+  {
+    std::lock_guard<std::mutex> lock(P.m);
+    out = ofp::take_out(P, [](const ofp::Kept&) { return true; });
+  }
+  size_t sum = 0;
+  for (const ofp::Kept& k : out) sum += k.cap;
+  ofp::give_back(out);
+  if (bytes) *bytes = sum;
+  return OFP_OK;
+}
 
 // Test hook (not in the public header), see test_fails.
 int ofp_test_fail_alloc_(size_t lo, size_t hi, int count) {

@@ -60,9 +60,9 @@ void bump_realloc_epoch();
 //    submitted before the block's release (one wait covers all earlier releases;
 //    hipFree waits the same way), so its former users may have run on any stream and
 //    been called from any thread.
-//  * Kept blocks are bounded (1/32 of the device's memory; the oldest go first),
-//    given back when an allocation fails, and all given back when the library's
-//    last handle is destroyed.
+//  * Kept blocks are bounded (1/128 of the device's memory; the oldest go first),
+//    given back when an allocation fails or the program asks (ofp_trim), and all
+//    given back when the library's last handle is destroyed.
 int block_alloc(void** p, size_t bytes, size_t* cap, int* dev);
 void block_free(void* p, size_t cap, int dev);
 

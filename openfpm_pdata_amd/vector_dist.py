@@ -89,6 +89,14 @@ def plane_array(pl: list):
     return arr
 
 
+def trim() -> int:
+    """Gives the device memory of destroyed lists back that the library keeps for its
+    next ones; returns the bytes."""
+    n = C.c_size_t(0)
+    L.call("ofp_trim", C.byref(n))
+    return int(n.value)
+
+
 class _DevArray:
     """Exposes a raw device pointer through __cuda_array_interface__."""
 
