@@ -29,6 +29,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <mutex>
 #include <type_traits>
 
 struct ofp_vl {
@@ -37,6 +38,7 @@ struct ofp_vl {
   ofp::DevBuf rmask;  // thread-per-row build: the rows' hit masks, count pass to fill
   ofp::DevBuf aux;  // pair kernels' per-particle gather stream over the rows
   ofp::DevBuf rec;  // the density pass's 12-byte records
+  std::mutex rec_lock;  // its allocation: passes over one list may come from several threads
   size_t mask_cap = 0;  // pairs of mask words (8 bytes) the buffer holds (0: not sized yet)
   bool rows_path = false;  // the last build ran the thread-per-row kernels
   uint64_t n_rows = 0, n_entries = 0;
@@ -1043,6 +1045,7 @@ int ofp_vl_rec_(const ofp_vl* h, size_t bytes, void** p, hipStream_t s) {
   OFP_CHECK(h && p, OFP_E_ARG, "ofp_vl_rec_: null argument");
   ofp_vl* m = const_cast<ofp_vl*>(h);
   *p = nullptr;
+  std::lock_guard<std::mutex> lock(m->rec_lock);
   if (m->rec.cap < bytes) {
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     OFP_HIP(hipStreamIsCapturing(s, &cap));
