@@ -52,7 +52,10 @@ __device__ __forceinline__ int wrap_diff(int gq, int gp) { return int(uint32_t(g
 // a pass needs no cut-off decision (both go to zero with the distance to 2h, as
 // (1 - r/2h)^3 and (1 - r/2h)^2; a pair that one rounding puts on either side
 // adds less than any rounding of the sums).  The particle itself has
-// t = u = 1: W = 1, dW = 0.
+// t = u = 1: W = 1.  A force needs dW/dq / r: (u^2 - t^2) / r taken as it stands
+// cancels for close pairs (relative error 2e-16 / q); as (u + t) (u - t) / r, where
+// (u - t) / r is -1/(2h) below r = h and -t / r from there on, the larger of the two,
+// it does not.
 // max(min(1 + a b, 1), 0) in one instruction: the FMA's clamp modifier (a NaN
 // gives 0 in the clamp mode kernels run in).
 __device__ __forceinline__ double sat1(double a, double b) {
@@ -64,10 +67,16 @@ struct Spline {
   double n2, n1;  // -1/(2h), -1/h in the unit of the pass
   __device__ __forceinline__ double t(double r) const { return sat1(r, n2); }
   __device__ __forceinline__ double u(double r) const { return sat1(r, n1); }
+  // dW/dq / (3 r), inv = 1 / r
+  __device__ __forceinline__ double slope(double r, double inv) const {
+    const double t_ = t(r);
+    return (u(r) + t_) * __builtin_fmax(n2, -t_ * inv);
+  }
 };
-// sqrt(x) and 1/sqrt(x) of an FP64 pass (x > 0) to the last bit or so:
-// Goldschmidt's iteration from the hardware estimate (2^-23), then one
-// correction of each by its residual.
+// sqrt(x) and 1/sqrt(x) of an FP64 pass (x > 0): Goldschmidt's iteration from the
+// hardware estimate (2^-23), then one correction of each by its residual, which
+// leaves 2^-90 before the last rounding: the IEEE root in each of 2e7 samples, its
+// reciprocal as near to the true one as the IEEE quotient (1.49 units in the last place).
 __device__ __forceinline__ double sqrt_full(double x) {
   const double y = __builtin_amdgcn_rsq(x);
   double g = x * y, h = 0.5 * y;
@@ -201,8 +210,7 @@ struct Force64 {
   __device__ __forceinline__ void pair(St& s, double pj, double rx, double ry, double rz, double d2) const {
     double inv;
     const double r = sqrt_full(d2, &inv);
-    const double t = sp.t(r), u = sp.u(r);
-    const double c = (s.pi + pj) * (__builtin_fma(u, u, -(t * t)) * inv);
+    const double c = (s.pi + pj) * sp.slope(r, inv);
     s.fx = __builtin_fma(c, rx, s.fx);
     s.fy = __builtin_fma(c, ry, s.fy);
     s.fz = __builtin_fma(c, rz, s.fz);
@@ -475,13 +483,12 @@ struct Force32 {
   };
   __device__ __forceinline__ void start(St& s, uint32_t p) const { s.pi = pterm[p]; }
   __device__ __forceinline__ float aux(uint32_t j) const { return pterm[j]; }
-  // (P_p/rho_p^2 + P_q/rho_q^2) dW/dq / (3 r); coincident particles have
-  // u^2 - t^2 = 0
+  // (P_p/rho_p^2 + P_q/rho_q^2) dW/dq / (3 r); coincident particles have no
+  // separation to multiply it with
   __device__ __forceinline__ void pair(St& s, float pj, double dx, double dy, double dz, double r2) const {
     const double inv = rsqrt_refined(r2);
     const double r = r2 * inv;
-    const double t = sp.t(r), u = sp.u(r);
-    const double c = (s.pi + double(pj)) * (__builtin_fma(u, u, -(t * t)) * inv);
+    const double c = (s.pi + double(pj)) * sp.slope(r, inv);
     s.fx = __builtin_fma(c, dx, s.fx);
     s.fy = __builtin_fma(c, dy, s.fy);
     s.fz = __builtin_fma(c, dz, s.fz);
