@@ -870,11 +870,13 @@ __global__ __launch_bounds__(256) void k_pairs_f32c(ClDev c, QGeom qg, const uns
 }
 
 // ------------------------------------------- smooth physics, Verlet rows
-// SPH passes over Verlet rows, 16 lanes per row.  A row holds the particle
-// itself (unless its position is not a number: then the row is empty, which
-// counts as W(0)), and its skin's entries vanish by themselves, so the whole
-// steps of 64 entries run without a decision, a mask or a branch; only the row's
-// last, partial step masks its lanes past the end (their square becomes kFar).
+// SPH passes over Verlet rows, 16 lanes per row.  A row holds the particle itself
+// (unless its position was not a number at the build: then the row is empty, which
+// counts as W(0)), and its skin's entries vanish by themselves.  In FP32C, whose
+// separations are integers, whole steps of 64 entries so run without a decision, a
+// mask or a branch; only the row's last, partial step masks its lanes past the end
+// (their square becomes kFar).  In FP64 a pair is decided: a value of the skin, or a
+// position since the build, may be infinite or no number, which zero does not undo.
 // The rows' entries of the next step are loaded before the current step's
 // gathers are used.
 // A pass was bound by VALU issue (62 and 45 instructions per entry in the force
@@ -883,6 +885,17 @@ __global__ __launch_bounds__(256) void k_pairs_f32c(ClDev c, QGeom qg, const uns
 // 4.4e9 entries (clustered, 4.2e6 particles): density 8.8 -> 7.2 ms, force 9.9 ->
 // 8.2 ms.
 constexpr double kFar = 1e200;
+
+// A pair of plain FP64 positions: taken within the cut-off (which a square that is no
+// number is not), coincident particles by the densities alone, as r = 1e-154.
+template <class Ph>
+__device__ __forceinline__ bool plain_pair(const Ph& ph, typename Ph::St& st, double aux, double rx, double ry,
+                                           double rz, double r2) {
+  if (!(r2 < ph.rc2)) return false;
+  if (Ph::kAux && r2 == 0.0) return false;
+  ph.pair(st, aux, rx, ry, rz, __builtin_fmax(r2, __DBL_MIN__));
+  return true;
+}
 
 // FP32C: 12-byte (q_x, q_y, q_z) or 16-byte (q, pterm) records; kWide: the
 // quantised stream itself, where there is no room for 12-byte records.
@@ -895,6 +908,8 @@ struct QuantRows {
   Ph ph;
   __device__ __forceinline__ Rec target(uint32_t p) const { return rec[p]; }
   __device__ __forceinline__ Rec gather(uint32_t j) const { return rec[j]; }
+  // whether a row's own entry was taken
+  __device__ __forceinline__ bool holds_itself(const Rec&) const { return true; }
   template <bool kMask>
   __device__ __forceinline__ void eval(St& st, const Rec& P, const Rec& Q, bool ok) const {
     const double dx = double(wrap_diff(Q.x, P.x));
@@ -928,13 +943,17 @@ struct PlainRows {
     if constexpr (Ph::kAux) r.a = ph.aux(j);
     return r;
   }
+  // not if the particle's position is infinite or not a number (inf - inf)
+  __device__ __forceinline__ bool holds_itself(const Rec& P) const {
+    const double rx = double(P.x) - double(P.x), ry = double(P.y) - double(P.y), rz = double(P.z) - double(P.z);
+    return rx + ry + rz == 0.0;
+  }
   template <bool kMask>
   __device__ __forceinline__ void eval(St& st, const Rec& P, const Rec& Q, bool ok) const {
     const double rx = double(P.x) - double(Q.x), ry = double(P.y) - double(Q.y), rz = double(P.z) - double(Q.z);
-    // coincident particles (and squares that underflow): any r far below h
-    double r2 = __builtin_fmax(__builtin_fma(rx, rx, __builtin_fma(ry, ry, rz * rz)), 1e-280);
-    if constexpr (kMask) r2 = ok ? r2 : kFar;
-    ph.pair(st, Q.a, rx, ry, rz, r2);
+    const double r2 = __builtin_fma(rx, rx, __builtin_fma(ry, ry, rz * rz));
+    if (kMask && !ok) return;
+    plain_pair(ph, st, Q.a, rx, ry, rz, r2);
   }
 };
 
@@ -990,7 +1009,7 @@ __global__ __launch_bounds__(256) void k_rows_smooth(ClDev c, const unsigned lon
     }
   }
   w.ph.reduce(st, kRowLanes);
-  if (valid && lane == 0) w.ph.finish(st, p, len == 0 ? 1.0 : 0.0);
+  if (valid && lane == 0) w.ph.finish(st, p, len == 0 || !w.holds_itself(P) ? 1.0 : 0.0);
 }
 
 // ---------------------------------------------- LDS-staged cell tiles
@@ -1284,15 +1303,12 @@ __global__ __launch_bounds__(kTileBlock, 4) void k_tile_f64(ClDev c, const T* __
             const Pos3<T> Q = buf[k];
             const uint32_t j = bufj[k];
             const double rx = xp - double(Q.x), ry = yp - double(Q.y), rz = zp - double(Q.z);
-            double d2 = dist2_unfused<double>(rx, ry, rz);
-            if (!(d2 < ph.rc2)) return;
+            const double d2 = dist2_unfused<double>(rx, ry, rz);
             if constexpr (Ph::kSmooth) {
-              d2 = __builtin_fmax(d2, 1e-280);  // coincident particles, and the particle itself
-              seen = true;
+              seen |= plain_pair(ph, st, ph.aux(j), rx, ry, rz, d2);  // (the particle itself too)
             } else {
-              if (j == p) return;
+              if (d2 < ph.rc2 && j != p) ph.pair(st, ph.aux(j), rx, ry, rz, d2);
             }
-            ph.pair(st, ph.aux(j), rx, ry, rz, d2);
           });
         });
     if constexpr (Ph::kSmooth) {
