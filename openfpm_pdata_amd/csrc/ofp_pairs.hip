@@ -471,6 +471,7 @@ struct Force32 {
   // the passes gather (q_x, q_y, q_z, pterm) as one 16-byte record per pair
   static constexpr bool kAuxInQuant = true;
   float rc2;
+  double cut2;  // (2h / q0)^2
   Spline sp;
   double fscale;       // 3 m / (pi h^4): of the separation x_q - x_p
   const float* pterm;  // P / rho^2
@@ -556,13 +557,21 @@ __device__ __forceinline__ QPair quant_geom(const QGeom& qg, int ix, int iy, int
 // an integer, or for non-cubic cells at least the squared axis ratio, to which
 // adding kTiny changes nothing), so 1/r stays finite.
 constexpr double kTiny = 1e-30;
+// careful (wave-uniform): the pairs may come with values that are infinite or no
+// number, so the particle itself and pairs beyond the cut-off, which the candidate
+// masks let through, are left out rather than multiplied by zero.  (Deciding every
+// pair: 16 us of the 400 of a force pass of 1.09e6 particles on a lattice, this 4.)
 template <class Ph, bool kCubic>
 __device__ __forceinline__ void smooth_pair(const Ph& ph, typename Ph::St& st, const QGeom& qg, float aux, int ix,
-                                            int iy, int iz) {
+                                            int iy, int iz, bool careful) {
   const double dx = double(ix);
   const double dy = kCubic ? double(iy) : double(iy) * qg.ryd;
   const double dz = kCubic ? double(iz) : double(iz) * qg.rzd;
-  ph.pair(st, aux, dx, dy, dz, __builtin_fma(dx, dx, __builtin_fma(dy, dy, __builtin_fma(dz, dz, kTiny))));
+  const double r2 = __builtin_fma(dx, dx, __builtin_fma(dy, dy, __builtin_fma(dz, dz, kTiny)));
+  if constexpr (Ph::kAuxInQuant) {
+    if (careful && ((ix | iy | iz) == 0 || r2 >= ph.cut2)) return;
+  }
+  ph.pair(st, aux, dx, dy, dz, r2);
 }
 
 template <class Ph>
@@ -1195,16 +1204,20 @@ __global__ __launch_bounds__(kTileBlock, 4) void k_tile_f32c(ClDev c, QGeom qg1,
     MatrixTest mt;
     const bool fast = mt.targets<true>(tx, ty, tz, rt2, rc2, pre2, ti.n > 32u);
     bool seen = false;
+    bool odd = false;  // a value that is infinite or no number
+    if constexpr (Ph::kAuxInQuant) odd = !__builtin_isfinite(ph.aux(p));
     for_each_chunk<kChunk>(
         c, G, lane,
         [&](uint32_t k, uint32_t j) {
           int4 Q = rec[j];
           if constexpr (!Ph::kAuxInQuant) Q.w = int(j);
+          if constexpr (Ph::kAuxInQuant) odd |= !__builtin_isfinite(__int_as_float(Q.w));
           buf[k] = Q;
         },
         [&](uint32_t m) {
           chunk_hits(mt, fast, buf, m, lane, valid, mk,
                      [&](const int4& Q, float* x, float* y, float* z) { sep(Q, ox, oy, oz, x, y, z); }, test);
+          const bool careful = Ph::kAuxInQuant && __ballot(odd) != 0ull;
           for_each_hit(mk, (m + 63u) / 64u, lane, [&](uint32_t k) {
             seen = true;
             const int4 Q = buf[k];
@@ -1212,7 +1225,7 @@ __global__ __launch_bounds__(kTileBlock, 4) void k_tile_f32c(ClDev c, QGeom qg1,
             if constexpr (Ph::kSmooth) {  // (the particle itself too)
               float a = 0.f;
               if constexpr (Ph::kAuxInQuant) a = __int_as_float(Q.w);
-              smooth_pair<Ph, kCubic>(ph, st, qg, a, ix, iy, iz);
+              smooth_pair<Ph, kCubic>(ph, st, qg, a, ix, iy, iz, careful);
             } else {
               const uint32_t j = uint32_t(Q.w);
               if (j != p) quant_pair<Ph, kCubic>(ph, st, qg, ph.aux(j), ix, iy, iz, p, j);
@@ -2302,6 +2315,7 @@ int ofp_sph_force(const ofp_cl* cl, const ofp_vl* vl, const void* pos, size_t st
   OFP_TRY(exact_cut(pos, stride, x.v.dtype == OFP_F64 ? 1 : 0, 2 * h, 4 * h * h, q0, quantum_ratio(qg.ryd, qg.rzd),
                     ph.rc2, &xc));
   ph.sp = spline(h, q0);
+  ph.cut2 = (2 * h / q0) * (2 * h / q0);
   ph.fscale = 3.0 * sd_m;
   ph.pterm = (const float*)pterm;
   ph.fx = (float*)fx;

@@ -1,4 +1,4 @@
-"""FP64 SPH passes with values and positions that are infinite or no number, over
+"""SPH passes with values and positions that are infinite or no number, over
 Verlet rows and over cells: what lies beyond 2h, or at no distance that can be said,
 adds nothing.  Reference: direct sums over the pairs within 2h, in FP64 (a sum of at
 most n terms of about ten roundings each: relative to the sum of their sizes, 1e-13)."""
@@ -110,3 +110,43 @@ def test_units_of_length(exponent, walk):
     n, h = 500, 0.1 * scale
     vd, cl, vl, _ = setup(n, torch.float64, h, walk, scale, seed=3)
     check_densities(vd, cl, vl, walk, h, n)
+
+
+@pytest.mark.parametrize("box", [(1.0, 1.0, 1.0), (1.0, 1.1, 1.3)])
+@pytest.mark.parametrize("value", [math.inf, math.nan])
+def test_values_fp32c_cells(value, box):
+    """FP32C over cells: pairs at the cut-off to within what the candidate masks decide,
+    a particle on its own and two in one place, all with the value.  (Over rows a
+    particle's value reaches those whose rows hold it.)"""
+    h, k = 0.05, 40
+    gen = torch.Generator(device="cuda").manual_seed(6)
+    g = torch.arange(4, device="cuda", dtype=torch.float64) * 0.25 + 0.125
+    c = torch.stack(torch.meshgrid(g, g, g, indexing="ij")).reshape(3, -1)[:, :k]
+    v = torch.randn((3, k), generator=gen, device="cuda", dtype=torch.float64)
+    v = v / v.norm(dim=0) * 2.0 * h * (1.0 + torch.logspace(-7, -2, k, device="cuda", dtype=torch.float64))
+    alone = torch.tensor([[0.9, 0.9, 0.9], [0.2, 0.8, 0.8], [0.2, 0.8, 0.8]], device="cuda", dtype=torch.float64)
+    x = torch.cat([c, c + v, c[:, :1] + 0.02, alone], dim=1).float()
+    n = x.shape[1]
+    vd = vdm.VectorDistGPU(n, (-0.2,) * 3, tuple(b + 0.2 for b in box), (0, 0, 0), 2 * h, dtype=torch.float32)
+    vd.pos[:, :n] = x
+    cl = vd.updateCellListGPU(vd.getCellListGPU(2 * h, vdm.CL_NON_SYMMETRIC | vdm.CL_GPU_REORDER_POSITION | vdm.CL_QUANT))
+    n2s = cl.arrays()["n2s"].long()[:n]
+    bad = torch.zeros(n, dtype=torch.bool, device="cuda")
+    bad[k:2 * k] = True
+    bad[-3:] = True
+    F = []
+    for other in (value, 0.7):
+        pt = torch.full((n,), 0.6, device="cuda")
+        pt[bad] = other
+        ps = torch.zeros(vd.cap, device="cuda")
+        ps[n2s] = pt
+        f = torch.full((3, vd.cap), 7.0, device="cuda")
+        L.call("ofp_sph_force", cl.h, None, vd.pos.data_ptr(), vd.cap, L.OFP_PREC_F32C, L.SPHParams(h, MASS, 1000.0, 10.0),
+               ps.data_ptr(), f[0].data_ptr(), f[1].data_ptr(), f[2].data_ptr(), vdm._stream())
+        F.append(f[:, n2s])
+    _, d2 = squares(x, n)
+    near = (d2 < 4 * h * h * (1 + 1e-6)) & (d2 > 0)
+    apart = ~(near & bad[None, :]).any(dim=1) & ~(bad & near.any(dim=1))
+    assert int(apart[:k].sum()) > 10 and apart[-3:].all()
+    assert torch.equal(F[0][:, apart], F[1][:, apart])
+    assert torch.isfinite(F[0][:, apart]).all()
