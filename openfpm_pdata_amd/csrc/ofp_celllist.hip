@@ -1501,9 +1501,14 @@ int ofp::cl_construct_many(ofp_cl* h, const void* pos, size_t stride, const uint
   return ofp::cl_construct_many_t<double>(h, pos, stride, n_cap, n_dev, gm, pos_sorted, sorted_stride, s);
 }
 
-int ofp::cl_far(const ofp_cl* h, size_t n, bool* far, hipStream_t s) {
+int ofp::cl_far(const ofp_cl* hc, size_t n, bool* far, hipStream_t s) {
   *far = false;
+  ofp_cl* h = const_cast<ofp_cl*>(hc);  // its scratch only
   if (!h->built || n < kFarFrom || n > kFarTo || h->payload.cap < kFarScratch * (n + 8)) return OFP_OK;
+  if (h->cursors.ensure(kFarRanges * 4) != OFP_OK) {
+    clear_error();
+    return OFP_OK;
+  }
   unsigned long long desc = 0;
   OFP_HIP(hipMemcpyAsync(&desc, h->packed.as<unsigned long long>() + h->n_cells, sizeof(desc), hipMemcpyDeviceToHost,
                          s));
@@ -1518,11 +1523,8 @@ int ofp::cl_permute(const ofp_cl* hc, const uint32_t* idx, size_t n, const Plane
   ofp_cl* h = const_cast<ofp_cl*>(hc);  // its scratch only
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   OFP_HIP(hipStreamIsCapturing(s, &cap));
-  if (cap != hipStreamCaptureStatusNone || n > kFarTo || h->payload.cap < kFarScratch * (n + 8)) return OFP_OK;
-  {
-    std::lock_guard<std::mutex> lock(h->far_lock);
-    OFP_TRY(h->cursors.ensure(kFarRanges * 4));
-  }
+  if (cap != hipStreamCaptureStatusNone || n > kFarTo || h->payload.cap < kFarScratch * (n + 8) || !h->cursors.p)
+    return OFP_OK;
   OFP_TRY(go_far(h, idx, uint32_t(n), pa, s));
   *done = true;
   return OFP_OK;

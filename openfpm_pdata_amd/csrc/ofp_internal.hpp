@@ -626,7 +626,7 @@ int cl_construct_many(ofp_cl* h, const void* pos, size_t stride, const uint32_t*
                       const uint32_t* n_dev, size_t gm, void* pos_sorted, size_t sorted_stride, hipStream_t s);
 int cl_sid_sorted(const ofp_cl* h, const uint32_t** sid_sorted);
 // Whether the last build found its n particles many and far from cell order, and the
-// list holds scratch for cl_permute (read from the device: synchronous).
+// list holds all scratch for cl_permute (read from the device: synchronous).
 int cl_far(const ofp_cl* h, size_t n, bool* far, hipStream_t s);
 // out[idx[j]] = in[j] (pa.src 0: in[j] = j), idx a permutation of n, by ranges of
 // destinations in the list's scratch; *done = false: not done (captured, no scratch).

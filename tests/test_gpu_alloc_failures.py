@@ -8,6 +8,7 @@ import pytest
 import torch
 
 from openfpm_pdata_amd import _lib as L
+from openfpm_pdata_amd import ensemble as E
 from openfpm_pdata_amd import vector_dist as vdm
 
 pytestmark = pytest.mark.gpu
@@ -81,3 +82,28 @@ def test_a_refused_call_leaves_no_error_behind():
     for a, b in zip((off, nbr), made[2].arrays()):
         assert torch.equal(a, b)
     torch.cuda.synchronize()
+
+
+def random_gas(n, seed=2):
+    m = round(n ** (1.0 / 3.0)) + 1
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    c = torch.randperm(m ** 3, generator=g, device="cuda")[:n]
+    x = (torch.stack([c % m, (c // m) % m, c // (m * m)]).double() + 0.5) / m
+    v = torch.randn((3, n), generator=g, device="cuda", dtype=torch.float64)
+    ens = E.Ensemble([E.System(n, 1.6 / m, 0.8 / m, 1.0, 1.0)], torch.float32, E.Options(skin=0.1, sub=1, lanes=1))
+    ens.set(x.float().contiguous(), v.float().contiguous())
+    return ens
+
+
+def test_far_run_without_its_cursors():
+    n = (1 << 22) + 77
+    out = []
+    for k in (0, 1):
+        ens = random_gas(n)
+        ens.force_pass(L.OFP_PREC_F64)
+        with refused(12288, 12288, k):
+            ens.run(L.OFP_PREC_F64, 1e-7, 3)
+        out.append(ens.get())
+        del ens
+    for a, b in zip(*out):
+        assert torch.equal(a, b)
