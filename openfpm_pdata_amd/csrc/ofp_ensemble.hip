@@ -1263,7 +1263,7 @@ int ofp_ens_run(ofp_ens* e, int precision, double dt, int n_steps, int use_graph
   // particles still in the caller's order: one reordering pays from the first
   // step that kicks inside the pair kernel (every step but a run's last), see
   // ens_relabel; a run of one step has none
-  if (!e->ordered && e->at_build && n_steps >= 2) OFP_TRY(ens_relabel(e, e->force_prec == precision, s));
+  if (!e->ordered && e->at_build && n_steps >= 2) OFP_TRY(ens_relabel(e, e->force_prec >= 0, s));
   if (e->force_prec != precision) {
     OFP_TRY(ens_forces(e, precision, nullptr, s));
     e->force_prec = precision;

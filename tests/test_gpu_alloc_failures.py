@@ -107,3 +107,16 @@ def test_far_run_without_its_cursors():
         del ens
     for a, b in zip(*out):
         assert torch.equal(a, b)
+
+
+def test_forces_after_a_refused_run():
+    """A run in another precision that fails before its steps leaves the forces of
+    the last pass, each with its particle."""
+    ens = random_gas(3000)
+    want = ens.forces(L.OFP_PREC_F64)
+    assert float(want.abs().max()) > 0
+    with refused(1, 4096, 1):  # the other precision's tables
+        with pytest.raises(L.OfpError):
+            ens.run(L.OFP_PREC_F32C, 1e-7, 3)
+    assert torch.equal(ens.get()[2], want)
+    ens.run(L.OFP_PREC_F32C, 1e-7, 3)
