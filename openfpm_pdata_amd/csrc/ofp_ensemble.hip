@@ -81,8 +81,8 @@ __global__ __launch_bounds__(256) void k_ens_map(uint32_t N, size_t cap, const u
 // stored particle k; written to the *2 arrays and copied back, for a run moves no
 // buffer unless it rebuilds).  inv[old storage index] = new one, for
 // k_ens_relabel_ghosts.
-// Called with positions that are those of the build (xb equals them).  It is paid
-// once, against nine gathered and six scattered values per particle in every later
+// xb, the positions of the build, move with their particles: the stored positions are
+// the caller's to change (ofp_ens_arrays_get).  It is paid once, against nine gathered and six scattered values per particle in every later
 // step: 40 steps of 2^23 particles given in random order 108.7 -> 28.7 ms.  Bound by
 // the gather from the caller's order; where that is far from cell order (cl_far) the
 // particles go by ranges of destinations instead, and back so in ofp_ens_get: both
@@ -94,16 +94,16 @@ __global__ __launch_bounds__(256) void k_ens_relabel(uint32_t N, size_t cap, con
                                                      const T* __restrict__ frc, const uint32_t* __restrict__ gid,
                                                      T* __restrict__ pos2, T* __restrict__ vel2,
                                                      T* __restrict__ frc2, uint32_t* __restrict__ gid2,
-                                                     T* __restrict__ xb, uint32_t* __restrict__ inv) {
+                                                     const T* __restrict__ xb, T* __restrict__ xb2,
+                                                     uint32_t* __restrict__ inv) {
   const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= N) return;
   const uint32_t f = dom[k];
   const uint32_t i = s2n[f];
 #pragma unroll
   for (int d = 0; d < 3; ++d) {
-    const T x = pos[d * cap + i];
-    pos2[d * cap + k] = x;
-    xb[d * cap + k] = x;
+    pos2[d * cap + k] = pos[d * cap + i];
+    xb2[d * cap + k] = xb[d * cap + i];
     vel2[d * cap + k] = vel[d * cap + i];
     if (frc) frc2[d * cap + k] = frc[d * cap + i];
   }
@@ -425,7 +425,8 @@ struct ofp_ens {
   // particle arrays (3 planes of cap unless noted)
   DevBuf pos, vel, frc, xb, pos2, vel2, frc2, gid, gid2, sid, spos, fsorted, esorted, energy_tmp, nn;
   // the second set of sorted positions and FP32C records a run's steps
-  // alternate with (set 0: spos and the cell list's records)
+  // alternate with (set 0: spos and the cell list's records); before a run's first
+  // step spos2 also serves the reordering (xb)
   DevBuf spos2, quant2;
   int rec_set = 0;  // the set holding the current sorted positions and records
   DevBuf gcnt, gstart, gtmp, opid, osid;
@@ -437,7 +438,7 @@ struct ofp_ens {
   // the caller's order is far from the stored one: gid's neighbours lie far apart
   bool far = false;
   bool ordered = false;   // the stored particles are in cell order (a build's rows)
-  bool at_build = false;  // the stored positions are those of the last build
+  bool at_build = false;  // no drift since the last build
   int force_prec = -1;  // precision of the forces in frc (-1: none)
   uint64_t n_ghost = 0, n_entries = 0, rebuilds = 0, steps = 0, recaptures = 0;
   // graphs: [step variant][precision] step (variants: see step_variant),
@@ -814,19 +815,17 @@ static int ens_relabel_t(ofp_ens* e, bool keep_frc, hipStream_t s) {
     for (size_t d = 0; d < 3; ++d) {
       add_plane(&pa, e->pos.as<T>() + d * cap, e->pos2.as<T>() + d * cap);
       add_plane(&pa, e->vel.as<T>() + d * cap, e->vel2.as<T>() + d * cap);
+      add_plane(&pa, e->xb.as<T>() + d * cap, e->spos2.as<T>() + d * cap);
       if (keep_frc) add_plane(&pa, e->frc.as<T>() + d * cap, e->frc2.as<T>() + d * cap);
     }
     add_plane(&pa, e->gid.as<uint32_t>(), e->gid2.as<uint32_t>());
     OFP_TRY(cl_permute(e->cl, inv, N, pa, &done, s));
     OFP_CHECK(done, OFP_E_STATE, "ens_relabel: no scratch");
-    for (size_t d = 0; d < 3; ++d)
-      OFP_HIP(hipMemcpyAsync(e->xb.as<T>() + d * cap, e->pos2.as<T>() + d * cap, N * sizeof(T),
-                             hipMemcpyDeviceToDevice, s));
   } else {
     k_ens_relabel<T><<<grid_for(N, 256), 256, 0, s>>>(
         N, cap, v.dom_sort_ids, s2n, n2s, e->pos.as<T>(), e->vel.as<T>(), keep_frc ? e->frc.as<T>() : nullptr,
         e->gid.as<uint32_t>(), e->pos2.as<T>(), e->vel2.as<T>(), keep_frc ? e->frc2.as<T>() : nullptr,
-        e->gid2.as<uint32_t>(), e->xb.as<T>(), inv);
+        e->gid2.as<uint32_t>(), e->xb.as<T>(), e->spos2.as<T>(), inv);
     OFP_LAUNCHED();
   }
   if (e->gcap > 0) {
@@ -836,9 +835,10 @@ static int ens_relabel_t(ofp_ens* e, bool keep_frc, hipStream_t s) {
   }
   // the stored particles keep their buffers (pointers taken after ofp_ens_set)
   if (keep_frc)
-    OFP_TRY(ens_copy_back<T>(e, {{&e->pos, &e->pos2}, {&e->vel, &e->vel2}, {&e->frc, &e->frc2}}, &e->gid, &e->gid2, s));
+    OFP_TRY(ens_copy_back<T>(
+        e, {{&e->pos, &e->pos2}, {&e->vel, &e->vel2}, {&e->xb, &e->spos2}, {&e->frc, &e->frc2}}, &e->gid, &e->gid2, s));
   else
-    OFP_TRY(ens_copy_back<T>(e, {{&e->pos, &e->pos2}, {&e->vel, &e->vel2}}, &e->gid, &e->gid2, s));
+    OFP_TRY(ens_copy_back<T>(e, {{&e->pos, &e->pos2}, {&e->vel, &e->vel2}, {&e->xb, &e->spos2}}, &e->gid, &e->gid2, s));
   e->ordered = true;
   return OFP_OK;
 }

@@ -72,3 +72,28 @@ def test_arrays_of_a_run_without_rebuild(n, with_forces):
     for ptr, want in zip((a.pos, a.vel, a.force), ens.get()):
         got = vdm.device_view(ptr, 3 * int(a.cap), torch.float32).view(3, -1)[:, :n]
         assert torch.equal(got, want[:, gid])
+
+
+@pytest.mark.parametrize("n", [2000, (1 << 22) + 3])
+def test_positions_changed_by_their_pointer(n):
+    """Particles that the caller moves after a build, by more than the skin allows: the
+    next run rebuilds, in three steps at once as in three runs of one step."""
+    m = round(n ** (1.0 / 3.0)) + 1
+    systems = [E.System(n, 1.5 / m, 0.5 / m, 1.0, 1.0)]
+    x, v = gas(systems, m, 4)
+    out = []
+    for split in (False, True):
+        ens = E.Ensemble(systems, torch.float32, E.Options(skin=0.1, sub=1, lanes=1))
+        ens.set(x, v)
+        ens.rebuild()
+        a = ens.arrays()
+        pos = vdm.device_view(a.pos, 3 * int(a.cap), torch.float32).view(3, -1)
+        pos[0, :n:5] += 0.6 / m
+        before = ens.status()["rebuilds"]
+        for _ in range(3 if split else 1):
+            ens.run(L.OFP_PREC_F64, 1e-7 / m, 1 if split else 3)
+        assert ens.status()["rebuilds"] == before + 1
+        out.append(ens.get())
+        del ens
+    for a, b in zip(*out):
+        assert torch.equal(a, b)
