@@ -16,7 +16,8 @@ struct ofp_ghost {
   ofp::GhostBoxes<float> bf;
   ofp::GhostBoxes<double> bd;
   ofp::DevBuf cnt, starts, tmp, opid, osid;
-  ofp::DevBuf boxes;  // bf or bd on the device (uploaded by the first label)
+  ofp::DevBuf boxes;  // bf or bd on the device, uploaded by the first label
+  bool boxes_there = false;  // (an upload that fails is made again)
   size_t n_dom = 0;    // ghost marker at the last label
   size_t n_ghost = 0;  // ghosts of the last label
   bool labelled = false;
@@ -179,10 +180,14 @@ __global__ __launch_bounds__(256) void k_apply_bc(T* __restrict__ pos, size_t st
 template <class T>
 static int ghost_label(ofp_ghost* h, const GhostBoxes<T>& B, const void* pos, size_t stride,
                        size_t n_dom, size_t* n_ghost, hipStream_t s) {
-  if (!h->boxes.p) {
+  if (!h->boxes_there) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    OFP_HIP(hipStreamIsCapturing(s, &cap));
+    OFP_CHECK(cap == hipStreamCaptureStatusNone, OFP_E_HIP, "ofp_ghost_label: synchronous, not for a captured stream");
     OFP_TRY(h->boxes.ensure(sizeof(B)));
     OFP_HIP(hipMemcpyAsync(h->boxes.p, &B, sizeof(B), hipMemcpyHostToDevice, s));
     OFP_HIP(hipStreamSynchronize(s));  // any stream may use them from here on
+    h->boxes_there = true;
   }
   OFP_TRY(h->cnt.ensure((n_dom + 1) * sizeof(uint32_t)));
   OFP_TRY(h->starts.ensure((n_dom + 1) * sizeof(uint32_t)));
