@@ -864,12 +864,17 @@ static int ens_tables_lj(ofp_ens* e, int prec) {
   const size_t cap = e->cap;
   uint32_t* nn = e->nn.as<uint32_t>();
   const int f64 = e->dtype == OFP_F64 ? 1 : 0;
-  if (prec == OFP_PREC_F64)
-    return lj_tables_many(prec, e->S, prm.data(), e->csp.data(), fs, fs + cap, fs + 2 * cap, e->esorted.p, nn,
-                          e->spos.p, cap, f64, &e->ljtab[prec], &e->ljq[prec], &e->lj_cubic[prec]);
   float* f32 = e->fsorted.as<float>();
-  return lj_tables_many(prec, e->S, prm.data(), e->csp.data(), f32, f32 + cap, f32 + 2 * cap, e->esorted.p, nn,
-                        e->spos.p, cap, f64, &e->ljtab[prec], &e->ljq[prec], &e->lj_cubic[prec]);
+  const bool d = prec == OFP_PREC_F64;
+  const int rc = lj_tables_many(prec, e->S, prm.data(), e->csp.data(), d ? (void*)fs : f32,
+                                d ? (void*)(fs + cap) : f32 + cap, d ? (void*)(fs + 2 * cap) : f32 + 2 * cap,
+                                e->esorted.p, nn, e->spos.p, cap, f64, &e->ljtab[prec], &e->ljq[prec],
+                                &e->lj_cubic[prec]);
+  if (rc != OFP_OK) {  // the next call makes them
+    e->ljtab[prec].release();
+    e->ljq[prec].release();
+  }
+  return rc;
 }
 
 // The sorted positions and FP32C records of set k (0: spos and the cell

@@ -120,3 +120,23 @@ def test_forces_after_a_refused_run():
             ens.run(L.OFP_PREC_F32C, 1e-7, 3)
     assert torch.equal(ens.get()[2], want)
     ens.run(L.OFP_PREC_F32C, 1e-7, 3)
+
+
+@pytest.mark.parametrize("size", [1, 24])  # any first table, and the second one (24 bytes a system)
+def test_tables_of_many_systems(size):
+    S = 200
+    gen = torch.Generator(device="cuda").manual_seed(9)
+    x = torch.rand((3, 20 * S), generator=gen, device="cuda")
+    systems = [E.System(20, 0.2, 0.02, 1.0, 1.0) for _ in range(S)]
+    out = []
+    for k in (0, 1):
+        ens = E.Ensemble(systems, torch.float32, E.Options(skin=0.1, sub=1))
+        ens.set(x)
+        ens.rebuild()
+        if k:
+            lo, hi = (24 * S, 24 * S) if size == 24 else (24 * S + 1, 400 * S)
+            with refused(lo, hi, 1):
+                with pytest.raises(L.OfpError):
+                    ens.force_pass(L.OFP_PREC_F32C)
+        out.append(ens.forces(L.OFP_PREC_F32C))
+    assert torch.equal(*out)
