@@ -1084,7 +1084,7 @@ static int cl_build_t(ofp_cl* h, const Key& key, const EmitArgs<T>& A0, size_t n
   const uint32_t n_tiles = uint32_t((n_cap + kRxTile - 1) / kRxTile);
   const size_t hist_n = size_t(kRxBins) * (n_tiles ? n_tiles : 1);
   const bool first = g1 != nullptr && n_dev == nullptr;
-  if (first) {  // a build of a count on the host is none for a graph: the count and the buffers are this call's
+  if (first && n_tiles > 0) {  // a build of a count on the host is none for a graph: the count and the buffers are this call's
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     OFP_HIP(hipStreamIsCapturing(s, &cap));
     if (cap != hipStreamCaptureStatusNone) OFP_HIP(hipErrorStreamCaptureUnsupported);
