@@ -73,7 +73,6 @@ struct ofp_cl {
   unsigned long long* desc = nullptr;
   hipEvent_t checked = nullptr;
   ofp::DevBuf items;
-  uint64_t heads_at = 0;  // word of packed: the consumers' queue heads (kQueueWords), then the item count
   ofp::DevBuf aux;            // pair kernels' per-particle record stream (cell tiles)
   // sparse view (ofp_cl_build_sparse): non-empty cells only
   ofp::DevBuf nz_flag, nz_key, nz_start, nz_nn, nz_inv;
@@ -1091,17 +1090,17 @@ static int cl_build_t(ofp_cl* h, const Key& key, const EmitArgs<T>& A0, size_t n
   }
   int widths[4];
   const int passes = radix_plan(C, widths);
-  // the descents counted, the chunks' sums, the items' queue heads and their count
-  // lie behind the cells' counts, cleared with them
+  // behind the cells' counts, and cleared with them: the descents counted, the items'
+  // queue heads and their count (captured pair passes name these: their place must not
+  // depend on the particles, nor the buffer grow with them), the chunks' sums
   const int direct = n_tiles <= kRxChunked ? 1 : 0;
   const bool chunked = direct && n_tiles > kRxDirect;
   // the [tile][digit] table in at most kColChunks chunks of ch tiles
   const uint32_t ch = std::max((n_tiles + kColChunks - 1) / kColChunks, kColBatch);
   const uint32_t n_chunks = (n_tiles + ch - 1) / ch;
-  const uint64_t heads_at = C + 1 + (chunked ? uint64_t(passes) * n_chunks * (kRxBins / 2) : 0);
-  const uint64_t n_clear = heads_at + kQueueWords / 2 + 1;
-  OFP_TRY(h->packed.ensure(n_clear * 8));
-  h->heads_at = heads_at;
+  const uint64_t sums_at = C + 1 + kQueueWords / 2 + 1;
+  const uint64_t n_clear = sums_at + (chunked ? uint64_t(passes) * n_chunks * (kRxBins / 2) : 0);
+  OFP_TRY(h->packed.ensure((sums_at + uint64_t(passes) * kColChunks * (kRxBins / 2)) * 8));
   OFP_TRY(h->scan64.ensure((C + 1) * 8));
   OFP_TRY(h->scantmp.ensure(scan_tmp_bytes(C)));
   if (!direct) OFP_TRY(h->colpart.ensure(size_t(kColChunks) * kRxBins * 4));
@@ -1200,7 +1199,7 @@ static int cl_build_t(ofp_cl* h, const Key& key, const EmitArgs<T>& A0, size_t n
       pout = last ? A0.pos_sorted : pbuf[p % 2];
       so = last ? A0.sorted_stride : n_cap;
     }
-    uint32_t* part = chunked ? reinterpret_cast<uint32_t*>(packed + C + 1) + size_t(p) * n_chunks * kRxBins
+    uint32_t* part = chunked ? reinterpret_cast<uint32_t*>(packed + sums_at) + size_t(p) * n_chunks * kRxBins
                              : h->colpart.as<uint32_t>();
     k_rx_hist<Key, kIters><<<n_tiles, kRxBlock, 0, s>>>(
         key, p ? kin : nullptr, p ? nullptr : kin, n_host, n_dev, shift, bits, n_tiles, hist,
@@ -1643,7 +1642,8 @@ int ofp_cl_items_(const ofp_cl* hc, const TargetItem** items, const uint32_t** n
                   uint32_t** counter, size_t* cap, hipStream_t s) {
   ofp_cl* h = const_cast<ofp_cl*>(hc);
   OFP_CHECK(h && h->built, OFP_E_STATE, "cell list not constructed");
-  uint32_t* heads = reinterpret_cast<uint32_t*>(h->packed.as<unsigned long long>() + h->heads_at);
+  // the consumers' queue heads (kQueueWords), then the item count: see cl_build_t
+  uint32_t* heads = reinterpret_cast<uint32_t*>(h->packed.as<unsigned long long>() + h->n_cells + 1);
   if (!h->items_valid) {
     size_t need = size_t(h->gm) + 1;
     OFP_TRY(h->items.ensure(need * sizeof(TargetItem)));
