@@ -185,6 +185,7 @@ SIGNATURES = {
     "ofp_ens_status": (_i, [_vp, C.POINTER(EnsState), _vp]),
     # test hook exported by the library but not declared in the public header
     "ofp_vl_test_rows_": (_i, [_vp, C.POINTER(_i)]),
+    "ofp_test_queue_grid_": (_i, [C.c_uint, C.c_uint, C.POINTER(C.c_uint), C.POINTER(C.c_uint)]),
     "ofp_test_fail_alloc_": (_i, [_sz, _sz, _i]),
     "ofp_ens_test_masks_": (_i, [_vp, _sz, _i, C.POINTER(_sz)]),
 }

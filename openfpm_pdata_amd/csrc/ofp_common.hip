@@ -478,6 +478,13 @@ int ofp_test_fail_alloc_(size_t lo, size_t hi, int count) {
   return OFP_OK;
 }
 
+// Test hook (not in the public header): queue_grid.
+int ofp_test_queue_grid_(unsigned blocks, unsigned waves_per_block, unsigned* grid, unsigned* queues) {
+  *grid = ofp::queue_grid(blocks, waves_per_block);
+  *queues = ofp::kQueues;
+  return OFP_OK;
+}
+
 int ofp_device_info(int* device, int* n_cu, char* arch, size_t arch_len) {
   int dev = 0;
   OFP_HIP(hipGetDevice(&dev));

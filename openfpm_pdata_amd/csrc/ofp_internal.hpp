@@ -400,6 +400,12 @@ __device__ __forceinline__ uint32_t xcd_tile(uint32_t b, uint32_t n_blocks) {
 constexpr uint32_t kQueues = 64;
 constexpr uint32_t kQueueStride = 32;  // u32 words between heads
 constexpr uint32_t kQueueWords = kQueues * kQueueStride;
+// A queue that no wave draws from keeps its units: blocks of such a launch, no fewer
+// than bring a wave to every queue (few CUs, as in a partition of the card).
+inline unsigned queue_grid(unsigned blocks, unsigned waves_per_block) {
+  const unsigned least = (kQueues + waves_per_block - 1) / waves_per_block;
+  return blocks < least ? least : blocks;
+}
 __device__ __forceinline__ uint32_t next_unit(uint32_t* __restrict__ heads) {
   const uint32_t q =
       __builtin_amdgcn_readfirstlane((blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave) % kQueues);

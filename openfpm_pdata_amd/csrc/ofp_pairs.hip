@@ -1732,7 +1732,7 @@ static unsigned tile_grid() {
   if (!g) {
     int dev = 0, ncu = 256;
     if (ofp_device_info(&dev, &ncu, nullptr, 0) != OFP_OK || ncu <= 0) ncu = 256;
-    g = unsigned(ncu) * 8u;
+    g = queue_grid(unsigned(ncu) * 8u, kTileWaves);
   }
   return g;
 }

@@ -845,7 +845,7 @@ static int vl_build_t(ofp_vl* h, const ofp_cl* cl, const void* pos_v, size_t str
   uint32_t* counter;  // the cell tiles' queue heads; a list's passes have their own
   size_t cap;
   OFP_TRY(ofp_cl_items_(cl, &items, &n_items, &counter, &cap, s));
-  if (grid == 0) grid = persistent_grid();
+  grid = queue_grid(grid ? grid : persistent_grid(), kVlWaves);
   const VlSplit sp = vl_split(n);
   const bool add = sp.parts > 1;  // the parts add their hits to the counts
   k_vl_pack<T><<<grid_for(std::max<size_t>(v.n_part, kCtl), 256), 256, 0, s>>>(
