@@ -316,8 +316,6 @@ struct ExactCut {
 template <bool kU>
 struct LJ32T {
   static constexpr bool kSmooth = false;
-  static constexpr bool kExact = true;  // the (sigma/r)^12 chain needs the exact square
-  static constexpr bool kRefine = true;
   static constexpr bool kAuxInQuant = false;
   float rc2;      // (r_c / q0)^2
   double sig2;    // (sigma / q0)^2
@@ -514,42 +512,30 @@ struct QGeom {
 
 // A pair gets x_p - x_q in FP64 (integer components; for non-cubic cells times
 // the FP64 axis ratio, rounded once) and its square in FP64 (products summed
-// with FMAs); the cut-off test compares the square rounded to FP32 (physics
-// without kExact: the FP32 square of the rounded components), and a square in
-// the ExactCut band is decided on the stored positions as the FP64 form decides.
+// with FMAs; the (sigma/r)^12 chain needs the exact square); the cut-off test compares
+// the square rounded to FP32, and a square in the ExactCut band is decided on the
+// stored positions as the FP64 form decides.
 // The cell walk first drops candidates whose FP32 square exceeds the cut-off by
 // more than any rounding and the band (pre_cut), then decides like the Verlet
 // rows.
 // kCubic: cubic cells (q_y = q_z = q_0), no component scaling.
-// Physics with close-pair refinement (LJ) replaces the quantised separation of
-// a hit closer than close2 by the exact one from the stored positions.
+// The quantised separation of a hit closer than close2 is replaced by the exact one
+// from the stored positions.
 constexpr float kPreCut = 1.0f + 1.0f / 65536.0f;
 
-template <class Ph, bool kCubic>
+template <bool kCubic>
 __device__ __forceinline__ QPair quant_geom(const QGeom& qg, int ix, int iy, int iz, float* d2f) {
   QPair p;
-  if constexpr (Ph::kExact) {
-    const double dx = double(ix);
-    const double dy = kCubic ? double(iy) : double(iy) * qg.ryd;
-    const double dz = kCubic ? double(iz) : double(iz) * qg.rzd;
-    const double r2 = __builtin_fma(dx, dx, __builtin_fma(dy, dy, dz * dz));
-    p.rx = -dx;
-    p.ry = -dy;
-    p.rz = -dz;
-    p.r2 = r2;
-    p.d2 = float(r2);
-    *d2f = p.d2;
-  } else {
-    const float fx = float(ix);
-    const float fy = kCubic ? float(iy) : float(iy) * qg.ry;
-    const float fz = kCubic ? float(iz) : float(iz) * qg.rz;
-    p.rx = -double(fx);
-    p.ry = -double(fy);
-    p.rz = -double(fz);
-    p.d2 = __builtin_fmaf(fx, fx, __builtin_fmaf(fy, fy, fz * fz));
-    p.r2 = p.d2;
-    *d2f = p.d2;
-  }
+  const double dx = double(ix);
+  const double dy = kCubic ? double(iy) : double(iy) * qg.ryd;
+  const double dz = kCubic ? double(iz) : double(iz) * qg.rzd;
+  const double r2 = __builtin_fma(dx, dx, __builtin_fma(dy, dy, dz * dz));
+  p.rx = -dx;
+  p.ry = -dy;
+  p.rz = -dz;
+  p.r2 = r2;
+  p.d2 = float(r2);
+  *d2f = p.d2;
   return p;
 }
 // kSmooth physics: x_q - x_p and its square in FP64 from the integer separation.
@@ -576,9 +562,7 @@ __device__ __forceinline__ void smooth_pair(const Ph& ph, typename Ph::St& st, c
 
 template <class Ph>
 __device__ __forceinline__ void refine_close(const Ph& ph, QPair& p, bool hit, uint32_t ip, uint32_t jq) {
-  if constexpr (Ph::kRefine) {
-    if (hit && p.d2 < ph.close2) ph.refine(p, ip, jq);  // rare, divergent
-  }
+  if (hit && p.d2 < ph.close2) ph.refine(p, ip, jq);  // rare, divergent
 }
 
 template <class Ph, bool kCubic>
@@ -590,7 +574,7 @@ __device__ __forceinline__ void quant_pair(const Ph& ph, typename Ph::St& st, co
   const float pre = __builtin_fmaf(fx, fx, __builtin_fmaf(fy, fy, fz * fz));
   if (pre < ph.rc2 * kPreCut) {
     float d2;
-    QPair p = quant_geom<Ph, kCubic>(qg, ix, iy, iz, &d2);
+    QPair p = quant_geom<kCubic>(qg, ix, iy, iz, &d2);
     bool hit = d2 < ph.rc2;
     if (ph.xc.in_band(d2)) hit = ph.xc.hit(ip, jq);  // rare, divergent
     if (hit) {
@@ -608,7 +592,7 @@ __device__ __forceinline__ void quant_pair_masked(const Ph& ph, typename Ph::St&
                                                   int ix, int iy, int iz, bool not_self, uint32_t ip,
                                                   uint32_t jq) {
   float d2;
-  QPair p = quant_geom<Ph, kCubic>(qg, ix, iy, iz, &d2);
+  QPair p = quant_geom<kCubic>(qg, ix, iy, iz, &d2);
   bool hit = not_self && d2 < ph.rc2;
   if (not_self && ph.xc.in_band(d2)) hit = ph.xc.hit(ip, jq);  // rare, divergent
   refine_close(ph, p, hit, ip, jq);
@@ -631,13 +615,12 @@ __device__ __forceinline__ void quant_group_masked(const Ph& ph, typename Ph::St
                                                    const float (&aux)[4], const int4 (&Q)[4], const int4& P,
                                                    const uint32_t (&j)[4], const bool (&not_self)[4],
                                                    const T (&pp)[3], const T* __restrict__ sref, size_t sstride) {
-  static_assert(Ph::kRefine, "grouped evaluation is for physics with close-pair refinement");
   bool hit[4], band[4], need[4];
 #pragma unroll
   for (int u = 0; u < 4; ++u) {
     float d2;
     const QPair r =
-        quant_geom<Ph, kCubic>(qg, wrap_diff(Q[u].x, P.x), wrap_diff(Q[u].y, P.y), wrap_diff(Q[u].z, P.z), &d2);
+        quant_geom<kCubic>(qg, wrap_diff(Q[u].x, P.x), wrap_diff(Q[u].y, P.y), wrap_diff(Q[u].z, P.z), &d2);
     hit[u] = not_self[u] && d2 < ph.rc2;
     band[u] = not_self[u] && ph.xc.in_band(d2);
     // close pairs are refined; a band pair's final decision may still be a hit
@@ -661,7 +644,7 @@ __device__ __forceinline__ void quant_group_masked(const Ph& ph, typename Ph::St
     // than kept from the first pass
     asm volatile("" : "+v"(ix), "+v"(iy), "+v"(iz));
     float d2;
-    QPair r = quant_geom<Ph, kCubic>(qg, ix, iy, iz, &d2);
+    QPair r = quant_geom<kCubic>(qg, ix, iy, iz, &d2);
     if (hit[u] && r.d2 < ph.close2) ph.refine_from(r, pp, xq[u]);
     ph.pair_masked(st, aux[u], r, hit[u]);
     __builtin_amdgcn_sched_barrier(0);
@@ -699,13 +682,12 @@ __device__ __forceinline__ void quant_group_defer(const Ph& ph, typename Ph::St&
                                                   const uint32_t (&j)[4], const bool (&not_self)[4],
                                                   const T (&pp)[3], const T* __restrict__ sref, size_t sstride,
                                                   Deferred& df) {
-  static_assert(Ph::kRefine, "deferred refinement is for physics with close-pair refinement");
   bool hit[4], need[4], close[4];
 #pragma unroll
   for (int u = 0; u < 4; ++u) {
     float d2;
     const QPair r =
-        quant_geom<Ph, kCubic>(qg, wrap_diff(Q[u].x, P.x), wrap_diff(Q[u].y, P.y), wrap_diff(Q[u].z, P.z), &d2);
+        quant_geom<kCubic>(qg, wrap_diff(Q[u].x, P.x), wrap_diff(Q[u].y, P.y), wrap_diff(Q[u].z, P.z), &d2);
     hit[u] = not_self[u] && d2 < ph.rc2;
     const bool band = not_self[u] && ph.xc.in_band(d2);
     close[u] = hit[u] && !band && r.d2 < ph.close2;
@@ -730,7 +712,7 @@ __device__ __forceinline__ void quant_group_defer(const Ph& ph, typename Ph::St&
     int ix = wrap_diff(Q[u].x, P.x), iy = wrap_diff(Q[u].y, P.y), iz = wrap_diff(Q[u].z, P.z);
     asm volatile("" : "+v"(ix), "+v"(iy), "+v"(iz));  // recomputed, not kept from the first pass
     float d2;
-    QPair r = quant_geom<Ph, kCubic>(qg, ix, iy, iz, &d2);
+    QPair r = quant_geom<kCubic>(qg, ix, iy, iz, &d2);
     if (close[u]) ph.refine_from(r, pp, xq[u]);
     ph.pair_masked(st, aux[u], r, hit[u]);
     __builtin_amdgcn_sched_barrier(0);
@@ -854,13 +836,8 @@ __global__ __launch_bounds__(256) void k_pairs_f32c(ClDev c, QGeom qg, const uns
       }
 #pragma unroll
       for (int u = 0; u < kUnroll; ++u) {
-        if constexpr (Ph::kAuxInQuant) {
-          Q[u] = ph.qaux[j[u]];
-          a[u] = __int_as_float(Q[u].w);
-        } else {
-          Q[u] = c.quant[j[u]];
-          a[u] = ph.aux(j[u]);
-        }
+        Q[u] = c.quant[j[u]];
+        a[u] = ph.aux(j[u]);
       }
       load_j(e + kUnroll * kRowLanes);
       // one entry's evaluation at a time (its FP64 temporaries are what sets
