@@ -71,6 +71,8 @@ def parse():
     ap.add_argument("--dyn-n", type=int, default=1 << 26, help="particles of the dynamic run")
     ap.add_argument("--ens-boxes", type=int, default=256)
     ap.add_argument("--tune-budget", type=float, default=40.0, help="autotuner time budget (s)")
+    ap.add_argument("--candidates", default="", metavar="DIR",
+                    help="write every candidate the autotuner measured to DIR/candidates_<run>.json")
     ap.add_argument("--verbose", action="store_true")
     ap.add_argument("--pmc-summary", nargs=3, metavar=("FETCH_DIR", "WRITE_DIR", "OUT_JSON"), default=None,
                     help="no benchmark: summarise two rocprofv3 --pmc runs of this benchmark (FETCH_SIZE, then "
@@ -604,6 +606,19 @@ def _mean_std(xs):
     return float(a.mean()), float(a.std(ddof=1)) if len(a) > 1 else 0.0
 
 
+def candidates(args, run, log):
+    """The autotuner's log for the result line, which has to stay short enough to be
+    kept whole: the fastest candidates, and how many there were."""
+    if not isinstance(log, list):
+        return {"candidates": log}
+    if args.candidates:
+        os.makedirs(args.candidates, exist_ok=True)
+        with open(os.path.join(args.candidates, f"candidates_{run}.json"), "w") as f:
+            json.dump(log, f, indent=1)
+    best = sorted((c for c in log if c.get("step_ms") is not None), key=lambda c: c["step_ms"])
+    return {"candidates_measured": len(log), "best_candidates": best[:4]}
+
+
 def dynamic_headline(args):
     """The dynamic run (see the module docstring).  Returns (fields of the
     headline line, context kept for the cell-list section and the CPU
@@ -739,7 +754,7 @@ def dynamic_headline(args):
                                        "drift_over_kinetic": abs(e1 - e0) / ek0},
                     "init": {"seconds": t_init, "redraw_rounds": rounds, "pairs_below_min": n_close,
                              "min_distance": wl.params["d_min"]},
-                    "autotune": {"seconds": t_tune, "candidates": log}},
+                    "autotune": {"seconds": t_tune, **candidates(args, "dynamic_run", log)}},
         "fp64": {"value": pairs * K / (ms64 * 1e-3), "ms_per_step": ms64 / K, "rebuilds_in_timed_region": reb64 + 1,
                  "lj_kernel_ms": t_lj64, "speedup_fp32_storage_over_fp64": ms64 / ms,
                  "lj_kernel_speedup": t_lj64 / t_lj},
@@ -835,7 +850,7 @@ def ensemble_section(args):
     out = {"workload": "ensemble of periodic LJ boxes", "n_boxes": len(wls), "n_particles": n_tot,
            "n_min": int(min(s.n for s in systems)), "n_max": int(max(s.n for s in systems)),
            "autotune": {"chosen": dict(vars(opts)), "objective": "force pass + rebuild / steps between rebuilds "
-                        f"(v_max {vmax}, dt {dt})", "candidates": log}}
+                        f"(v_max {vmax}, dt {dt})", **candidates(args, "ensemble", log)}}
     ens = E.Ensemble(systems, torch.float32, opts)
     ens.set(pos)
     ens.rebuild()
