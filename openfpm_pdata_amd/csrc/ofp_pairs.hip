@@ -867,9 +867,9 @@ __global__ __launch_bounds__(256) void k_pairs_f32c(ClDev c, QGeom qg, const uns
 // gathers are used.
 // A pass was bound by VALU issue (62 and 45 instructions per entry in the force
 // and density passes); without the decisions and with the clamped spline it is
-// 32 and 26, and the gathers through the L1 (busy 85 % of the pass) come next.
-// 4.4e9 entries (clustered, 4.2e6 particles): density 8.8 -> 7.2 ms, force 9.9 ->
-// 8.2 ms.
+// 33 and 26, and the texture path is what it waits for (data unit busy 97 %, address
+// unit 93 %, VALU 62-69 %).  4.4e9 entries (clustered, 4.2e6 particles): density
+// 8.8 -> 7.1 ms, force 9.9 -> 8.1 ms.
 constexpr double kFar = 1e200;
 
 // A pair of plain FP64 positions: taken within the cut-off (which a square that is no
@@ -1019,7 +1019,7 @@ __global__ __launch_bounds__(256) void k_rows_smooth(ClDev c, const unsigned lon
 // target's place in its cell; larger rounds even that out).  Tests in the vector
 // ALU, eleven instructions per candidate and wave, took half of the passes.
 // 1,092,727 particles on a lattice (FP32C, density and force): 632 and 682 -> 372
-// and 391 us (128 candidates a round 445 and 453, 320: 380 and 402); 65,536 of a
+// and 400 us (128 candidates a round 445 and 453); 65,536 of a
 // gas, FP64 LJ: 112 -> 55 us.
 //
 // FP32C separations: the union spans at most kItemMaxCells - 1 + B cells in x

@@ -370,9 +370,9 @@ __global__ __launch_bounds__(kVlBlock, 4) void k_vl_count(ClDev c, const T* __re
 // takes of the CU's address unit, for 8 entries on average.
 // e_total / e_cap: the list's entry count (device) and the capacity of nbr; a list
 // that does not fit, or whose masks did not, is not written.
-// 4.2e6 clustered particles (4.4e9 entries, 17.7 GB): 8.4 -> 6.5 ms (2.7 TB/s
-// written; instructions of the expansion, 40 % of whose lanes have bits left on
-// average, and their LDS conflicts); 3e5: 0.58 -> 0.35 ms; 4e5 in FP64 0.83 -> 0.55 ms.
+// 4.2e6 clustered particles (4.4e9 entries, 17.7 GB): 8.4 -> 6.4 ms (2.8 TB/s
+// written; instructions of the expansion, 45 % of the kernel's lanes on, and LDS
+// conflicts, 56 % of its LDS cycles); 3e5: 0.58 -> 0.35 ms; 4e5 in FP64 0.83 -> 0.55 ms.
 // LDS: 24 KB a block, six blocks per CU (32 KB and five: 6.8 ms).
 constexpr uint32_t kStage = 1024;  // entries staged per wave
 constexpr uint32_t kTab = 192;     // blocks tabulated per item (more: searched in its runs)
